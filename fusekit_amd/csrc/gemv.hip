@@ -76,6 +76,26 @@ uint32_t blocks_per_cu(const void* func, uint32_t lds_bytes) {
     return (uint32_t)it->second;
 }
 
+// The tile height and grid of a flat-stream launch, by everything they depend on.
+struct GemvTiling {
+    const void* func;
+    uint32_t n[kMaxMats], cpr;
+    uint32_t rows_per_tile, grid_blocks, grid_override;
+    uint32_t rows, blocks;  // the result
+    bool same_request(const GemvTiling& o) const {
+        return func == o.func && n[0] == o.n[0] && n[1] == o.n[1] && n[2] == o.n[2] && cpr == o.cpr &&
+               rows_per_tile == o.rows_per_tile && grid_blocks == o.grid_blocks && grid_override == o.grid_override;
+    }
+};
+
+// A thread's last tilings, one per slot (a colliding shape is searched for again): no lock, no growth.
+GemvTiling& gemv_tiling_slot(const GemvTiling& k) {
+    static thread_local GemvTiling slots[128];  // func null: empty
+    uint64_t h = (uint64_t)(uintptr_t)k.func;
+    for (uint32_t v : {k.n[0], k.n[1], k.n[2], k.cpr}) h = (h ^ v) * 0x9E3779B97F4A7C15ull;
+    return slots[h >> 57];
+}
+
 uint32_t ilog2(uint32_t v) {
     uint32_t r = 0;
     while ((1u << (r + 1)) <= v) ++r;
@@ -243,42 +263,63 @@ fk_status plan_gemv(const GemvRequest& rq, Launch* out) {
     // (argument fetch, activation staging).  Measured on the 4B-class gate/up pair
     // (2 x 9728 x 2560): 19 rows per tile = 512 blocks of three 97 %-full batches runs
     // 10.4 us where one-batch tiles of 6 rows on 1280 blocks ran 12.2 us.
-    const uint32_t pos = kGemvBlock * (kGemvUnroll / nseg);
-    uint32_t r_max = 8 * pos / cpr;  // up to eight batches per tile
-    if (r_max < 1) r_max = 1;
-    if (r_max > kGemvBlock) r_max = kGemvBlock;
-    uint32_t best_r = 1, best_blocks = 1;
-    uint64_t best_cost = ~0ull, best_waste = ~0ull;
-    for (uint32_t r = 1; r <= r_max; ++r) {
-        const uint32_t lds_r = lds_for(r);
-        if ((int)lds_r > dev->max_dyn_lds) continue;
-        const uint64_t tiles = tiles_for(r);
-        uint64_t cap = t_gemv_grid_override ? t_gemv_grid_override
-                       : (g_gemv_policy.grid_blocks ? g_gemv_policy.grid_blocks : resident_for(lds_r));
-        const uint64_t blocks = tiles < cap ? tiles : cap;
-        const uint64_t per_block = (tiles + blocks - 1) / blocks;
-        const uint64_t batches = ((uint64_t)r * cpr + pos - 1) / pos;
-        // fewer than two blocks (eight waves) on a CU cannot hide the load latency:
-        // such a choice is priced as if it ran two
-        uint64_t per_cu = (blocks + dev->cus - 1) / dev->cus;
-        if (per_cu < 512 / kGemvBlock) per_cu = 512 / kGemvBlock;
-        const uint64_t cost = per_cu * per_block * batches;
-        const uint64_t waste = tiles * batches + blocks;
-        if (cost < best_cost || (cost == best_cost && waste < best_waste)) {
-            best_cost = cost;
-            best_waste = waste;
-            best_r = r;
-            best_blocks = (uint32_t)blocks;
+    // The search tries up to a few hundred tile heights, several microseconds on the host: more than a small launch
+    // takes on the GPU.  What it finds depends on the shape alone, so a direct call looks it up (4864 x 896 int4, called
+    // back to back: 6.9 us of host time per call with the search, 4.0 us without, as long as the runtime takes for an empty kernel).
+    GemvTiling key;
+    memset(&key, 0, sizeof(key));
+    key.func = func;
+    for (int m = 0; m < nm; ++m) key.n[m] = rq.mats[m]->n;
+    key.cpr = cpr;
+    key.rows_per_tile = g_gemv_policy.rows_per_tile;
+    key.grid_blocks = g_gemv_policy.grid_blocks;
+    key.grid_override = t_gemv_grid_override;
+    GemvTiling& tiling = gemv_tiling_slot(key);
+    if (!tiling.same_request(key)) {
+        const uint32_t pos = kGemvBlock * (kGemvUnroll / nseg);
+        uint32_t r_max = 8 * pos / cpr;  // up to eight batches per tile
+        if (r_max < 1) r_max = 1;
+        if (r_max > kGemvBlock) r_max = kGemvBlock;
+        uint32_t best_r = 1, best_blocks = 1;
+        uint64_t best_cost = ~0ull, best_waste = ~0ull;
+        for (uint32_t r = 1; r <= r_max; ++r) {
+            const uint32_t lds_r = lds_for(r);
+            if ((int)lds_r > dev->max_dyn_lds) continue;
+            const uint64_t tiles = tiles_for(r);
+            uint64_t cap = t_gemv_grid_override ? t_gemv_grid_override
+                           : (g_gemv_policy.grid_blocks ? g_gemv_policy.grid_blocks : resident_for(lds_r));
+            const uint64_t blocks = tiles < cap ? tiles : cap;
+            const uint64_t per_block = (tiles + blocks - 1) / blocks;
+            const uint64_t batches = ((uint64_t)r * cpr + pos - 1) / pos;
+            // fewer than two blocks (eight waves) on a CU cannot hide the load latency:
+            // such a choice is priced as if it ran two
+            uint64_t per_cu = (blocks + dev->cus - 1) / dev->cus;
+            if (per_cu < 512 / kGemvBlock) per_cu = 512 / kGemvBlock;
+            const uint64_t cost = per_cu * per_block * batches;
+            const uint64_t waste = tiles * batches + blocks;
+            if (cost < best_cost || (cost == best_cost && waste < best_waste)) {
+                best_cost = cost;
+                best_waste = waste;
+                best_r = r;
+                best_blocks = (uint32_t)blocks;
+            }
         }
+        if (best_cost == ~0ull) return set_error(FK_ERR_UNSUPPORTED, "gemv: K too large for LDS staging");
+        if (g_gemv_policy.rows_per_tile) {
+            best_r = g_gemv_policy.rows_per_tile;
+            const uint64_t tiles = tiles_for(best_r);
+            const uint64_t cap = t_gemv_grid_override ? t_gemv_grid_override
+                                 : (g_gemv_policy.grid_blocks ? g_gemv_policy.grid_blocks : resident_for(lds_for(best_r)));
+            best_blocks = (uint32_t)(tiles < cap ? tiles : cap);
+        }
+        if ((int)lds_for(best_r) > dev->max_dyn_lds) return set_error(FK_ERR_UNSUPPORTED, "gemv: K too large for LDS staging");
+        if (lds_for(best_r) > 48 * 1024)
+            FK_HIP(hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_for(best_r)));
+        tiling = key;
+        tiling.rows = best_r;
+        tiling.blocks = best_blocks;
     }
-    if (best_cost == ~0ull) return set_error(FK_ERR_UNSUPPORTED, "gemv: K too large for LDS staging");
-    if (g_gemv_policy.rows_per_tile) {
-        best_r = g_gemv_policy.rows_per_tile;
-        const uint64_t tiles = tiles_for(best_r);
-        const uint64_t cap = t_gemv_grid_override ? t_gemv_grid_override
-                             : (g_gemv_policy.grid_blocks ? g_gemv_policy.grid_blocks : resident_for(lds_for(best_r)));
-        best_blocks = (uint32_t)(tiles < cap ? tiles : cap);
-    }
+    const uint32_t best_r = tiling.rows, best_blocks = tiling.blocks;
     const uint32_t R = best_r;
     const uint64_t tiles = tiles_for(R);
     if (tiles > 0x7fffffffull) return set_error(FK_ERR_UNSUPPORTED, "gemv: too many tiles");
@@ -317,7 +358,6 @@ fk_status plan_gemv(const GemvRequest& rq, Launch* out) {
     a.y_scale = 1.0f;
 
     const uint32_t lds = lds_for(R);
-    if ((int)lds > dev->max_dyn_lds) return set_error(FK_ERR_UNSUPPORTED, "gemv: K too large for LDS staging");
     out->func = func;
     out->grid = dim3(best_blocks, 1, 1);
     out->block = dim3(kGemvBlock, 1, 1);
@@ -327,9 +367,6 @@ fk_status plan_gemv(const GemvRequest& rq, Launch* out) {
     out->add_lead(a.x);
     out->add_lead(a.norm_w);
     out->add_lead(a.K);
-    if (lds > 48 * 1024) {
-        FK_HIP(hipFuncSetAttribute(out->func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    }
     return FK_OK;
 }
 
