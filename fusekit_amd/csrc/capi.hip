@@ -61,6 +61,15 @@ fk_status run_launch(const Launch& l, hipStream_t s) {
     return FK_OK;
 }
 
+fk_status raise_dynamic_lds(const void* func, uint32_t bytes) {
+    static thread_local struct { const void* func; uint32_t bytes; } seen[64];
+    auto& slot = seen[((uintptr_t)func >> 4) & 63u];
+    if (slot.func == func && slot.bytes >= bytes) return FK_OK;
+    FK_HIP(hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    slot = {func, bytes};
+    return FK_OK;
+}
+
 }  // namespace fk
 
 using namespace fk;
@@ -195,7 +204,7 @@ fk_status fk_event_elapsed_ms(fk_event start, fk_event stop, float* ms) {
 }
 
 fk_status fk_set_qgemm_wide(int enabled) {
-    set_qgemm_wide(enabled != 0);
+    (void)enabled;   // one form serves these row counts
     return FK_OK;
 }
 
@@ -264,9 +273,19 @@ fk_status fk_rmsnorm_qkv_rows(const uint16_t* x, uint32_t rows, uint32_t x_row_s
                               fk_stream s) {
     if (!Wq) return set_error(FK_ERR_INVALID, "fk_rmsnorm_qkv_rows: null Wq");
     if (!Wk && Wv) return set_error(FK_ERR_INVALID, "fk_rmsnorm_qkv_rows: Wv without Wk");
-    WideSeg segs[3] = {{Wq, q, q_row_stride}, {Wk, k, k_row_stride}, {Wv, v, v_row_stride}};
+    if (rows < 2 || rows > 8 || Wq->group != 64 || (Wq->bits != 4 && Wq->bits != 8))
+        return set_error(FK_ERR_UNSUPPORTED, "fk_rmsnorm_qkv_rows: 2..8 rows, 4- or 8-bit weights, group size 64");
+    RowsRequest rq;
+    rq.W[0] = Wq; rq.W[1] = Wk; rq.W[2] = Wv;
+    rq.y[0] = q; rq.y[1] = k; rq.y[2] = v;
+    rq.y_stride[0] = q_row_stride; rq.y_stride[1] = k_row_stride; rq.y_stride[2] = v_row_stride;
+    rq.n_mats = Wv ? 3u : (Wk ? 2u : 1u);
+    for (uint32_t i = 0; i < rq.n_mats; ++i)
+        if (rq.y_stride[i] < rq.W[i]->n) return set_error(FK_ERR_INVALID, "fk_rmsnorm_qkv_rows: output row stride below the matrix's rows");
+    if (x_row_stride < Wq->k) return set_error(FK_ERR_INVALID, "fk_rmsnorm_qkv_rows: x_row_stride below K");
+    rq.x = x; rq.M = rows; rq.x_stride = x_row_stride; rq.norm_w = norm_w; rq.eps = eps;
     Launch l;
-    FK_TRY(plan_qgemm_wide_fan(x, x_row_stride, rows, norm_w, eps, segs, Wv ? 3u : (Wk ? 2u : 1u), &l));
+    FK_TRY(plan_qgemm_rows(rq, &l));
     return run_launch(l, (hipStream_t)s);
 }
 
@@ -279,7 +298,10 @@ fk_status fk_gateup_swiglu_rows(const uint16_t* x, uint32_t rows, const uint16_t
     if (rows < 2 || rows > 8 || Wg->group != 64 || (Wg->bits != 4 && Wg->bits != 8))
         return set_error(FK_ERR_UNSUPPORTED, "fk_gateup_swiglu_rows: 2..8 rows, 4- or 8-bit weights, group size 64");
     Launch l;
-    FK_TRY(plan_qgemm_wide(Wg, Wu, x, rows, nullptr, nullptr, variant, out, &l, norm_w, eps));
+    RowsRequest rq;
+    rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true;
+    rq.x = x; rq.M = rows; rq.norm_w = norm_w; rq.eps = eps; rq.variant = variant; rq.y[0] = out;
+    FK_TRY(plan_qgemm_rows(rq, &l));
     return run_launch(l, (hipStream_t)s);
 }
 
@@ -396,6 +418,13 @@ fk_status fk_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint
                    uint16_t* y, void* workspace, fk_stream s) {
     if (W && W->bits == 16) {  // dense bf16 weights: the plain library GEMM with this library's epilogue
         if (!x || !y || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm: null activation, output or workspace");
+        if (qgemm_takes_rows(m, 16, 0, W->k)) {
+            RowsRequest rq;
+            rq.W[0] = W; rq.x = x; rq.M = m; rq.bias[0] = bias; rq.res = residual; rq.y[0] = y;
+            Launch l;
+            FK_TRY(plan_qgemm_rows(rq, &l));
+            return run_launch(l, (hipStream_t)s);
+        }
         if (!gemm_library_available()) return set_error(FK_ERR_UNSUPPORTED, "fk_qgemm: bf16 weights need rocBLAS (librocblas.so.5 not found)");
         return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, (hipStream_t)s);
     }
@@ -429,6 +458,13 @@ fk_status fk_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint16
         if (!x || !out || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: null activation, output or workspace");
         if (Wg->n != Wu->n || Wg->k != Wu->k) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: gate and up need the same shape");
         if (variant < 0 || variant > 2) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: variant must be 0, 1 or 2");
+        if (qgemm_takes_rows(m, 16, 0, Wg->k)) {
+            RowsRequest rq;
+            rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true; rq.x = x; rq.M = m; rq.variant = variant; rq.y[0] = out;
+            Launch l;
+            FK_TRY(plan_qgemm_rows(rq, &l));
+            return run_launch(l, (hipStream_t)s);
+        }
         if (!gemm_library_available()) return set_error(FK_ERR_UNSUPPORTED, "fk_qgemm_swiglu: bf16 weights need rocBLAS (librocblas.so.5 not found)");
         return run_qgemm_library(Wg, Wu, x, m, nullptr, nullptr, variant, out, workspace, (hipStream_t)s);
     }

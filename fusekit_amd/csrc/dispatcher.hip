@@ -174,26 +174,34 @@ fk_status plan_qkv(const Dispatch& d, Launch* l, SlotRW* rw) {
     const uint32_t rows = d.u("rows", 1);
     if (rows > 1) {
         // Row form (2 .. 8 token rows, the prefill_mN variants' and the multi-row passes' shape): x [rows, x_row_stride],
-        // outputs [rows, q / k / v_row_stride] (defaults: dense rows), one shared-stream launch for the three matrices
+        // outputs [rows, q / k / v_row_stride] (defaults: dense rows), one launch for the three matrices
         // with the norm applied while the rows are staged.
         if (has_bias) return set_error(FK_ERR_UNSUPPORTED, d.kernel + ": the row form takes no bias");
         const uint32_t xs = d.u("x_row_stride", hidden);
         const uint32_t ys[3] = {d.u("q_row_stride", n_q), d.u("k_row_stride", n_kv), d.u("v_row_stride", n_kv)};
         if (xs < hidden) return set_error(FK_ERR_INVALID, d.kernel + ": x_row_stride below hidden");
         FK_TRY(need_bytes(d, 0, ((size_t)(rows - 1) * xs + hidden) * 2));
-        WideSeg segs[3];
+        RowsRequest rr;
         for (int m = 0; m < 3; ++m) {
             if (ys[m] < ns[m]) return set_error(FK_ERR_INVALID, d.kernel + ": output row stride below the matrix's rows");
             FK_TRY(need_bytes(d, out_slot + m, ((size_t)(rows - 1) * ys[m] + ns[m]) * 2));
-            segs[m] = WideSeg{&W[m], arg_ptr<uint16_t>(d, out_slot + m), ys[m]};
+            rr.W[m] = &W[m];
+            rr.y[m] = arg_ptr<uint16_t>(d, out_slot + m);
+            rr.y_stride[m] = ys[m];
         }
-        const uint16_t* nw = nullptr;
         if (has_norm) {
             FK_TRY(need_bytes(d, norm_slot, (size_t)hidden * 2));
-            nw = arg_ptr<const uint16_t>(d, norm_slot);
+            rr.norm_w = arg_ptr<const uint16_t>(d, norm_slot);
         }
         all_but_last(s, 3, rw);
-        return plan_qgemm_wide_fan(arg_ptr<const uint16_t>(d, 0), xs, rows, nw, (float)d.param("eps", 1e-6), segs, 3, l);
+        if (rows > 8 || group != 64 || bits == 16)
+            return set_error(FK_ERR_UNSUPPORTED, d.kernel + ": the row form takes 2..8 rows, 4- or 8-bit weights and group size 64");
+        rr.n_mats = 3;
+        rr.x = arg_ptr<const uint16_t>(d, 0);
+        rr.M = rows;
+        rr.x_stride = xs;
+        rr.eps = (float)d.param("eps", 1e-6);
+        return plan_qgemm_rows(rr, l);
     }
     FK_TRY(need_bytes(d, 0, (size_t)hidden * 2));
     rq.x = arg_ptr<const uint16_t>(d, 0);
@@ -230,8 +238,8 @@ fk_status plan_gateup(const Dispatch& d, Launch* l, SlotRW* rw) {
     rq.swiglu_variant = variant;
     const uint32_t rows = d.u("rows", 1);
     if (rows > 1) {
-        // Row form (2 .. 8 token rows): x [rows, hidden], out [rows, inter]; the pair streamed once for all rows by the
-        // shared-stream matmul, the norm applied while the rows are staged.
+        // Row form (2 .. 8 token rows): x [rows, hidden], out [rows, inter]; the pair streamed once for all rows,
+        // the norm applied while the rows are staged.
         if (bits == 16) return set_error(FK_ERR_UNSUPPORTED, d.kernel + ": the row form takes 4- or 8-bit weights");
         FK_TRY(need_bytes(d, 0, (size_t)rows * hidden * 2));
         FK_TRY(need_bytes(d, out_slot, (size_t)rows * inter * 2));
@@ -242,8 +250,15 @@ fk_status plan_gateup(const Dispatch& d, Launch* l, SlotRW* rw) {
         }
         all_but_last(s, 1, rw);
         if (rows > 8 || group != 64) return set_error(FK_ERR_UNSUPPORTED, d.kernel + ": the row form takes 2..8 rows and group size 64");
-        return plan_qgemm_wide(&W[0], &W[1], arg_ptr<const uint16_t>(d, 0), rows, nullptr, nullptr, variant,
-                               arg_ptr<uint16_t>(d, out_slot), l, nw, (float)d.param("eps", 1e-6));
+        RowsRequest rr;
+        rr.W[0] = &W[0]; rr.W[1] = &W[1]; rr.n_mats = 2; rr.pair = true;
+        rr.x = arg_ptr<const uint16_t>(d, 0);
+        rr.M = rows;
+        rr.norm_w = nw;
+        rr.eps = (float)d.param("eps", 1e-6);
+        rr.variant = variant;
+        rr.y[0] = arg_ptr<uint16_t>(d, out_slot);
+        return plan_qgemm_rows(rr, l);
     }
     FK_TRY(need_bytes(d, 0, (size_t)hidden * 2));
     FK_TRY(need_bytes(d, out_slot, (size_t)inter * 2));
@@ -1391,7 +1406,7 @@ fk_status plan_qgemm_d(const Dispatch& d, Launch* l, SlotRW* rw) {
 // The q / k / v projections of several token rows (fk_qgemm_fanout): x, W_q, W_k, W_v, s_q, s_k, s_v, b_q, b_k, b_v,
 // [bias_q, bias_k, bias_v], q, k, v, workspace (fk_qgemm_workspace_bytes(rows, n_q + 2 n_kv, hidden, group)).
 // Parameters: hidden (= K), n_q, n_kv, rows, bits, group, has_bias.  One launch of the fused kernel's tile form (plus the
-// fan-out's second kernel when k is split); FK_ERR_UNSUPPORTED where that form does not apply (fewer than 65 rows, an n
+// fan-out's second kernel when k is split); up to 64 rows one launch of the row form.  FK_ERR_UNSUPPORTED where neither applies (from 65 rows an n
 // that is no multiple of 4): the caller dispatches fusekit_qgemm per matrix then.
 fk_status plan_qgemm_fanout_d(const Dispatch& d, Launch* l, SlotRW* rw) {
     const uint32_t bits = d.u("bits", 4), group = d.u("group", 64), K = d.u("hidden"), rows = d.u("rows");
@@ -1405,6 +1420,8 @@ fk_status plan_qgemm_fanout_d(const Dispatch& d, Launch* l, SlotRW* rw) {
     const size_t ws_slot = s++;
     FK_TRY(need_args(d, s));
     if (bits != 4 && bits != 8) return set_error(FK_ERR_UNSUPPORTED, d.kernel + ": bits must be 4 or 8");
+    if (rows != 0 && rows <= 64)
+        return set_error(FK_ERR_UNSUPPORTED, d.kernel + ": the fan-out takes 65 rows or more; dispatch fusekit_qgemm per matrix instead");
     if (rows == 0 || K == 0 || ns[0] == 0 || ns[1] == 0) return set_error(FK_ERR_INVALID, d.kernel + ": hidden / n_q / n_kv / rows parameters missing");
     fk_weight W[3];
     const fk_weight* Wp[3];

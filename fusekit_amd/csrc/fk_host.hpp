@@ -64,6 +64,8 @@ fk_status device_facts(const DeviceFacts** out);
 fk_status set_error(fk_status code, const std::string& msg);
 fk_status hip_error(hipError_t e, const char* what);
 fk_status run_launch(const Launch& l, hipStream_t s);
+// Allows `func` that much dynamic LDS (needed above 48 KB); asked of the runtime once per kernel and size.
+fk_status raise_dynamic_lds(const void* func, uint32_t bytes);
 
 #define FK_HIP(call)                                            \
     do {                                                        \
@@ -170,21 +172,25 @@ fk_status plan_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint
 void set_gemm_library_rows(uint32_t rows);  // 0: never
 fk_status run_dequantize_bf16(const fk_weight* W, uint16_t* out, hipStream_t s);
 bool qgemm_takes_library(uint32_t m);
-// 2..10 activation rows at group size 64 run the shared-stream kernel (qgemm_wide.hip): one launch, epilogue
-// included.  plan_qgemm / plan_qgemm_swiglu then leave their other launches empty (func == nullptr), which
-// run_launch and the graph builder skip.
-bool qgemm_takes_wide(uint32_t M, uint32_t group);
-void set_qgemm_wide(bool on);
-struct WideSeg {
-    const fk_weight* W;
-    uint16_t* y;
-    uint32_t y_stride;   // elements between the rows of y
+// Up to 64 activation rows (qgemm_rows.hip): one launch, epilogue included, no workspace; bits 4 / 8 (group 64 / 128) and
+// dense bf16.  plan_qgemm / plan_qgemm_swiglu then leave their other launches empty (func == nullptr), which run_launch
+// and the graph builder skip.
+struct RowsRequest {
+    const fk_weight* W[3] = {nullptr, nullptr, nullptr};
+    uint32_t n_mats = 1;
+    bool pair = false;                 // W[0] = gate, W[1] = up: SwiGLU of the two into y[0]
+    const uint16_t* x = nullptr;
+    uint32_t M = 0, x_stride = 0;      // x_stride 0: K
+    const uint16_t* norm_w = nullptr;  // RMSNorm of the rows on the way in
+    float eps = 0.f;
+    const uint16_t* bias[3] = {nullptr, nullptr, nullptr};
+    const uint16_t* res = nullptr;
+    int variant = 0;
+    uint16_t* y[3] = {nullptr, nullptr, nullptr};
+    uint32_t y_stride[3] = {0, 0, 0};  // 0: the matrix's N
 };
-fk_status plan_qgemm_wide_fan(const uint16_t* x, uint32_t x_stride, uint32_t M, const uint16_t* norm_w, float eps,
-                              const WideSeg* segs, uint32_t n_seg, Launch* out);
-fk_status plan_qgemm_wide(const fk_weight* W0, const fk_weight* W1, const uint16_t* x, uint32_t M, const uint16_t* bias,
-                          const uint16_t* res, int variant, uint16_t* y, Launch* out, const uint16_t* norm_w = nullptr,
-                          float eps = 0.f);
+bool qgemm_takes_rows(uint32_t M, uint32_t bits, uint32_t group, uint32_t K);
+fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out);
 bool gemm_library_available();
 size_t qgemm_library_sums_bytes(uint32_t m, uint32_t n, uint32_t k);
 size_t qgemm_library_workspace_bytes(uint32_t m, uint32_t n, uint32_t k);

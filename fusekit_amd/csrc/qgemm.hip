@@ -1,7 +1,8 @@
 // Multi-row quantised matmul y[M, N] = T(x[M, K] @ dequant(W)^T) on the gfx950
-// matrix cores: the path for 2 .. a few hundred activation rows (multi-token
-// prediction, batched decode, prefill), where the weight stream is still the
-// dominant traffic and must be read once for all rows.
+// matrix cores: the path for many activation rows (prefill), where the weight
+// stream must be read once for all rows.  Up to 64 rows run qgemm_rows.hip; of the
+// first kernel below the exact forms (MT = 1, 2) are left for what that one does not
+// take, a gate / up pair of unlike bits.
 //
 // v_mfma_f32_32x32x16_bf16 with the WEIGHTS as the B operand: a lane then owns one
 // weight row n (output column) for all 16 accumulator registers, so the affine
@@ -826,9 +827,11 @@ fk_status plan_qgemm(const fk_weight* W, const uint16_t* x, uint32_t M, const ui
     FK_TRY(device_facts(&dev));
     FK_TRY(check_weight(W, "qgemm"));
     if (!x || !y || !workspace) return set_error(FK_ERR_INVALID, "qgemm: null activation, output or workspace");
-    if (qgemm_takes_wide(M, W->group)) {  // 2..10 rows: one launch, no split-k sums (reduce stays empty)
+    if (qgemm_takes_rows(M, W->bits, W->group, W->k)) {  // up to 64 rows: one launch, no split-k sums (reduce stays empty)
+        RowsRequest rq;
+        rq.W[0] = W; rq.x = x; rq.M = M; rq.bias[0] = bias; rq.res = res; rq.y[0] = y;
         *reduce = Launch();
-        return plan_qgemm_wide(W, nullptr, x, M, bias, res, 0, y, main);
+        return plan_qgemm_rows(rq, main);
     }
     QgemmShape s;
     const QgemmDirect direct{y, bias, res};
@@ -859,6 +862,20 @@ fk_status plan_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const ui
         if (!y[i]) return set_error(FK_ERR_INVALID, "qgemm fan-out: null output");
         if (W[i]->k != W[0]->k || W[i]->bits != W[0]->bits || W[i]->group != W[0]->group)
             return set_error(FK_ERR_INVALID, "qgemm fan-out: the matrices need the same K, bits and group size");
+    }
+    if (qgemm_takes_rows(M, W[0]->bits, W[0]->group, W[0]->k)) {   // up to 64 rows
+        *fused = true;
+        *reduce = Launch();
+        RowsRequest rq;
+        for (uint32_t i = 0; i < n_mats; ++i) {
+            rq.W[i] = W[i];
+            rq.bias[i] = bias ? bias[i] : nullptr;
+            rq.y[i] = y[i];
+        }
+        rq.n_mats = n_mats; rq.x = x; rq.M = M;
+        return plan_qgemm_rows(rq, main);
+    }
+    for (uint32_t i = 0; i < n_mats; ++i) {
         if (W[i]->n % 4u) return FK_OK;
         n_total += W[i]->n;
         blocks_n += (W[i]->n + kTileN - 1) / kTileN;
@@ -938,10 +955,12 @@ fk_status plan_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint
         return set_error(FK_ERR_INVALID, "qgemm_swiglu: gate and up need the same shape and group size");
     if (variant < 0 || variant > 2) return set_error(FK_ERR_INVALID, "qgemm_swiglu: variant must be 0, 1 or 2");
     if (!x || !out || !workspace) return set_error(FK_ERR_INVALID, "qgemm_swiglu: null activation, output or workspace");
-    if (qgemm_takes_wide(M, Wg->group)) {  // 2..10 rows: gate, up and SwiGLU in one launch (up, reduce stay empty)
+    if (Wg->bits == Wu->bits && qgemm_takes_rows(M, Wg->bits, Wg->group, Wg->k)) {  // gate, up and SwiGLU in one launch
+        RowsRequest rq;
+        rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true; rq.x = x; rq.M = M; rq.variant = variant; rq.y[0] = out;
         *up = Launch();
         *reduce = Launch();
-        return plan_qgemm_wide(Wg, Wu, x, M, nullptr, nullptr, variant, out, gate);
+        return plan_qgemm_rows(rq, gate);
     }
     QgemmShape s;
     float* p0 = static_cast<float*>(workspace);

@@ -259,8 +259,8 @@ void fk_set_routed_fused_reduce(int on);
  *     reference's qMM-T / NAX tile path (src/codegen/msl.rs:2318-2440, 3821-4330;
  *     admission src/codegen/kernels/mod.rs:1442-1475) and its small-M shared-stream
  *     GEMVs (fusekit_qmv_wide_impl, src/codegen/msl.rs:461-546).  Any m >= 1; bits 4
- *     or 8, group 64 or 128; bits 16 (dense bf16 rows, k a multiple of 8): the plain
- *     library GEMM (rocBLAS) with the same epilogue, direct calls only.  workspace: fk_qgemm_workspace_bytes() bytes of device
+ *     or 8, group 64 or 128; bits 16 (dense bf16 rows, k a multiple of 8; direct calls only): up to
+ *     64 rows with k a multiple of 64 the same kernel, else the plain library GEMM (rocBLAS) with the same epilogue.  workspace: fk_qgemm_workspace_bytes() bytes of device
  *     memory (fp32 split-k partial sums; from fk_set_gemm_library_rows() rows up the fp32
  *     sums and the matrix dequantised to bf16, N*K*2 bytes; group 0 = dense bf16 weights: the
  *     fp32 sums only); the SwiGLU pair needs twice that.
@@ -809,11 +809,10 @@ fk_status fk_set_gemv_flat_only(int flat_only);
  * kernel's LDS-tiled form is the faster one on the benchmark model's projections); 0 = never.
  * Set it BEFORE sizing workspaces: fk_qgemm_workspace_bytes covers the route that will be taken. */
 fk_status fk_set_gemm_library_rows(uint32_t rows);
-/* 2..10 activation rows at group size 64 run fk_qgemm / fk_qgemm_swiglu as ONE launch that streams the weights
+/* Up to 64 activation rows run fk_qgemm / fk_qgemm_swiglu / fk_qgemm_fanout as ONE launch that streams the weights
  * once for all rows and includes the epilogue (the reference's small-M kernels: src/codegen/msl.rs:462-546,
- * :1307-1485, policy src/codegen/kernels/mod.rs:164-186).  fk_set_qgemm_wide(0) sends those row counts through
- * the split-k kernel + reduction instead (measurements, tests); 1 restores the default.  Process-wide; takes
- * effect for launches planned afterwards. */
+ * :1307-1485, policy src/codegen/kernels/mod.rs:164-186).  fk_set_qgemm_wide is accepted and changes nothing: it chose
+ * between two forms of 2..10 rows, of which one is left. */
 fk_status fk_set_qgemm_wide(int enabled);
 /* An MLX-affine matrix (bits 4 / 8, group 64 / 128) as dense bf16 [n, k], every element T(code * scale + bias):
  * the values the library route of fk_qgemm multiplies with.  With 288 GB of HBM a runtime may keep the bf16 copy

@@ -28,3 +28,39 @@ def test_gemv_tiling_is_looked_up_by_shape_and_policy(fk):
 def test_attention_tiles_of_groups_of_more_than_four_heads(fk, heads, length):
     n_heads, n_kv, dim = heads
     _sdpa_case(fk, n_heads, n_kv, dim, dim, length, length + 3, seed=length)
+
+
+@pytest.mark.parametrize("bits,group", [(4, 64), (8, 64), (4, 128), (16, 64)])
+@pytest.mark.parametrize("m,n,k", [(1, 17, 64), (15, 333, 896), (17, 4112, 128), (33, 4100, 384), (48, 16, 2048), (64, 40, 4864), (49, 8200, 128)])
+def test_matmul_of_up_to_64_rows(fk, bits, group, m, n, k):
+    """Row tiles, weight-row tiles, waves without a group, both block forms; bias and residual; against the oracle."""
+    if k % group:
+        pytest.skip("K is whole groups")
+    W = make_qweight(11 + bits, n, k, bits, group=group)
+    x, bias, res = normal_bf16(12, (m, k)), normal_bf16(13, n), normal_bf16(14, (m, n))
+    y, ws = fk.DeviceBuffer(2 * m * n), fk.DeviceBuffer(fk.qgemm_workspace_bytes(m, n, k, 0 if bits == 16 else group))
+    up = fk.DeviceBuffer.from_numpy
+    fk.qgemm(to_device(fk, W), up(x), m, up(bias), up(res), y, ws)
+    got = y.to_numpy(np.uint16, (m, n))
+    for r in sorted({0, m // 2, m - 1}):
+        want = oracle.linear_acc(W, x[r]) + oracle.bf16_to_f32(bias) + oracle.bf16_to_f32(res[r])
+        assert rel_l2(got[r], want) <= 4e-3
+
+
+@pytest.mark.parametrize("bits", [4, 8, 16])
+@pytest.mark.parametrize("m", [12, 37, 64])
+def test_pair_and_fan_out_of_up_to_64_rows(fk, bits, m):
+    k, inter, ns = 896, 1000, (896, 130, 128)
+    x = normal_bf16(21, (m, k))
+    up = fk.DeviceBuffer.from_numpy
+    g, u = make_qweight(22, inter, k, bits), make_qweight(23, inter, k, bits)
+    out, ws = fk.DeviceBuffer(2 * m * inter), fk.DeviceBuffer(2 * fk.qgemm_workspace_bytes(m, 2048, k, 0 if bits == 16 else 64))
+    fk.qgemm_swiglu(to_device(fk, g), to_device(fk, u), up(x), m, 1, out, ws)
+    Ws, biases = [make_qweight(24 + i, n, k, bits) for i, n in enumerate(ns)], [normal_bf16(30 + i, n) for i, n in enumerate(ns)]
+    ys = [fk.DeviceBuffer(2 * m * n) for n in ns]
+    fk.qgemm_fanout([to_device(fk, W) for W in Ws], up(x), m, [up(b) for b in biases], ys, ws)
+    for r in (0, m - 1):
+        want = oracle.gateup_swiglu(x[r], None, 0.0, g, u, 1)
+        assert rel_l2(out.to_numpy(np.uint16, (m, inter))[r], oracle.bf16_to_f32(want)) <= 1e-2
+        for W, b, y in zip(Ws, biases, ys):
+            assert rel_l2(y.to_numpy(np.uint16, (m, W.n))[r], oracle.linear_acc(W, x[r]) + oracle.bf16_to_f32(b)) <= 4e-3
