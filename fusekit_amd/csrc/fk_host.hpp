@@ -160,13 +160,14 @@ fk_status plan_route_reduce(const uint16_t* parts, const uint16_t* route_weight,
 
 // Multi-row quantised matmul on the matrix cores (main kernel(s) + split-k reduction).
 fk_status qgemm_workspace_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t group, size_t* bytes);
+// (split_k: the split-k kernel also where the form of up to 64 rows would run; its sums are added in another order)
 fk_status plan_qgemm(const fk_weight* W, const uint16_t* x, uint32_t M, const uint16_t* bias, const uint16_t* res,
-                     uint16_t* y, void* workspace, Launch* main, Launch* reduce);
+                     uint16_t* y, void* workspace, Launch* main, Launch* reduce, bool split_k = false);
 fk_status plan_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const uint16_t* x, uint32_t M,
                             const uint16_t* const* bias, uint16_t* const* y, void* workspace, Launch* main, Launch* reduce,
                             bool* fused);
 fk_status plan_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint16_t* x, uint32_t M, int variant,
-                            uint16_t* out, void* workspace, Launch* gate, Launch* up, Launch* reduce);
+                            uint16_t* out, void* workspace, Launch* gate, Launch* up, Launch* reduce, bool split_k = false);
 
 // Large row counts, direct calls only: dequantise to bf16 once, library GEMM, the same epilogue.
 void set_gemm_library_rows(uint32_t rows);  // 0: never
@@ -183,12 +184,15 @@ struct RowsRequest {
     uint32_t M = 0, x_stride = 0;      // x_stride 0: K
     const uint16_t* norm_w = nullptr;  // RMSNorm of the rows on the way in
     float eps = 0.f;
+    const float* ssq_in = nullptr;     // with norm_w: the rows' sums of squares as the launch that wrote the rows left them
+    float* ssq_out = nullptr;          // single matrix: leave those of the outputs, rows_ssq_parts(N) floats per row
     const uint16_t* bias[3] = {nullptr, nullptr, nullptr};
     const uint16_t* res = nullptr;
     int variant = 0;
     uint16_t* y[3] = {nullptr, nullptr, nullptr};
     uint32_t y_stride[3] = {0, 0, 0};  // 0: the matrix's N
 };
+inline uint32_t rows_ssq_parts(uint32_t n) { return (n + 15u) / 16u; }
 bool qgemm_takes_rows(uint32_t M, uint32_t bits, uint32_t group, uint32_t K);
 fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out);
 bool gemm_library_available();
@@ -312,8 +316,9 @@ fk_status plan_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const ui
                             uint32_t capacity, float scale, Launch* out_launch, const uint32_t* kv_len_ptr = nullptr);
 fk_status plan_embed(const fk_weight* E, const uint32_t* token_ptr, uint32_t token_imm, float out_scale,
                      uint16_t* x, Launch* out, uint32_t rows = 1);
+// (strided: the form that adds a row's squares 256 elements apart also where the one in 16-byte pieces would run)
 fk_status plan_rmsnorm_rows(const uint16_t* x, const uint16_t* w, float eps, uint32_t rows, uint32_t hidden, uint16_t* y,
-                            Launch* out);
+                            Launch* out, bool strided = false);
 // workspace: 8 bytes (counter, zeroed once) + 8 bytes per block (<= 160 blocks)
 constexpr size_t kArgmaxWorkspaceBytes = 8 + 8 * 160;
 fk_status plan_argmax(const uint16_t* logits, uint32_t n, uint32_t* next_token, uint32_t* history,

@@ -2,7 +2,7 @@
 // matrix cores: the path for many activation rows (prefill), where the weight
 // stream must be read once for all rows.  Up to 64 rows run qgemm_rows.hip; of the
 // first kernel below the exact forms (MT = 1, 2) are left for what that one does not
-// take, a gate / up pair of unlike bits.
+// take: a gate / up pair of unlike bits, and passes into a quantised cache (prompt.hip).
 //
 // v_mfma_f32_32x32x16_bf16 with the WEIGHTS as the B operand: a lane then owns one
 // weight row n (output column) for all 16 accumulator registers, so the affine
@@ -822,12 +822,12 @@ fk_status qgemm_workspace_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t gro
 }
 
 fk_status plan_qgemm(const fk_weight* W, const uint16_t* x, uint32_t M, const uint16_t* bias, const uint16_t* res,
-                     uint16_t* y, void* workspace, Launch* main, Launch* reduce) {
+                     uint16_t* y, void* workspace, Launch* main, Launch* reduce, bool split_k) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
     FK_TRY(check_weight(W, "qgemm"));
     if (!x || !y || !workspace) return set_error(FK_ERR_INVALID, "qgemm: null activation, output or workspace");
-    if (qgemm_takes_rows(M, W->bits, W->group, W->k)) {  // up to 64 rows: one launch, no split-k sums (reduce stays empty)
+    if (!split_k && qgemm_takes_rows(M, W->bits, W->group, W->k)) {  // up to 64 rows: one launch, no split-k sums (reduce stays empty)
         RowsRequest rq;
         rq.W[0] = W; rq.x = x; rq.M = M; rq.bias[0] = bias; rq.res = res; rq.y[0] = y;
         *reduce = Launch();
@@ -946,7 +946,7 @@ fk_status plan_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const ui
 }
 
 fk_status plan_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint16_t* x, uint32_t M, int variant,
-                            uint16_t* out, void* workspace, Launch* gate, Launch* up, Launch* reduce) {
+                            uint16_t* out, void* workspace, Launch* gate, Launch* up, Launch* reduce, bool split_k) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
     FK_TRY(check_weight(Wg, "qgemm_swiglu"));
@@ -955,7 +955,7 @@ fk_status plan_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint
         return set_error(FK_ERR_INVALID, "qgemm_swiglu: gate and up need the same shape and group size");
     if (variant < 0 || variant > 2) return set_error(FK_ERR_INVALID, "qgemm_swiglu: variant must be 0, 1 or 2");
     if (!x || !out || !workspace) return set_error(FK_ERR_INVALID, "qgemm_swiglu: null activation, output or workspace");
-    if (Wg->bits == Wu->bits && qgemm_takes_rows(M, Wg->bits, Wg->group, Wg->k)) {  // gate, up and SwiGLU in one launch
+    if (!split_k && Wg->bits == Wu->bits && qgemm_takes_rows(M, Wg->bits, Wg->group, Wg->k)) {  // gate, up and SwiGLU in one launch
         RowsRequest rq;
         rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true; rq.x = x; rq.M = M; rq.variant = variant; rq.y[0] = out;
         *up = Launch();

@@ -43,6 +43,11 @@ struct QgemmRowsArgs {
     const uint16_t* x;        // M rows of K values, x_stride apart
     const uint16_t* res;      // like y[0], or null (single matrix)
     const uint16_t* norm_w;   // the rows enter as T(w * T(x * r)), r = 1 / rms of the row; null: as they are
+    // sums of squares of the rows, as the launch that wrote them left them (or null: formed here, in one more pass over
+    // the rows): ssq_in[row * ssq_n + i], i < ssq_n; and where this launch leaves those of its outputs (single matrix)
+    const float* ssq_in;
+    float* ssq_out;
+    uint32_t ssq_n;
     float eps;
     uint32_t M, K, n_seg, x_stride;
     uint32_t gshift;          // 64-code groups per scale: 0 (group 64), 1 (group 128)
@@ -93,7 +98,8 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
         if (a.n_seg > 1 && blockIdx.x >= a.blk0[1]) seg = 1;
         if (a.n_seg > 2 && blockIdx.x >= a.blk0[2]) seg = 2;
     }
-    const uint32_t blk = blockIdx.x - a.blk0[seg], N = a.n[seg], K = a.K, M = a.M, G = K >> 6, gpr = G >> a.gshift;
+    const uint32_t m0 = blockIdx.y * (MT * 16u), M = a.M - m0 < MT * 16u ? a.M - m0 : MT * 16u;   // this block's activation rows
+    const uint32_t blk = blockIdx.x - a.blk0[seg], N = a.n[seg], K = a.K, G = K >> 6, gpr = G >> a.gshift;
     const uint32_t g0 = wave * G / WAVES, g1 = (wave + 1u) * G / WAVES;
     u32x4_t* xs = reinterpret_cast<u32x4_t*>(reinterpret_cast<char*>(lds_raw) + wave * rows_wave_lds(MT, NT));   // [MT * 16][kRowsLine]
     u32x4_t* wl = xs + MT * 16 * kRowsLine;                                                                    // [NT * 16][kRowsLine]
@@ -115,7 +121,7 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
         for (int h = 0; h < 2; ++h) woff[t][h] = row(r8 + 8u * (uint32_t)h) * row_bytes;
         soff[t] = row(lane >> 2) * gpr * 2u;
     }
-    const unsigned char* xbase = reinterpret_cast<const unsigned char*>(a.x);
+    const unsigned char* xbase = reinterpret_cast<const unsigned char*>(a.x + (size_t)m0 * a.x_stride);
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -224,7 +230,35 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     float rr[MT][2];   // 1 / rms of the rows this lane parks
 #pragma unroll
     for (int i = 0; i < MT; ++i) rr[i][0] = rr[i][1] = 1.f;
-    if (normed) {
+    if (normed && a.ssq_in) {
+        float* tot = reinterpret_cast<float*>(reinterpret_cast<char*>(lds_raw) + WAVES * rows_wave_lds(MT, NT));   // [MT * 16]
+        // sixteen lanes a row, four rows a wave and step, every step's requests made before the first is used
+        constexpr int STEPS = (MT * 16 + 4 * WAVES - 1) / (4 * WAVES);
+        float v[STEPS];
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) v[i] = 0.f;
+        for (uint32_t c = lane & 15u; c < a.ssq_n / 4u; c += 16u)
+#pragma unroll
+            for (int i = 0; i < STEPS; ++i) {
+                const uint32_t m = ((uint32_t)i * WAVES + wave) * 4u + kq;
+                const float4 p = reinterpret_cast<const float4*>(a.ssq_in + (size_t)(m0 + (m < M ? m : M - 1)) * a.ssq_n)[c];
+                v[i] += (p.x + p.y) + (p.z + p.w);
+            }
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+            const uint32_t m = ((uint32_t)i * WAVES + wave) * 4u + kq;
+            const float t = group_sum(v[i], 16);
+            if (c16 == 0 && m < MT * 16u) tot[m] = 1.0f / sqrtf(t / (float)K + a.eps);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t m = (uint32_t)i * 16u + r8 + 8u * (uint32_t)h;
+                rr[i][h] = tot[m];
+            }
+    } else if (normed) {
         // the squares of the wave's own columns, the first weights on their way meanwhile; the waves add them up in LDS
         float ss[MT][2];
 #pragma unroll
@@ -320,28 +354,37 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
                 meet[wave * PER_WAVE + ((uint32_t)i * 16u + kq * 4u + (uint32_t)r) * COLS + (uint32_t)t * 16u + c16] = acc[i][t][r];
     __syncthreads();
     constexpr uint32_t OUT = 16u * CT;
-    uint16_t* yo = a.y[seg];
     const uint32_t yst = a.y_stride[seg];
+    uint16_t* yo = a.y[seg] + (size_t)m0 * yst;
+    const uint16_t* res = a.res ? a.res + (size_t)m0 * yst : nullptr;
     const uint16_t* bias = a.bias[seg];
-    for (uint32_t e = threadIdx.x; e < M * OUT; e += WAVES * kWave) {
-        const uint32_t m = e / OUT, col = e % OUT, n = blk * OUT + col;
-        if (n >= N) continue;
-        const float* at = meet + m * COLS + col;
-        float s0 = 0.f, s1 = 0.f;
+    for (uint32_t e0 = 0; e0 < M * OUT; e0 += WAVES * kWave) {
+        const uint32_t e = e0 + threadIdx.x, m = e / OUT, col = e % OUT, n = blk * OUT + col;
+        const bool live = m < M && n < N;
+        uint32_t o = 0;
+        if (live) {
+            const float* at = meet + m * COLS + col;
+            float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            s0 += at[(uint32_t)w * PER_WAVE];
-            if constexpr (PAIR) s1 += at[(uint32_t)w * PER_WAVE + OUT];
+            for (int w = 0; w < WAVES; ++w) {
+                s0 += at[(uint32_t)w * PER_WAVE];
+                if constexpr (PAIR) s1 += at[(uint32_t)w * PER_WAVE + OUT];
+            }
+            if constexpr (PAIR) {
+                o = swiglu_bits(s0, s1, a.variant, 1.0f);
+            } else {
+                if (bias) s0 += bf16_bits_to_f32(bias[n]);
+                if (res) s0 += bf16_bits_to_f32(res[(size_t)m * yst + n]);
+                o = f32_to_bf16_bits(s0);
+            }
+            yo[(size_t)m * yst + n] = (uint16_t)o;
         }
-        uint32_t o;
-        if constexpr (PAIR) {
-            o = swiglu_bits(s0, s1, a.variant, 1.0f);
-        } else {
-            if (bias) s0 += bf16_bits_to_f32(bias[n]);
-            if (a.res) s0 += bf16_bits_to_f32(a.res[(size_t)m * yst + n]);
-            o = f32_to_bf16_bits(s0);
+        if constexpr (!PAIR) {
+            if (a.ssq_out) {   // block-uniform; the 16 lanes of a tile's row are neighbours (columns past N: zero)
+                const float v = bf16_bits_to_f32(o), t = group_sum(v * v, 16);
+                if (m < M && (col & 15u) == 0) a.ssq_out[(size_t)(m0 + m) * a.ssq_n + blk * CT + (col >> 4)] = t;
+            }
         }
-        yo[(size_t)m * yst + n] = (uint16_t)o;
     }
 }
 
@@ -402,14 +445,21 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
         if (a.y_stride[i] < W->n) return set_error(FK_ERR_INVALID, "qgemm (rows): output row stride below the matrix's rows");
         b16 += (W->n + 15u) / 16u;
     }
+    if (rq.ssq_out && (rq.pair || rq.n_mats != 1)) return set_error(FK_ERR_INVALID, "qgemm (rows): sums of squares come from a single matrix");
     a.x = rq.x; a.res = rq.res; a.norm_w = rq.norm_w; a.eps = rq.eps;
+    a.ssq_in = rq.ssq_in; a.ssq_out = rq.ssq_out;
+    a.ssq_n = rq.ssq_out ? rows_ssq_parts(W0->n) : rows_ssq_parts(K);
     a.M = M; a.K = K; a.x_stride = x_stride; a.variant = rq.variant;
     a.n_seg = rq.pair ? 1u : rq.n_mats;
     a.gshift = W0->bits != 16 && W0->group == 128 ? 1u : 0u;
+    // Few blocks: the tiles of 16 activation rows go to blocks of their own (their weights come from the L2), which shortens
+    // what one block does (37 rows: 896 x 4864 12.5 -> 8.0 us, 896 x 896 5.0 -> 4.0, 2048 x 2048 7.6 -> 6.7).
+    const uint32_t cus = (uint32_t)dev->cus, tiles = (M + 15u) / 16u;
+    const uint32_t m_blocks = tiles > 1u && b16 * tiles <= cus ? tiles : (tiles > 2u && b16 * 2u <= cus ? 2u : 1u);
+    const uint32_t mt = (tiles + m_blocks - 1u) / m_blocks;
     // Eight waves per block where the blocks do not fill the chip and K is deep enough for them; else four, of which two
-    // blocks share a CU and cover each other's start (64 / 37 rows of int4, eight / four waves: 896 x 4864 12.1 / 13.3 us,
+    // blocks share a CU and cover each other's start (37 rows of int4, eight / four waves: 896 x 4864 12.1 / 13.3 us,
     // 2560 x 4096 11.1 / 12.1, 896 x 896 5.7 / 5.2, 4864 x 896 pair 14.0 / 9.7, 6144 x 2560 17.6 / 14.0).
-    const uint32_t cus = (uint32_t)dev->cus, mt = (M + 15u) / 16u;
     const uint32_t waves = b16 <= cus && K >= 2048u ? 8u : 4u;
     // Two tiles of weight rows per block -- half the blocks, each of which reads all activation rows -- once three or four
     // tiles of those make that traffic count (9728 x 2560: 37 rows 20.3 / 18.2 us with one / two, 12 rows 11.1 / 11.7; 64
@@ -422,7 +472,7 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
     }
     out->func = W0->bits == 4 ? rows_func<W_Q4>(rq.pair, two, mt, waves)
                               : (W0->bits == 8 ? rows_func<W_Q8>(rq.pair, two, mt, waves) : rows_func<W_BF16>(rq.pair, two, mt, waves));
-    out->grid = dim3(blocks, 1, 1);
+    out->grid = dim3(blocks, m_blocks, 1);
     out->block = dim3(waves * kWave, 1, 1);
     out->shmem = rows_lds_bytes(mt, rq.pair || two ? 2u : 1u, waves);
     out->set_args(a);

@@ -114,8 +114,9 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     if (same_lanes && G >= 2 && G <= 4) gt = max_len <= 2048 ? 1 : (kvq ? gt : 2);
     // Larger groups (the tile of 8 goes through LDS, three block barriers per range).  14 q / 2 kv heads x 64, time of the
     // task alone with tiles of 8 / 4 / 2 / 1 heads: 544 positions 15.8 / 11.9 / 10.7 / 9.8 us, 4096 18.4 / 14.2 / 14.2 /
-    // 13.4, 12032 30.6 / 19.1 / 17.7 / 18.6; an 8-bit cache at 8192 25.1 / 19.3 / 16.6 / 16.8.
-    if (same_lanes && G > 4) gt = max_len <= 4096 ? 1 : 2;
+    // 13.4, 12032 30.6 / 19.1 / 17.7 / 18.6.  (Not over a quantised cache: the two forms differ in the last bit, and what
+    // follows from that -- a key whose group takes the other sign of its scale -- stays in the cache.)
+    if (same_lanes && G > 4 && !kvq) gt = max_len <= 4096 ? 1 : 2;
     // Long contexts: a block walks several consecutive ranges (online softmax, the next
     // range's rows in flight), so that the grid stays near one to two blocks per CU and
     // the final merge, which costs one memory round trip per 16 partials, stays short.

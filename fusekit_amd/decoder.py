@@ -439,17 +439,19 @@ class DecoderRuntime:
         causal inside the group (fk_sdpa_prefill for the bf16 cache with head dimension 64 or 128,
         else the single-row kernel once per row).  Leaves the KV
         caches, step counter and history as token-by-token `prefill` would, and returns the greedy
-        first token.  Dense bf16 weights take the library GEMM for every row count.
+        first token.  Dense bf16 weights take the library GEMM beyond 64 rows.
         keep_bf16_weights: passes of at least 256 rows multiply with a bf16 copy of every projection that stays
         resident after its first use (2 bytes per weight: 7.3 GB for the 4B-class model) instead of
         dequantising each matrix again in every pass; the results of the dequantise + library route, bit for bit."""
-        c, w = self.cfg, self.w
+        c = self.cfg
         prompt = list(prompt)
+        if not prompt:
+            raise ValueError("empty prompt")
         if start_offset + len(prompt) > c.capacity:
             raise ValueError("prompt exceeds the KV-cache capacity")
-        # buffers follow the prompt (next power of two), so a short prompt does not allocate for 4096 rows
+        # buffers follow the longest pass so far (next power of two), so a short prompt does not allocate for 4096 rows
         R = max(1, min(rows_per_pass, 4096, 1 << max(5, (len(prompt) - 1).bit_length())))
-        if getattr(self, "_rows_R", 0) != R:
+        if getattr(self, "_rows_R", 0) < R:
             self._rows_R = R
             # the split of k differs between the kernel forms (<= 32, <= 64, more rows) and with the
             # number of 128-row tiles; the last pass of a prompt may have any row count up to R
@@ -469,78 +471,60 @@ class DecoderRuntime:
             if c.kv_bits and c.head_dim in (64, 128):  # the dequantised prefix of one layer's cache, reused by every layer
                 self._rows["kdq"] = DeviceBuffer(c.n_kv * c.capacity * c.head_dim * 2)
                 self._rows["vdq"] = DeviceBuffer(c.n_kv * c.capacity * c.head_dim * 2)
-        b = self._rows
-        emb = w.mats["embed_tokens"]
-        head = w.mats.get("lm_head", emb)
-        pos = start_offset
-        scale = 1.0 / float(np.sqrt(c.head_dim))
+            self._prompt_models = {}
+        # passes of at least 256 rows with the resident bf16 copies, the others with the quantised matrices
+        copies = bool(keep_bf16_weights and c.bits != 16 and native.gemm_library_available())
+        first = next((i for i in range(0, len(prompt), R) if copies and min(R, len(prompt) - i) < 256), len(prompt)) if copies else 0
+        nxt = 0
+        if first:
+            nxt = native.prompt_run(self._prompt_model(True), prompt[:first], start_offset, R)
+        if first < len(prompt):
+            nxt = native.prompt_run(self._prompt_model(False), prompt[first:], start_offset + first, R)
+        return nxt
 
-        def mat(name: str, m: int):
+    def _prompt_model(self, copies: bool) -> "native.PromptModel":
+        """The model as fk_prompt_run takes it, over the row buffers of the present size."""
+        if copies in self._prompt_models:
+            return self._prompt_models[copies]
+        c, w, b = self.cfg, self.w, self._rows
+
+        def mat(name: str):
             W = w.mats[name]
-            if not keep_bf16_weights or W.bits == 16 or m < 256 or not native.gemm_library_available():
-                return W
+            if not copies:
+                return W.c
             if name not in self._bf16_weights:
                 self._bf16_weights[name] = native.dequantize_bf16(W)
-            return self._bf16_weights[name]
+            return self._bf16_weights[name].c
 
-        while pos < start_offset + len(prompt):
-            chunk = prompt[pos - start_offset: pos - start_offset + R]
-            m = len(chunk)
-            b["tok"].upload(np.asarray(chunk, np.uint32))
-            native.embed_lookup_rows(emb, b["tok"], m, c.embed_scale, b["x"])
-            native.rope_table_rows(b["rope"], c.head_dim, c.theta, pos, m)  # once per pass, for every layer and head
-            for l in range(c.n_layers):
-                p = f"layers.{l}."
-                native.rmsnorm_rows(b["x"], w.vecs[p + "input_layernorm"], c.eps, m, c.hidden, b["xn"])
-                # q, k and v over the same rows: one call (one launch of the fused kernel where its tile form applies)
-                qkv = [mat(p + f"self_attn.{nm}_proj", m) for nm in "qkv"]
-                qkv_bias = [w.vecs.get(p + f"self_attn.{nm}_proj.bias") for nm in "qkv"] if c.qkv_bias else None
-                if all(W.bits != 16 for W in qkv):
-                    native.qgemm_fanout(qkv, b["xn"], m, qkv_bias, [b["q"], b["k"], b["v"]], b["ws"])
-                else:
-                    for i, dst in enumerate((b["q"], b["k"], b["v"])):
-                        native.qgemm(qkv[i], b["xn"], m, qkv_bias[i] if qkv_bias else None, None, dst, b["ws"])
-                qn = w.vecs.get(p + "self_attn.q_norm") if c.qk_norm else None
-                kn = w.vecs.get(p + "self_attn.k_norm") if c.qk_norm else None
-                if c.kv_bits:
-                    native.qkv_rope_store_rows(b["q"], None, None, qn, None, c.n_heads, 0, c.head_dim, c.head_dim,
-                                               c.theta, c.eps, m, pos, c.capacity, None, None, rope_tab=b["rope"])
-                    native.kv_cache_store_quant(b["k"], b["v"], kn, c.n_kv, c.head_dim, c.head_dim, c.theta, c.eps,
-                                                None, pos, m, self.cache_k[l], self.cache_v[l])
-                    if c.head_dim in (64, 128):
-                        # the visible prefix as bf16 (a few MB per layer), then the matrix-core attention
-                        native.kv_cache_dequant(self.cache_k[l], pos + m, b["kdq"], c.capacity)
-                        native.kv_cache_dequant(self.cache_v[l], pos + m, b["vdq"], c.capacity)
-                        native.sdpa_prefill(b["q"], b["kdq"], b["vdq"], b["att"], m, pos + m, c.n_heads, c.n_kv, c.head_dim,
-                                            c.capacity, scale)
-                    else:
-                        native.sdpa_decode_quant(b["q"], self.cache_k[l], self.cache_v[l], b["att"], None, pos + 1,
-                                                 pos + m, m, c.n_heads, scale, b["part"], b["cnt"])
-                else:
-                    native.qkv_rope_store_rows(b["q"], b["k"], b["v"], qn, kn, c.n_heads, c.n_kv, c.head_dim, c.head_dim,
-                                               c.theta, c.eps, m, pos, c.capacity, self.cache_k[l], self.cache_v[l],
-                                               rope_tab=b["rope"])
-                    if c.head_dim in (64, 128):  # causal attention of the whole group on the matrix cores
-                        native.sdpa_prefill(b["q"], self.cache_k[l], self.cache_v[l], b["att"], m, pos + m, c.n_heads,
-                                            c.n_kv, c.head_dim, c.capacity, scale)
-                    else:
-                        native.sdpa_decode_rows(b["q"], self.cache_k[l], self.cache_v[l], b["att"], m, pos + 1, c.n_heads,
-                                                c.n_kv, c.head_dim, c.head_dim, c.capacity, scale, b["part"], b["cnt"])
-                native.qgemm(mat(p + "self_attn.o_proj", m), b["att"], m, None, b["x"], b["x2"], b["ws"])
-                native.rmsnorm_rows(b["x2"], w.vecs[p + "post_attention_layernorm"], c.eps, m, c.hidden, b["xn"])
-                native.qgemm_swiglu(mat(p + "mlp.gate_proj", m), mat(p + "mlp.up_proj", m), b["xn"], m, c.swiglu_variant,
-                                    b["mid"], b["ws"])
-                native.qgemm(mat(p + "mlp.down_proj", m), b["mid"], m, None, b["x2"], b["x"], b["ws"])
-            pos += m
-        # the last row's hidden state -> logits -> greedy token, and the decode loop's uniforms
-        last = DeviceBuffer(c.hidden * 2)
-        native.copy(last, b["x"].ptr + (m - 1) * c.hidden * 2, c.hidden * 2)
-        native.final_rmsnorm_lm_head(last, w.vecs["final_norm"], c.eps, head, self.logits)
-        native.argmax_logits_decode(self.logits, c.vocab, self.token, None, None, 0, self.argmax_ws)
-        native.sync()
-        total = start_offset + len(prompt)
-        self.step_counter.upload(np.array([total], np.uint32))
-        return int(self.token.to_numpy(np.uint32)[0])
+        layers = (native.PromptLayer * c.n_layers)()
+        for l, L in enumerate(layers):
+            p = f"layers.{l}."
+            for field, name in (("q", "self_attn.q_proj"), ("k", "self_attn.k_proj"), ("v", "self_attn.v_proj"), ("o", "self_attn.o_proj"),
+                                ("gate", "mlp.gate_proj"), ("up", "mlp.up_proj"), ("down", "mlp.down_proj")):
+                setattr(L, field, mat(p + name))
+            L.input_norm, L.post_norm = w.vecs[p + "input_layernorm"].ptr, w.vecs[p + "post_attention_layernorm"].ptr
+            if c.qk_norm:
+                L.q_norm, L.k_norm = w.vecs[p + "self_attn.q_norm"].ptr, w.vecs[p + "self_attn.k_norm"].ptr
+            if c.qkv_bias:
+                L.q_bias, L.k_bias, L.v_bias = (w.vecs[p + f"self_attn.{n}_proj.bias"].ptr for n in "qkv")
+            if c.kv_bits:
+                L.cache_kq, L.cache_vq = self.cache_k[l].c, self.cache_v[l].c
+            else:
+                L.cache_k, L.cache_v = self.cache_k[l].ptr, self.cache_v[l].ptr
+        emb = w.mats["embed_tokens"]
+        m = native.PromptModel()
+        m.embed, m.head, m.final_norm, m.layers = emb.c, w.mats.get("lm_head", emb).c, w.vecs["final_norm"].ptr, layers
+        for n in ("n_layers", "hidden", "n_heads", "n_kv", "head_dim", "inter", "vocab", "capacity", "eps", "theta", "embed_scale",
+                  "swiglu_variant", "kv_bits", "kv_group"):
+            setattr(m, n, getattr(c, n))
+        for field, name in (("tokens", "tok"), ("x", "x"), ("x2", "x2"), ("xn", "xn"), ("q", "q"), ("k", "k"), ("v", "v"), ("att", "att"),
+                            ("mid", "mid"), ("workspace", "ws"), ("rope_tab", "rope"), ("partials", "part"), ("counters", "cnt"),
+                            ("k_rows", "kdq"), ("v_rows", "vdq")):
+            if name in b:
+                setattr(m, field, b[name].ptr)
+        m.logits, m.token, m.argmax_workspace, m.step_counter = self.logits.ptr, self.token.ptr, self.argmax_ws.ptr, self.step_counter.ptr
+        self._prompt_models[copies] = m
+        return m
 
     def generate(self, prompt: Sequence[int], max_tokens: int):
         """Greedy decode.  Returns (tokens, gpu_seconds of the decode chunks, decode steps timed)."""

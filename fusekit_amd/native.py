@@ -499,6 +499,32 @@ def sdpa_prefill(q, cache_k, cache_v, out, rows, kv_len, n_heads, n_kv, head_dim
                               C.c_float(scale), _ptr(stream)))
 
 
+class PromptLayer(C.Structure):
+    """fk_prompt_layer."""
+    _fields_ = ([(n, Weight) for n in ("q", "k", "v", "o", "gate", "up", "down")] +
+                [(n, C.c_void_p) for n in ("input_norm", "post_norm", "q_norm", "k_norm", "q_bias", "k_bias", "v_bias", "cache_k", "cache_v")] +
+                [("cache_kq", _KvQuantCache), ("cache_vq", _KvQuantCache)])
+
+
+class PromptModel(C.Structure):
+    """fk_prompt_model."""
+    _fields_ = ([("embed", Weight), ("head", Weight), ("final_norm", C.c_void_p), ("layers", C.POINTER(PromptLayer))] +
+                [(n, C.c_uint32) for n in ("n_layers", "hidden", "n_heads", "n_kv", "head_dim", "inter", "vocab", "capacity")] +
+                [(n, C.c_float) for n in ("eps", "theta", "embed_scale")] + [("swiglu_variant", C.c_int)] +
+                [(n, C.c_uint32) for n in ("kv_bits", "kv_group")] +
+                [(n, C.c_void_p) for n in ("tokens", "x", "x2", "xn", "q", "k", "v", "att", "mid", "workspace", "rope_tab", "partials",
+                                           "counters", "k_rows", "v_rows", "logits", "token", "argmax_workspace", "step_counter")])
+
+
+def prompt_run(model: PromptModel, tokens, start: int, rows_per_pass: int, stream=None) -> int:
+    """A prompt through the dense decoder (fk_prompt_run); returns the greedy next token."""
+    t = np.ascontiguousarray(tokens, dtype=np.uint32)
+    nxt = C.c_uint32()
+    check(lib.fk_prompt_run(C.byref(model), t.ctypes.data_as(C.c_void_p), C.c_uint32(t.size), C.c_uint32(start),
+                            C.c_uint32(rows_per_pass), C.byref(nxt), _ptr(stream)))
+    return nxt.value
+
+
 def gemm_library_available() -> bool:
     return bool(lib.fk_gemm_library_available())
 

@@ -523,6 +523,45 @@ fk_status fk_sdpa_prefill(const uint16_t *q, const uint16_t *cache_k, const uint
                           uint32_t rows, uint32_t kv_len, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
                           uint32_t capacity, float scale, fk_stream s);
 
+/* A whole prompt through a dense decoder, rows_per_pass token rows at a time (the reference's prefill variants as its
+ * runtime drives them, src/commands/patch.rs:112-150, python/fusekit_runtime/__init__.py:4782-4900): per pass embedding
+ * rows, rotary table, then per layer norm + q / k / v, RoPE + cache store, causal attention, o_proj + residual, norm +
+ * gate / up + SwiGLU, down_proj + residual -- the operator launches above, issued natively -- and behind the last pass the
+ * final norm, the LM head on the last row and the argmax.  tokens is host memory; *next_token (host) is the greedy token.
+ * step_counter (may be null) is set to start + count.  kv_bits 0: bf16 caches cache_k / cache_v; 4 / 8: cache_kq / cache_vq,
+ * with k_rows / v_rows ([n_kv, capacity, head_dim] bf16) where head_dim is 64 or 128.  Buffers hold rows_per_pass rows;
+ * workspace: twice the largest fk_qgemm_workspace_bytes of the projections for any row count up to that; partials /
+ * counters: fk_sdpa_decode_rows', for other head dims.  Returns when the token is there. */
+typedef struct fk_prompt_layer {
+    fk_weight q, k, v, o, gate, up, down;
+    const uint16_t *input_norm, *post_norm;
+    const uint16_t *q_norm, *k_norm;            /* or null */
+    const uint16_t *q_bias, *k_bias, *v_bias;   /* or null */
+    uint16_t *cache_k, *cache_v;
+    fk_kv_quant_cache cache_kq, cache_vq;
+} fk_prompt_layer;
+typedef struct fk_prompt_model {
+    fk_weight embed, head;
+    const uint16_t *final_norm;
+    const fk_prompt_layer *layers;
+    uint32_t n_layers, hidden, n_heads, n_kv, head_dim, inter, vocab, capacity;
+    float eps, theta, embed_scale;
+    int swiglu_variant;
+    uint32_t kv_bits, kv_group;
+    uint32_t *tokens;
+    uint16_t *x, *x2, *xn, *q, *k, *v, *att, *mid;
+    void *workspace;
+    float *rope_tab, *partials;
+    uint32_t *counters;
+    uint16_t *k_rows, *v_rows;
+    uint16_t *logits;
+    uint32_t *token;
+    void *argmax_workspace;
+    uint32_t *step_counter;
+} fk_prompt_model;
+fk_status fk_prompt_run(const fk_prompt_model *model, const uint32_t *tokens, uint32_t count, uint32_t start,
+                        uint32_t rows_per_pass, uint32_t *next_token, fk_stream s);
+
 /* E   x = T(embed[token] * out_scale), dense bf16 or MLX-affine table.  Replaces
  *     src/codegen/kernels/embed_lookup_decode.rs:17-108. */
 fk_status fk_embed_lookup_decode(const fk_weight *E, const uint32_t *d_token, uint32_t token, float out_scale,

@@ -64,3 +64,32 @@ def test_pair_and_fan_out_of_up_to_64_rows(fk, bits, m):
         assert rel_l2(out.to_numpy(np.uint16, (m, inter))[r], oracle.bf16_to_f32(want)) <= 1e-2
         for W, b, y in zip(Ws, biases, ys):
             assert rel_l2(y.to_numpy(np.uint16, (m, W.n))[r], oracle.linear_acc(W, x[r]) + oracle.bf16_to_f32(b)) <= 4e-3
+
+
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (3, 2048), (5, 2056), (2, 4104), (2, 12288), (2, 16392), (2, 100)])
+def test_norm_of_rows_in_16_byte_pieces(fk, rows, hidden):
+    """One, two, four and eight pieces per thread, ragged last pieces, and the widths the strided form keeps."""
+    x, w = normal_bf16(41, (rows, hidden)), normal_bf16(42, hidden, 0.1, 1.0)
+    y = fk.DeviceBuffer(2 * rows * hidden)
+    fk.rmsnorm_rows(fk.DeviceBuffer.from_numpy(x), fk.DeviceBuffer.from_numpy(w), 1e-6, rows, hidden, y)
+    got = y.to_numpy(np.uint16, (rows, hidden))
+    for r in range(rows):
+        ref = oracle.rmsnorm(x[r], w, 1e-6)
+        assert np.mean(got[r] != ref) <= 0.01 and rel_l2(got[r], oracle.bf16_to_f32(ref)) <= 1e-3
+
+
+@pytest.mark.parametrize("kv_bits,bits,n", [(0, 4, 9), (0, 8, 40), (0, 16, 64), (0, 4, 65), (8, 4, 40), (8, 16, 20)])
+def test_prompt_pass_is_the_single_token_pass(fk, kv_bits, bits, n):
+    """A prompt in one pass and token by token: the same greedy token, close logits (the norms inside the projections, the
+    forms up to 64 rows, the kept summation orders of a quantised cache)."""
+    from fusekit_amd.decoder import DecoderConfig, DecoderRuntime, DecoderWeights
+    cfg = DecoderConfig(n_layers=2, hidden=512, n_heads=14, n_kv=2, head_dim=64, inter=1024, vocab=800, capacity=128, bits=bits,
+                        kv_bits=kv_bits, qkv_bias=True)
+    W = DecoderWeights.random_init(cfg, seed=3)
+    a, b = DecoderRuntime(cfg, W), DecoderRuntime(cfg, W)
+    prompt = np.random.default_rng(n).integers(0, 800, n).tolist()
+    b.prefill(prompt)
+    for _ in range(2):
+        a.prefill_rows(prompt)
+        assert rel_l2(a.logits.to_numpy(np.uint16), oracle.bf16_to_f32(b.logits.to_numpy(np.uint16))) <= 2e-2
+        assert a.step_counter.to_numpy(np.uint32)[0] == n
