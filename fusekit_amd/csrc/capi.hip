@@ -74,6 +74,100 @@ fk_status raise_dynamic_lds(const void* func, uint32_t bytes) {
 
 using namespace fk;
 
+namespace fk {
+
+fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint16_t* bias, const uint16_t* residual, uint16_t* y,
+                    void* workspace, bool kept_order, hipStream_t s) {
+    if (W && W->bits == 16) {  // dense bf16 weights: the plain library GEMM with this library's epilogue
+        if (!x || !y || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm: null activation, output or workspace");
+        if (qgemm_takes_rows(m, 16, 0, W->k)) {
+            RowsRequest rq;
+            rq.W[0] = W; rq.x = x; rq.M = m; rq.bias[0] = bias; rq.res = residual; rq.y[0] = y;
+            Launch l;
+            FK_TRY(plan_qgemm_rows(rq, &l));
+            return run_launch(l, s);
+        }
+        if (!gemm_library_available()) return set_error(FK_ERR_UNSUPPORTED, "fk_qgemm: bf16 weights need rocBLAS (librocblas.so.5 not found)");
+        return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, s);
+    }
+    Launch main, reduce;
+    if (!kept_order && !qgemm_takes_library(m)) {
+        DmaRequest rq;
+        rq.W[0] = W; rq.x = x; rq.M = m; rq.bias[0] = bias; rq.res = residual; rq.y[0] = y; rq.workspace = workspace;
+        if (qgemm_takes_dma(rq)) {
+            FK_TRY(plan_qgemm_dma(rq, &main, &reduce));
+            FK_TRY(run_launch(main, s));
+            return run_launch(reduce, s);
+        }
+    }
+    FK_TRY(plan_qgemm(W, x, m, bias, residual, y, workspace, &main, &reduce));  // validates the arguments for both routes
+    if (qgemm_takes_library(m)) return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, s);
+    FK_TRY(run_launch(main, s));
+    return run_launch(reduce, s);
+}
+
+fk_status run_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const uint16_t* x, uint32_t m, const uint16_t* const* bias,
+                           uint16_t* const* y, void* workspace, bool kept_order, hipStream_t s) {
+    if (!W || !y || n_mats < 1 || n_mats > 3) return set_error(FK_ERR_INVALID, "fk_qgemm_fanout: one to three matrices");
+    if (n_mats > 1 && W[0] && W[0]->bits != 16 && !qgemm_takes_library(m)) {
+        Launch main, reduce;
+        DmaRequest rq;
+        rq.n_mats = n_mats; rq.x = x; rq.M = m; rq.workspace = workspace;
+        for (uint32_t i = 0; i < n_mats; ++i) {
+            rq.W[i] = W[i];
+            rq.bias[i] = bias ? bias[i] : nullptr;
+            rq.y[i] = y[i];
+        }
+        bool fused = !kept_order && qgemm_takes_dma(rq);
+        if (fused)
+            FK_TRY(plan_qgemm_dma(rq, &main, &reduce));
+        else
+            FK_TRY(plan_qgemm_fanout(W, n_mats, x, m, bias, y, workspace, &main, &reduce, &fused));
+        if (fused) {
+            FK_TRY(run_launch(main, s));
+            return run_launch(reduce, s);
+        }
+    }
+    for (uint32_t i = 0; i < n_mats; ++i)   // one by one, in stream order (they share the workspace)
+        FK_TRY(run_qgemm(W[i], x, m, bias ? bias[i] : nullptr, nullptr, y[i], workspace, kept_order, s));
+    return FK_OK;
+}
+
+fk_status run_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint16_t* x, uint32_t m, int variant, uint16_t* out,
+                           void* workspace, bool kept_order, hipStream_t s) {
+    if (Wg && Wu && Wg->bits == 16 && Wu->bits == 16) {
+        if (!x || !out || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: null activation, output or workspace");
+        if (Wg->n != Wu->n || Wg->k != Wu->k) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: gate and up need the same shape");
+        if (variant < 0 || variant > 2) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: variant must be 0, 1 or 2");
+        if (qgemm_takes_rows(m, 16, 0, Wg->k)) {
+            RowsRequest rq;
+            rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true; rq.x = x; rq.M = m; rq.variant = variant; rq.y[0] = out;
+            Launch l;
+            FK_TRY(plan_qgemm_rows(rq, &l));
+            return run_launch(l, s);
+        }
+        if (!gemm_library_available()) return set_error(FK_ERR_UNSUPPORTED, "fk_qgemm_swiglu: bf16 weights need rocBLAS (librocblas.so.5 not found)");
+        return run_qgemm_library(Wg, Wu, x, m, nullptr, nullptr, variant, out, workspace, s);
+    }
+    Launch gate, up, reduce;
+    if (!kept_order && !qgemm_takes_library(m, true) && variant >= 0 && variant <= 2) {
+        DmaRequest rq;
+        rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true; rq.x = x; rq.M = m; rq.variant = variant; rq.y[0] = out; rq.workspace = workspace;
+        if (qgemm_takes_dma(rq)) {
+            FK_TRY(plan_qgemm_dma(rq, &gate, &reduce));
+            FK_TRY(run_launch(gate, s));
+            return run_launch(reduce, s);
+        }
+    }
+    FK_TRY(plan_qgemm_swiglu(Wg, Wu, x, m, variant, out, workspace, &gate, &up, &reduce));
+    if (qgemm_takes_library(m)) return run_qgemm_library(Wg, Wu, x, m, nullptr, nullptr, variant, out, workspace, s);
+    FK_TRY(run_launch(gate, s));
+    FK_TRY(run_launch(up, s));
+    return run_launch(reduce, s);
+}
+
+}  // namespace fk
+
 extern "C" {
 
 const char* fk_last_error(void) { return t_last_error.c_str(); }
@@ -416,64 +510,17 @@ fk_status fk_qgemm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t 
 
 fk_status fk_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint16_t* bias, const uint16_t* residual,
                    uint16_t* y, void* workspace, fk_stream s) {
-    if (W && W->bits == 16) {  // dense bf16 weights: the plain library GEMM with this library's epilogue
-        if (!x || !y || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm: null activation, output or workspace");
-        if (qgemm_takes_rows(m, 16, 0, W->k)) {
-            RowsRequest rq;
-            rq.W[0] = W; rq.x = x; rq.M = m; rq.bias[0] = bias; rq.res = residual; rq.y[0] = y;
-            Launch l;
-            FK_TRY(plan_qgemm_rows(rq, &l));
-            return run_launch(l, (hipStream_t)s);
-        }
-        if (!gemm_library_available()) return set_error(FK_ERR_UNSUPPORTED, "fk_qgemm: bf16 weights need rocBLAS (librocblas.so.5 not found)");
-        return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, (hipStream_t)s);
-    }
-    Launch main, reduce;
-    FK_TRY(plan_qgemm(W, x, m, bias, residual, y, workspace, &main, &reduce));  // validates the arguments for both routes
-    if (qgemm_takes_library(m)) return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, (hipStream_t)s);
-    FK_TRY(run_launch(main, (hipStream_t)s));
-    return run_launch(reduce, (hipStream_t)s);
+    return run_qgemm(W, x, m, bias, residual, y, workspace, false, (hipStream_t)s);
 }
 
 fk_status fk_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const uint16_t* x, uint32_t m,
                           const uint16_t* const* bias, uint16_t* const* y, void* workspace, fk_stream s) {
-    if (!W || !y || n_mats < 1 || n_mats > 3) return set_error(FK_ERR_INVALID, "fk_qgemm_fanout: one to three matrices");
-    bool fused = false;
-    if (n_mats > 1 && W[0] && W[0]->bits != 16 && !qgemm_takes_library(m)) {
-        Launch main, reduce;
-        FK_TRY(plan_qgemm_fanout(W, n_mats, x, m, bias, y, workspace, &main, &reduce, &fused));
-        if (fused) {
-            FK_TRY(run_launch(main, (hipStream_t)s));
-            return run_launch(reduce, (hipStream_t)s);
-        }
-    }
-    for (uint32_t i = 0; i < n_mats; ++i)   // one by one, in stream order (they share the workspace)
-        FK_TRY(fk_qgemm(W[i], x, m, bias ? bias[i] : nullptr, nullptr, y[i], workspace, s));
-    return FK_OK;
+    return run_qgemm_fanout(W, n_mats, x, m, bias, y, workspace, false, (hipStream_t)s);
 }
 
 fk_status fk_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint16_t* x, uint32_t m, int variant,
                           uint16_t* out, void* workspace, fk_stream s) {
-    if (Wg && Wu && Wg->bits == 16 && Wu->bits == 16) {
-        if (!x || !out || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: null activation, output or workspace");
-        if (Wg->n != Wu->n || Wg->k != Wu->k) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: gate and up need the same shape");
-        if (variant < 0 || variant > 2) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: variant must be 0, 1 or 2");
-        if (qgemm_takes_rows(m, 16, 0, Wg->k)) {
-            RowsRequest rq;
-            rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true; rq.x = x; rq.M = m; rq.variant = variant; rq.y[0] = out;
-            Launch l;
-            FK_TRY(plan_qgemm_rows(rq, &l));
-            return run_launch(l, (hipStream_t)s);
-        }
-        if (!gemm_library_available()) return set_error(FK_ERR_UNSUPPORTED, "fk_qgemm_swiglu: bf16 weights need rocBLAS (librocblas.so.5 not found)");
-        return run_qgemm_library(Wg, Wu, x, m, nullptr, nullptr, variant, out, workspace, (hipStream_t)s);
-    }
-    Launch gate, up, reduce;
-    FK_TRY(plan_qgemm_swiglu(Wg, Wu, x, m, variant, out, workspace, &gate, &up, &reduce));
-    if (qgemm_takes_library(m)) return run_qgemm_library(Wg, Wu, x, m, nullptr, nullptr, variant, out, workspace, (hipStream_t)s);
-    FK_TRY(run_launch(gate, (hipStream_t)s));
-    FK_TRY(run_launch(up, (hipStream_t)s));
-    return run_launch(reduce, (hipStream_t)s);
+    return run_qgemm_swiglu(Wg, Wu, x, m, variant, out, workspace, false, (hipStream_t)s);
 }
 
 fk_status fk_final_rmsnorm_lm_head(const uint16_t* x, const uint16_t* norm_w, float eps, const fk_weight* W,

@@ -172,7 +172,15 @@ fk_status plan_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint
 // Large row counts, direct calls only: dequantise to bf16 once, library GEMM, the same epilogue.
 void set_gemm_library_rows(uint32_t rows);  // 0: never
 fk_status run_dequantize_bf16(const fk_weight* W, uint16_t* out, hipStream_t s);
-bool qgemm_takes_library(uint32_t m);
+bool qgemm_takes_library(uint32_t m, bool pair = false);
+// What fk_qgemm, fk_qgemm_fanout and fk_qgemm_swiglu run.  kept_order: the launches whose sums are added in the order that
+// quantised caches have been filled with (see prompt.hip).
+fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint16_t* bias, const uint16_t* residual, uint16_t* y,
+                    void* workspace, bool kept_order, hipStream_t s);
+fk_status run_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const uint16_t* x, uint32_t m, const uint16_t* const* bias,
+                           uint16_t* const* y, void* workspace, bool kept_order, hipStream_t s);
+fk_status run_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint16_t* x, uint32_t m, int variant, uint16_t* out,
+                           void* workspace, bool kept_order, hipStream_t s);
 // Up to 64 activation rows (qgemm_rows.hip): one launch, epilogue included, no workspace; bits 4 / 8 (group 64 / 128) and
 // dense bf16.  plan_qgemm / plan_qgemm_swiglu then leave their other launches empty (func == nullptr), which run_launch
 // and the graph builder skip.
@@ -195,6 +203,24 @@ struct RowsRequest {
 inline uint32_t rows_ssq_parts(uint32_t n) { return (n + 15u) / 16u; }
 bool qgemm_takes_rows(uint32_t M, uint32_t bits, uint32_t group, uint32_t K);
 fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out);
+// From 65 activation rows, 4- or 8-bit weights of group 64 (qgemm_dma.hip): one to three matrices over the same rows, or a
+// gate / up pair; `reduce` stays empty where k is not split.
+struct DmaRequest {
+    const fk_weight* W[3] = {nullptr, nullptr, nullptr};
+    uint32_t n_mats = 1;
+    bool pair = false;                 // W[0] = gate, W[1] = up: SwiGLU of the two into y[0]
+    const uint16_t* x = nullptr;
+    uint32_t M = 0;
+    const uint16_t* bias[3] = {nullptr, nullptr, nullptr};
+    const uint16_t* res = nullptr;
+    int variant = 0;
+    uint16_t* y[3] = {nullptr, nullptr, nullptr};
+    void* workspace = nullptr;
+};
+bool qgemm_takes_dma(const DmaRequest& rq);
+uint32_t qgemm_dma_split(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, bool pair);
+fk_status plan_qgemm_dma(const DmaRequest& rq, Launch* main, Launch* reduce);
+void plan_qgemm_dma_reduce(const DmaRequest& rq, uint32_t n_total, uint32_t ksplit, Launch* out);
 bool gemm_library_available();
 size_t qgemm_library_sums_bytes(uint32_t m, uint32_t n, uint32_t k);
 size_t qgemm_library_workspace_bytes(uint32_t m, uint32_t n, uint32_t k);

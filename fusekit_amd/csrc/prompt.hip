@@ -30,7 +30,7 @@ fk_status run_rows(const RowsRequest& rq, hipStream_t s) {
 // Passes into a QUANTISED cache keep the summation orders such caches have been filled with: a key that differs in its last
 // bit can turn the sign of its group's scale (MLX's rule takes it from the end of the range that is larger in magnitude) and
 // shift the group's codes, and a cache is kept and compared for longer than a pass.  So, up to 64 rows: split-k sums, the
-// library GEMM for dense bf16 weights; and the strided norm.
+// library GEMM for dense bf16 weights; beyond, the tiles of qgemm.hip and the library (`kept` of run_qgemm); and the strided norm.
 fk_status norm_rows(const fk_prompt_model& m, const uint16_t* x, const uint16_t* w, uint32_t rows, hipStream_t s) {
     Launch l;
     FK_TRY(plan_rmsnorm_rows(x, w, m.eps, rows, m.hidden, m.xn, &l, m.kv_bits != 0));
@@ -41,7 +41,7 @@ bool kept_order(const fk_prompt_model& m, const fk_weight& W, uint32_t rows) {
 }
 fk_status matmul(const fk_prompt_model& m, const fk_weight& W, const uint16_t* x, uint32_t rows, const uint16_t* bias, const uint16_t* res,
                  uint16_t* y, hipStream_t s) {
-    if (!kept_order(m, W, rows)) return fk_qgemm(&W, x, rows, bias, res, y, m.workspace, s);
+    if (!kept_order(m, W, rows)) return run_qgemm(&W, x, rows, bias, res, y, m.workspace, m.kv_bits != 0, s);
     if (W.bits == 16) return run_qgemm_library(&W, nullptr, x, rows, bias, res, 0, y, m.workspace, s);
     Launch main, reduce;
     FK_TRY(plan_qgemm(&W, x, rows, bias, res, y, m.workspace, &main, &reduce, true));
@@ -82,7 +82,7 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* s
         if (kept_order(m, l.q, rows))
             for (int i = 0; i < 3; ++i) FK_TRY(matmul(m, *W[i], m.xn, rows, bias[i], nullptr, y[i], (hipStream_t)s));
         else
-            FK_TRY(fk_qgemm_fanout(W, 3, m.xn, rows, l.q_bias ? bias : nullptr, y, m.workspace, s));
+            FK_TRY(run_qgemm_fanout(W, 3, m.xn, rows, l.q_bias ? bias : nullptr, y, m.workspace, m.kv_bits != 0, (hipStream_t)s));
     }
     if (m.kv_bits) {
         FK_TRY(fk_qkv_rope_store_rows(m.q, nullptr, nullptr, l.q_norm, nullptr, m.n_heads, 0, dim, dim, m.theta, m.eps, rows, pos,
@@ -125,7 +125,7 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* s
             FK_TRY(run_launch(up, (hipStream_t)s));
             FK_TRY(run_launch(reduce, (hipStream_t)s));
         } else {
-            FK_TRY(fk_qgemm_swiglu(&l.gate, &l.up, m.xn, rows, m.swiglu_variant, m.mid, m.workspace, s));
+            FK_TRY(run_qgemm_swiglu(&l.gate, &l.up, m.xn, rows, m.swiglu_variant, m.mid, m.workspace, m.kv_bits != 0, (hipStream_t)s));
         }
     }
     return residual_rows(m, l.down, m.mid, rows, m.x2, m.x, ssq, (hipStream_t)s);

@@ -801,6 +801,34 @@ void plan_qgemm_epilogue(const float* p0, const float* p1, const uint16_t* bias,
     plan_reduce(p0, p1, bias, res, y, M, N, ksplit, variant, out);
 }
 
+// the second kernel of qgemm_dma.hip's split-k sums
+void plan_qgemm_dma_reduce(const DmaRequest& rq, uint32_t n_total, uint32_t ksplit, Launch* out) {
+    const float* p = static_cast<const float*>(rq.workspace);
+    if (rq.pair) return plan_reduce(p, p + (size_t)ksplit * rq.M * n_total, nullptr, nullptr, rq.y[0], rq.M, n_total, ksplit, rq.variant, out);
+    if (rq.n_mats == 1) return plan_reduce(p, nullptr, rq.bias[0], rq.res, rq.y[0], rq.M, n_total, ksplit, 0, out);
+    QgemmFanReduceArgs r;
+    memset(&r, 0, sizeof(r));
+    r.p = p;
+    r.M = rq.M;
+    r.n_total = n_total;
+    r.ksplit = ksplit;
+    r.n_seg = rq.n_mats;
+    uint32_t col = 0;
+    for (uint32_t i = 0; i < 3; ++i) {
+        const uint32_t j = i < rq.n_mats ? i : rq.n_mats - 1u;
+        r.y[i] = rq.y[j];
+        r.bias[i] = rq.bias[j];
+        r.col0[i] = i < rq.n_mats ? col : 0xffffffffu;
+        r.N[i] = rq.W[j]->n;
+        if (i < rq.n_mats) col += rq.W[i]->n;
+    }
+    out->func = reinterpret_cast<const void*>(&qgemm_fan_reduce_kernel);
+    out->grid = dim3((rq.M * n_total / 4u + 255u) / 256u, 1, 1);
+    out->block = dim3(256, 1, 1);
+    out->shmem = 0;
+    out->set_args(r);
+}
+
 fk_status qgemm_workspace_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t group, size_t* bytes) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
@@ -814,6 +842,11 @@ fk_status qgemm_workspace_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t gro
     FK_TRY(qgemm_shape(dev, M, N, K, group, 4, &s4));
     FK_TRY(qgemm_shape(dev, M, N, K, group, 8, &s8));
     *bytes = (size_t)(s4.ksplit > s8.ksplit ? s4.ksplit : s8.ksplit) * M * N * sizeof(float);
+    for (uint32_t bits : {4u, 8u})
+        for (bool pair : {false, true}) {
+            const size_t dma = (size_t)qgemm_dma_split(bits, M, N, K, pair) * M * N * sizeof(float);   // (per matrix of a pair)
+            if (dma > *bytes) *bytes = dma;
+        }
     // direct calls with many rows may take the library route, which also parks the dequantised matrix
     // here; dense bf16 weights always take it and need the fp32 sums only
     const size_t lib = qgemm_takes_library(M) ? qgemm_library_workspace_bytes(M, N, K) : qgemm_library_sums_bytes(M, N, K);

@@ -93,3 +93,23 @@ def test_prompt_pass_is_the_single_token_pass(fk, kv_bits, bits, n):
         a.prefill_rows(prompt)
         assert rel_l2(a.logits.to_numpy(np.uint16), oracle.bf16_to_f32(b.logits.to_numpy(np.uint16))) <= 2e-2
         assert a.step_counter.to_numpy(np.uint32)[0] == n
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(65, 4, 768), (128, 132, 896), (129, 1000, 1024), (300, 2052, 2048), (257, 8200, 896), (640, 96, 4864)])
+def test_matmul_from_65_rows(fk, bits, m, n, k):
+    """Tiles of 128 and 256 activation rows, one to eight k splits, ragged rows and weight rows: one matrix with bias and
+    residual, a gate / up pair, a fan-out of three."""
+    x, bias, res = normal_bf16(41, (m, k)), normal_bf16(42, n), normal_bf16(43, (m, n))
+    Ws = [make_qweight(44 + i, n, k, bits) for i in range(3)]
+    dW, up = [to_device(fk, W) for W in Ws], fk.DeviceBuffer.from_numpy
+    dx, ws = up(x), fk.DeviceBuffer(2 * fk.qgemm_workspace_bytes(m, 3 * n, k))
+    ys = [fk.DeviceBuffer(2 * m * n) for _ in range(5)]
+    fk.qgemm(dW[0], dx, m, up(bias), up(res), ys[0], ws)
+    fk.qgemm_swiglu(dW[0], dW[1], dx, m, 1, ys[1], ws)
+    fk.qgemm_fanout(dW, dx, m, [None, up(bias), None], ys[2:], ws)
+    acc = [oracle.qgemm_bf16w(W, x, None, want_acc=True)[1].astype(np.float64) for W in Ws]
+    b, r = oracle.bf16_to_f32(bias).astype(np.float64), oracle.bf16_to_f32(res).astype(np.float64)
+    g, u = (oracle.bf16_to_f32(oracle.f32_to_bf16(a.astype(np.float32))).astype(np.float64) for a in acc[:2])
+    for y, want in zip(ys, (acc[0] + b + r, g / (1 + np.exp(-g)) * u, acc[0], acc[1] + b, acc[2])):
+        assert rel_l2(y.to_numpy(np.uint16, (m, n)), want) <= 4e-3
