@@ -656,9 +656,10 @@ fk_status plan_rmsnorm_rows_d(const Dispatch& d, Launch* l, SlotRW* rw) {
 
 // Q, K, V, [q_weight, k_weight], cache_k, cache_v, kv_len, out, partials, counters, [rope_tab]
 // (one launch for the rope/store stage and the attention of a layer)
-fk_status plan_rope_store_sdpa(const Dispatch& d, Launch* l, SlotRW* rw) {
+// kv_bits (families .._q4, .._q8): a quantised cache, its K then V slots as packed, scales, biases; parameter group
+fk_status plan_rope_store_sdpa(const Dispatch& d, Launch* l, SlotRW* rw, uint32_t kv_bits) {
     const bool norm = d.u("has_norm", 0) != 0, table = d.u("has_table", 0) != 0;
-    const size_t c0 = norm ? 5 : 3, n = c0 + 6 + (table ? 1 : 0);
+    const size_t k0 = norm ? 5 : 3, per = kv_bits ? 3 : 1, c0 = k0 + 2 * per - 2, n = c0 + 6 + (table ? 1 : 0);   // c0 + 2: kv_len
     FK_TRY(need_args(d, n));
     const uint32_t n_heads = d.u("n_heads"), n_kv = d.u("n_kv"), dim = d.u("head_dim");
     const uint32_t capacity = d.u("capacity"), max_len = d.u("max_len", capacity);
@@ -680,8 +681,22 @@ fk_status plan_rope_store_sdpa(const Dispatch& d, Launch* l, SlotRW* rw) {
         f.q_norm = arg_ptr<const uint16_t>(d, 3);
         f.k_norm = arg_ptr<const uint16_t>(d, 4);
     }
-    FK_TRY(need_bytes(d, c0, (size_t)n_kv * capacity * dim * 2));
-    FK_TRY(need_bytes(d, c0 + 1, (size_t)n_kv * capacity * dim * 2));
+    KvQuant qz;
+    qz.bits = kv_bits;
+    qz.group = d.u("group", 64);
+    if (kv_bits && (qz.group == 0 || dim % qz.group)) return set_error(FK_ERR_INVALID, d.kernel + ": group parameter inconsistent with head_dim");
+    for (size_t c = 0; c < 2; ++c) {
+        FK_TRY(need_bytes(d, k0 + c * per, (size_t)n_kv * capacity * dim * (kv_bits ? kv_bits : 16u) / 8u));
+        if (!kv_bits) continue;
+        FK_TRY(need_bytes(d, k0 + c * per + 1, (size_t)n_kv * capacity * (dim / qz.group) * 2));
+        FK_TRY(need_bytes(d, k0 + c * per + 2, (size_t)n_kv * capacity * (dim / qz.group) * 2));
+    }
+    if (kv_bits) {
+        qz.k_scales = arg_ptr<const uint16_t>(d, k0 + 1);
+        qz.k_biases = arg_ptr<const uint16_t>(d, k0 + 2);
+        qz.v_scales = arg_ptr<const uint16_t>(d, k0 + 4);
+        qz.v_biases = arg_ptr<const uint16_t>(d, k0 + 5);
+    }
     FK_TRY(need_bytes(d, c0 + 2, 4));
     FK_TRY(need_bytes(d, c0 + 3, (size_t)n_heads * dim * 2));
     size_t pb = 0, cb = 0;
@@ -694,11 +709,12 @@ fk_status plan_rope_store_sdpa(const Dispatch& d, Launch* l, SlotRW* rw) {
     }
     for (uint32_t i = 0; i < n; ++i)
         if (i != c0 + 3) rw->reads.push_back(i);
-    rw->writes = {(uint32_t)c0, (uint32_t)c0 + 1, (uint32_t)c0 + 3, (uint32_t)c0 + 4, (uint32_t)c0 + 5};
-    return plan_sdpa_decode(arg_ptr<const uint16_t>(d, 0), arg_ptr<const uint16_t>(d, c0),
-                            arg_ptr<const uint16_t>(d, c0 + 1), arg_ptr<uint16_t>(d, c0 + 3),
+    for (uint32_t i = (uint32_t)k0; i < c0 + 2; ++i) rw->writes.push_back(i);
+    for (uint32_t i : {3u, 4u, 5u}) rw->writes.push_back((uint32_t)c0 + i);
+    return plan_sdpa_decode(arg_ptr<const uint16_t>(d, 0), arg_ptr<const uint16_t>(d, k0),
+                            arg_ptr<const uint16_t>(d, k0 + per), arg_ptr<uint16_t>(d, c0 + 3),
                             arg_ptr<const uint32_t>(d, c0 + 2), 0, max_len, n_heads, n_kv, dim, dim, capacity, scale,
-                            arg_ptr<float>(d, c0 + 4), arg_ptr<uint32_t>(d, c0 + 5), l, 1, nullptr, &f);
+                            arg_ptr<float>(d, c0 + 4), arg_ptr<uint32_t>(d, c0 + 5), l, 1, kv_bits ? &qz : nullptr, &f);
 }
 
 // ---- XCD-resident layer (xcd_layer.hpp): two launches per layer -------------------------------------
@@ -1545,7 +1561,9 @@ const Family kFamilies[] = {
     {"fusekit_sdpa_decode", plan_sdpa_d},
     {"fusekit_sdpa_prefill", plan_sdpa_prefill_d},
     {"fusekit_rmsnorm_rows", plan_rmsnorm_rows_d},
-    {"fusekit_rope_store_sdpa_decode", plan_rope_store_sdpa},
+    {"fusekit_rope_store_sdpa_decode", [](const Dispatch& d, Launch* l, SlotRW* rw) { return plan_rope_store_sdpa(d, l, rw, 0); }},
+    {"fusekit_rope_store_sdpa_decode_q4", [](const Dispatch& d, Launch* l, SlotRW* rw) { return plan_rope_store_sdpa(d, l, rw, 4); }},
+    {"fusekit_rope_store_sdpa_decode_q8", [](const Dispatch& d, Launch* l, SlotRW* rw) { return plan_rope_store_sdpa(d, l, rw, 8); }},
     {"fusekit_split_store_sdpa_decode", plan_split_store_sdpa},
     {"fusekit_rope_kv_cache_store_decode_q4",
      [](const Dispatch& d, Launch* l, SlotRW* rw) { return plan_rope_kv_quant(d, l, rw, 4); }},

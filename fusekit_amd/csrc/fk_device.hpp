@@ -120,6 +120,14 @@ __device__ __forceinline__ void pin_u128(uint4& v) {
 // and an agent-scope fence adds a write-back of the whole L2.
 __device__ __forceinline__ void wait_memory_ops_done() { __builtin_amdgcn_s_waitcnt(0x0070); }
 
+// LDS traffic of ONE wave with itself: the hardware runs a wave's LDS instructions in order, the fence keeps the compiler from
+// reordering them.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Reads one word of every 64-byte line of the kernel's argument block (BYTES from its start) and makes the wave wait
 // for them once.  A long kernel otherwise fetches its arguments where it first uses them, phase by phase, and each
 // first touch of a line is a scalar-cache miss -- a trip to the L2 -- in the middle of that phase; after this the

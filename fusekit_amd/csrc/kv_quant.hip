@@ -5,8 +5,7 @@
 // src/codegen/kernels/rope_kv_cache_store_decode_quant.rs:100-260: as there, the rotated K value
 // is NOT rounded to bf16 before it is quantised.  One wave per (K or V head, token row).
 #include "fk_host.hpp"
-#include "fk_device.hpp"
-#include "rope_device.hpp"
+#include "kv_quant_device.hpp"
 
 namespace fk {
 
@@ -22,78 +21,21 @@ __global__ __launch_bounds__(kWave) void kv_store_quant_kernel(const KvQuantStor
     const uint32_t crow = (a.write_offset_ptr ? *a.write_offset_ptr + tr : pos) % a.capacity;
     const uint16_t* src = (is_v ? a.v : a.k) + ((size_t)tr * a.n_kv + h) * a.dim;
 
-    if (is_v) {
+    if (is_v)
         for (uint32_t d = lane; d < a.dim; d += kWave) row[d] = bf16_bits_to_f32(src[d]);
-    } else {
-        float r = 1.f;
-        if (a.k_norm) {
-            float ss = 0.f;
-            for (uint32_t d = lane; d < a.dim; d += kWave) {
-                const float x = bf16_bits_to_f32(src[d]);
-                ss = fmaf(x, x, ss);
-            }
-            ss = wave_sum(ss);
-            r = 1.0f / sqrtf(ss / (float)a.dim + a.eps);
-        }
-        auto value = [&](uint32_t d) {
-            const float x = bf16_bits_to_f32(src[d]);
-            return a.k_norm ? round_bf16(bf16_bits_to_f32(a.k_norm[d]) * round_bf16(x * r)) : x;
-        };
-        const uint32_t half = a.rope_dims / 2;
-        for (uint32_t d = lane; d < half; d += kWave) {
-            float lo, hi;
-            rope_rotate(value(d), value(d + half), d, half, pos, a.base_log2, lo, hi);
-            row[d] = lo;
-            row[d + half] = hi;
-        }
-        for (uint32_t d = 2 * half + lane; d < a.dim; d += kWave) row[d] = value(d);
-    }
+    else
+        kv_key_row(src, a.k_norm, row, a.dim, a.rope_dims, pos, a.base_log2, a.eps, lane, nullptr);
     __syncthreads();
-
-    // Per group: min / max over the wave, then the quantiser's arithmetic statement for statement
-    // (see quantize_affine_kernel); every lane derives the same scale and bias.
-    const uint32_t groups = a.dim / a.group, per_word = 32u / a.bits;
-    const int mask = (1 << a.bits) - 1;
-    uint32_t* packed = (is_v ? a.cv_packed : a.ck_packed) + ((size_t)h * a.capacity + crow) * (a.dim / per_word);
+    const uint32_t groups = a.dim / a.group, wpr = a.dim * a.bits / 32u;
+    uint32_t* packed = (is_v ? a.cv_packed : a.ck_packed) + ((size_t)h * a.capacity + crow) * wpr;
     uint16_t* scales = (is_v ? a.cv_scales : a.ck_scales) + ((size_t)h * a.capacity + crow) * groups;
     uint16_t* biases = (is_v ? a.cv_biases : a.ck_biases) + ((size_t)h * a.capacity + crow) * groups;
-    for (uint32_t g = 0; g < groups; ++g) {
-        const float* x = row + g * a.group;
-        float vmin = INFINITY, vmax = -INFINITY;
-        for (uint32_t i = lane; i < a.group; i += kWave) {
-            vmin = fminf(vmin, x[i]);
-            vmax = fmaxf(vmax, x[i]);
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            vmin = fminf(vmin, __shfl_xor(vmin, o, kWave));
-            vmax = fmaxf(vmax, __shfl_xor(vmax, o, kWave));
-        }
-        const float scale_abs = fmaxf((vmax - vmin) / (float)mask, 1.0e-7f);
-        const bool lo_anchor = fabsf(vmin) > fabsf(vmax);
-        float scale = lo_anchor ? scale_abs : -scale_abs;
-        const float edge = lo_anchor ? vmin : vmax;
-        const float q0 = roundf(edge / scale);
-        const bool at_zero = (q0 == 0.0f);
-        scale = at_zero ? scale : (edge / q0);
-        const float bias = at_zero ? 0.0f : edge;
-        const float inv_scale = (scale != 0.0f) ? (1.0f / scale) : 0.0f;
-        for (uint32_t i = lane; i < a.group; i += kWave) {
-            int qi = (int)roundf((x[i] - bias) * inv_scale);
-            qi = qi < 0 ? 0 : (qi > mask ? mask : qi);
-            codes[g * a.group + i] = (uint8_t)qi;
-        }
-        if (lane == 0) {
-            scales[g] = (uint16_t)f32_to_bf16_bits(scale);
-            biases[g] = (uint16_t)f32_to_bf16_bits(bias);
-        }
-    }
+    kv_quantize_row(row, codes, a.dim, a.group, a.bits, lane, [&](uint32_t g, uint32_t sc, uint32_t bi) {
+        scales[g] = (uint16_t)sc;
+        biases[g] = (uint16_t)bi;
+    });
     __syncthreads();
-    for (uint32_t wi = lane; wi < a.dim / per_word; wi += kWave) {
-        uint32_t word = 0;
-        for (uint32_t el = 0; el < per_word; ++el) word |= (uint32_t)codes[wi * per_word + el] << (el * a.bits);
-        packed[wi] = word;
-    }
+    kv_pack_row(codes, a.dim, a.bits, lane, [&](uint32_t wi, uint32_t word) { packed[wi] = word; });
 }
 
 fk_status plan_kv_store_quant(const KvQuantStore& in, Launch* out) {

@@ -77,7 +77,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
             return set_error(FK_ERR_UNSUPPORTED, "sdpa: cache group size must be 32, 64 or 128 and divide the head dims");
     }
     if (fusion) {
-        if (kvq || rows != 1) return set_error(FK_ERR_UNSUPPORTED, "sdpa: the fused rope/store form takes one row and a bf16 cache");
+        if (rows != 1 || (kvq && fusion->q0_dim)) return set_error(FK_ERR_UNSUPPORTED, "sdpa: the fused rope/store form takes one row, split heads a bf16 cache");
         if (!fusion->k_new || !fusion->v_new) return set_error(FK_ERR_INVALID, "sdpa: null new k / v row");
         if (fusion->rope_dims % 2 || fusion->rope_dims > qk_dim)
             return set_error(FK_ERR_INVALID, "sdpa: rope_dims must be even and within the head");
@@ -177,19 +177,29 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     }
     if (fusion) {
         // whole-width rotation of at most 128 dims with a table: the form whose loads run ahead
-        const bool fast = fusion->rope_tab && fusion->rope_dims == qk_dim && qk_dim <= 128;
-#define FK_SDPA_FUSED(F)                                                                           \
-    switch (gt) {                                                                                  \
-        case 1: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<1, F>); break;        \
-        case 2: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<2, F>); break;        \
-        case 4: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<4, F>); break;        \
-        default: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<8, F>); break;       \
+        // (heads of fewer than 128 dims add their squares in another order there: a quantised cache keeps the one it has)
+        const bool fast = fusion->rope_tab && fusion->rope_dims == qk_dim && qk_dim <= 128 && !(kvq && fusion->q_norm && qk_dim != 128);
+#define FK_SDPA_FUSED(F, Q)                                                                           \
+    switch (gt) {                                                                                     \
+        case 1: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<1, F, Q>); break;        \
+        case 2: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<2, F, Q>); break;        \
+        case 4: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<4, F, Q>); break;        \
+        default: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<8, F, Q>); break;       \
+    }
+#define FK_SDPA_FUSED_Q(F)              \
+    if (kvq == 4) {                     \
+        FK_SDPA_FUSED(F, 4)             \
+    } else if (kvq == 8) {              \
+        FK_SDPA_FUSED(F, 8)             \
+    } else {                            \
+        FK_SDPA_FUSED(F, 0)             \
     }
         if (fast) {
-            FK_SDPA_FUSED(true)
+            FK_SDPA_FUSED_Q(true)
         } else {
-            FK_SDPA_FUSED(false)
+            FK_SDPA_FUSED_Q(false)
         }
+#undef FK_SDPA_FUSED_Q
 #undef FK_SDPA_FUSED
     } else if (kvq == 4) {
         FK_SDPA_PICK(4)
@@ -202,7 +212,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     out_launch->func = func;
     out_launch->grid = dim3(n_splits, n_kv, ((G + gt - 1) / gt) * rows);
     out_launch->block = dim3(kSdpaBlock, 1, 1);
-    out_launch->shmem = (uint32_t)(sdpa_lds_floats(gt, chunk, qk_dim, v_dim, fusion != nullptr) * sizeof(float));
+    out_launch->shmem = (uint32_t)(sdpa_lds_floats(gt, chunk, qk_dim, v_dim, fusion != nullptr, kvq != 0) * sizeof(float));
     out_launch->set_args(a);
     return FK_OK;
 }

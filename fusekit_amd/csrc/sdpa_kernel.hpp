@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "fk_device.hpp"
+#include "kv_quant_device.hpp"
 #include "rope_device.hpp"
 
 // Hook for timing probes: a build may define FK_SDPA_STAMP(i) to record a clock at
@@ -69,13 +70,18 @@ struct SdpaArgs {
 // wave-local form: per-wave maxima [wave][8] at 32 and per-wave sums [wave][8] at 64.
 constexpr uint32_t kSdpaStatFloats = 96;
 
+// The new row of a quantised cache in the block that appends it, floats behind the transformed heads: the rows in fp32, their
+// packed words, scale | bias << 16 per group, their codes as bytes.
+__host__ __device__ inline uint32_t sdpa_quant_row_floats(uint32_t qk_dim, uint32_t v_dim) { return 2u * (qk_dim + v_dim); }
+
 // LDS floats one block needs.
 __host__ __device__ inline uint32_t sdpa_lds_floats(uint32_t gt, uint32_t chunk, uint32_t qk_dim, uint32_t v_dim,
-                                                     bool fused) {
+                                                     bool fused, bool quant = false) {
     uint32_t lpv = 1;
     while (lpv < v_dim / 8) lpv <<= 1;
     const uint32_t slots = kSdpaBlock / lpv;  // key rows handled side by side in the value phase
-    return gt * chunk + slots * gt * v_dim + kSdpaStatFloats + (fused ? (gt + 1) * qk_dim / 2 + 8 : 0);
+    return gt * chunk + slots * gt * v_dim + kSdpaStatFloats + (fused ? (gt + 1) * qk_dim / 2 + 8 : 0) +
+           (fused && quant ? sdpa_quant_row_floats(qk_dim, v_dim) : 0);
 }
 
 // One (range, kv head, head tile) work item.  Uniform per block; `kv_len` already read.
@@ -103,7 +109,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // the ranges of a block need no barrier; the waves meet once, after the last range.
     constexpr bool WAVES = MODE != 1 && GT <= 4;
     constexpr int kSteps = FUSED ? kSdpaStepsFused : kSdpaSteps;
-    static_assert(!(XFORM && KVQ != 0), "the fused forms read a bf16 cache");
+    static_assert(!(FUSED && KVQ != 0), "the whole-token kernel reads a bf16 cache");
     const uint32_t span = a.chunk_len * a.chunks_per_block;  // cache positions per block
     const uint32_t blk0 = split * span;
     const uint32_t G = a.n_heads / a.n_kv;
@@ -139,6 +145,11 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     float* stat = red + (kSdpaBlock / a.lpv) * GT * a.v_dim;  // m[GT], l[GT], misc
     uint16_t* qn = reinterpret_cast<uint16_t*>(stat + kSdpaStatFloats);  // fused: [GT][qk_dim] + k row
     uint16_t* kn = qn + GT * a.qk_dim;
+    // quantised cache: the new K and V rows (k, then v): fp32, packed words, scale | bias << 16 of a group, codes
+    float* nrow = reinterpret_cast<float*>(kn + a.qk_dim);
+    uint32_t* nword = reinterpret_cast<uint32_t*>(nrow + a.qk_dim + a.v_dim);
+    uint32_t* nmeta = nword + (a.qk_dim + a.v_dim) / 4u;
+    uint8_t* ncode = reinterpret_cast<uint8_t*>(nmeta + (a.qk_dim + a.v_dim) / 32u);
     bool blk_owner = false;
 
     // Head norm + RoPE of this block's q heads (one wave per head), and of the new k row
@@ -147,7 +158,37 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     auto head_dst = [&](uint32_t h) { return h < gcount ? qn + h * a.qk_dim : kn; };
     auto transform_heads = [&](uint32_t h_first) {
         blk_owner = pos >= blk0 && pos < blk0 + blk_keys;
-        for (uint32_t h = h_first + wave; h < gcount + (blk_owner ? 1u : 0u); h += kSdpaWaves) {
+        if constexpr (KVQ != 0) {
+            if (blk_owner && wave < 2u) {   // wave 0 the key, wave 1 the value; the first head tile's block writes them to the cache
+                const bool is_v = wave != 0u;
+                const uint32_t dim = is_v ? a.v_dim : a.qk_dim, at = is_v ? a.qk_dim : 0u, bits = (uint32_t)KVQ, groups = dim / a.kv_group;
+                float* row = nrow + at;
+                uint32_t *word = nword + at / 4u, *meta = nmeta + at / 32u;
+                uint8_t* code = ncode + at;
+                if (is_v)
+                    for (uint32_t d = lane; d < dim; d += kWave) row[d] = bf16_bits_to_f32(a.v_new[(size_t)kvh * dim + d]);
+                else
+                    kv_key_row(a.k_new + (size_t)kvh * dim, a.k_norm, row, dim, a.rope_dims, pos, a.base_log2, a.eps, lane, a.rope_tab);
+                const size_t crow = (size_t)kvh * a.capacity + (pos % a.capacity);
+                uint32_t* packed = reinterpret_cast<uint32_t*>(const_cast<uint16_t*>(is_v ? a.v : a.k)) + crow * (dim * bits / 32u);
+                uint16_t* scales = const_cast<uint16_t*>(is_v ? a.v_scales : a.k_scales) + crow * groups;
+                uint16_t* biases = const_cast<uint16_t*>(is_v ? a.v_biases : a.k_biases) + crow * groups;
+                wave_lds_order();
+                kv_quantize_row(row, code, dim, a.kv_group, bits, lane, [&](uint32_t g, uint32_t sc, uint32_t bi) {
+                    meta[g] = sc | (bi << 16);
+                    if (gz == 0) {
+                        scales[g] = (uint16_t)sc;
+                        biases[g] = (uint16_t)bi;
+                    }
+                });
+                wave_lds_order();
+                kv_pack_row(code, dim, bits, lane, [&](uint32_t wi, uint32_t w) {
+                    word[wi] = w;
+                    if (gz == 0) packed[wi] = w;
+                });
+            }
+        }
+        for (uint32_t h = h_first + wave; h < gcount + (blk_owner && KVQ == 0 ? 1u : 0u); h += kSdpaWaves) {
             if (a.q0_dim) {
                 const uint32_t d1 = a.qk_dim - a.q0_dim;
                 if (h < gcount) {
@@ -167,7 +208,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
             }
         }
         __syncthreads();
-        if (blk_owner && gz == 0) {
+        if (KVQ == 0 && blk_owner && gz == 0) {
             const size_t row = (size_t)kvh * a.capacity + (pos % a.capacity);
             for (uint32_t d = tid; d < a.qk_dim; d += kSdpaBlock) a.cache_k_w[row * a.qk_dim + d] = kn[d];
             for (uint32_t d = tid; d < a.v_dim; d += kSdpaBlock)
@@ -246,7 +287,11 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // Stand-alone: every row that exists in the cache allocation is requested, whether
     // or not it is below kv_len (rows past kv_len are masked where they are used).
     uint4 kc[kSteps], vc[kSteps];
-    uint4 kn_[kSteps], vn_[kSteps];  // stand-alone: the next range, in flight while this one is consumed
+    // Stand-alone: the next range, in flight while this one is consumed; of a quantised cache, whose ranges are a quarter to a
+    // half of the bytes, the one behind it too (12016 positions of an 8-bit cache, three ranges a block, cold: the last range
+    // starts 8.8 us into the launch instead of 13.6; a bf16 cache is bound by the bytes and was 5 % slower with it).
+    constexpr bool DEEP = MODE != 1 && WAVES && KVQ != 0;
+    uint4 kn_[kSteps], vn_[kSteps], kf_[DEEP ? kSteps : 1], vf_[DEEP ? kSteps : 1];
     auto request_rows = [&](uint4(&kd)[kSteps], uint4(&vd)[kSteps], uint32_t key0, uint32_t nkeys, bool owner,
                             uint32_t jpos) {
         const uint16_t* kbase = a.k + ((size_t)kvh * a.capacity + key0) * a.qk_dim + 8 * ck;
@@ -349,14 +394,14 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         }
         request_rows(kc, vc, blk0, 0, false, 0);
         if constexpr (MODE == 0) settle_q();
-        if constexpr (MODE == 2)
+        if constexpr (MODE == 2 && KVQ == 0)
             vnew = *reinterpret_cast<const uint4*>(a.v_new + (size_t)kvh * a.v_stride + (vcol_ok ? 8 * cv : 0u));
         asm volatile("" : "+v"(kv_raw));
         settle();
         if (split >= n_active) return;  // uniform: whole block leaves before any barrier
         if constexpr (MODE == 2) {
             if constexpr (FASTHEAD) {
-                const bool own = pos >= blk0 && pos < blk0 + blk_keys;
+                const bool own = KVQ == 0 && pos >= blk0 && pos < blk0 + blk_keys;
                 head_pair_apply(ha, head_dst(hi_a), a.q_norm != nullptr, half, a.eps, lane,
                                 hi_a < gcount || (hi_a == gcount && own));
                 head_pair_apply(hb, head_dst(hi_b), a.q_norm != nullptr, half, a.eps, lane,
@@ -372,6 +417,8 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         }
     }
 
+    if constexpr (DEEP)
+        if (n_chunks > 1) request_rows(kn_, vn_, blk0 + a.chunk_len, 0, false, 0);
     for (uint32_t c = 0; c < n_chunks; ++c) {
     const uint32_t key0 = blk0 + c * a.chunk_len;
     const uint32_t nkeys = (kv_len - key0) < a.chunk_len ? (kv_len - key0) : a.chunk_len;
@@ -379,13 +426,26 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     const uint32_t jpos = pos - key0;
     if constexpr (FUSED) {
         request_rows(kc, vc, key0, nkeys, owner, jpos);
+    } else if constexpr (DEEP) {
+        if (c + 2 < n_chunks) request_rows(kf_, vf_, key0 + 2 * a.chunk_len, 0, false, 0);
     } else {
         if (c + 1 < n_chunks) request_rows(kn_, vn_, key0 + a.chunk_len, 0, false, 0);
     }
 
     FK_SDPA_STAMP(1);
     if constexpr (XFORM) {
-        if (owner && kcol_ok) {
+        if constexpr (KVQ != 0) {
+            if (owner) {
+                constexpr uint32_t WPL = KVQ == 4 ? 1u : 2u;
+                const uint32_t kcol = kcol_ok ? ck : 0u, vcol = vcol_ok ? cv : 0u;
+                const uint32_t *kw = nword + kcol * WPL, *vw = nword + a.qk_dim / 4u + vcol * WPL;
+#pragma unroll
+                for (int u = 0; u < kSteps; ++u) {
+                    if (kslot + u * kslots == jpos) kc[u] = make_uint4(kw[0], kw[WPL - 1u], nmeta[8u * kcol / a.kv_group], 0u);
+                    if (vslot + u * vslots == jpos) vc[u] = make_uint4(vw[0], vw[WPL - 1u], nmeta[a.qk_dim / 32u + 8u * vcol / a.kv_group], 0u);
+                }
+            }
+        } else if (owner && kcol_ok) {
 #pragma unroll
             for (int u = 0; u < kSteps; ++u)
                 if (kslot + u * kslots == jpos) kc[u] = *reinterpret_cast<const uint4*>(kn + 8 * ck);
@@ -608,6 +668,10 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
             for (int u = 0; u < kSteps; ++u) {
                 kc[u] = kn_[u];
                 vc[u] = vn_[u];
+                if constexpr (DEEP) {
+                    kn_[u] = kf_[u];
+                    vn_[u] = vf_[u];
+                }
             }
         }
     }
@@ -713,19 +777,30 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // own two output dims of each of the 16 ranges; the next batch's loads are in flight
     // while the current one is folded in.
     constexpr uint32_t kBatch = 16;
+    const uint32_t ranges = __builtin_amdgcn_readfirstlane(n_active);   // (the length came through a vector register)
     const uint32_t row = a.v_dim + 2;
-    for (uint32_t h = wave; h < gcount; h += kSdpaWaves) {
+    // (the head is the same for the whole wave, which the compiler has to be told: the rows' addresses then are scalars)
+    for (uint32_t h = __builtin_amdgcn_readfirstlane(wave); h < gcount; h += kSdpaWaves) {
         const float* ph = a.partials + (size_t)(h0 + h) * a.n_splits * row;
         for (uint32_t d2 = lane; d2 < ((a.v_dim >> 1) + kWave - 1) / kWave * kWave; d2 += kWave) {
             const bool live = d2 < (a.v_dim >> 1);
-            const float* pd = ph + 2 + 2 * (live ? d2 : 0u);
+            const uint32_t at = 2u + 2u * (live ? d2 : 0u);
             float M = -INFINITY, L = 0.f, o0 = 0.f, o1 = 0.f;
+            // two floats at ph + (uniform) + (per lane), as a GLOBAL access with a scalar base and a 32-bit lane offset: the generic
+            // form keeps a 64-bit address in registers for every load in flight
+            auto ld_partial = [&](uint32_t uniform, uint32_t per_lane) {
+                typedef const __attribute__((address_space(1))) char* gptr;
+                typedef const __attribute__((address_space(1))) unsigned long long* gptr8;
+                const gptr base = (gptr)(uintptr_t)(ph + uniform);
+                const unsigned long long v = __hip_atomic_load((gptr8)(base + 4u * per_lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+            };
             auto fetch = [&](uint32_t base, float2& ml, float2(&po)[kBatch]) {
                 const uint32_t mine = base + (lane & (kBatch - 1));
-                ml = ld_f32x2<true>(ph + (size_t)(mine < n_active ? mine : base) * row);
+                ml = ld_partial(0u, (mine < ranges ? mine : base) * row);
 #pragma unroll
                 for (uint32_t i = 0; i < kBatch; ++i)
-                    po[i] = ld_f32x2<true>(pd + (size_t)(base + i < n_active ? base + i : base) * row);
+                    po[i] = ld_partial((base + i < ranges ? base + i : base) * row, at);
             };
             auto fold = [&](uint32_t base, const float2& ml, const float2(&po)[kBatch]) {
                 float pm[kBatch], pl[kBatch];
@@ -736,14 +811,14 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
                 }
                 float mn = fmaxf(M, pm[0]);
 #pragma unroll
-                for (uint32_t i = 1; i < kBatch; ++i) mn = base + i < n_active ? fmaxf(mn, pm[i]) : mn;
+                for (uint32_t i = 1; i < kBatch; ++i) mn = base + i < ranges ? fmaxf(mn, pm[i]) : mn;
                 const float alpha = base ? expf(M - mn) : 0.f;
                 L *= alpha;
                 o0 *= alpha;
                 o1 *= alpha;
 #pragma unroll
                 for (uint32_t i = 0; i < kBatch; ++i) {
-                    const float w = base + i < n_active ? expf(pm[i] - mn) : 0.f;
+                    const float w = base + i < ranges ? expf(pm[i] - mn) : 0.f;
                     L = fmaf(pl[i], w, L);
                     o0 = fmaf(po[i].x, w, o0);
                     o1 = fmaf(po[i].y, w, o1);
@@ -753,7 +828,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
             float2 ml_a, ml_b, po_a[kBatch], po_b[kBatch];
             uint32_t base = 0;
             fetch(0, ml_a, po_a);
-            while (base + kBatch < n_active) {  // straight-line body: request the next batch, fold this one
+            while (base + kBatch < ranges) {  // straight-line body: request the next batch, fold this one
                 fetch(base + kBatch, ml_b, po_b);
                 fold(base, ml_a, po_a);
                 ml_a = ml_b;
@@ -790,7 +865,7 @@ __device__ __forceinline__ uint32_t sdpa_load_kv_len(const SdpaArgs& a) {
 }
 
 template <int GT, int KVQ = 0>
-__global__ __launch_bounds__(kSdpaBlock) void sdpa_decode_kernel(const SdpaArgs a) {
+__global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_decode_kernel(const SdpaArgs a) {
     extern __shared__ __align__(16) float lds[];
     // One unconditional load (the immediate is read from the kernel-argument segment
     // when there is no device scalar): a load under a branch would be waited for at
@@ -817,12 +892,13 @@ __global__ __launch_bounds__(kSdpaBlock) void sdpa_decode_kernel(const SdpaArgs 
 // RoPE (+ head norm) of q and of the new k row, the cache append and the attention in one
 // launch: a.q / a.k_new / a.v_new are the raw projection outputs of the token at position
 // kv_len - 1, a.k / a.v the cache it is appended to.
-template <int GT, bool FASTHEAD>
-__global__ __launch_bounds__(kSdpaBlock) void sdpa_rope_store_kernel(const SdpaArgs a) {
+// KVQ: a quantised cache; the new rows are quantised by the block whose range holds them.
+template <int GT, bool FASTHEAD, int KVQ = 0>
+__global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_rope_store_kernel(const SdpaArgs a) {
     extern __shared__ __align__(16) float lds[];
     kernarg_warm<(int)sizeof(SdpaArgs)>();
     const uint32_t kv_len0 = sdpa_load_kv_len(a);
-    sdpa_block<GT, 2, SdpaArgs, 0, FASTHEAD>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
+    sdpa_block<GT, 2, SdpaArgs, KVQ, FASTHEAD>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
 }
 
 }  // namespace fk

@@ -77,14 +77,6 @@ __device__ __forceinline__ float both_halves_sum(float v) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// LDS traffic of ONE wave with itself: the hardware runs a wave's LDS instructions in order,
-// the fence keeps the compiler from reordering them.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The rescale of the output accumulators, in place in the accumulation registers of the matrix unit.
 // Written as plain C++ this multiply makes the compiler copy all of them to vector registers at the
 // head of EVERY pass, taken or not; spelled out, the copies stay inside the rare branch that calls
@@ -253,7 +245,7 @@ __global__ __launch_bounds__(kPrefillBlock) void sdpa_prefill_kernel(const SdpaP
         uint32_t pk[16];
         softmax_step<DT>(s, a.scale2, kv0 + kPrefillStep > first_limit, kv0, kb, q_limit, m_run, l_run, oacc, pk);
 
-        wave_lds_fence();  // the transposed tile is complete
+        wave_lds_order();  // the transposed tile is complete
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const uint4 pb = make_uint4(pk[c * 4 + 0], pk[c * 4 + 1], pk[c * 4 + 2], pk[c * 4 + 3]);
@@ -264,7 +256,7 @@ __global__ __launch_bounds__(kPrefillBlock) void sdpa_prefill_kernel(const SdpaP
                                                                   __builtin_bit_cast(pf_bf16x8_t, pb), oacc[i], 0, 0, 0);
             }
         }
-        wave_lds_fence();  // the tile has been read before the next pass overwrites it
+        wave_lds_order();  // the tile has been read before the next pass overwrites it
     }
 
     // ---- merge of the four waves, in wave order --------------------------------------------
@@ -514,7 +506,7 @@ __global__ __launch_bounds__(kPrefillBlock) void sdpa_prefill_tile_kernel(const 
         for (int g = 0; g < 4; ++g)
             *reinterpret_cast<float4*>(ob + nl * OS + (uint32_t)(i * 32 + 8 * g) + 4u * kb) =
                 make_float4(oacc[i][4 * g + 0] * f, oacc[i][4 * g + 1] * f, oacc[i][4 * g + 2] * f, oacc[i][4 * g + 3] * f);
-    wave_lds_fence();
+    wave_lds_order();
     for (uint32_t idx = lane; idx < kPrefillRows * (uint32_t)VP; idx += 64u) {
         const uint32_t row = idx / (uint32_t)VP, pc = idx % (uint32_t)VP;
         if (row >= live) continue;

@@ -218,10 +218,10 @@ class DecoderRuntime:
         self.persistent = persistent
         # one launch per layer for rope/store + attention: the task graph only (the whole-token kernel
         # fuses them itself and is built from the plain task list)
-        self.fused_attention = bool(cfg.fuse_attention and not persistent and not cfg.kv_bits)
+        self.fused_attention = bool(cfg.fuse_attention and not persistent)
         self.rope_tab = DeviceBuffer(cfg.head_dim * 4) if self.fused_attention else None
         # a layer as two XCD-resident launches (8 KV heads, one per XCD): graph mode, bf16 cache, no projection bias
-        self.xcd = bool(cfg.xcd_layers and self.fused_attention and not cfg.qkv_bias and
+        self.xcd = bool(cfg.xcd_layers and self.fused_attention and not cfg.kv_bits and not cfg.qkv_bias and
                         native.xcd_layer_supported(cfg.hidden, cfg.inter, cfg.n_heads, cfg.n_kv, cfg.head_dim, cfg.capacity,
                                                    cfg.bits, cfg.group))
         if self.xcd:
@@ -293,10 +293,11 @@ class DecoderRuntime:
                 a = [arg(self.q), arg(self.k), arg(self.v)]
                 if c.qk_norm:
                     a += [arg(w.vecs[p + "self_attn.q_norm"]), arg(w.vecs[p + "self_attn.k_norm"])]
-                a += [arg(self.cache_k[l]), arg(self.cache_v[l]), arg(self.kv_len), arg(self.att),
-                      arg(self.sdpa_partials), arg(self.sdpa_counters), arg(self.rope_tab)]
-                t.append(Dispatch(name("rope_store_sdpa_decode"), a,
-                                  dict(rope, has_norm=int(c.qk_norm), has_table=1, max_len=c.capacity)))
+                for C in (self.cache_k[l], self.cache_v[l]):
+                    a += [arg(b) for b in (C.packed, C.scales, C.biases)] if c.kv_bits else [arg(C)]
+                a += [arg(self.kv_len), arg(self.att), arg(self.sdpa_partials), arg(self.sdpa_counters), arg(self.rope_tab)]
+                t.append(Dispatch(name("rope_store_sdpa_decode" + (f"_q{c.kv_bits}" if c.kv_bits else "")), a,
+                                  dict(rope, has_norm=int(c.qk_norm), has_table=1, max_len=c.capacity, group=c.kv_group)))
             elif c.kv_bits:
                 # quantised cache: rotate q in place, then quantise the rotated K row and the V row
                 qa = [arg(self.q)] + ([arg(w.vecs[p + "self_attn.q_norm"])] if c.qk_norm else []) + [arg(self.offset)]

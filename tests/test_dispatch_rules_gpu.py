@@ -113,3 +113,24 @@ def test_matmul_from_65_rows(fk, bits, m, n, k):
     g, u = (oracle.bf16_to_f32(oracle.f32_to_bf16(a.astype(np.float32))).astype(np.float64) for a in acc[:2])
     for y, want in zip(ys, (acc[0] + b + r, g / (1 + np.exp(-g)) * u, acc[0], acc[1] + b, acc[2])):
         assert rel_l2(y.to_numpy(np.uint16, (m, n)), want) <= 4e-3
+
+
+@pytest.mark.parametrize("heads,qk_norm", [((8, 2, 128), True), ((4, 2, 64), True), ((14, 2, 64), False), ((2, 2, 128), False)])
+@pytest.mark.parametrize("kv_bits", [4, 8])
+def test_quantised_cache_rows_appended_inside_the_attention(fk, heads, qk_norm, kv_bits):
+    """One launch for rotation, quantisation, append and attention leaves the bits of the three launches it replaces: one,
+    two and four heads a tile and eight, the first position, range boundaries, several ranges."""
+    from fusekit_amd.decoder import DecoderConfig, DecoderRuntime, DecoderWeights
+    n_heads, n_kv, dim = heads
+    cfg = dict(n_layers=2, hidden=256, n_heads=n_heads, n_kv=n_kv, head_dim=dim, inter=512, vocab=500, capacity=2304, kv_bits=kv_bits,
+               qk_norm=qk_norm)
+    W = DecoderWeights.random_init(DecoderConfig(**cfg), seed=5)
+    a, b = (DecoderRuntime(DecoderConfig(**cfg, fuse_attention=f), W) for f in (True, False))
+    assert len(a.tasks) == len(b.tasks) - 2 * cfg["n_layers"]
+    bufs = lambda rt: [x for c in rt.cache_k + rt.cache_v for x in (c.packed, c.scales, c.biases)]
+    for pos in (0, 1, 31, 63, 64, 130, 700, 2303):
+        for rt in (a, b):
+            rt.d.decode_host_loop(rt.graph, rt.uniforms, pos, [7 + pos % 400])
+        assert np.array_equal(a.logits.to_numpy(np.uint16), b.logits.to_numpy(np.uint16)), pos
+        for x, y in zip(bufs(a), bufs(b)):
+            assert np.array_equal(x.to_numpy(np.uint8), y.to_numpy(np.uint8)), pos
