@@ -76,6 +76,13 @@ using namespace fk;
 
 namespace fk {
 
+fk_status run_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const uint16_t* cache_v, uint16_t* out, uint32_t rows, uint32_t kv_len,
+                           uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t capacity, float scale, bool kept_order, hipStream_t s) {
+    Launch l;
+    FK_TRY(plan_sdpa_prefill(q, cache_k, cache_v, out, rows, kv_len, n_heads, n_kv, head_dim, capacity, scale, &l, nullptr, kept_order));
+    return run_launch(l, s);
+}
+
 fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint16_t* bias, const uint16_t* residual, uint16_t* y,
                     void* workspace, bool kept_order, hipStream_t s) {
     if (W && W->bits == 16) {  // dense bf16 weights: the plain library GEMM with this library's epilogue
@@ -785,9 +792,7 @@ fk_status fk_sdpa_decode_rows(const uint16_t* q, const uint16_t* cache_k, const 
 fk_status fk_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const uint16_t* cache_v, uint16_t* out,
                           uint32_t rows, uint32_t kv_len, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
                           uint32_t capacity, float scale, fk_stream s) {
-    Launch l;
-    FK_TRY(plan_sdpa_prefill(q, cache_k, cache_v, out, rows, kv_len, n_heads, n_kv, head_dim, capacity, scale, &l));
-    return run_launch(l, (hipStream_t)s);
+    return run_sdpa_prefill(q, cache_k, cache_v, out, rows, kv_len, n_heads, n_kv, head_dim, capacity, scale, false, (hipStream_t)s);
 }
 
 fk_status fk_sdpa_workspace_bytes(uint32_t n_heads, uint32_t n_kv, uint32_t qk_dim, uint32_t v_dim, uint32_t max_len,

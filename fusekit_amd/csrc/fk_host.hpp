@@ -175,6 +175,8 @@ fk_status run_dequantize_bf16(const fk_weight* W, uint16_t* out, hipStream_t s);
 bool qgemm_takes_library(uint32_t m, bool pair = false);
 // What fk_qgemm, fk_qgemm_fanout and fk_qgemm_swiglu run.  kept_order: the launches whose sums are added in the order that
 // quantised caches have been filled with (see prompt.hip).
+fk_status run_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const uint16_t* cache_v, uint16_t* out, uint32_t rows, uint32_t kv_len,
+                           uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t capacity, float scale, bool kept_order, hipStream_t s);
 fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint16_t* bias, const uint16_t* residual, uint16_t* y,
                     void* workspace, bool kept_order, hipStream_t s);
 fk_status run_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const uint16_t* x, uint32_t m, const uint16_t* const* bias,
@@ -336,10 +338,12 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
                            const KvQuant* quant = nullptr, const SdpaFusion* fusion = nullptr);
 // Causal attention of a group of rows on the matrix cores (head dimension 64 or 128, bf16 cache):
 // kv_len counts the rows of the group, row r sees the first kv_len - rows + r + 1 positions.  With
-// kv_len_ptr the count is read on the device at run time (clamped to rows .. capacity).
+// kv_len_ptr the count is read on the device at run time (clamped to rows .. capacity).  kept_order: sums in the order of
+// the kernels for short groups and of 128-row tiles staged through registers.
 fk_status plan_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const uint16_t* cache_v, uint16_t* out,
                             uint32_t rows, uint32_t kv_len, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
-                            uint32_t capacity, float scale, Launch* out_launch, const uint32_t* kv_len_ptr = nullptr);
+                            uint32_t capacity, float scale, Launch* out_launch, const uint32_t* kv_len_ptr = nullptr,
+                            bool kept_order = false);
 fk_status plan_embed(const fk_weight* E, const uint32_t* token_ptr, uint32_t token_imm, float out_scale,
                      uint16_t* x, Launch* out, uint32_t rows = 1);
 // (strided: the form that adds a row's squares 256 elements apart also where the one in 16-byte pieces would run)

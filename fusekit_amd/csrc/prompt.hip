@@ -92,7 +92,7 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* s
         if (tiled) {   // the visible prefix as bf16, then the matrix-core attention
             FK_TRY(fk_kv_cache_dequant(&l.cache_kq, m.n_kv, dim, m.capacity, m.kv_bits, m.kv_group, len, m.k_rows, m.capacity, s));
             FK_TRY(fk_kv_cache_dequant(&l.cache_vq, m.n_kv, dim, m.capacity, m.kv_bits, m.kv_group, len, m.v_rows, m.capacity, s));
-            FK_TRY(fk_sdpa_prefill(m.q, m.k_rows, m.v_rows, m.att, rows, len, m.n_heads, m.n_kv, dim, m.capacity, scale, s));
+            FK_TRY(run_sdpa_prefill(m.q, m.k_rows, m.v_rows, m.att, rows, len, m.n_heads, m.n_kv, dim, m.capacity, scale, true, (hipStream_t)s));
         } else {
             FK_TRY(fk_sdpa_decode_quant(m.q, &l.cache_kq, &l.cache_vq, m.att, nullptr, pos + 1, len, rows, m.n_heads, m.n_kv, dim, dim,
                                         m.capacity, m.kv_bits, m.kv_group, scale, m.partials, m.counters, s));

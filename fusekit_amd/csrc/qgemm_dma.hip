@@ -19,24 +19,14 @@
 
 #include <type_traits>
 
+#include "dma_device.hpp"
 #include "fk_host.hpp"
 #include "gemv_kernel.hpp"
 
 namespace fk {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-
-// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>): every index is a constant, whatever the unroller thinks of
-// the body (an accumulator indexed by a loop variable goes to scratch).
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<N, I + 1>(f);
-    }
-}
 
 // acc += weights x activations with the accumulators in the AGPR half of the register file (left to itself the compiler keeps
 // what is beyond 256 registers there and moves it back and forth).  The statement hides the instruction from the hazard
@@ -45,14 +35,6 @@ __device__ __forceinline__ void mfma_acc(f32x4_t& acc, const uint32_t (&w)[4], c
     const fk_u32x4_t wv = {w[0], w[1], w[2], w[3]};
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(wv), "v"(x));
 }
-// a finished sum, where it is used (a plain read lets the compiler copy all of them out at once)
-__device__ __forceinline__ f32x4_t take(const f32x4_t& acc) {
-    float v[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[r]) : "a"(acc[r]));
-    return f32x4_t{v[0], v[1], v[2], v[3]};
-}
-__device__ __forceinline__ void settle_matrix_ops() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
 struct QgemmDmaArgs {
     const uint16_t* x;  // [M, K] bf16
@@ -74,22 +56,6 @@ struct QgemmDmaArgs {
         uint32_t N, nb_end, col0, pad;
     } seg[3];   // a fan-out's matrices, or gate and up
 };
-
-// 16 (4) bytes per lane from `base + off` (`ptr`) to LDS at `to` + 16 (4) * lane; counted in vmcnt.  As statements the
-// compiler does not look into: its own form waits for every such load in flight ahead of each LDS read.
-__device__ __forceinline__ void dma16(uint32_t to, uint32_t off, const void* base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory");
-}
-__device__ __forceinline__ void dma16(uint32_t to, const unsigned char* ptr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(ptr) : "memory");
-}
-__device__ __forceinline__ void dma4(uint32_t to, const unsigned char* ptr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(to), "v"(ptr) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 // Eight int4 codes as bf16 weights T(s q + b).  A nibble in the low bits of a half word is the fp16 subnormal code * 2^-24
 // (* 2^-20 four bits higher), so one mixed-precision FMA takes it as it lies: fma(code * 2^-24, s * 2^24, b) is

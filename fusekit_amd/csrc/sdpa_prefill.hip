@@ -6,12 +6,12 @@
 // with all scores in threadgroup memory (kv_len <= 4096); here the scores never leave
 // registers and kv_len is bounded by the cache only.
 //
-// Two forms share the arithmetic.  Up to 64 rows (few rows, possibly a long cache):
+// The forms share the arithmetic.  Few rows, possibly a long cache:
 // one block = one query head x 32 consecutive rows; its four waves take the 64-position
 // steps of the visible range round-robin (wave w: steps w, w + 4, ...), each with its own
 // running (reference, sum, output), and the four are merged once at the end in wave order.
-// More rows: one block = one head x 128 rows, a 32-row tile per wave, K and V shared through
-// LDS (described at sdpa_prefill_tile_kernel below).
+// More rows: blocks of 64 or 128 rows of a head, a 32-row tile per wave, K and V shared through
+// LDS (described at sdpa_prefill_tile_kernel and sdpa_prefill_dma_kernel below).
 //
 // Per step a wave computes, with v_mfma_f32_32x32x16_bf16,
 //     S^T[kv, q] = K[kv, :] . Q[q, :]        A = K rows (read from the cache as they lie),
@@ -28,7 +28,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "fk_device.hpp"
+#include "dma_device.hpp"
 #include "fk_host.hpp"
 
 namespace fk {
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(kPrefillBlock) void sdpa_prefill_kernel(const SdpaP
     }
 }
 
-// ---- the form for more than 64 rows ------------------------------------------------------------
+// ---- 128 rows a block, K and V staged through registers (passes that keep their sums: see the plan) ----
 // One block = one query head x 128 consecutive rows, one 32-row tile per wave.  The four waves
 // walk the SAME 64-position steps, so a step's K and V rows are fetched once per block, with
 // coalesced 16-byte loads, and shared through LDS (two buffers: the next step is written while
@@ -321,15 +321,6 @@ constexpr uint32_t prefill_tile_lds_bytes(uint32_t d) {
     const uint32_t stage = 2u * prefill_tile_buf(d) * 2u;
     const uint32_t outb = kPrefillWaves * kPrefillRows * (d + 4u) * 4u;
     return stage > outb ? stage : outb;
-}
-
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 // value of the thread that holds the neighbouring cache row (lane ^ PIECES) -> (even row's, odd row's)
@@ -517,9 +508,250 @@ __global__ __launch_bounds__(kPrefillBlock) void sdpa_prefill_tile_kernel(const 
     }
 }
 
+// ---- the form whose operands go straight into LDS -----------------------------------------------------------------
+// One head x 128 rows a block, a 32-row tile per wave (SPLIT 1); or 64 rows (SPLIT 2): 128 positions a step, waves 0 and 1
+// take their first 64, waves 2 and 3 the second on the same rows, merged at the end -- twice the blocks and half the chain of
+// steps, where 128-row blocks would leave CUs idle.  The products and the softmax are those of the form above; what differs is
+// how the operands arrive.  K and V rows go from memory into LDS as they lie (16-byte pieces XOR-swizzled by the row, so that
+// the fragment reads meet all banks): no registers in flight, no LDS stores, no transposition.  V^T fragments are read with
+// ds_read_b64_tr_b16: in each group of 16 lanes, lane i receives column i of the 4 x 16 values that the group's lanes address
+// (lane s: row s / 4, columns 4 (s % 4) ..).  Every fragment of a product is asked for before its first matrix instruction, V's
+// behind the first product so that they arrive during the softmax; the probabilities of 16 positions are formed between the
+// matrix instructions of the 16 before.  Matrix instructions are statements on VGPRs: with AGPRs in use the compiler halves
+// the file and copies the scores.  That makes 226 registers: two waves a SIMD (the form above has one), so that with SPLIT 1
+// the softmax of one block runs beside the products of another.  Bound by the matrix units and the softmax's vector
+// instructions together (1024 and about 1300 cycles of a 64-position step).
+//     us at 32 query / 8 KV heads x 128, form above -> this: 512 rows 19.4 -> 11.5 (SPLIT 2; 15.0 with SPLIT 1), behind 3000
+//     positions 95 -> 55; 1024 rows 32.6 -> 25.6; 2048 rows 71 -> 54 (SPLIT 1); 4096 rows 246 -> 163, 840 TFLOP/s
+//     14 / 2 heads x 64, 2000 rows behind 500 positions: 41.4 -> 26.9
+constexpr uint32_t prefill_dma_lds_bytes(uint32_t d, uint32_t split) {
+    const uint32_t stage = 2u * 2u * split * kPrefillStep * d * 2u, outb = kPrefillWaves * kPrefillRows * (d + 4u) * 4u;
+    return stage > outb ? stage : outb;
+}
+typedef short pf_s16x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void mfma32_acc(pf_f32x16_t& acc, const pf_u32x4_t& a, const pf_u32x4_t& b) {
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+
+// scores stay in VGPRs, where the softmax takes them
+template <bool FIRST>
+__device__ __forceinline__ void mfma32_scores(pf_f32x16_t& s, const pf_u32x4_t& a, const pf_u32x4_t& b) {
+    if constexpr (FIRST) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(a), "v"(b));
+}
+
+template <int D, int SPLIT>
+__global__ __launch_bounds__(kPrefillBlock, 2) void sdpa_prefill_dma_kernel(const SdpaPrefillArgs a) {
+    constexpr int KB = D / 16, DT = D / 32, VP = D / 8;
+    constexpr uint32_t STEP = kPrefillStep * SPLIT, TILES = kPrefillWaves / SPLIT;        // positions of a step, 32-row tiles of a block
+    constexpr uint32_t ROW = D * 2u, TILE = STEP * ROW, STAGE = 2u * TILE;               // bytes: a row, K (or V) of a step, both
+    constexpr uint32_t RPI = 1024u / ROW;                                            // rows of one wave's request
+    constexpr int REQ = (int)(STEP / RPI / kPrefillWaves);                   // requests of a wave, matrix and step
+    extern __shared__ uint4 lds_raw[];
+    unsigned char* const lds = reinterpret_cast<unsigned char*>(lds_raw);
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kb = lane >> 5, nl = lane & 31u;
+    const uint32_t head = blockIdx.x % a.n_heads;
+    const uint32_t grp = a.row_tiles - 1u - blockIdx.x / a.n_heads;   // longest first
+    const uint32_t kvh = head / a.heads_per_kv;
+    const uint32_t part = wave / TILES, r0 = (grp * TILES + wave % TILES) * kPrefillRows;
+    const uint32_t live = r0 < a.rows ? (a.rows - r0 < kPrefillRows ? a.rows - r0 : kPrefillRows) : 0u;
+    const uint32_t prior = prefill_kv_len(a) - a.rows;
+    const uint32_t grp_end = (grp + 1u) * TILES * kPrefillRows;
+    const uint32_t kv_end_blk = prior + (grp_end < a.rows ? grp_end : a.rows);   // positions the block's last row sees
+    const uint32_t first_limit = prior + r0 + 1u;
+    const uint32_t n_steps = __builtin_amdgcn_readfirstlane((kv_end_blk + STEP - 1u) / STEP);
+
+    uint32_t rq = r0 + (nl < live ? nl : (live ? live - 1u : 0u));
+    rq = rq < a.rows ? rq : a.rows - 1u;   // a wave without rows repeats the last one and stores nothing
+    const uint32_t q_limit = prior + rq + 1u;
+    pf_u32x4_t qreg[KB];
+    {
+        const pf_u32x4_t* qp = reinterpret_cast<const pf_u32x4_t*>(a.q + ((size_t)rq * a.n_heads + head) * D + kb * 8u);
+#pragma unroll
+        for (int j = 0; j < KB; ++j) qreg[j] = qp[2 * j];
+    }
+
+    // the 16-byte piece of a row that lies at place `at`: K reads 16 rows of one piece at a time, V 8 rows of 64 bytes
+    auto k_swizzle = [](uint32_t row) { return D == 128 ? row & 15u : (row >> 1) & 7u; };
+    auto v_swizzle = [](uint32_t row) { return D == 128 ? (row & 3u) << 2 : ((row >> 1) & 1u) << 2; };
+    const unsigned char* kbase = reinterpret_cast<const unsigned char*>(a.k + (size_t)kvh * a.capacity * D);
+    const unsigned char* vbase = reinterpret_cast<const unsigned char*>(a.v + (size_t)kvh * a.capacity * D);
+    const uint32_t irow = lane / (uint32_t)VP, place = lane % (uint32_t)VP;
+    auto issue = [&](uint32_t step, uint32_t stage) {
+#pragma unroll
+        for (int i = 0; i < REQ; ++i) {
+            const uint32_t idx = wave * (uint32_t)REQ + (uint32_t)i, row = idx * RPI + irow;
+            uint32_t kv = step * STEP + row;
+            kv = kv < kv_end_blk ? kv : kv_end_blk - 1u;   // (past the range: masked scores, zero probabilities)
+            dma16(stage * STAGE + idx * 1024u, kv * ROW + ((place ^ k_swizzle(row)) * 16u), kbase);
+            dma16(stage * STAGE + TILE + idx * 1024u, kv * ROW + ((place ^ v_swizzle(row)) * 16u), vbase);
+        }
+    };
+
+    float m_run = -INFINITY, l_run = 0.f;
+    pf_f32x16_t oacc[DT];
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
+
+    // fragments: K row nl (+ 32), piece 2 j + kb; V rows 4 kb + (0..3) (+ 8) of 16, columns 32 i + nl
+    const uint32_t vrow = 4u * kb + ((lane & 15u) >> 2), vcol = ((lane >> 4) & 1u) * 2u + ((lane & 3u) >> 1), vlow = (lane & 1u) * 8u;
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    issue(0, 0);
+    uint32_t stage = 0;
+#pragma unroll 1
+    for (uint32_t step = 0; step < n_steps; ++step, stage ^= 1u) {
+        wait_loads<0>();
+        barrier();   // this step's rows are everybody's; the other stage has been read
+        if (step + 1u < n_steps) issue(step + 1u, stage ^ 1u);
+        const uint32_t kv0 = step * STEP + part * kPrefillStep;
+        if (kv0 >= first_limit + kPrefillRows - 1u) continue;   // all of it in the future of this wave's rows
+        const unsigned char *ks = lds + stage * STAGE + part * kPrefillStep * ROW, *vs = ks + TILE;
+        // all of a product's fragments are asked for before its first matrix instruction
+        pf_u32x4_t kf[KB][2];
+#pragma unroll
+        for (int j = 0; j < KB; ++j)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const uint32_t row = (uint32_t)t * 32u + nl;
+                kf[j][t] = *reinterpret_cast<const pf_u32x4_t*>(ks + row * ROW + (((uint32_t)(2 * j) + kb) ^ k_swizzle(row)) * 16u);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        pf_f32x16_t s[2];
+        static_for<KB>([&](auto j) __attribute__((always_inline)) {
+            mfma32_scores<j() == 0>(s[0], kf[j()][0], qreg[j()]);
+            mfma32_scores<j() == 0>(s[1], kf[j()][1], qreg[j()]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        pf_s16x4_t vf[4][DT][2];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int i = 0; i < DT; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t row = (uint32_t)(c * 16 + h * 8) + vrow;
+                    const unsigned char* at = vs + row * ROW + (((uint32_t)(4 * i) + vcol) ^ v_swizzle(row)) * 16u + vlow;
+                    typedef __attribute__((address_space(3))) pf_s16x4_t* lds_ptr;
+                    vf[c][i][h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(pf_s16x4_t*)at);
+                }
+        __builtin_amdgcn_sched_barrier(0);
+        settle_matrix_ops();
+        asm volatile("" : "+v"(s[0]), "+v"(s[1]));
+        if (kv0 + kPrefillStep > first_limit) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (kv0 + (uint32_t)(t * 32 + r % 4 + 8 * (r / 4)) + 4u * kb >= q_limit) s[t][r] = -INFINITY;
+        }
+        // as softmax_step, with the scale (positive) inside the exponent's multiply-add
+        float mt = s[0][0];
+#pragma unroll
+        for (int i = 1; i < 32; ++i) mt = fmaxf(mt, s[i / 16][i % 16]);
+        mt = other_half_max(mt) * a.scale2;
+        const bool grow = mt > m_run + 8.0f;
+        const float m_new = grow ? mt : m_run, m_ref = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = grow ? __builtin_amdgcn_exp2f(m_run - m_ref) : 1.0f;
+        m_run = m_new;
+        l_run *= alpha;
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+            settle_matrix_ops();
+#pragma unroll
+            for (int i = 0; i < DT; ++i) {
+                asm volatile("" : "+v"(oacc[i]));
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[i][r] *= alpha;
+            }
+        }
+        // the second product of 16 positions, and between its matrix instructions the probabilities of the next 16
+        pf_u32x4_t pb[4];
+        auto probabilities = [&](auto c, auto w) __attribute__((always_inline)) {
+            constexpr int at = c() * 8 + w() * 2;
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(s[at / 16][at % 16], a.scale2, -m_ref));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(s[at / 16][at % 16 + 1], a.scale2, -m_ref));
+            l_run += p0 + p1;
+            pb[c()][w()] = pack_bf16(p0, p1);
+        };
+        static_for<4>([&](auto w) __attribute__((always_inline)) { probabilities(std::integral_constant<int, 0>{}, w); });
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_nop 1");
+        static_for<4>([&](auto c) __attribute__((always_inline)) {
+            static_for<DT>([&](auto i) __attribute__((always_inline)) {
+                const pf_u32x2_t lo = __builtin_bit_cast(pf_u32x2_t, vf[c()][i()][0]), hi = __builtin_bit_cast(pf_u32x2_t, vf[c()][i()][1]);
+                mfma32_acc(oacc[i()], pf_u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pb[c()]);
+                if constexpr (c() < 3)
+                    static_for<4 / DT>([&](auto w) __attribute__((always_inline)) {
+                        probabilities(std::integral_constant<int, c() + 1>{}, std::integral_constant<int, i() * (4 / DT) + w()>{});
+                    });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            asm volatile("s_nop 1");
+        });
+    }
+    settle_matrix_ops();
+#pragma unroll
+    for (int i = 0; i < DT; ++i) asm volatile("" : "+v"(oacc[i]));
+    barrier();
+
+    // ---- output: through this wave's own LDS rows, so that the stores are whole 16-byte pieces ----
+    l_run = both_halves_sum(l_run);
+    constexpr uint32_t OS = D + 4;
+    float* const ob = reinterpret_cast<float*>(lds_raw) + wave * kPrefillRows * OS;
+    float f = SPLIT == 1 ? 1.0f / l_run : 1.0f, f_other = 0.f;
+    auto put = [&]() {
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                float4* const to = reinterpret_cast<float4*>(ob + nl * OS + (uint32_t)(i * 32 + 8 * g) + 4u * kb);
+                float4 o = make_float4(oacc[i][4 * g + 0] * f, oacc[i][4 * g + 1] * f, oacc[i][4 * g + 2] * f, oacc[i][4 * g + 3] * f);
+                if (SPLIT == 2 && part == 0) {
+                    const float4 p = to[TILES * kPrefillRows * OS / 4u];
+                    o = make_float4(fmaf(p.x, f_other, o.x), fmaf(p.y, f_other, o.y), fmaf(p.z, f_other, o.z), fmaf(p.w, f_other, o.w));
+                }
+                *to = o;
+            }
+    };
+    if constexpr (SPLIT == 2) {   // the second half's sums, its reference and its denominator (in the padding) to the first
+        if (part == 1) {
+            put();
+            if (kb == 0) *reinterpret_cast<float2*>(ob + nl * OS + D) = make_float2(m_run, l_run);
+        }
+        __syncthreads();
+        if (part == 1) return;
+        const float2 other = *reinterpret_cast<const float2*>(ob + (TILES * kPrefillRows + nl) * OS + D);
+        const float m = fmaxf(m_run, other.x), w0 = __builtin_amdgcn_exp2f(m_run - m), w1 = __builtin_amdgcn_exp2f(other.x - m);
+        f = 1.0f / (l_run * w0 + other.y * w1);
+        f_other = f * w1;
+        f *= w0;
+    }
+    if (live == 0) return;
+    put();
+    wave_lds_order();
+    for (uint32_t idx = lane; idx < kPrefillRows * (uint32_t)VP; idx += 64u) {
+        const uint32_t row = idx / (uint32_t)VP, pc = idx % (uint32_t)VP;
+        if (row >= live) continue;
+        const float4 lo = *reinterpret_cast<const float4*>(ob + row * OS + pc * 8u);
+        const float4 hi = *reinterpret_cast<const float4*>(ob + row * OS + pc * 8u + 4u);
+        *reinterpret_cast<uint4*>(a.out + ((size_t)(r0 + row) * a.n_heads + head) * D + pc * 8u) =
+            make_uint4(pack_bf16(lo.x, lo.y), pack_bf16(lo.z, lo.w), pack_bf16(hi.x, hi.y), pack_bf16(hi.z, hi.w));
+    }
+}
+
 fk_status plan_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const uint16_t* cache_v, uint16_t* out,
                             uint32_t rows, uint32_t kv_len, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
-                            uint32_t capacity, float scale, Launch* l, const uint32_t* kv_len_ptr) {
+                            uint32_t capacity, float scale, Launch* l, const uint32_t* kv_len_ptr, bool kept_order) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
     if (!q || !cache_k || !cache_v || !out) return set_error(FK_ERR_INVALID, "sdpa_prefill: null pointer");
@@ -537,27 +769,42 @@ fk_status plan_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const ui
     if (rows > capacity) return set_error(FK_ERR_INVALID, "sdpa_prefill: more rows than the cache holds");
     a.rows = rows; a.kv_len = kv_len; a.n_heads = n_heads; a.heads_per_kv = n_heads / n_kv; a.capacity = capacity;
     a.scale2 = scale * 1.4426950408889634f;
-    // Two forms: a block per 32 rows whose waves split the positions, or a block per 128 rows whose
-    // waves share every step's K and V through LDS.  The second does a 64-position step of its 128
-    // rows in 1.65 us against 4 x 0.93 us, but has a quarter of the blocks: it is taken when the first
-    // form would need more rounds over the CUs than that advantage is worth (measured at head
-    // dimension 128: 128 rows x 32 heads 65 against 105 us, 512 rows 118 against 106 us at 4096 positions).
-    const uint64_t blocks_split = (uint64_t)n_heads * ((rows + kPrefillRows - 1u) / kPrefillRows);
-    const uint64_t blocks_tile = (uint64_t)n_heads * ((rows + kPrefillWaves * kPrefillRows - 1u) / (kPrefillWaves * kPrefillRows));
+    // Four forms: a block per 32 rows whose waves split the positions; a block per 128 rows, or per 64 with the positions in
+    // halves, whose waves share the rows through LDS; and, where a caller needs the sums of earlier passes over the same rows
+    // (kept_order: a quantised cache rounds what follows from them), the older kernel of 128 rows.
     const uint64_t cus = (uint64_t)(dev->cus > 0 ? dev->cus : 1);
-    const bool shared_tiles = ((blocks_tile + cus - 1) / cus) * 165u < ((blocks_split + cus - 1) / cus) * 93u;
-    const uint32_t rows_per_block = shared_tiles ? kPrefillWaves * kPrefillRows : kPrefillRows;
+    auto blocks = [&](uint32_t rows_per_block) { return (uint64_t)n_heads * ((rows + rows_per_block - 1u) / rows_per_block); };
+    uint32_t rows_per_block = kPrefillRows;
+    uint32_t split = 0;   // the parts of a step in the kernel that loads into LDS; 0: another kernel
+    if (kept_order || !(scale > 0.f)) {
+        // A 64-position step of 128 rows takes 1.65 us against 4 x 0.93 us, but there is a quarter of the blocks: taken when the
+        // first form would need more rounds over the CUs than that advantage is worth (measured at head dimension 128: 128 rows
+        // x 32 heads 65 against 105 us, 512 rows 118 against 106 us at 4096 positions).
+        if (((blocks(kPrefillWaves * kPrefillRows) + cus - 1) / cus) * 165u < ((blocks(kPrefillRows) + cus - 1) / cus) * 93u)
+            rows_per_block = kPrefillWaves * kPrefillRows;
+    } else if (head_dim == 128 || 2u * blocks(kPrefillRows) > cus) {
+        // At head dimension 64, 32-row blocks while there are two CUs for each (14 heads, 200 rows at 1200 positions 12.9
+        // against 13.8 us; 512 rows 8.3 either way); at 128 the shared rows win from the first (100 rows at 3100 positions 50.4 -> 44.9).
+        // 64-row blocks until 128-row ones fill the places that the former have, 1 a CU (2 at head dimension 64): 32 heads x 128,
+        // 1024 rows 25.6 / 25.7 us, 1200 rows 35.6 / 31.7; 14 heads x 64, 4096 rows 49.8 / 70.2, 8192 rows 173 / 163.
+        split = blocks(kPrefillWaves * kPrefillRows) > cus * (128u / head_dim) ? 1u : 2u;
+        rows_per_block = kPrefillWaves / split * kPrefillRows;
+    }
     a.row_tiles = (rows + rows_per_block - 1u) / rows_per_block;
     if ((uint64_t)a.row_tiles * n_heads > 0x7fffffffull) return set_error(FK_ERR_UNSUPPORTED, "sdpa_prefill: too many rows");
-    if (shared_tiles)
-        l->func = head_dim == 64 ? reinterpret_cast<const void*>(&sdpa_prefill_tile_kernel<64, kPrefillTileDepth>)
-                                 : reinterpret_cast<const void*>(&sdpa_prefill_tile_kernel<128, kPrefillTileDepth>);
+    auto at = [&](const void* d64, const void* d128) { return head_dim == 64 ? d64 : d128; };
+    if (split == 1)
+        l->func = at(reinterpret_cast<const void*>(&sdpa_prefill_dma_kernel<64, 1>), reinterpret_cast<const void*>(&sdpa_prefill_dma_kernel<128, 1>));
+    else if (split == 2)
+        l->func = at(reinterpret_cast<const void*>(&sdpa_prefill_dma_kernel<64, 2>), reinterpret_cast<const void*>(&sdpa_prefill_dma_kernel<128, 2>));
+    else if (rows_per_block > kPrefillRows)
+        l->func = at(reinterpret_cast<const void*>(&sdpa_prefill_tile_kernel<64, kPrefillTileDepth>),
+                     reinterpret_cast<const void*>(&sdpa_prefill_tile_kernel<128, kPrefillTileDepth>));
     else
-        l->func = head_dim == 64 ? reinterpret_cast<const void*>(&sdpa_prefill_kernel<64>)
-                                 : reinterpret_cast<const void*>(&sdpa_prefill_kernel<128>);
+        l->func = at(reinterpret_cast<const void*>(&sdpa_prefill_kernel<64>), reinterpret_cast<const void*>(&sdpa_prefill_kernel<128>));
     l->grid = dim3(a.row_tiles * n_heads, 1, 1);
     l->block = dim3(kPrefillBlock, 1, 1);
-    l->shmem = shared_tiles ? prefill_tile_lds_bytes(head_dim) : prefill_lds_bytes(head_dim);
+    l->shmem = split ? prefill_dma_lds_bytes(head_dim, split) : rows_per_block > kPrefillRows ? prefill_tile_lds_bytes(head_dim) : prefill_lds_bytes(head_dim);
     if ((int)l->shmem > dev->max_dyn_lds) return set_error(FK_ERR_UNSUPPORTED, "sdpa_prefill: LDS tile does not fit");
     if (l->shmem > 48 * 1024) FK_HIP(hipFuncSetAttribute(l->func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l->shmem));
     l->set_args(a);

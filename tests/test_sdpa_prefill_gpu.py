@@ -69,6 +69,14 @@ def test_large_groups_many_heads(fk, rows, kv_len, n_heads, n_kv, D):
     _case(fk, rows, kv_len, n_heads, n_kv, D, 1600, seed=17)
 
 
+@pytest.mark.parametrize("rows,kv_len,n_heads,n_kv,D", [
+    (1, 129, 4, 4, 128), (33, 96, 4, 2, 128), (64, 64, 5, 1, 128), (65, 193, 4, 4, 128),   # 64 rows a block, positions in halves
+    (63, 191, 140, 2, 64), (65, 129, 130, 65, 64),
+    (129, 129, 129, 3, 128), (127, 255, 257, 1, 128), (129, 321, 258, 2, 64)])             # 128 rows a block
+def test_rows_straight_into_lds(fk, rows, kv_len, n_heads, n_kv, D):
+    _case(fk, rows, kv_len, n_heads, n_kv, D, kv_len + 3, seed=23)
+
+
 def test_first_row_of_fresh_group_is_v0(fk):
     q, ck, cv, got = _case(fk, 40, 40, 32, 8, 128, 64, seed=11)
     v0 = cv.reshape(8, 64, 128)[:, 0]  # softmax over the one visible position is 1
