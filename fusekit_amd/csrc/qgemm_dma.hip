@@ -11,10 +11,10 @@
 // the same tile took 20 % longer, with the unpacking where the compiler puts it 35 %.  The rest is the requests: 38 cycles of
 // a wave for each kilobyte, spread over a step's tiles.
 //     us (before: the tiles of qgemm.hip; from 1024 rows dequantise + library), 4-bit weights, warm:
-//     gate / up pair 9728 x 2560:    128 rows 34.8 -> 30.3   512 rows 99.2 -> 67.5   2048 rows 284 -> 242   4096 rows 446 -> 419
+//     gate / up pair 9728 x 2560:    128 rows 34.8 -> 29.5   512 rows 99.2 -> 65.3   2048 rows 284 -> 222   4096 rows 446 -> 375
 //     q / k / v 6144 x 2560:         512 rows 41.9 -> 33.6   768 rows 63.8 -> 50.2
 //     2560 x 9728:                   512 rows 50.4 -> 46.8;  0.5B class, pair 4864 x 896, 200 rows: 39.6 -> 12.9
-// (4096 rows of the pair are 1.04 PFLOP/s of the 1.16 that a large library product reaches on this card.)
+// (4096 rows of the pair are 1.09 PFLOP/s of the 1.16 that a large library product reaches on this card.)
 #include <string.h>
 
 #include <type_traits>
@@ -77,22 +77,32 @@ constexpr uint32_t dma_stage_bytes(WKind kind, int gk, uint32_t wtn) { return 32
 constexpr uint32_t dma_stages(WKind kind, int gk, uint32_t wtn) { return 4u * dma_stage_bytes(kind, gk, wtn) <= 163840u ? 4u : 3u; }
 constexpr uint32_t dma_lds_bytes(WKind kind, int gk, uint32_t wtn) { return dma_stages(kind, gk, wtn) * dma_stage_bytes(kind, gk, wtn); }
 
-// SiLU(g) * u of the rounded sums, the variant with one rounding at the end: 1 / (1 + e^-g) with e^x as 2^(x log2 e), the
-// product in two parts, and the hardware's reciprocal with one Newton step -- about an ulp each, as expf and the divide that
-// swiglu_bits uses, in a third of their instructions (128 outputs a lane: 8 us of a 90 us launch).
+// SiLU(g) * u of the rounded sums, the variant with one rounding at the end, as swiglu_bits has it, with e^x and 1 / d from the
+// hardware's 2^x and reciprocal instead of expf and a divide (128 outputs a lane: those take 8 us of a 90 us launch).
+//     e^x 2^-32 = 2^(e - 32) 2^a: e is the nearest integer to x log2 e (adding 1.5 2^23, here less 32, rounds to integers and
+//     leaves e - 32 in the low bits, from where it goes into the exponent of 2^a), a what is left, with log2 e in two parts:
+//     the float next to it and the rest.  |a| <= 1/2, so 2^a keeps its last bits whatever x is.
+//     x is held to -64 .. 110: below, 1 + e^x is 1; above, the result is zero (g < -110).  So nothing is infinite on the way.
+//     d = (1 + e^x) 2^-32, 1 / d by the reciprocal and one Newton step: the reciprocal of 1 + e^x itself is subnormal from
+//     2^126 on, which the instruction gives as zero; of d it is so only for results that are zero.
+// Against 64 bits over all bf16 gates no further off than expf and the divide, in every range (largest error, units in the last
+// place of fp32, here / there: gates in -4 .. -1 1.49 / 1.57, -20 .. -4 1.39 / 1.40, -88.7 .. -20 1.33 / 1.33, -1 .. 0 2.19 / 2.19,
+// above zero 1.82 / 1.82; below -88.7, where expf overflows and leaves -0 u, this still has the value).
 __device__ __forceinline__ float swiglu_fast(float acc_g, float acc_u) {
+    constexpr float kRound = 12582912.0f - 32.0f;
     const float g = round_bf16(acc_g), u = round_bf16(acc_u);
-    const float x = -g, t = x * 1.44269504f, lo = fmaf(x, 1.44269504f, -t) + x * 1.92596299e-8f;
-    const float p = __builtin_amdgcn_exp2f(t);
-    const float d = 1.0f + fmaf(p, lo * 0.693147181f, p);
-    const float r0 = __builtin_amdgcn_rcpf(d);
-    const float r = d < 1e30f ? fmaf(fmaf(-d, r0, 1.0f), r0, r0) : r0;
-    return (r * g) * u;
+    const float x = __builtin_amdgcn_fmed3f(-g, -64.0f, 110.0f);
+    const float y = fmaf(x, 1.44269504f, kRound), e = y - kRound;
+    const float a = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269504f, -e));
+    const float d = __uint_as_float(__float_as_uint(__builtin_amdgcn_exp2f(a)) + (__float_as_uint(y) << 23)) + 0x1p-32f;
+    const float r0 = __builtin_amdgcn_rcpf(d), r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
+    return ((r * 0x1p-32f) * g) * u;
 }
+template <bool FAST>
 __device__ __forceinline__ void store_swiglu(const QgemmDmaArgs& a, uint32_t m, uint32_t n, uint32_t N, const f32x4_t& g, const f32x4_t& u) {
     if (m >= a.M || n >= N) return;
     uint2 o;
-    if (a.variant == 1)
+    if constexpr (FAST)
         o = make_uint2(pack_bf16(swiglu_fast(g[0], u[0]), swiglu_fast(g[1], u[1])), pack_bf16(swiglu_fast(g[2], u[2]), swiglu_fast(g[3], u[3])));
     else
         o = make_uint2(swiglu_bits(g[0], u[0], a.variant, 1.0f) | (swiglu_bits(g[1], u[1], a.variant, 1.0f) << 16),
@@ -391,29 +401,39 @@ __global__ __launch_bounds__(256 * GK, GK) void qgemm_dma_kernel(const QgemmDmaA
             if ((wn >= 2u) != (I % 2 != 0)) static_for<NJ>([&](auto j) { ex[(I * NJ + decltype(j)::value) * 64] = take(acc[I][decltype(j)::value]); });
         });
         __syncthreads();
-        static_for<NR / 2>([&](auto i) {
-            static_for<NJ>([&](auto j) {
-                constexpr int I = decltype(i)::value * 2, J = decltype(j)::value;
-                const bool up = wn >= 2u;
-                const f32x4_t own = up ? take(acc[I + 1][J]) : take(acc[I][J]), o = ex[((up ? I + 1 : I) * NJ + J) * 64];
-                const uint32_t m = mrow0 + (up ? I + 1 : I) * 16u + l16, n = n0 + (wn & 1u) * (uint32_t)WTN + J * 16u + 4u * kb;
-                store_swiglu(a, m, n, N, up ? o : own, up ? own : o);
+        auto finish = [&](auto fast) {
+            static_for<NR / 2>([&](auto i) {
+                static_for<NJ>([&](auto j) {
+                    constexpr int I = decltype(i)::value * 2, J = decltype(j)::value;
+                    const bool up = wn >= 2u;
+                    const f32x4_t own = up ? take(acc[I + 1][J]) : take(acc[I][J]), o = ex[((up ? I + 1 : I) * NJ + J) * 64];
+                    const uint32_t m = mrow0 + (up ? I + 1 : I) * 16u + l16, n = n0 + (wn & 1u) * (uint32_t)WTN + J * 16u + 4u * kb;
+                    store_swiglu<decltype(fast)::value>(a, m, n, N, up ? o : own, up ? own : o);
+                });
             });
-        });
+        };
+        a.variant == 1 ? finish(std::true_type{}) : finish(std::false_type{});
     } else if constexpr (PAIR) {
-        static_for<NR>([&](auto i) {
-            static_for<NJ / 2>([&](auto j) {
-                constexpr int I = decltype(i)::value, J = decltype(j)::value;
-                const uint32_t m = mrow0 + I * 16u + l16, n = n0 + wn * (WTN / 2u) + J * 16u + 4u * kb;
-                const f32x4_t g = take(acc[I][J]), u = take(acc[I][J + NJ / 2]);
-                if (finished) {
-                    store_swiglu(a, m, n, N, g, u);
-                } else if (m < a.M && n < N) {
-                    *reinterpret_cast<f32x4_t*>(a.partial + ((size_t)ks * a.M + m) * N + n) = g;
-                    *reinterpret_cast<f32x4_t*>(a.partial2 + ((size_t)ks * a.M + m) * N + n) = u;
-                }
+        // (What is done with the sums is chosen once: chosen at every output, the code that a tile's end runs through lies
+        // scattered over 110 KB, more than the instruction cache holds: 4096 rows of the 9728 x 2560 pair 402 us, this way 372.)
+        auto each = [&](auto store) {
+            static_for<NR>([&](auto i) {
+                static_for<NJ / 2>([&](auto j) {
+                    constexpr int I = decltype(i)::value, J = decltype(j)::value;
+                    store(mrow0 + I * 16u + l16, n0 + wn * (WTN / 2u) + J * 16u + 4u * kb, take(acc[I][J]), take(acc[I][J + NJ / 2]));
+                });
             });
-        });
+        };
+        if (!finished)
+            each([&](uint32_t m, uint32_t n, const f32x4_t& g, const f32x4_t& u) {
+                if (m >= a.M || n >= N) return;
+                *reinterpret_cast<f32x4_t*>(a.partial + ((size_t)ks * a.M + m) * N + n) = g;
+                *reinterpret_cast<f32x4_t*>(a.partial2 + ((size_t)ks * a.M + m) * N + n) = u;
+            });
+        else if (a.variant == 1)
+            each([&](uint32_t m, uint32_t n, const f32x4_t& g, const f32x4_t& u) { store_swiglu<true>(a, m, n, N, g, u); });
+        else
+            each([&](uint32_t m, uint32_t n, const f32x4_t& g, const f32x4_t& u) { store_swiglu<false>(a, m, n, N, g, u); });
     } else {
         uint16_t* y = a.seg[si].y;
         const uint16_t* bias = a.seg[si].bias;

@@ -134,3 +134,40 @@ def test_quantised_cache_rows_appended_inside_the_attention(fk, heads, qk_norm, 
         assert np.array_equal(a.logits.to_numpy(np.uint16), b.logits.to_numpy(np.uint16)), pos
         for x, y in zip(bufs(a), bufs(b)):
             assert np.array_equal(x.to_numpy(np.uint8), y.to_numpy(np.uint8)), pos
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m", [65, 300, 1024])
+def test_swiglu_of_every_finite_gate(fk, bits, m):
+    """All finite bf16 gates (and, in a row that doubles them, infinite ones) through the pair's one-launch form: the finite
+    values against 64 bits, infinities and NaN as the form of up to 64 rows (expf and a divide) gives them."""
+    n, k = 4096, 1024
+    rng = np.random.default_rng(m)
+    zeros = np.zeros((n, k // 64), np.uint16)
+    # a weight is T(0 code + bias): a row that is one in group j and zero elsewhere selects gate n, j and its factor u
+    gate = rng.permutation(np.arange(65536, dtype=np.uint16)).reshape(n, k // 64)
+    gate[(gate & 0x7F80) == 0x7F80] = 0x42B5                      # (infinities and NaN: another 90.5)
+    factor = oracle.f32_to_bf16(rng.normal(0, 1, (n, k // 64)).astype(np.float32))
+    codes = np.zeros((n, k * bits // 32), np.uint32)
+    g, u = (to_device(fk, oracle.QWeight(codes, zeros, b, n, k, bits)) for b in (gate, factor))
+    x = np.zeros((m, k), np.float32)
+    x[np.arange(m), 64 * (np.arange(m) % 16) + 5] = np.where(np.arange(m) == m - 1, 2.0, 1.0)
+    x = oracle.f32_to_bf16(x)
+    def run(rows):
+        out, ws = fk.DeviceBuffer(2 * len(rows) * n), fk.DeviceBuffer(2 * fk.qgemm_workspace_bytes(len(rows), n, k))
+        fk.qgemm_swiglu(g, u, fk.DeviceBuffer.from_numpy(x[rows]), len(rows), 1, out, ws)
+        return oracle.bf16_to_f32(out.to_numpy(np.uint16, (len(rows), n))).astype(np.float64)
+    got, sel = run(np.arange(m)), [r % 16 for r in range(m)]
+    with np.errstate(all="ignore"):
+        scale = np.where(np.arange(m) == m - 1, 2.0, 1.0)[:, None]
+        gv, uv = (oracle.bf16_to_f32(oracle.f32_to_bf16(oracle.bf16_to_f32(b).T[sel] * np.float32(scale))).astype(np.float64) for b in (gate, factor))
+        want = gv / (1 + np.exp(-gv)) * uv
+        # half a unit of bf16, a few of fp32; below -88.73 e^-g overflows and the result may be -0 u, at most 88.8 2^-128 u away
+        off = np.abs(got - want) > (2.0 ** -8 + 2.0 ** -20) * np.abs(want) + 3e-37 * np.abs(uv) + 1e-40
+    plain = np.isfinite(gv) & (np.abs(want) < 3.3e38)
+    assert plain.mean() > 0.99 and not (off & plain).any(), (gv[off & plain][:8], got[off & plain][:8])
+    assert np.isfinite(got[plain]).all()
+    few = np.r_[0:63, m - 1]
+    ref = run(few)
+    assert np.isposinf(gv[m - 1]).any() and np.isneginf(gv[m - 1]).any()
+    assert np.array_equal(np.isnan(got[few]), np.isnan(ref)) and np.array_equal(np.isinf(got[few]), np.isinf(ref))
