@@ -17,8 +17,10 @@ namespace {
 // 0.4 us per million values it normalises, where the norm as a launch of its own costs some 3.5 us.  37 rows of K = 896:
 // 1152 outputs (2.4 million) 5.4 us against 4.1 + 4.1, a 4864 pair (10 million) 15.2 against 10.1 + 4.1; 50 rows of
 // K = 2560, a 9728 pair (78 million) 54 against 30 + 5.
-bool takes_norm(const fk_weight& W, uint32_t rows, uint32_t n_total) {
-    return qgemm_takes_rows(rows, W.bits, W.group, W.k) && (uint64_t)rows * W.k * ((n_total + 15u) / 16u) < 8000000ull;
+// (Rows and norm weights that are not 16-byte aligned take the norm's own launch.)
+bool takes_norm(const fk_weight& W, uint32_t rows, uint32_t n_total, const uint16_t* x, const uint16_t* norm_w) {
+    return qgemm_takes_rows(rows, W.bits, W.group, W.k) && (uint64_t)rows * W.k * ((n_total + 15u) / 16u) < 8000000ull &&
+           (((uintptr_t)x | (uintptr_t)norm_w) & 15u) == 0;
 }
 
 fk_status run_rows(const RowsRequest& rq, hipStream_t s) {
@@ -53,7 +55,7 @@ fk_status matmul(const fk_prompt_model& m, const fk_weight& W, const uint16_t* x
 // place, free between a projection's launch and the next norm).
 fk_status residual_rows(const fk_prompt_model& m, const fk_weight& W, const uint16_t* x, uint32_t rows, const uint16_t* res, uint16_t* y,
                         bool* ssq, hipStream_t s) {
-    *ssq = m.kv_bits == 0 && qgemm_takes_rows(rows, W.bits, W.group, W.k) && W.n % 64u == 0;
+    *ssq = m.kv_bits == 0 && qgemm_takes_rows(rows, W.bits, W.group, W.k) && W.n % 64u == 0 && ((uintptr_t)m.xn & 15u) == 0;
     if (!*ssq) return matmul(m, W, x, rows, nullptr, res, y, s);
     RowsRequest rq;
     rq.W[0] = &W; rq.x = x; rq.M = rows; rq.res = res; rq.y[0] = y;
@@ -66,7 +68,7 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* s
     const float scale = (float)(1.0 / sqrt((double)dim));
     const bool tiled = dim == 64 || dim == 128;
     if (m.kv_bits == 0 && l.k.bits == l.q.bits && l.v.bits == l.q.bits && l.k.group == l.q.group && l.v.group == l.q.group &&
-        takes_norm(l.q, rows, l.q.n + l.k.n + l.v.n)) {
+        takes_norm(l.q, rows, l.q.n + l.k.n + l.v.n, m.x, l.input_norm)) {
         RowsRequest rq;
         rq.W[0] = &l.q; rq.W[1] = &l.k; rq.W[2] = &l.v; rq.n_mats = 3;
         rq.x = m.x; rq.M = rows; rq.norm_w = l.input_norm; rq.eps = m.eps;
@@ -107,7 +109,7 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* s
                                        m.partials, m.counters, s));
     }
     FK_TRY(residual_rows(m, l.o, m.att, rows, m.x, m.x2, ssq, (hipStream_t)s));
-    if (*ssq && l.gate.bits == l.up.bits && l.gate.group == l.up.group && takes_norm(l.gate, rows, l.gate.n)) {
+    if (*ssq && l.gate.bits == l.up.bits && l.gate.group == l.up.group && takes_norm(l.gate, rows, l.gate.n, m.x2, l.post_norm)) {
         RowsRequest rq;
         rq.W[0] = &l.gate; rq.W[1] = &l.up; rq.n_mats = 2; rq.pair = true;
         rq.x = m.x2; rq.M = rows; rq.norm_w = l.post_norm; rq.eps = m.eps; rq.variant = m.swiglu_variant;

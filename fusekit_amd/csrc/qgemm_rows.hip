@@ -29,6 +29,9 @@ namespace {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+// 16 bytes of an operand, which need not lie on their own alignment (a row of a larger tensor, a matrix inside a file): the
+// vector memory unit takes any address, and the type keeps the compiler from assuming more.  The same instructions.
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
 
 constexpr uint32_t kRowsMax = 64;   // activation rows: four tiles of 16
 
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) s.w[t][h] = *reinterpret_cast<const u32x4_t*>(wbase[t] + (woff[t][h] + at));
+            for (int h = 0; h < 2; ++h) s.w[t][h] = *reinterpret_cast<const u32x4_any_t*>(wbase[t] + (woff[t][h] + at));
             if constexpr (KIND != W_BF16) {
                 const uint32_t gm = g + (lane & 3u), gmc = (gm < gl ? gm : gl) >> a.gshift;
                 s.sc[t] = *reinterpret_cast<const uint16_t*>(sbase[t] + (soff[t] + gmc * 2u));
@@ -167,8 +170,8 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) s.x[t][h] = *reinterpret_cast<const u32x4_t*>(xbase + (xoff[t][h] + gc * 128u));
-        s.nw = *reinterpret_cast<const u32x4_t*>(nbase + (l8 * 16u + gc * 128u));
+            for (int h = 0; h < 2; ++h) s.x[t][h] = *reinterpret_cast<const u32x4_any_t*>(xbase + (xoff[t][h] + gc * 128u));
+        s.nw = *reinterpret_cast<const u32x4_any_t*>(nbase + (l8 * 16u + gc * 128u));
     };
     const uint4 ones4 = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
     const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, ones4);
@@ -409,7 +412,7 @@ const void* rows_func(bool pair, bool two, uint32_t mt, uint32_t waves) {
 }  // namespace
 
 bool qgemm_takes_rows(uint32_t M, uint32_t bits, uint32_t group, uint32_t K) {
-    return M >= 1 && M <= kRowsMax && K >= 64u && K % 64u == 0 &&
+    return M >= 1 && M <= kRowsMax && K >= 64u && K % 64u == 0 && K < (1u << 24) &&   // (32-bit offsets)
            (bits == 16 || ((bits == 4 || bits == 8) && (group == 64 || (group == 128 && K % 128u == 0))));
 }
 
@@ -421,8 +424,10 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
     if (!W0 || !rq.x) return set_error(FK_ERR_INVALID, "qgemm (rows): null weight or activations");
     const uint32_t M = rq.M, K = W0->k, x_stride = rq.x_stride ? rq.x_stride : K;
     if (!qgemm_takes_rows(M, W0->bits, W0->group, K)) return set_error(FK_ERR_UNSUPPORTED, "qgemm (rows): 1..64 rows, whole groups of 64 columns");
-    if (x_stride >= (1u << 24) || K >= (1u << 24)) return set_error(FK_ERR_UNSUPPORTED, "qgemm (rows): rows too long");   // 32-bit offsets
-    if (x_stride < K || x_stride % 8u || (((uintptr_t)rq.x | (uintptr_t)rq.norm_w) & 15u))
+    if (x_stride >= (1u << 24)) return set_error(FK_ERR_UNSUPPORTED, "qgemm (rows): rows too far apart");
+    if (x_stride < K) return set_error(FK_ERR_INVALID, "qgemm (rows): row stride below K");
+    // (normalised or strided rows: the entry points for those have always asked for it)
+    if ((rq.norm_w || rq.x_stride) && (x_stride % 8u || (((uintptr_t)rq.x | (uintptr_t)rq.norm_w) & 15u)))
         return set_error(FK_ERR_INVALID, "qgemm (rows): rows and norm weights must be 16-byte aligned");
     QgemmRowsArgs a;
     memset(&a, 0, sizeof(a));
@@ -432,7 +437,6 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
         if (!W || !W->w || W->n == 0 || (W->bits != 16 && (!W->scales || !W->biases))) return set_error(FK_ERR_INVALID, "qgemm (rows): null weight");
         if (W->k != K || W->bits != W0->bits || (W->bits != 16 && W->group != W0->group) || (rq.pair && W->n != W0->n))
             return set_error(FK_ERR_INVALID, "qgemm (rows): the matrices must share K, bits and group size (a pair: N too)");
-        if ((uintptr_t)W->w & 15u) return set_error(FK_ERR_INVALID, "qgemm (rows): weights must be 16-byte aligned");
         a.w[i] = reinterpret_cast<const uint4*>(W->w);
         a.sc[i] = W->scales;
         a.bi[i] = W->biases;
