@@ -518,7 +518,7 @@ __global__ __launch_bounds__(kPrefillBlock) void sdpa_prefill_tile_kernel(const 
 // (lane s: row s / 4, columns 4 (s % 4) ..).  Every fragment of a product is asked for before its first matrix instruction, V's
 // behind the first product so that they arrive during the softmax; the probabilities of 16 positions are formed between the
 // matrix instructions of the 16 before.  Matrix instructions are statements on VGPRs: with AGPRs in use the compiler halves
-// the file and copies the scores.  That makes 226 registers: two waves a SIMD (the form above has one), so that with SPLIT 1
+// the file and copies the scores.  That makes 228 registers (235 with SPLIT 2): two waves a SIMD (the form above has one), so that with SPLIT 1
 // the softmax of one block runs beside the products of another.  Bound by the matrix units and the softmax's vector
 // instructions together (1024 and about 1300 cycles of a 64-position step).
 //     us at 32 query / 8 KV heads x 128, form above -> this: 512 rows 19.4 -> 11.5 (SPLIT 2; 15.0 with SPLIT 1), behind 3000
@@ -579,14 +579,16 @@ __global__ __launch_bounds__(kPrefillBlock, 2) void sdpa_prefill_dma_kernel(cons
     const unsigned char* kbase = reinterpret_cast<const unsigned char*>(a.k + (size_t)kvh * a.capacity * D);
     const unsigned char* vbase = reinterpret_cast<const unsigned char*>(a.v + (size_t)kvh * a.capacity * D);
     const uint32_t irow = lane / (uint32_t)VP, place = lane % (uint32_t)VP;
+    // (a step's first row is a 64-bit address: the rows of a head may lie more than 4 GB apart)
     auto issue = [&](uint32_t step, uint32_t stage) {
+        const uint32_t left = kv_end_blk - step * STEP;
+        const unsigned char *kstep = kbase + (size_t)step * TILE, *vstep = vbase + (size_t)step * TILE;
 #pragma unroll
         for (int i = 0; i < REQ; ++i) {
             const uint32_t idx = wave * (uint32_t)REQ + (uint32_t)i, row = idx * RPI + irow;
-            uint32_t kv = step * STEP + row;
-            kv = kv < kv_end_blk ? kv : kv_end_blk - 1u;   // (past the range: masked scores, zero probabilities)
-            dma16(stage * STAGE + idx * 1024u, kv * ROW + ((place ^ k_swizzle(row)) * 16u), kbase);
-            dma16(stage * STAGE + TILE + idx * 1024u, kv * ROW + ((place ^ v_swizzle(row)) * 16u), vbase);
+            const uint32_t kv = row < left ? row : left - 1u;   // (past the range: masked scores, zero probabilities)
+            dma16(stage * STAGE + idx * 1024u, kv * ROW + ((place ^ k_swizzle(row)) * 16u), kstep);
+            dma16(stage * STAGE + TILE + idx * 1024u, kv * ROW + ((place ^ v_swizzle(row)) * 16u), vstep);
         }
     };
 

@@ -77,6 +77,24 @@ def test_rows_straight_into_lds(fk, rows, kv_len, n_heads, n_kv, D):
     _case(fk, rows, kv_len, n_heads, n_kv, D, kv_len + 3, seed=23)
 
 
+@pytest.mark.parametrize("rows,n_heads,D", [(100, 2, 128), (640, 8, 64)])
+def test_positions_more_than_four_gigabytes_into_a_head(fk, rows, n_heads, D):
+    """One key that every query meets lies beyond 4 GB of its head; the rows 4 GB below it hold another value."""
+    wrap = (1 << 32) // (2 * D)
+    at, kv_len = wrap + 37, wrap + 37 + rows
+    ck, cv = (fk.zeros(2 * D * (kv_len + 11)) for _ in range(2))
+    value = normal_bf16(7, D)
+    ck.upload(np.full(D, 0x40C0, np.uint16), 2 * D * at)                # 6: a score of 6 sqrt(D), e^48 of the zeros' weight
+    cv.upload(value, 2 * D * at)
+    cv.upload(np.full(D, 0x40E0, np.uint16), 2 * D * (at - wrap))       # 7
+    out = fk.DeviceBuffer(2 * rows * n_heads * D)
+    q = fk.DeviceBuffer.from_numpy(np.full(rows * n_heads * D, 0x3F80, np.uint16))
+    fk.sdpa_prefill(q, ck, cv, out, rows, kv_len, n_heads, 1, D, kv_len + 11, 1.0 / np.sqrt(D))
+    fk.sync()
+    got = out.to_numpy(np.uint16, (rows * n_heads, D))
+    assert (got == value).all()
+
+
 def test_first_row_of_fresh_group_is_v0(fk):
     q, ck, cv, got = _case(fk, 40, 40, 32, 8, 128, 64, seed=11)
     v0 = cv.reshape(8, 64, 128)[:, 0]  # softmax over the one visible position is 1
