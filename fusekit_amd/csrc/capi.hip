@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "fk_host.hpp"
+#include "lds_limit.hpp"
 #include "xcd_layer.hpp"
 
 namespace fk {
@@ -62,10 +63,15 @@ fk_status run_launch(const Launch& l, hipStream_t s) {
 }
 
 fk_status raise_dynamic_lds(const void* func, uint32_t bytes) {
+    if (bytes <= 48u * 1024u) return FK_OK;
+    // what this thread knows to be allowed (it stays so: limits only rise), without the lock
     static thread_local struct { const void* func; uint32_t bytes; } seen[64];
     auto& slot = seen[((uintptr_t)func >> 4) & 63u];
     if (slot.func == func && slot.bytes >= bytes) return FK_OK;
-    FK_HIP(hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    static LdsLimits limits;
+    FK_HIP((hipError_t)limits.raise(func, bytes, [&](uint32_t b) {
+        return (int)hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
+    }));
     slot = {func, bytes};
     return FK_OK;
 }

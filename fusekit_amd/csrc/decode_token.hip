@@ -260,7 +260,7 @@ fk_status token_kernel_max_grid(int kind, int gt, uint32_t lds_bytes, uint32_t* 
     const void* f = pick(kind, gt);
     if (!f) return set_error(FK_ERR_UNSUPPORTED, "token kernel: unsupported weight kind or GQA group size");
     if ((int)lds_bytes > dev->max_dyn_lds) return set_error(FK_ERR_UNSUPPORTED, "token kernel: LDS need exceeds the CU");
-    if (lds_bytes > 48 * 1024) FK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+    FK_TRY(raise_dynamic_lds(f, lds_bytes));
     int per_cu = 0;
     FK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kGemvBlock, lds_bytes));
     if (per_cu < 1) return set_error(FK_ERR_UNSUPPORTED, "token kernel: does not fit on a compute unit");

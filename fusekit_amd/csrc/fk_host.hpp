@@ -64,7 +64,8 @@ fk_status device_facts(const DeviceFacts** out);
 fk_status set_error(fk_status code, const std::string& msg);
 fk_status hip_error(hipError_t e, const char* what);
 fk_status run_launch(const Launch& l, hipStream_t s);
-// Allows `func` that much dynamic LDS (needed above 48 KB); asked of the runtime once per kernel and size.
+// Allows `func` that much dynamic LDS (nothing to do up to 48 KB).  A limit that another launch needs is never lowered; every
+// planner of a kernel above 48 KB calls this for every launch it plans (lds_limit.hpp).
 fk_status raise_dynamic_lds(const void* func, uint32_t bytes);
 
 #define FK_HIP(call)                                            \

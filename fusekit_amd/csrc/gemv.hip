@@ -66,8 +66,7 @@ uint32_t blocks_per_cu(const void* func, uint32_t lds_bytes) {
     auto key = std::make_pair(func, lds_bytes);
     auto it = cache.find(key);
     if (it == cache.end()) {
-        if (lds_bytes > 48 * 1024)
-            (void)hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+        (void)raise_dynamic_lds(func, lds_bytes);
         int per_cu = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, func, kGemvBlock, lds_bytes) != hipSuccess || per_cu < 1)
             per_cu = 1;
@@ -230,8 +229,7 @@ fk_status plan_gemv(const GemvRequest& rq, Launch* out) {
             out->add_lead(a.x);
             out->add_lead(a.norm_w);
             out->add_lead(a.K);
-            if (lds > 48 * 1024) FK_HIP(hipFuncSetAttribute(out->func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            return FK_OK;
+            return raise_dynamic_lds(out->func, lds);
         }
     }
     if (rq.argmax) return set_error(FK_ERR_UNSUPPORTED, "gemv: head argmax needs a shape the row-group form takes");
@@ -313,8 +311,6 @@ fk_status plan_gemv(const GemvRequest& rq, Launch* out) {
             best_blocks = (uint32_t)(tiles < cap ? tiles : cap);
         }
         if ((int)lds_for(best_r) > dev->max_dyn_lds) return set_error(FK_ERR_UNSUPPORTED, "gemv: K too large for LDS staging");
-        if (lds_for(best_r) > 48 * 1024)
-            FK_HIP(hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_for(best_r)));
         tiling = key;
         tiling.rows = best_r;
         tiling.blocks = best_blocks;
@@ -367,7 +363,7 @@ fk_status plan_gemv(const GemvRequest& rq, Launch* out) {
     out->add_lead(a.x);
     out->add_lead(a.norm_w);
     out->add_lead(a.K);
-    return FK_OK;
+    return raise_dynamic_lds(func, lds);
 }
 
 }  // namespace fk

@@ -690,7 +690,7 @@ uint32_t qgemm_resident(const DeviceFacts* dev, uint32_t bits, int mt) {
     if (slot == 0) {
         const void* f = qgemm_func(bits, mt);
         const uint32_t lds = qgemm_form_lds_bytes(mt);
-        if (lds > 48 * 1024) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        (void)raise_dynamic_lds(f, lds);
         int per_cu = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, mt == 8 ? kTileBlock : kQgemmBlock, lds) != hipSuccess || per_cu < 1) per_cu = 1;
         if (mt == 8) per_cu = 1;         // the tile form: one block (two LDS buffers, 128 accumulator registers per lane) per CU
@@ -774,9 +774,7 @@ fk_status plan_qgemm_main(const DeviceFacts* dev, const fk_weight* W, const uint
     out->block = dim3(shape->mt == 8 ? kTileBlock : kQgemmBlock, 1, 1);
     out->shmem = qgemm_form_lds_bytes(shape->form(false));
     out->set_args(a);
-    if (out->shmem > 48 * 1024)
-        FK_HIP(hipFuncSetAttribute(out->func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)out->shmem));
-    return FK_OK;
+    return raise_dynamic_lds(out->func, out->shmem);
 }
 
 void plan_reduce(const float* p0, const float* p1, const uint16_t* bias, const uint16_t* res, uint16_t* y, uint32_t M,
@@ -960,7 +958,7 @@ fk_status plan_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const ui
     main->block = dim3(kTileBlock, 1, 1);
     main->shmem = qgemm_form_lds_bytes(s.form(false));
     main->set_args(a);
-    FK_HIP(hipFuncSetAttribute(main->func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)main->shmem));
+    FK_TRY(raise_dynamic_lds(main->func, main->shmem));
     *reduce = Launch();
     if (s.ksplit > 1) {
         r.p = a.partial;
@@ -1014,7 +1012,7 @@ fk_status plan_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint
         gate->func = qgemm_func(Wg->bits, s.form(true));
         gate->shmem = qgemm_form_lds_bytes(s.form(true));
         gate->set_args(a);
-        FK_HIP(hipFuncSetAttribute(gate->func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gate->shmem));
+        FK_TRY(raise_dynamic_lds(gate->func, gate->shmem));
         *up = Launch();
         if (s.ksplit == 1)
             *reduce = Launch();

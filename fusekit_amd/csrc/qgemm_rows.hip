@@ -480,8 +480,7 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
     out->block = dim3(waves * kWave, 1, 1);
     out->shmem = rows_lds_bytes(mt, rq.pair || two ? 2u : 1u, waves);
     out->set_args(a);
-    if (out->shmem > 48 * 1024) FK_TRY(raise_dynamic_lds(out->func, out->shmem));
-    return FK_OK;
+    return raise_dynamic_lds(out->func, out->shmem);
 }
 
 }  // namespace fk

@@ -371,8 +371,7 @@ uint32_t resident_blocks(const void* func, uint32_t lds_bytes, int cus) {
     auto key = std::make_pair(func, lds_bytes);
     auto it = cache.find(key);
     if (it == cache.end()) {
-        if (lds_bytes > 48 * 1024)
-            (void)hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+        (void)raise_dynamic_lds(func, lds_bytes);
         int per_cu = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, func, kGemvBlock, lds_bytes) != hipSuccess || per_cu < 1)
             per_cu = 1;
@@ -485,9 +484,7 @@ fk_status plan_routed_gemv(const uint16_t* x, uint32_t n_x_rows, const fk_weight
     out->block = dim3(kGemvBlock, 1, 1);
     out->shmem = base.shmem;
     out->set_args(a);
-    if (base.shmem > 48 * 1024)
-        FK_HIP(hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)base.shmem));
-    return FK_OK;
+    return raise_dynamic_lds(func, base.shmem);
 }
 
 fk_status plan_route_reduce(const uint16_t* parts, const uint16_t* route_weight, const uint16_t* residual,
@@ -574,9 +571,7 @@ fk_status plan_routed_reduce_chain(const uint16_t* h, uint32_t n_h_rows, const f
         out->block = dim3(kDrBlock, 1, 1);
         out->shmem = (uint32_t)lds;
         out->set_args(a);
-        if (lds > 48 * 1024)
-            FK_HIP(hipFuncSetAttribute(out->func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        return FK_OK;
+        return raise_dynamic_lds(out->func, (uint32_t)lds);
     }
     if (!parts) return set_error(FK_ERR_INVALID, "routed reduce: workspace required");
     FK_TRY(plan_routed_gemv(h, n_h_rows, Wd, nullptr, n_experts, row_idx, expert_idx, nullptr, n_routes, parts, out, nullptr,

@@ -808,7 +808,7 @@ fk_status plan_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const ui
     l->block = dim3(kPrefillBlock, 1, 1);
     l->shmem = split ? prefill_dma_lds_bytes(head_dim, split) : rows_per_block > kPrefillRows ? prefill_tile_lds_bytes(head_dim) : prefill_lds_bytes(head_dim);
     if ((int)l->shmem > dev->max_dyn_lds) return set_error(FK_ERR_UNSUPPORTED, "sdpa_prefill: LDS tile does not fit");
-    if (l->shmem > 48 * 1024) FK_HIP(hipFuncSetAttribute(l->func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l->shmem));
+    FK_TRY(raise_dynamic_lds(l->func, l->shmem));
     l->set_args(a);
     return FK_OK;
 }

@@ -700,8 +700,7 @@ inline fk_status set_lds_limit(const void* func, uint32_t lds) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
     if ((int)lds > dev->max_dyn_lds) return set_error(FK_ERR_UNSUPPORTED, "xcd layer: LDS need exceeds the CU");
-    if (lds > 48 * 1024) FK_HIP(hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    return FK_OK;
+    return raise_dynamic_lds(func, lds);
 }
 
 // Both launches need their 512 workgroups resident TOGETHER, two per CU: a block that has not started cannot publish
@@ -717,7 +716,7 @@ inline fk_status require_two_blocks_per_cu(const void* func, uint32_t lds, const
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
     if ((int)lds > dev->max_dyn_lds) return set_error(FK_ERR_UNSUPPORTED, "xcd layer: LDS need exceeds the CU");
-    if (lds > 48 * 1024) FK_HIP(hipFuncSetAttribute(func, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    FK_TRY(raise_dynamic_lds(func, lds));
     int per_cu = 0;
     FK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, func, kBlock, lds));
     if ((long long)per_cu * dev->cus < (long long)kXcdGrid)

@@ -228,3 +228,13 @@ def test_prompt_with_norm_weights_at_any_address(fk):
     other = DecoderRuntime(cfg, W)
     other.prefill_rows(prompt)
     assert rel_l2(other.logits.to_numpy(np.uint16), want) <= 2e-2   # (the norm in a launch of its own: sums in another order)
+
+
+@pytest.mark.parametrize("bits", [4, 16])
+def test_two_shapes_of_one_kernel_beyond_48_kilobytes_in_turn(fk, bits):
+    """Each launch is allowed the LDS it needs, whichever shape was planned before it."""
+    kept = [(W := make_qweight(90 + i, 40, k, bits), to_device(fk, W), normal_bf16(91 + i, k), fk.DeviceBuffer(80))
+            for i, k in enumerate((40960, 25600, 32768))]
+    for W, dW, x, y in kept + kept[:2] + kept[::-1]:
+        fk.qgemv(dW, fk.DeviceBuffer.from_numpy(x), None, y)
+        assert rel_l2(y.to_numpy(np.uint16), oracle.linear_acc(W, x)) <= 5e-3
