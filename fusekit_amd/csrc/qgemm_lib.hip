@@ -49,10 +49,12 @@ struct RocblasApi {
     std::mutex mu;  // one handle, one stream binding at a time
 };
 RocblasApi g_rb;
-// row count from which direct calls take this route (0: never): below it the fused kernel's tile form is the faster
-// one on the 4B-class projections (passes of 256 / 512 / 768 rows: +16 / +3..9 / +7 % prompt rate), from 1024 rows this route
-constexpr uint32_t kLibraryRowsDefault = 1024;
-uint32_t g_library_rows = kLibraryRowsDefault;
+// Row count from which direct calls take this route (0: never; FK_GEMM_LIBRARY_ROWS_DEFAULT: the choice below).  Single matrices
+// from 1024 rows: below, the fused kernel is the faster one on the 4B-class projections (passes of 256 / 512 / 768 rows:
+// +16 / +3..9 / +7 % prompt rate).  A gate / up pair that qgemm_dma.hip takes, never: 4096 rows of 9728 x 2560 take two
+// dequantisations, two library products and the SwiGLU kernel 489 us, its one launch 375.
+constexpr uint32_t kLibraryRows = 1024;
+uint32_t g_library_rows = FK_GEMM_LIBRARY_ROWS_DEFAULT;
 
 bool rocblas_ready() {
     if (g_rb.tried) return g_rb.ok;
@@ -221,10 +223,10 @@ fk_status run_dequantize_bf16(const fk_weight* W, uint16_t* out, hipStream_t s) 
 
 void set_gemm_library_rows(uint32_t rows) { g_library_rows = rows; }
 
-// (a gate / up pair only where a caller has set the threshold: 4096 rows of 9728 x 2560, both matrices dequantised, two library
-// products and the SwiGLU kernel 489 us, qgemm_dma.hip's one launch 393)
 bool qgemm_takes_library(uint32_t m, bool pair) {
-    if (g_library_rows == 0 || m < g_library_rows || (pair && g_library_rows == kLibraryRowsDefault)) return false;
+    const bool own = g_library_rows == FK_GEMM_LIBRARY_ROWS_DEFAULT;
+    const uint32_t rows = own ? (pair ? 0u : kLibraryRows) : g_library_rows;
+    if (rows == 0 || m < rows) return false;
     std::lock_guard<std::mutex> lk(g_rb.mu);
     return rocblas_ready();
 }

@@ -538,7 +538,7 @@ def dequantize_bf16(W: DeviceWeight, stream=None) -> DeviceWeight:
     return D
 
 
-GEMM_LIBRARY_ROWS_DEFAULT = 1024  # fk_set_gemm_library_rows' default
+GEMM_LIBRARY_ROWS_DEFAULT = 0xFFFFFFFF  # the library's own choice (from 1024 rows, pairs as include/fusekit_hip.h says)
 
 
 def set_gemm_library_rows(rows: int):

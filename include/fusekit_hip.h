@@ -844,9 +844,13 @@ fk_status fk_set_gemv_policy(uint32_t rows_per_tile, uint32_t grid_blocks);
 int fk_gemv_form(uint32_t n, uint32_t k, uint32_t bits, uint32_t group);
 fk_status fk_set_gemv_flat_only(int flat_only);
 /* Row count from which fk_qgemm / fk_qgemm_swiglu dequantise the matrix to bf16 once and hand the
- * product to rocBLAS (opened on first use; absent: the fused kernel is kept).  Default 1024 (below it the fused
- * kernel's LDS-tiled form is the faster one on the benchmark model's projections); 0 = never.
+ * product to rocBLAS (opened on first use; absent: the fused kernel is kept); 0 = never.  A count that is set holds for single
+ * matrices and gate / up pairs alike.  FK_GEMM_LIBRARY_ROWS_DEFAULT, what a process starts with and what restores it, is the
+ * library's own choice: single matrices from 1024 rows (below, the fused kernel is the faster one on the benchmark model's
+ * projections), pairs only where the fused launch does not take them (group 128, K below 768 or no multiple of 128, N no
+ * multiple of 4): where it does, it is the faster one at every row count.
  * Set it BEFORE sizing workspaces: fk_qgemm_workspace_bytes covers the route that will be taken. */
+#define FK_GEMM_LIBRARY_ROWS_DEFAULT 0xffffffffu
 fk_status fk_set_gemm_library_rows(uint32_t rows);
 /* Up to 64 activation rows run fk_qgemm / fk_qgemm_swiglu / fk_qgemm_fanout as ONE launch that streams the weights
  * once for all rows and includes the epilogue (the reference's small-M kernels: src/codegen/msl.rs:462-546,

@@ -238,3 +238,22 @@ def test_two_shapes_of_one_kernel_beyond_48_kilobytes_in_turn(fk, bits):
     for W, dW, x, y in kept + kept[:2] + kept[::-1]:
         fk.qgemv(dW, fk.DeviceBuffer.from_numpy(x), None, y)
         assert rel_l2(y.to_numpy(np.uint16), oracle.linear_acc(W, x)) <= 5e-3
+
+
+def test_a_library_threshold_that_is_set_holds_for_pairs(fk):
+    """Every count that a caller sets, 1024 among them, sends pairs from there on to the library route; the default never does."""
+    m, hidden, inter = 1024, 896, 1216
+    Wg, Wu = make_qweight(76, inter, hidden, 4), make_qweight(77, inter, hidden, 4)
+    x, dg, du = fk.DeviceBuffer.from_numpy(normal_bf16(78, (m, hidden))), to_device(fk, Wg), to_device(fk, Wu)
+    def run(rows):
+        fk.set_gemm_library_rows(rows)
+        out, ws = fk.DeviceBuffer(2 * m * inter), fk.DeviceBuffer(2 * fk.qgemm_workspace_bytes(m, inter, hidden, 64))
+        fk.qgemm_swiglu(dg, du, x, m, 1, out, ws)
+        return out.to_numpy(np.uint16)
+    try:
+        fused, library = run(0), run(1023)
+        assert not np.array_equal(fused, library)   # (sums in another order: how the routes are told apart)
+        assert np.array_equal(run(1024), library) and np.array_equal(run(1025), fused)
+    finally:
+        default = run(fk.GEMM_LIBRARY_ROWS_DEFAULT)
+    assert np.array_equal(default, fused)
