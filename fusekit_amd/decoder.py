@@ -13,6 +13,7 @@ back on the GPU.
 from __future__ import annotations
 
 import ctypes as C
+import operator
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence
 
@@ -185,6 +186,14 @@ class DecoderWeights:
         return sum(m.nbytes for m in self.mats.values()) + sum(v.nbytes for v in self.vecs.values())
 
 
+# the device buffers inside a matrix and a quantised cache; the fields of native.PromptModel that come from the configuration
+_matrix_buffers = operator.attrgetter("w", "scales", "biases")
+_cache_buffers = operator.attrgetter("packed", "scales", "biases")
+_PROMPT_SCALARS = ("n_layers", "hidden", "n_heads", "n_kv", "head_dim", "inter", "vocab", "capacity", "eps", "theta", "embed_scale",
+                   "swiglu_variant", "kv_bits", "kv_group")
+_prompt_scalars = operator.attrgetter(*_PROMPT_SCALARS)
+
+
 class DecoderRuntime:
     """Scratch arena, KV caches, uniforms and the captured decode graph of one model."""
 
@@ -244,6 +253,10 @@ class DecoderRuntime:
                         self.xcd_kmeta[name] = (native.xcd_kslice_meta(W.scales, W.n, W.k // W.group),
                                                 native.xcd_kslice_meta(W.biases, W.n, W.k // W.group))
         self._bf16_weights: Dict[str, DeviceWeight] = {}   # resident bf16 copies for prompt passes (prefill_rows)
+        self._bf16_sources: Dict[str, DeviceBuffer] = {}   # the codes that each was made from
+        self._prompt_held: list = []                       # what the kept prompt models are made from
+        self._prompt_buffers: list = []                    # and the buffers of its matrices
+        self._prompt_assigned = -1                         # DeviceWeight.assigned when the last of them was made
         self.tasks = self.build_tasks()
         # persistent: the same task list, run by one whole-token kernel per replay
         self.graph = (self.d.build_decode_graph(self.tasks, True, spin_limit) if persistent
@@ -473,6 +486,10 @@ class DecoderRuntime:
                 self._rows["kdq"] = DeviceBuffer(c.n_kv * c.capacity * c.head_dim * 2)
                 self._rows["vdq"] = DeviceBuffer(c.n_kv * c.capacity * c.head_dim * 2)
             self._prompt_models = {}
+        held = self._prompt_sources()
+        if held != self._prompt_held or DeviceWeight.assigned != self._prompt_assigned:   # something was replaced since the last prompt
+            self._prompt_models, self._prompt_held = {}, held
+            self._prompt_buffers = [*map(_matrix_buffers, self.w.mats.values())]
         # passes of at least 256 rows with the resident bf16 copies, the others with the quantised matrices
         copies = bool(keep_bf16_weights and c.bits != 16 and native.gemm_library_available())
         first = next((i for i in range(0, len(prompt), R) if copies and min(R, len(prompt) - i) < 256), len(prompt)) if copies else 0
@@ -482,6 +499,14 @@ class DecoderRuntime:
         if first < len(prompt):
             nxt = native.prompt_run(self._prompt_model(False), prompt[first:], start_offset + first, R)
         return nxt
+
+    def _prompt_sources(self) -> list:
+        """What a prompt model is made from: the matrices, vectors and caches, the few other buffers it writes, the configuration.
+        It holds their addresses, so it is kept as long as these are the same objects (and no matrix has been given another buffer),
+        and they live as long as it is kept."""
+        caches = [*self.cache_k, *self.cache_v]
+        return [_prompt_scalars(self.cfg), self.logits, self.token, self.argmax_ws, self.step_counter, *self.w.mats.values(),
+                *self.w.vecs.values(), *caches, *(map(_cache_buffers, caches) if self.cfg.kv_bits else ())]
 
     def _prompt_model(self, copies: bool) -> "native.PromptModel":
         """The model as fk_prompt_run takes it, over the row buffers of the present size."""
@@ -493,8 +518,8 @@ class DecoderRuntime:
             W = w.mats[name]
             if not copies:
                 return W.c
-            if name not in self._bf16_weights:
-                self._bf16_weights[name] = native.dequantize_bf16(W)
+            if self._bf16_sources.get(name) is not W.w:
+                self._bf16_weights[name], self._bf16_sources[name] = native.dequantize_bf16(W), W.w
             return self._bf16_weights[name].c
 
         layers = (native.PromptLayer * c.n_layers)()
@@ -515,16 +540,15 @@ class DecoderRuntime:
         emb = w.mats["embed_tokens"]
         m = native.PromptModel()
         m.embed, m.head, m.final_norm, m.layers = emb.c, w.mats.get("lm_head", emb).c, w.vecs["final_norm"].ptr, layers
-        for n in ("n_layers", "hidden", "n_heads", "n_kv", "head_dim", "inter", "vocab", "capacity", "eps", "theta", "embed_scale",
-                  "swiglu_variant", "kv_bits", "kv_group"):
-            setattr(m, n, getattr(c, n))
         for field, name in (("tokens", "tok"), ("x", "x"), ("x2", "x2"), ("xn", "xn"), ("q", "q"), ("k", "k"), ("v", "v"), ("att", "att"),
                             ("mid", "mid"), ("workspace", "ws"), ("rope_tab", "rope"), ("partials", "part"), ("counters", "cnt"),
                             ("k_rows", "kdq"), ("v_rows", "vdq")):
             if name in b:
                 setattr(m, field, b[name].ptr)
         m.logits, m.token, m.argmax_workspace, m.step_counter = self.logits.ptr, self.token.ptr, self.argmax_ws.ptr, self.step_counter.ptr
-        self._prompt_models[copies] = m
+        for n, v in zip(_PROMPT_SCALARS, _prompt_scalars(c)):
+            setattr(m, n, v)
+        self._prompt_models[copies], self._prompt_assigned = m, DeviceWeight.assigned
         return m
 
     def generate(self, prompt: Sequence[int], max_tokens: int):

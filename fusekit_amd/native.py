@@ -152,6 +152,13 @@ class DeviceBuffer:
 class DeviceWeight:
     """A weight matrix resident in HBM (packed + scales + biases, or dense bf16)."""
 
+    assigned = 0   # how often a buffer of any matrix has been assigned: unchanged, no matrix has been given another buffer
+
+    def __setattr__(self, name: str, value) -> None:
+        object.__setattr__(self, name, value)
+        if name in ("w", "scales", "biases"):
+            DeviceWeight.assigned += 1
+
     def __init__(self, w: np.ndarray, scales, biases, n: int, k: int, bits: int, group: int = 64):
         self.n, self.k, self.bits, self.group = int(n), int(k), int(bits), int(group)
         self.w = DeviceBuffer.from_numpy(w)
