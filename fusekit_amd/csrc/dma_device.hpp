@@ -20,15 +20,19 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // 16 (4) bytes per lane from `base + off` (`ptr`) to LDS at `to` + 16 (4) * lane; counted in vmcnt.  As statements the
-// compiler does not look into: its own form waits for every such load in flight ahead of each LDS read.
+// compiler does not look into: its own form waits for every such load in flight ahead of each LDS read.  m0, which the
+// statement writes, is an output (the compiler refuses it as a clobber).
 __device__ __forceinline__ void dma16(uint32_t to, uint32_t off, const void* base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory");
+    uint32_t m0;
+    asm volatile("s_mov_b32 %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" : "=&{m0}"(m0) : "s"(to), "v"(off), "s"(base) : "memory");
 }
 __device__ __forceinline__ void dma16(uint32_t to, const unsigned char* ptr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(ptr) : "memory");
+    uint32_t m0;
+    asm volatile("s_mov_b32 %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off" : "=&{m0}"(m0) : "s"(to), "v"(ptr) : "memory");
 }
 __device__ __forceinline__ void dma4(uint32_t to, const unsigned char* ptr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(to), "v"(ptr) : "memory");
+    uint32_t m0;
+    asm volatile("s_mov_b32 %0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, off" : "=&{m0}"(m0) : "s"(to), "v"(ptr) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() {

@@ -143,3 +143,11 @@ def test_expert_and_low_rank_attention_launch_admission_rules_need_no_device():
     assert mla(2048, 16, 512, 64, 128, 128, 1024, 8, 64) == fk.FK_ERR_UNSUPPORTED and b"4-bit" in fk.lib.fk_last_error()
     assert mla(2048, 16, 448, 64, 128, 128, 1024, 4, 64) == fk.FK_ERR_UNSUPPORTED and b"latent" in fk.lib.fk_last_error()
     assert fk.xcd_moe_scratch_bytes(1408) == 8 * 64 * 4 + 8 * 1408 * 2
+
+
+def test_asm_statements_declare_the_m0_they_write():
+    """m0 is the compiler's register too: a statement that sets it names it among its outputs ("{m0}") instead of in its text."""
+    sources = [os.path.join(ROOT, "fusekit_amd", "csrc", f) for f in os.listdir(os.path.join(ROOT, "fusekit_amd", "csrc")) if f.endswith((".hip", ".hpp"))]
+    for path in sources:
+        for statement in re.findall(r"\basm\b[^;]*;", open(path).read(), flags=re.S):
+            assert not re.search(r"\bm0\b", re.sub(r'"=&\{m0\}"\(m0\)', "", statement)), (path, statement)
