@@ -93,7 +93,7 @@ fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uin
                     void* workspace, bool kept_order, hipStream_t s) {
     if (W && W->bits == 16) {  // dense bf16 weights: the plain library GEMM with this library's epilogue
         if (!x || !y || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm: null activation, output or workspace");
-        if (qgemm_takes_rows(m, 16, 0, W->k)) {
+        if (qgemm_takes_rows(m, 16, 0, W->k) && (g_rows_form || !gemm_library_available())) {
             RowsRequest rq;
             rq.W[0] = W; rq.x = x; rq.M = m; rq.bias[0] = bias; rq.res = residual; rq.y[0] = y;
             Launch l;
@@ -152,7 +152,7 @@ fk_status run_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint1
         if (!x || !out || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: null activation, output or workspace");
         if (Wg->n != Wu->n || Wg->k != Wu->k) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: gate and up need the same shape");
         if (variant < 0 || variant > 2) return set_error(FK_ERR_INVALID, "fk_qgemm_swiglu: variant must be 0, 1 or 2");
-        if (qgemm_takes_rows(m, 16, 0, Wg->k)) {
+        if (qgemm_takes_rows(m, 16, 0, Wg->k) && (g_rows_form || !gemm_library_available())) {
             RowsRequest rq;
             rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true; rq.x = x; rq.M = m; rq.variant = variant; rq.y[0] = out;
             Launch l;
@@ -311,7 +311,7 @@ fk_status fk_event_elapsed_ms(fk_event start, fk_event stop, float* ms) {
 }
 
 fk_status fk_set_qgemm_wide(int enabled) {
-    (void)enabled;   // one form serves these row counts
+    g_rows_form = enabled != 0;
     return FK_OK;
 }
 

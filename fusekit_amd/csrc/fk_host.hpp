@@ -203,6 +203,9 @@ struct RowsRequest {
     uint16_t* y[3] = {nullptr, nullptr, nullptr};
     uint32_t y_stride[3] = {0, 0, 0};  // 0: the matrix's N
 };
+// fk_set_qgemm_wide: whether fk_qgemm, _swiglu and _fanout (and the task families) take it; else the routes that passes into a
+// quantised cache keep (split k and a second kernel; dense bf16: the library)
+extern bool g_rows_form;
 inline uint32_t rows_ssq_parts(uint32_t n) { return (n + 15u) / 16u; }
 bool qgemm_takes_rows(uint32_t M, uint32_t bits, uint32_t group, uint32_t K);
 fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out);

@@ -793,6 +793,8 @@ void plan_reduce(const float* p0, const float* p1, const uint16_t* bias, const u
 
 }  // namespace
 
+bool g_rows_form = true;
+
 // the epilogue of a product whose fp32 sums are complete (the library route)
 void plan_qgemm_epilogue(const float* p0, const float* p1, const uint16_t* bias, const uint16_t* res, uint16_t* y,
                          uint32_t M, uint32_t N, uint32_t ksplit, int variant, Launch* out) {
@@ -858,7 +860,7 @@ fk_status plan_qgemm(const fk_weight* W, const uint16_t* x, uint32_t M, const ui
     FK_TRY(device_facts(&dev));
     FK_TRY(check_weight(W, "qgemm"));
     if (!x || !y || !workspace) return set_error(FK_ERR_INVALID, "qgemm: null activation, output or workspace");
-    if (!split_k && qgemm_takes_rows(M, W->bits, W->group, W->k)) {  // up to 64 rows: one launch, no split-k sums (reduce stays empty)
+    if (!split_k && g_rows_form && qgemm_takes_rows(M, W->bits, W->group, W->k)) {  // up to 64 rows: one launch, no split-k sums (reduce stays empty)
         RowsRequest rq;
         rq.W[0] = W; rq.x = x; rq.M = M; rq.bias[0] = bias; rq.res = res; rq.y[0] = y;
         *reduce = Launch();
@@ -894,7 +896,7 @@ fk_status plan_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const ui
         if (W[i]->k != W[0]->k || W[i]->bits != W[0]->bits || W[i]->group != W[0]->group)
             return set_error(FK_ERR_INVALID, "qgemm fan-out: the matrices need the same K, bits and group size");
     }
-    if (qgemm_takes_rows(M, W[0]->bits, W[0]->group, W[0]->k)) {   // up to 64 rows
+    if (g_rows_form && qgemm_takes_rows(M, W[0]->bits, W[0]->group, W[0]->k)) {   // up to 64 rows
         *fused = true;
         *reduce = Launch();
         RowsRequest rq;
@@ -986,7 +988,7 @@ fk_status plan_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint
         return set_error(FK_ERR_INVALID, "qgemm_swiglu: gate and up need the same shape and group size");
     if (variant < 0 || variant > 2) return set_error(FK_ERR_INVALID, "qgemm_swiglu: variant must be 0, 1 or 2");
     if (!x || !out || !workspace) return set_error(FK_ERR_INVALID, "qgemm_swiglu: null activation, output or workspace");
-    if (!split_k && Wg->bits == Wu->bits && qgemm_takes_rows(M, Wg->bits, Wg->group, Wg->k)) {  // gate, up and SwiGLU in one launch
+    if (!split_k && g_rows_form && Wg->bits == Wu->bits && qgemm_takes_rows(M, Wg->bits, Wg->group, Wg->k)) {  // gate, up and SwiGLU in one launch
         RowsRequest rq;
         rq.W[0] = Wg; rq.W[1] = Wu; rq.n_mats = 2; rq.pair = true; rq.x = x; rq.M = M; rq.variant = variant; rq.y[0] = out;
         *up = Launch();

@@ -854,8 +854,10 @@ fk_status fk_set_gemv_flat_only(int flat_only);
 fk_status fk_set_gemm_library_rows(uint32_t rows);
 /* Up to 64 activation rows run fk_qgemm / fk_qgemm_swiglu / fk_qgemm_fanout as ONE launch that streams the weights
  * once for all rows and includes the epilogue (the reference's small-M kernels: src/codegen/msl.rs:462-546,
- * :1307-1485, policy src/codegen/kernels/mod.rs:164-186).  fk_set_qgemm_wide is accepted and changes nothing: it chose
- * between two forms of 2..10 rows, of which one is left. */
+ * :1307-1485, policy src/codegen/kernels/mod.rs:164-186).  fk_set_qgemm_wide(0) sends those row counts through
+ * the split-k kernel + reduction (dense bf16: the library GEMM where it is present) instead, the routes that prompt passes into
+ * a quantised cache keep (measurements, tests); 1 restores the default.  Process-wide; takes effect for launches planned
+ * afterwards. */
 fk_status fk_set_qgemm_wide(int enabled);
 /* An MLX-affine matrix (bits 4 / 8, group 64 / 128) as dense bf16 [n, k], every element T(code * scale + bias):
  * the values the library route of fk_qgemm multiplies with.  With 288 GB of HBM a runtime may keep the bf16 copy

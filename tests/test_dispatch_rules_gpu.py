@@ -257,3 +257,31 @@ def test_a_library_threshold_that_is_set_holds_for_pairs(fk):
     finally:
         default = run(fk.GEMM_LIBRARY_ROWS_DEFAULT)
     assert np.array_equal(default, fused)
+
+
+@pytest.mark.parametrize("bits,group", [(4, 64), (8, 128), (16, 0)])
+@pytest.mark.parametrize("m", [1, 12, 33, 64])
+def test_up_to_64_rows_by_the_routes_of_quantised_caches(fk, bits, group, m):
+    """Split k and a second kernel (dense bf16: the library), one matrix, a pair and a fan-out: another kernel, the same values."""
+    k, n = 2560, 320
+    Ws = [make_qweight(70 + i, n, k, bits, group=group or 64) for i in range(3)]
+    x, bias, res = normal_bf16(73, (m, k)), normal_bf16(74, n), normal_bf16(75, (m, n))
+    dW, up = [to_device(fk, W) for W in Ws], fk.DeviceBuffer.from_numpy
+    def run(wide):
+        ws, ys = fk.DeviceBuffer(2 * fk.qgemm_workspace_bytes(m, 3 * n, k, group)), [fk.DeviceBuffer(2 * m * n) for _ in range(5)]
+        fk.set_qgemm_wide(wide)
+        try:
+            fk.qgemm(dW[0], up(x), m, up(bias), up(res), ys[0], ws)
+            fk.qgemm_swiglu(dW[0], dW[1], up(x), m, 1, ys[1], ws)
+            fk.qgemm_fanout(dW, up(x), m, [None, up(bias), None], ys[2:], ws)
+        finally:
+            fk.set_qgemm_wide(True)
+        return [y.to_numpy(np.uint16, (m, n)) for y in ys]
+    one, other = run(True), run(False)
+    # sums in another order are how the kernels are told apart (a bf16 result flips about once in a thousand)
+    assert m == 1 or any(not np.array_equal(a, b) for a, b in zip(one, other))
+    acc = [np.stack([oracle.linear_acc(W, r) for r in x]).astype(np.float64) for W in Ws]
+    b, r = oracle.bf16_to_f32(bias).astype(np.float64), oracle.bf16_to_f32(res).astype(np.float64)
+    g, u = (oracle.bf16_to_f32(oracle.f32_to_bf16(a.astype(np.float32))).astype(np.float64) for a in acc[:2])
+    for a, o, want in zip(one, other, (acc[0] + b + r, g / (1 + np.exp(-g)) * u, acc[0], acc[1] + b, acc[2])):
+        assert rel_l2(a, want) <= 4e-3 and rel_l2(o, want) <= 4e-3
