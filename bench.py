@@ -24,7 +24,7 @@ Prints ONE JSON line: value = generated tokens/s (wall clock around the K timed 
                   launch, three sets in rotation): the steady streaming rate of the int4 qGEMV,
   hbm_read_ceiling -- a plain read-and-XOR kernel over 1 GiB buffers: what a read-only kernel gets from
                   HBM on this device, the bound the GEMV figures are also stated against,
-  qgemm_rows   -- the multi-row matmul of the prompt path (9728 x 2560 int4 as a graph node, 512 and 2048
+  qgemm_rows   -- the multi-row matmul of the prefill variants (9728 x 2560 int4 as a graph node, 512 and 2048
                   activation rows): TFLOP/s and fraction of the dense bf16 MFMA peak,
   moe_cfg5_decode -- configs[4]'s mixture-of-experts decoder: tokens/s of its decode loop,
   cpu_baseline -- the CPU oracle (C restatement of the reference semantics) decoding the same
@@ -340,7 +340,7 @@ def main() -> int:
             out["qgemv_steady"]["median_frac_of_read_ceiling"] = round(out["qgemv_steady"]["median_GBps"] / out["hbm_read_ceiling"]["GBps"], 4)
         del bufs
 
-        # ---- the multi-row matmul on the matrix cores (the prompt path's projection: 9728 x 2560 int4 g64 as a graph
+        # ---- the multi-row matmul on the matrix cores (a prefill variant's projection: 9728 x 2560 int4 g64 as a graph
         # node, 512 and 2048 activation rows), against the dense bf16 MFMA peak ----
         from fusekit_amd.kernel_bench import measure_qgemm
         out["qgemm_rows"] = {}

@@ -29,10 +29,14 @@ fk_status run_rows(const RowsRequest& rq, hipStream_t s) {
     return run_launch(l, s);
 }
 
-// Passes into a QUANTISED cache keep the summation orders such caches have been filled with: a key that differs in its last
-// bit can turn the sign of its group's scale (MLX's rule takes it from the end of the range that is larger in magnitude) and
-// shift the group's codes, and a cache is kept and compared for longer than a pass.  So, up to 64 rows: split-k sums, the
-// library GEMM for dense bf16 weights; beyond, the tiles of qgemm.hip and the library (`kept` of run_qgemm); and the strided norm.
+// Passes into a QUANTISED cache keep older kernels, whose sums are added in another order than those of the forms above: a key
+// that differs in its last bit can turn the sign of its group's scale (MLX's rule takes it from the end of the range that is
+// larger in magnitude) and shift the group's codes, so the same prompt would fill a cache with other bytes than before.  From 11
+// rows: split-k sums up to 64 rows (dense bf16 weights: the library GEMM), beyond, the tiles of qgemm.hip and the library
+// (kept_order of run_qgemm); at any row count the norm in a launch of its own, strided, and the older attention.  Passes of up to
+// 10 rows take the one-launch matmul (what they took before is gone), so it is longer passes only that fill a cache with the
+// bytes they always did.  The same prompt token by token differs in such bits either way.  What the newer kernels would give
+// these passes has not been measured.
 fk_status norm_rows(const fk_prompt_model& m, const uint16_t* x, const uint16_t* w, uint32_t rows, hipStream_t s) {
     Launch l;
     FK_TRY(plan_rmsnorm_rows(x, w, m.eps, rows, m.hidden, m.xn, &l, m.kv_bits != 0));

@@ -2,7 +2,7 @@
 // matrix cores: the path for many activation rows (prefill), where the weight
 // stream must be read once for all rows.  Up to 64 rows run qgemm_rows.hip; of the
 // first kernel below the exact forms (MT = 1, 2) are left for what that one does not
-// take: a gate / up pair of unlike bits, and passes into a quantised cache (prompt.hip).
+// take: a gate / up pair of unlike bits, and passes into a quantised cache (prompt.hip); fk_set_qgemm_wide(0) reaches them.
 //
 // v_mfma_f32_32x32x16_bf16 with the WEIGHTS as the B operand: a lane then owns one
 // weight row n (output column) for all 16 accumulator registers, so the affine

@@ -1,7 +1,8 @@
 // Multi-row quantised matmul from 65 activation rows: tiles whose operands come straight from memory into LDS
 // (global_load_lds: no registers, no LDS stores, nothing for the vector ALU to do) and whose weights are dequantised in
 // registers by the wave that multiplies them, T(s q + b), the arithmetic of qgemm.hip's tiles.  Direct calls and prompt
-// passes; a task list keeps the launch shapes it was written with (qgemm.hip).
+// passes into a bf16 cache.  The task families fusekit_qgemm* plan qgemm.hip's tiles: their launch geometry (fk_plan_geometry:
+// blocks, LDS, one kernel or two) is part of what a task list's owner sees and is tested; they have not been moved here.
 //
 // What bounds it is how much other work goes with the matrix instructions.  One v_mfma_f32_16x16x32_bf16 takes 16 cycles and
 // hides two vector instructions of its wave, no more (measured: 18.5 cycles with one or two behind each, 22.5 with three, 28

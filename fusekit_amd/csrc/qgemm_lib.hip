@@ -5,10 +5,10 @@
 // plain bf16 x bf16 -> fp32 product to rocBLAS; the epilogue kernel of the split-k path then
 // applies bias / residual / SwiGLU to the fp32 sums and rounds once.
 //
-// From about 512 rows the matrix product itself dominates and a tuned library GEMM (≈ 0.9 PFLOP/s
-// at 512 x 9728 x 2560, 1.1 at 1024 rows) beats the fused kernel, whose weight fragments are
-// unpacked by every block that uses them (0.35 PFLOP/s).  Below that the int4 stream and the
-// launch count matter more and the fused kernel is used.  rocBLAS is opened with dlopen on first
+// From 1024 rows of a single matrix the dequantisation (one pass over the weights) is small beside the
+// product, which a tuned library GEMM runs at 1.1 PFLOP/s and more; below, the launch count and the
+// bf16 copy matter more and the fused kernel is used, as it is for gate / up pairs at every row count.
+// Dense bf16 weights take this route beyond 64 rows.  rocBLAS is opened with dlopen on first
 // use: the decode path never touches it, and a box without it keeps the fused kernel.
 // Only direct calls take this route (fk_qgemm, fk_qgemm_swiglu); the dispatch families
 // fusekit_qgemm* stay kernel nodes of a hipGraph.

@@ -772,8 +772,8 @@ fk_status plan_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const ui
     a.rows = rows; a.kv_len = kv_len; a.n_heads = n_heads; a.heads_per_kv = n_heads / n_kv; a.capacity = capacity;
     a.scale2 = scale * 1.4426950408889634f;
     // Four forms: a block per 32 rows whose waves split the positions; a block per 128 rows, or per 64 with the positions in
-    // halves, whose waves share the rows through LDS; and, where a caller needs the sums of earlier passes over the same rows
-    // (kept_order: a quantised cache rounds what follows from them), the older kernel of 128 rows.
+    // halves, whose waves share the rows through LDS; and, for passes into a quantised cache (kept_order: prompt.hip has the
+    // reason) and scales that are not positive (the newer forms scale inside the exponent), the older kernel of 128 rows.
     const uint64_t cus = (uint64_t)(dev->cus > 0 ? dev->cus : 1);
     auto blocks = [&](uint32_t rows_per_block) { return (uint64_t)n_heads * ((rows + rows_per_block - 1u) / rows_per_block); };
     uint32_t rows_per_block = kPrefillRows;
@@ -786,7 +786,10 @@ fk_status plan_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const ui
             rows_per_block = kPrefillWaves * kPrefillRows;
     } else if (head_dim == 128 || 2u * blocks(kPrefillRows) > cus) {
         // At head dimension 64, 32-row blocks while there are two CUs for each (14 heads, 200 rows at 1200 positions 12.9
-        // against 13.8 us; 512 rows 8.3 either way); at 128 the shared rows win from the first (100 rows at 3100 positions 50.4 -> 44.9).
+        // against 13.8 us; 512 rows 8.3 either way); at 128 the shared rows win from the first (100 rows at 3100 positions 49.3 -> 44.4
+        // over a cache that stays in the last-level cache).  The rule does not look at the context, where it is not always right: over
+        // caches that come from memory 100 rows at 1024 / 3100 positions take 19.8 -> 17.4 / 51.9 -> 56.7, and at head dimension 64 the
+        // 64-row blocks of 300..512 rows (14 heads) take 26.3 -> 32.6 at 3100.
         // 64-row blocks until 128-row ones fill the places that the former have, 1 a CU (2 at head dimension 64): 32 heads x 128,
         // 1024 rows 25.6 / 25.7 us, 1200 rows 35.6 / 31.7; 14 heads x 64, 4096 rows 49.8 / 70.2, 8192 rows 173 / 163.
         split = blocks(kPrefillWaves * kPrefillRows) > cus * (128u / head_dim) ? 1u : 2u;

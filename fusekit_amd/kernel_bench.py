@@ -236,8 +236,8 @@ def measure_qgemm(d, reps, rows, n=9728, k=2560, bits=4):
 def case_qgemm(d, reps, rows, n=9728, k=2560, bits=4):
     sec, nbytes, flops, pool = measure_qgemm(d, reps, rows, n, k, bits)
     _emit(f"qgemm_rows{rows}_{n}x{k}_q{bits}", sec, nbytes, flops=flops, pool=pool,
-          note="2..10 rows: one shared-stream launch; 11..64 rows: MFMA main + split-k reduction; from 65 rows the "
-               "LDS-tiled form (finished outputs at one k split)")
+          note="up to 64 rows: one launch, epilogue included; from 65 rows the LDS-tiled form that graph nodes run (finished "
+               "outputs at one k split)")
 
 
 def case_qgemm_swiglu(d, reps, rows, hidden=2560, inter=9728, bits=4):

@@ -65,10 +65,10 @@ def test_qgemm_matches_oracle(fk, m, n, k, bits):
         _check(got[r], ref[r], acc[r], W, x[r])
 
 
-# The shared-stream kernel for 2..10 activation rows (one launch, no split-k sums): every row count of its range,
-# the projections of the 4B-class decoder and of the mixture-of-experts model (K = 1408 ends in half a slab),
-# a ragged N, few weight rows with a long K (16 waves per block), bias and residual, and the split-k route on the
-# same operands (both keep the single-row arithmetic: rounding-edge flips only).
+# The one-launch form (no split-k sums) at 2..10 activation rows: the projections of the 4B-class decoder and of the
+# mixture-of-experts model (K = 1408 ends in half a slab), a ragged N, few weight rows with a long K (eight waves per
+# block), bias and residual, and the split-k route (fk_set_qgemm_wide(0)) on the same operands (both keep the
+# single-row arithmetic: rounding-edge flips only).
 WIDE_SHAPES = [(2, 2560, 2560), (3, 6144, 2560), (4, 333, 1408), (5, 2560, 9728), (6, 2048, 1408), (7, 1408, 2048),
                (8, 9728, 2560), (9, 70, 4096), (10, 2560, 4096),
                # K of one, three and five groups (a slab's second double group partly or wholly past the end), few rows
@@ -298,10 +298,10 @@ def test_qgemm_swiglu_tile_form_takes_the_pair_in_one_launch(fk, bits, m, hidden
 @pytest.mark.parametrize("m,k,ns,with_bias", [(512, 256, (4096, 1024, 1024), False),   # one k split: finished in the launch
                                               (300, 1024, (1000, 520, 260), True),     # ragged, k split, the fan-out's second kernel
                                               (512, 512, (2048, 1024), True),          # two matrices
-                                              (40, 256, (512, 256, 256), False)])      # too few rows for the tile form: one by one
+                                              (40, 256, (512, 256, 256), False)])      # up to 64 rows: one launch of the row form
 def test_qgemm_fanout_of_the_prompt_projections(fk, bits, m, k, ns, with_bias):
-    """fk_qgemm_fanout: up to three matrices over the same rows (q / k / v of a prompt pass) as one launch of the tile
-    form whose blocks run through the matrices in turn; every output against the oracle form of its row count."""
+    """fk_qgemm_fanout: up to three matrices over the same rows (q / k / v of a prompt pass) as one launch
+    whose blocks run through the matrices in turn; every output against the oracle form of its row count."""
     Ws = [make_qweight(110 + bits + 3 * i, n, k, bits) for i, n in enumerate(ns)]
     x = normal_bf16(120, (m, k))
     biases = [normal_bf16(121 + i, n) if (with_bias and i != 1) else None for i, n in enumerate(ns)]
