@@ -253,7 +253,7 @@ class DecoderRuntime:
                         self.xcd_kmeta[name] = (native.xcd_kslice_meta(W.scales, W.n, W.k // W.group),
                                                 native.xcd_kslice_meta(W.biases, W.n, W.k // W.group))
         self._bf16_weights: Dict[str, DeviceWeight] = {}   # resident bf16 copies for prompt passes (prefill_rows)
-        self._bf16_sources: Dict[str, DeviceBuffer] = {}   # the codes that each was made from
+        self._bf16_sources: Dict[str, tuple] = {}          # the buffers that each was made from
         self._prompt_held: list = []                       # what the kept prompt models are made from
         self._prompt_buffers: list = []                    # and the buffers of its matrices
         self._prompt_assigned = -1                         # DeviceWeight.assigned when the last of them was made
@@ -519,8 +519,8 @@ class DecoderRuntime:
             W = w.mats[name]
             if not copies:
                 return W.c
-            if self._bf16_sources.get(name) is not W.w:
-                self._bf16_weights[name], self._bf16_sources[name] = native.dequantize_bf16(W), W.w
+            if self._bf16_sources.get(name) != _matrix_buffers(W):
+                self._bf16_weights[name], self._bf16_sources[name] = native.dequantize_bf16(W), _matrix_buffers(W)
             return self._bf16_weights[name].c
 
         layers = (native.PromptLayer * c.n_layers)()

@@ -152,5 +152,6 @@ def test_a_replaced_matrix_gets_a_new_bf16_copy(monkeypatch):
     rt.prefill_rows(prompt, keep_bf16_weights=True)
     kept = dict(rt._bf16_weights)
     _replace_matrix(rt, cache)
+    _replace_codes(rt, cache)
     rt.prefill_rows(prompt, keep_bf16_weights=True)
-    assert [n for n in kept if rt._bf16_weights[n] is not kept[n]] == ["layers.1.self_attn.o_proj"]
+    assert sorted(n for n in kept if rt._bf16_weights[n] is not kept[n]) == ["layers.0.mlp.up_proj", "layers.1.self_attn.o_proj"]
