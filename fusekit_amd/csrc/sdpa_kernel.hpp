@@ -679,16 +679,20 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     FK_SDPA_STAMP(5);
 
     if constexpr (WAVES) {
-        // The waves meet: maxima through LDS, every wave rescales its sums to the block's
-        // maximum (exp(-inf) = 0 for a wave that saw no live key) and publishes its share of l.
+        // The waves meet: maxima and sums through LDS, every wave rescales its value sums to the block's
+        // maximum (exp(-inf) = 0 for a wave that saw no live key).
         float* wm = stat + 32;
         float* wl = stat + 64;
-        if (lane == 0) {
+        const float inv_lanes = 1.0f / (float)lpk;  // a row's sum is held by each of its lpk lanes (power of two: exact)
 #pragma unroll
-            for (int h = 0; h < GT; ++h) wm[wave * 8 + h] = m_run[h];
+        for (int h = 0; h < GT; ++h) {
+            const float lw = wave_sum(l_run[h]) * inv_lanes;
+            if (lane == 0) {
+                wm[wave * 8 + h] = m_run[h];
+                wl[wave * 8 + h] = lw;
+            }
         }
         __syncthreads();
-        const float inv_lanes = 1.0f / (float)lpk;  // a row's sum is held by each of its lpk lanes (power of two: exact)
 #pragma unroll
         for (int h = 0; h < GT; ++h) {
             float M = wm[h];
@@ -698,9 +702,6 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
             accb[h] *= f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[h][i] *= f;
-            const float lw = wave_sum(l_run[h]) * inv_lanes * f;
-            if (lane == 0) wl[wave * 8 + h] = lw;
-            if (tid == 0) stat[h] = M * 0.693147180559945309f;  // back to natural units for the (m, l, o) partials
         }
     }
     // Every lane parks its sums in LDS, [value slot][head][dim]; the output loop below
@@ -720,32 +721,59 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         }
     }
     __syncthreads();
-    if constexpr (WAVES) {
-        if (tid < (uint32_t)GT) {
-            const float* wl = stat + 64;
-            float l = wl[tid];
-#pragma unroll
-            for (int w = 1; w < kSdpaWaves; ++w) l += wl[w * 8 + tid];
-            stat[8 + tid] = l;
-        }
-        __syncthreads();
-    }
 
     FK_SDPA_STAMP(6);
     const uint32_t n_out = gcount * a.v_dim;
     const bool direct = !NOMERGE && (n_active == 1);
+    // Maximum (natural units) and sum of a head over the block.  Wave-local form: of the waves' own, by whichever thread
+    // needs them (a few LDS reads that arrive with the value sums', instead of a round through LDS and a barrier).
+    auto head_stats = [&](uint32_t h, float& m, float& l) {
+        if constexpr (WAVES) {
+#pragma clang fp contract(off)
+            const float *wm = stat + 32, *wl = stat + 64;
+            float mw[kSdpaWaves], lw[kSdpaWaves];
+#pragma unroll
+            for (int w = 0; w < kSdpaWaves; ++w) {
+                mw[w] = wm[w * 8 + h];
+                lw[w] = wl[w * 8 + h];
+            }
+            float M = mw[0];
+#pragma unroll
+            for (int w = 1; w < kSdpaWaves; ++w) M = fmaxf(M, mw[w]);
+            l = lw[0] * __builtin_amdgcn_exp2f(mw[0] - M);
+#pragma unroll
+            for (int w = 1; w < kSdpaWaves; ++w) l += lw[w] * __builtin_amdgcn_exp2f(mw[w] - M);  // a product's rounding, then a sum's
+            m = M * 0.693147180559945309f;
+        } else {
+            m = stat[h];
+            l = stat[8 + h];
+        }
+    };
     for (uint32_t e = tid; e < n_out; e += kSdpaBlock) {
         const uint32_t h = e / a.v_dim, d = e - h * a.v_dim;
         float o = 0.f;
-        for (uint32_t sl = 0; sl < vslots; ++sl) o += red[(sl * GT + h) * a.v_dim + d];
+        // sixteen slots are read at once (every bf16 / quantised head of up to 128 dims has 16 or 32): read one by one, each
+        // waits out the LDS (heads of 128: 0.8 us of the launch, see the dispatch notes in sdpa.hip)
+        uint32_t sl = 0;
+        for (; sl + 16 <= vslots; sl += 16) {
+            float v[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[i] = red[((sl + i) * GT + h) * a.v_dim + d];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o += v[i];
+        }
+        for (; sl < vslots; ++sl) o += red[(sl * GT + h) * a.v_dim + d];
+        float m, l;
         if (direct) {
-            st_u16<FUSED>(a.out + (size_t)(h0 + h) * a.v_dim + d, f32_to_bf16_bits(o / stat[8 + h]));
+            head_stats(h, m, l);
+            st_u16<FUSED>(a.out + (size_t)(h0 + h) * a.v_dim + d, f32_to_bf16_bits(o / l));
         } else {
             float* p = a.partials + ((size_t)(h0 + h) * a.n_splits + split) * (a.v_dim + 2);
             st_f32<!NOMERGE>(p + 2 + d, o);
             if (d == 0) {
-                st_f32<!NOMERGE>(p, stat[h]);
-                st_f32<!NOMERGE>(p + 1, stat[8 + h]);
+                head_stats(h, m, l);
+                st_f32<!NOMERGE>(p, m);
+                st_f32<!NOMERGE>(p + 1, l);
             }
         }
     }
@@ -770,12 +798,11 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     if (tid == 0)  // ready for the next launch (or the next layer of this one)
         __hip_atomic_store(&a.counters[kvh * gz_count + gz], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
-    // One wave per head, no block barriers.  The ranges are taken 16 at a time and folded
-    // into a running (M, L, o) with the usual rescaling, in range order, so the result does
-    // not depend on arrival order.  Per batch a lane issues 17 eight-byte loads: (m, l) of
-    // range base + (lane % 16), handed to the other lanes through scalar registers, and its
-    // own two output dims of each of the 16 ranges; the next batch's loads are in flight
-    // while the current one is folded in.
+    // One wave per head, no block barriers.  The ranges are folded 16 at a time into a running (M, L, o) with the usual
+    // rescaling, in range order, so the result does not depend on arrival order.  For every 16 ranges a lane issues 17
+    // eight-byte loads: (m, l) of range base + (lane % 16), whose weight e^(m - M) that lane alone forms and hands to the
+    // others through scalar registers, and its own two output dims of each of the 16 ranges.  The loads pass every cache
+    // (some 1.2 us a trip), so all of up to 64 ranges are requested before the first is folded.
     constexpr uint32_t kBatch = 16;
     const uint32_t ranges = __builtin_amdgcn_readfirstlane(n_active);   // (the length came through a vector register)
     const uint32_t row = a.v_dim + 2;
@@ -796,47 +823,52 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
                 return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
             };
             auto fetch = [&](uint32_t base, float2& ml, float2(&po)[kBatch]) {
-                const uint32_t mine = base + (lane & (kBatch - 1));
-                ml = ld_partial(0u, (mine < ranges ? mine : base) * row);
+                const uint32_t first = base < ranges ? base : 0u, mine = base + (lane & (kBatch - 1));
+                ml = ld_partial(0u, (mine < ranges ? mine : first) * row);
 #pragma unroll
                 for (uint32_t i = 0; i < kBatch; ++i)
-                    po[i] = ld_partial((base + i < ranges ? base + i : base) * row, at);
+                    po[i] = ld_partial((base + i < ranges ? base + i : first) * row, at);
             };
             auto fold = [&](uint32_t base, const float2& ml, const float2(&po)[kBatch]) {
-                float pm[kBatch], pl[kBatch];
-#pragma unroll
-                for (uint32_t i = 0; i < kBatch; ++i) {
-                    pm[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ml.x), i));
-                    pl[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ml.y), i));
-                }
-                float mn = fmaxf(M, pm[0]);
-#pragma unroll
-                for (uint32_t i = 1; i < kBatch; ++i) mn = base + i < ranges ? fmaxf(mn, pm[i]) : mn;
+                // (a lane past the last range holds the batch's first: the maximum is that of the live ones)
+                float mx = dpp_max<0xB1>(ml.x);
+                mx = dpp_max<0x4E>(mx);
+                mx = dpp_max<0x141>(mx);
+                mx = dpp_max<0x140>(mx);
+                const float mn = fmaxf(M, mx);
+                const float w_mine = base + (lane & (kBatch - 1)) < ranges ? expf(ml.x - mn) : 0.f;
                 const float alpha = base ? expf(M - mn) : 0.f;
                 L *= alpha;
                 o0 *= alpha;
                 o1 *= alpha;
 #pragma unroll
                 for (uint32_t i = 0; i < kBatch; ++i) {
-                    const float w = base + i < ranges ? expf(pm[i] - mn) : 0.f;
-                    L = fmaf(pl[i], w, L);
+                    const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_mine), i));
+                    const float pl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ml.y), i));
+                    L = fmaf(pl, w, L);
                     o0 = fmaf(po[i].x, w, o0);
                     o1 = fmaf(po[i].y, w, o1);
                 }
                 M = mn;
             };
-            float2 ml_a, ml_b, po_a[kBatch], po_b[kBatch];
-            uint32_t base = 0;
-            fetch(0, ml_a, po_a);
-            while (base + kBatch < ranges) {  // straight-line body: request the next batch, fold this one
-                fetch(base + kBatch, ml_b, po_b);
-                fold(base, ml_a, po_a);
-                ml_a = ml_b;
+            // N batches requested together, then folded; batches past the last range are requested (clamped: a branch between
+            // the loads would make the first fold wait for all of them) and not folded.
+            auto merge = [&](auto n_const, uint32_t base) {
+                constexpr uint32_t N = decltype(n_const)::value;
+                float2 ml[N], po[N][kBatch];
 #pragma unroll
-                for (uint32_t i = 0; i < kBatch; ++i) po_a[i] = po_b[i];
-                base += kBatch;
+                for (uint32_t b = 0; b < N; ++b) fetch(base + b * kBatch, ml[b], po[b]);
+#pragma unroll
+                for (uint32_t b = 0; b < N; ++b)
+                    if (base + b * kBatch < ranges) fold(base + b * kBatch, ml[b], po[b]);
+            };
+            if (ranges <= kBatch) {
+                merge(std::integral_constant<uint32_t, 1>{}, 0u);
+            } else if (ranges <= 2 * kBatch) {
+                merge(std::integral_constant<uint32_t, 2>{}, 0u);
+            } else {
+                for (uint32_t base = 0; base < ranges; base += 4 * kBatch) merge(std::integral_constant<uint32_t, 4>{}, base);
             }
-            fold(base, ml_a, po_a);
             const float inv_l = 1.0f / L;
             if (live) {
                 uint16_t* dst = a.out + (size_t)(h0 + h) * a.v_dim + 2 * d2;

@@ -291,6 +291,43 @@ __device__ __forceinline__ void input_stage(const IN& in, const InputRegs& r, ui
     __syncthreads();
 }
 
+// ---- merge of a head's key ranges ----------------------------------------------------------------
+// One wave, one head: `ph` = its partial rows (maximum, sum, values), `row` floats apart, n_active <= 16 of them written; the
+// lane's two value dims are at `at`.  All requests first (clamped indices: straight-line; up to 4 or 8 ranges take fewer), then
+// the fold in range order.  Lane i (and i + 16 ..) alone fetches range i's pair and forms its weight e^(m - M); the wave takes
+// weight and sum through scalar registers (formed by every lane for every range, the exponentials were most of the fold).
+__device__ __forceinline__ void xcd_merge_ranges(const float* ph, uint32_t row, uint32_t at, uint32_t n_active, uint32_t lane,
+                                                 float& L, float& o0, float& o1) {
+    auto merge = [&](auto n_const) {
+        constexpr uint32_t N = decltype(n_const)::value;
+        float2 po[N];
+        const uint32_t li = lane & (kXcdMaxRanges - 1);
+        const float2 mine = ld_f32x2<true>(ph + (size_t)(li < n_active ? li : 0u) * row);
+#pragma unroll
+        for (uint32_t i = 0; i < N; ++i) po[i] = ld_f32x2<true>(ph + at + (size_t)(i < n_active ? i : 0u) * row);
+        float M = dpp_max<0xB1>(mine.x);
+        M = dpp_max<0x4E>(M);
+        M = dpp_max<0x141>(M);
+        M = dpp_max<0x140>(M);
+        const float w_mine = li < n_active ? expf(mine.x - M) : 0.f;
+        L = o0 = o1 = 0.f;
+#pragma unroll
+        for (uint32_t i = 0; i < N; ++i) {
+            const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w_mine), i));
+            const float l = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine.y), i));
+            L = fmaf(l, w, L);
+            o0 = fmaf(po[i].x, w, o0);
+            o1 = fmaf(po[i].y, w, o1);
+        }
+    };
+    if (n_active <= kXcdMaxRanges / 4)
+        merge(std::integral_constant<uint32_t, kXcdMaxRanges / 4>{});
+    else if (n_active <= kXcdMaxRanges / 2)
+        merge(std::integral_constant<uint32_t, kXcdMaxRanges / 2>{});
+    else
+        merge(std::integral_constant<uint32_t, kXcdMaxRanges>{});
+}
+
 // ---- projection tiles ----------------------------------------------------------------------------
 // A tile: rows [row0, row0 + rows) x chunks [col0, col0 + cs) of a matrix; flat position p = row * cs + col.
 // A pass covers NL * 256 positions; positions past the tile read the tile's first chunk (in bounds).

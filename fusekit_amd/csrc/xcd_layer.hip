@@ -235,40 +235,8 @@ __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, 
             const float* ph = a.sdpa.partials + (size_t)(sync.xcd * G + h) * a.sdpa.n_splits * row;
             for (uint32_t d2 = lane; d2 < ((a.sdpa.v_dim >> 1) + kWave - 1) / kWave * kWave; d2 += kWave) {
                 const bool live = d2 < (a.sdpa.v_dim >> 1);
-                const float* pd = ph + 2 + 2 * (live ? d2 : 0u);
-                float M = -INFINITY, L = 0.f, o0_ = 0.f, o1_ = 0.f;
-                // all requests first (clamped indices: straight-line), then the fold in range order; up to 8 ranges
-                // (a context of 8 x the range length) take half the requests.  The (maximum, sum) pair of range i is
-                // fetched by lane i alone and handed to the wave through scalar registers: one request, not N.
-                auto merge = [&](auto n_const) {
-                    constexpr uint32_t N = decltype(n_const)::value;
-                    float2 po[N];
-                    const float2 mine = ld_f32x2<true>(ph + (size_t)(lane < n_active ? lane : 0u) * row);
-#pragma unroll
-                    for (uint32_t i = 0; i < N; ++i) po[i] = ld_f32x2<true>(pd + (size_t)(i < n_active ? i : 0u) * row);
-                    float2 ml[N];
-#pragma unroll
-                    for (uint32_t i = 0; i < N; ++i) {
-                        ml[i].x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine.x), i));
-                        ml[i].y = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine.y), i));
-                    }
-                    M = ml[0].x;
-#pragma unroll
-                    for (uint32_t i = 1; i < N; ++i) M = i < n_active ? fmaxf(M, ml[i].x) : M;
-#pragma unroll
-                    for (uint32_t i = 0; i < N; ++i) {
-                        const float w = i < n_active ? expf(ml[i].x - M) : 0.f;
-                        L = fmaf(ml[i].y, w, L);
-                        o0_ = fmaf(po[i].x, w, o0_);
-                        o1_ = fmaf(po[i].y, w, o1_);
-                    }
-                };
-                if (n_active <= kXcdMaxRanges / 4)
-                    merge(std::integral_constant<uint32_t, kXcdMaxRanges / 4>{});
-                else if (n_active <= kXcdMaxRanges / 2)
-                    merge(std::integral_constant<uint32_t, kXcdMaxRanges / 2>{});
-                else
-                    merge(std::integral_constant<uint32_t, kXcdMaxRanges>{});
+                float L, o0_, o1_;
+                xcd_merge_ranges(ph, row, 2u + 2u * (live ? d2 : 0u), n_active, lane, L, o0_, o1_);
                 const float inv_l = 1.0f / L;
                 if (live) {
                     att[h * a.sdpa.v_dim + 2 * d2] = (uint16_t)f32_to_bf16_bits(o0_ * inv_l);
