@@ -179,9 +179,13 @@ __device__ __forceinline__ void stage_fetch(const ARGS& a, uint4 (&xr)[kStageReg
 // SHORT: the caller guarantees K <= kStageRegs * kGemvBlock * 8, so the loops over the rest of a long row are
 // left out (their loads, conditional and issued after the caller's prefetch, blur the compiler's account of which
 // registers still have a load outstanding).
-template <WKind KIND, typename ARGS, bool BLOCKED = false, bool SHORT = false>
+// before_sync: what the caller wants done ahead of the block barrier that ends the staging.
+struct StageNothing {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <WKind KIND, typename ARGS, bool BLOCKED = false, bool SHORT = false, typename BEFORE = StageNothing>
 __device__ __forceinline__ void stage_activations(const ARGS& a, uint4* xs, float* sx, float* scratch,
-                                                  uint4 (&xr)[kStageRegs], uint4 (&wr)[kStageRegs]) {
+                                                  uint4 (&xr)[kStageRegs], uint4 (&wr)[kStageRegs], BEFORE before_sync = BEFORE{}) {
     const bool NORM = a.norm_w != nullptr;  // uniform; one code path serves both
     const uint32_t K = a.K, cpr = a.cpr, n8 = K >> 3;
     const uint4* x8 = reinterpret_cast<const uint4*>(a.x);
@@ -272,6 +276,7 @@ __device__ __forceinline__ void stage_activations(const ARGS& a, uint4* xs, floa
         }
     }
     FK_GEMV_STAMP(7);
+    before_sync();
     __syncthreads();
 }
 

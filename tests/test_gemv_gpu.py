@@ -67,6 +67,56 @@ def test_qgemv_matches_oracle(fk, n, k, bits):
     assert rel_l2(got, ref64) <= REL_L2_BAR
 
 
+class _At:
+    """An array on the device, `shift` bytes behind an allocation's start."""
+
+    def __init__(self, fk, a, shift):
+        raw = np.concatenate([np.zeros(shift, np.uint8), a.reshape(-1).view(np.uint8)])
+        self.buf, self.nbytes = fk.DeviceBuffer.from_numpy(raw), a.nbytes
+        self.ptr = self.buf.ptr + shift
+
+
+# (n, k, bits, group): one row of four groups; a tile's groups no multiple of four (its last run is moved back); runs of four that
+# cross rows; a last tile of one row; groups of 32 and 128; long rows, one or a few a tile; three chunks a thread, two, eight
+ONE_TILE = [(1, 256, 4, 64), (5, 320, 4, 64), (3, 448, 8, 64), (257, 320, 8, 64), (37, 128, 4, 32), (65, 640, 8, 128),
+            (897, 896, 4, 64), (2561, 4096, 4, 64), (130, 10944, 4, 64), (515, 9728, 8, 64), (6145, 2560, 4, 64), (19, 64, 16, 0),
+            (1025, 1536, 16, 0), (300, 14336, 16, 0)]
+
+
+@pytest.mark.parametrize("n,k,bits,group", ONE_TILE)
+def test_one_tile_form_at_its_edges(fk, n, k, bits, group):
+    """Matrix, residual and (quantised) a pair and a fan-out of three with projection biases, scales and biases on two bytes:
+    the oracle's outputs, by the bars above, and nothing written past them."""
+    W = [make_qweight(900 + i, n if i < 2 else max(1, n // 3), k, bits, group or 64) for i in range(3)]
+    x, g, r, r2 = normal_bf16(3, k, 2.0), normal_bf16(4, k, 0.1, 1.0), normal_bf16(5, n), normal_bf16(6, n)
+    dx, dg, dr, dr2 = (fk.DeviceBuffer.from_numpy(a) for a in (x, g, r, r2))
+    dW = [to_device(fk, w) for w in W]
+    if bits != 16:
+        for d, w in zip(dW, W):
+            d.scales, d.biases = _At(fk, np.asarray(w.scales, np.uint16), 2), _At(fk, np.asarray(w.biases, np.uint16), 6)
+    dy = fk.DeviceBuffer.from_numpy(np.full(n + 8, 0x1234, np.uint16))
+
+    def outputs():
+        y = dy.to_numpy(np.uint16)
+        assert (y[n:] == 0x1234).all()
+        return y[:n]
+
+    fk.qgemv(dW[0], dx, None, dy)
+    _check(outputs(), oracle.qgemv(W[0], x), oracle.linear_acc(W[0], x), W[0], x)
+    fk.linear_residual(dW[0], dx, dr, dr2, dy)
+    ref = oracle.linear_residual(W[0], x, r, r2)
+    assert rel_l2(outputs(), oracle.bf16_to_f32(ref)) <= REL_L2_BAR and bf16_mismatch(outputs(), ref)[0] <= FLIP_FRACTION_BAR + 2.0 / n
+    fk.gateup_swiglu(dx, dg, 1e-6, dW[0], dW[1], 1, dy)
+    ref = oracle.gateup_swiglu(x, g, 1e-6, W[0], W[1], 1)
+    assert rel_l2(outputs(), oracle.bf16_to_f32(ref)) <= REL_L2_BAR
+    b = [normal_bf16(7 + i, w.n) for i, w in enumerate(W)]
+    db, dq = [fk.DeviceBuffer.from_numpy(a) for a in b], [fk.DeviceBuffer(2 * w.n) for w in W]
+    fk.rmsnorm_qkv(dx, dg, 1e-6, *dW, *db, *dq)
+    ny = oracle.rmsnorm(x, g, 1e-6)
+    for w, bias, d in zip(W, b, dq):
+        assert rel_l2(d.to_numpy(np.uint16), oracle.bf16_to_f32(oracle.qgemv(w, ny, bias))) <= REL_L2_BAR
+
+
 def test_qgemv_vocab_sized_matches_oracle(fk):
     """The 219 MB shape whose streaming rate the kernel bench reports (1536 blocks, many tiles per block)."""
     n, k = 151936, 2560
