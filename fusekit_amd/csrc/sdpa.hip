@@ -123,9 +123,13 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     // Measured (32 q / 8 kv heads x 128): 4096 positions are fastest with 32 splits,
     // 32768 with 64.
     // (several active rows multiply the tiles: each row then needs fewer ranges to fill the chip; 8 rows x 16 heads at
-    // a capacity of 1024 ran 16 ranges per row and head -- 2048 blocks, most of them past the context -- in 14.4 us)
+    // a capacity of 1024 ran 16 ranges per row and head -- 2048 blocks, most of them past the context -- in 14.4 us; with as
+    // many blocks as CUs a block of those walks its ranges alone on its CU, so from four rows on there are two a CU: a layer of
+    // the 16-head model, us, one / two / four a CU: 4 rows behind 480 positions 114 / 113 / 118, 8 rows behind 1500 156 / 143 / 145, 16
+    // rows 229 / 202 / 204, 16 behind 480 189 / 182 / 185; 2 rows 102 / 103 / 103.  A quantised cache keeps its ranges: their
+    // merge is the last bit of a row)
     const uint32_t tiles = n_kv * ((G + gt - 1) / gt) * rows;
-    uint32_t want = (n_chunks > 128 ? 2u : 1u) * (uint32_t)dev->cus / tiles;
+    uint32_t want = (n_chunks > 128 || (rows >= 4 && !kvq) ? 2u : 1u) * (uint32_t)dev->cus / tiles;
     if (want < 1) want = 1;
     if (want > 256) want = 256;
     const uint32_t cpb = (n_chunks + want - 1) / want;
