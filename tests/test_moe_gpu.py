@@ -256,6 +256,40 @@ def test_routed_reduce_tokens_and_row_idx(fk):
     assert frac <= FLIP_FRACTION_BAR and ulps <= 2.0, (frac, ulps)
 
 
+# (experts, outputs, K, tokens, top-k, bits, group): the fewest routes that are served together; outputs no multiple of 16; K of 11 and
+# of 3 groups (waves with more and fewer, and with none); a group of 128; more experts than a wave; 1024 routes, the most
+TOGETHER = [(8, 40, 704, 3, 2, 4, 64), (4, 333, 192, 40, 4, 4, 64), (16, 48, 256, 30, 6, 8, 64), (16, 32, 384, 17, 3, 8, 128),
+            (100, 16, 128, 64, 4, 4, 64), (5, 16, 64, 512, 2, 4, 64)]
+
+
+@pytest.mark.parametrize("E,O,K,tokens,top_k,bits,group", TOGETHER)
+def test_routes_of_an_expert_served_together(fk, E, O, K, tokens, top_k, bits, group):
+    """Three quarters of a route per expert and more: pair and single matrix against the oracle, by the bars of the other
+    routed tests; half of the routes go to one expert (several chunks of 16), one expert index and one row index lie beyond
+    the range, and nothing is written past the outputs."""
+    n = tokens * top_k
+    stack = lambda seed: oracle.StackedWeight([make_qweight(seed + e, O, K, bits, group) for e in range(E)])
+    Wg, Wu = stack(5000), stack(6000)
+    x, r = normal_bf16(5, (tokens, K)), rng(6)
+    expert_idx = np.where(r.random(n) < 0.5, E // 2, r.integers(0, E, n)).astype(np.uint32)
+    expert_idx[n // 3] = 100000                                       # clamps to E - 1 (routed_qmv_swiglu.rs:138)
+    row_idx = np.repeat(np.arange(tokens, dtype=np.uint32), top_k)
+    row_idx[-1] = tokens + 9                                          # reads the last row
+    rw = normal_bf16(7, n, 0.1, 0.3)
+    out = fk.DeviceBuffer.from_numpy(np.full(n * O + 64, 0x1234, np.uint16))
+    fk.routed_qmv_swiglu(_dev(fk, x), tokens, to_device(fk, Wg), to_device(fk, Wu), E, _dev(fk, row_idx), _dev(fk, expert_idx), _dev(fk, rw),
+                         n, out)
+    raw = out.to_numpy(np.uint16)
+    assert (raw[n * O:] == 0x1234).all()
+    ref = oracle.routed_qmv_swiglu(x, Wg, Wu, np.minimum(row_idx, tokens - 1), expert_idx, rw)
+    got = raw[:n * O].reshape(n, O)
+    assert rel_l2(got, oracle.bf16_to_f32(ref)) <= REL_L2_BAR and bf16_mismatch(got, ref)[0] <= FLIP_FRACTION_BAR
+    h, res = normal_bf16(8, (n, K), 0.0, 0.5), normal_bf16(9, (tokens, O))
+    got = _run_m2(fk, h, Wg, None, expert_idx, rw, None, None, res, tokens, top_k)
+    ref = oracle.routed_qmv_reduce(h, Wg, expert_idx, rw, res, tokens, top_k)
+    assert rel_l2(got, oracle.bf16_to_f32(ref)) <= REL_L2_BAR and bf16_mismatch(got, ref)[0] <= FLIP_FRACTION_BAR
+
+
 def test_routes_served_in_expert_order_give_the_same_bits(fk):
     """Several tokens whose routes share experts (config-5 widths, 8 tokens x top-6 over 16 experts): fk_route_order
     is numpy's stable sort by (clamped) expert, and the routed launches served in that order -- an expert's slice
