@@ -32,6 +32,7 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 // 16 bytes of an operand, which need not lie on their own alignment (a row of a larger tensor, a matrix inside a file): the
 // vector memory unit takes any address, and the type keeps the compiler from assuming more.  The same instructions.
 typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));
 
 constexpr uint32_t kRowsMax = 64;   // activation rows: four tiles of 16
 
@@ -60,8 +61,9 @@ struct QgemmRowsArgs {
 constexpr uint32_t kRowsLine = 9;   // uint4 per staged 128-byte line (8 used: the ninth spreads the banks)
 // groups of 64 columns per 128-byte line of a weight row
 __host__ __device__ constexpr uint32_t rows_slab_groups(uint32_t bits) { return bits == 4 ? 4u : (bits == 8 ? 2u : 1u); }
-// One wave: activation lines of a group, weight lines of a slab, (scale, bias) pairs of a slab.
-__host__ __device__ constexpr uint32_t rows_wave_lds(uint32_t mt, uint32_t nt) { return (mt + nt) * 16u * kRowsLine * 16u + nt * 16u * 4u * 4u; }
+// One wave: activation lines of a group, weight lines of a slab, (scale, bias) pairs of a slab (ONE: scales, then biases, of four
+// groups, and four groups of the norm weights).
+__host__ __device__ constexpr uint32_t rows_wave_lds(uint32_t mt, uint32_t nt) { return (mt + nt) * 16u * kRowsLine * 16u + nt * 16u * 4u * 4u + 4u * 128u; }
 __host__ __device__ constexpr uint32_t rows_lds_bytes(uint32_t mt, uint32_t nt, uint32_t waves) {
     const uint32_t stage = waves * (rows_wave_lds(mt, nt) + mt * 16u * 4u), meet = waves * mt * nt * 256u * 4u;   // one after the other
     return stage > meet ? stage : meet;
@@ -88,7 +90,14 @@ __device__ __forceinline__ uint4 rows_unpack(uint32_t w0, uint32_t w1) {
 }
 
 // MT tiles of 16 activation rows, NT tiles of 16 weight rows (PAIR: NT / 2 of the gate matrix and as many of the up matrix).
-template <WKind KIND, bool PAIR, int NT, int MT, int WAVES>
+// ONE: no wave has more than one slab of K (quantised; K up to 1024 int4 columns with four waves, 2048 with eight).  Everything
+// is then asked for exactly once, in straight line -- the loop below asks two slabs and two groups past its range, two thirds of
+// all requests at K = 896, and a CU issues one per 16 .. 20 cycles --, the four groups' scales and biases with one request for
+// all tiles, the norm weights with one.  Both forms ask for what the epilogue adds together with the first slab, not after the
+// waves have met.  The loop with its operands late / now, 37 rows of int4 with a residual, one call in a chain: 896 x 896 3.70 /
+// 3.42 us, 4864 x 896 7.48 / 6.98 (pair 8.98 / 8.61), 1024 x 2048 4.93 / 4.54, 2560 x 2048 7.56 / 6.84; the loop itself with
+// its operands early: 896 x 4864 7.55 / 7.14, 2560 x 4096 10.48 / 10.10.  The same sums in the same order.
+template <WKind KIND, bool PAIR, int NT, int MT, int WAVES, bool ONE>
 __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const QgemmRowsArgs a) {
     constexpr int CT = PAIR ? NT / 2 : NT;                                      // output tiles of a block
     constexpr uint32_t BITS = KIND == W_Q4 ? 4u : (KIND == W_Q8 ? 8u : 16u);
@@ -107,6 +116,8 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     u32x4_t* xs = reinterpret_cast<u32x4_t*>(reinterpret_cast<char*>(lds_raw) + wave * rows_wave_lds(MT, NT));   // [MT * 16][kRowsLine]
     u32x4_t* wl = xs + MT * 16 * kRowsLine;                                                                    // [NT * 16][kRowsLine]
     uint32_t* ml = reinterpret_cast<uint32_t*>(wl + NT * 16 * kRowsLine);                                    // [NT * 16][4]
+    [[maybe_unused]] uint16_t* sl = reinterpret_cast<uint16_t*>(ml);                                         // ONE: [NT][2][16][4]
+    [[maybe_unused]] u32x4_t* nl = reinterpret_cast<u32x4_t*>(ml + NT * 64);                                 // ONE: [4][8]
 
     // request roles: line `r8 + 8 h` of a tile, its piece l8; scale and bias of row lane / 4, group lane % 4
     // (uniform bases and 32-bit lane offsets: full pointers cost the registers that let a second wave share the SIMD)
@@ -148,6 +159,26 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     struct Acts {
         u32x4_t x[MT][2], nw;
     };
+    // ONE: four entries of each row's scales and biases, from the wave's first group or, at a row's end, the row's last four
+    [[maybe_unused]] const uint32_t e_first = ONE ? ((g0 >> a.gshift) + 4u <= gpr ? g0 >> a.gshift : gpr - 4u) : 0u;
+    // What the epilogue's first outputs of this thread add (a null operand reads the activations instead and is not used).
+    constexpr uint32_t OUT = 16u * CT;
+    constexpr int EARLY = 2;
+    const uint32_t yst = a.y_stride[seg];
+    const uint16_t* res = a.res ? a.res + (size_t)m0 * yst : nullptr;
+    const uint16_t* bias = a.bias[seg];
+    [[maybe_unused]] uint32_t e_bias[EARLY], e_res[EARLY];
+    auto fetch_epilogue = [&]() __attribute__((always_inline)) {
+        if constexpr (!PAIR) {
+#pragma unroll
+            for (int k = 0; k < EARLY; ++k) {
+                const uint32_t e = (uint32_t)k * (WAVES * kWave) + threadIdx.x, m = e / OUT, n = blk * OUT + e % OUT;
+                const uint32_t mc = m < M ? m : M - 1u, nc = n < N ? n : N - 1u;
+                e_bias[k] = *(bias ? bias + nc : a.x);
+                e_res[k] = *(res ? res + (size_t)mc * yst + nc : a.x);
+            }
+        }
+    };
     // Straight-line requests: what lies past the wave's range (or the row) is clamped to its last piece and never used.
     const uint32_t gl = g1 > g0 ? g1 - 1u : (g0 < G ? g0 : G - 1u);
     auto fetch_w = [&](uint32_t g, Slab& s) __attribute__((always_inline)) {   // groups g .. g + SG - 1
@@ -158,7 +189,7 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) s.w[t][h] = *reinterpret_cast<const u32x4_any_t*>(wbase[t] + (woff[t][h] + at));
-            if constexpr (KIND != W_BF16) {
+            if constexpr (KIND != W_BF16 && !ONE) {
                 const uint32_t gm = g + (lane & 3u), gmc = (gm < gl ? gm : gl) >> a.gshift;
                 s.sc[t] = *reinterpret_cast<const uint16_t*>(sbase[t] + (soff[t] + gmc * 2u));
                 s.bi[t] = *reinterpret_cast<const uint16_t*>(bbase[t] + (soff[t] + gmc * 2u));
@@ -171,7 +202,7 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
         for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int h = 0; h < 2; ++h) s.x[t][h] = *reinterpret_cast<const u32x4_any_t*>(xbase + (xoff[t][h] + gc * 128u));
-        s.nw = *reinterpret_cast<const u32x4_any_t*>(nbase + (l8 * 16u + gc * 128u));
+        if constexpr (!ONE) s.nw = *reinterpret_cast<const u32x4_any_t*>(nbase + (l8 * 16u + gc * 128u));
     };
     const uint4 ones4 = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
     const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, ones4);
@@ -210,8 +241,16 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
                     b0 = rows_unpack<KIND>(v.x, v.y);
                     b1 = rows_unpack<KIND>(v.z, v.w);
                 }
-                const uint32_t sb = ml[((uint32_t)t * 16u + c16) * 4u + u];
-                const float sf = bf16_lo(sb), bf = bf16_hi(sb);
+                float sf, bf;
+                if constexpr (ONE) {
+                    const uint16_t* at = sl + (uint32_t)t * 128u + c16 * 4u + (((g0 + u) >> a.gshift) - e_first);
+                    sf = bf16_bits_to_f32(at[0]);
+                    bf = bf16_bits_to_f32(at[64]);
+                } else {
+                    const uint32_t sb = ml[((uint32_t)t * 16u + c16) * 4u + u];
+                    sf = bf16_lo(sb);
+                    bf = bf16_hi(sb);
+                }
                 f32x4_t c[MT];
 #pragma unroll
                 for (int i = 0; i < MT; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][0], __builtin_bit_cast(bf16x8_t, b0), zero, 0, 0, 0);
@@ -224,12 +263,26 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
             }
         }
     };
-    Slab w0, w1;
+    Slab w0;
+    [[maybe_unused]] Slab w1;
     Acts x0, x1;
+    [[maybe_unused]] u32x2_any_t meta;
+    [[maybe_unused]] u32x4_t norms;
+    if constexpr (ONE) {
+        // lane: tile lane / 32, scales or biases, row lane % 16 (one tile: its upper half repeats it)
+        const uint32_t t = NT > 1 ? lane >> 5 : 0u;
+        const unsigned char *sfrom = NT > 1 && t ? sbase[NT - 1] : sbase[0], *bfrom = NT > 1 && t ? bbase[NT - 1] : bbase[0];
+        const unsigned char* from = lane & 16u ? bfrom : sfrom;
+        const uint32_t n0 = (blk * CT + (PAIR ? 0u : t)) * 16u, first = n0 < N ? n0 : N - 1u, r = first + c16 < N ? c16 : N - 1u - first;
+        meta = *reinterpret_cast<const u32x2_any_t*>(from + (r * gpr + e_first) * 2u);
+        const uint32_t gn = g0 + (r8 & 3u);
+        norms = *reinterpret_cast<const u32x4_any_t*>(nbase + (l8 * 16u + (gn < gl ? gn : gl) * 128u));
+    }
     fetch_w(g0, w0);
     fetch_x(g0, x0);
     fetch_x(g0 + 1u, x1);
-    fetch_w(g0 + SG, w1);
+    if constexpr (!ONE) fetch_w(g0 + SG, w1);
+    fetch_epilogue();
     float rr[MT][2];   // 1 / rms of the rows this lane parks
 #pragma unroll
     for (int i = 0; i < MT; ++i) rr[i][0] = rr[i][1] = 1.f;
@@ -300,6 +353,9 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
             }
     }
     auto step = [&](uint32_t g, uint32_t u, Acts& x) __attribute__((always_inline)) {
+        if constexpr (ONE) {
+            if (normed) x.nw = nl[u * 8u + l8];
+        }
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -314,7 +370,7 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
                 }
                 xs[((uint32_t)i * 16u + r8 + 8u * (uint32_t)h) * kRowsLine + l8] = v;
             }
-        fetch_x(g + u + 2u, x);
+        if (!ONE || u + 2u < SG) fetch_x(g + u + 2u, x);
         __builtin_amdgcn_wave_barrier();
         if (g + u < g1) consume(u);   // wave-uniform
         __builtin_amdgcn_wave_barrier();
@@ -324,9 +380,14 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) wl[((uint32_t)t * 16u + r8 + 8u * (uint32_t)h) * kRowsLine + l8] = s.w[t][h];
-            if constexpr (KIND != W_BF16) ml[(uint32_t)t * 64u + lane] = s.sc[t] | (s.bi[t] << 16);
+            if constexpr (KIND != W_BF16 && !ONE) ml[(uint32_t)t * 64u + lane] = s.sc[t] | (s.bi[t] << 16);
         }
-        fetch_w(g + 2u * SG, s);
+        if constexpr (ONE) {
+            if (NT > 1 || lane < 32u) *reinterpret_cast<u32x2_any_t*>(sl + (NT > 1 ? lane : lane & 31u) * 4u) = meta;
+            if (normed && r8 < 4u) nl[lane] = norms;
+        } else {
+            fetch_w(g + 2u * SG, s);
+        }
         step(g, 0u, xa);
         if constexpr (SG > 1) step(g, 1u, xb);
         if constexpr (SG > 2) {
@@ -334,13 +395,17 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
             step(g, 3u, xb);
         }
     };
-    for (uint32_t g = g0; g < g1; g += 2u * SG) {
-        slab(g, w0, x0, x1);
-        if (g + SG < g1) {
-            if constexpr (SG & 1u)
-                slab(g + SG, w1, x1, x0);
-            else
-                slab(g + SG, w1, x0, x1);
+    if constexpr (ONE) {
+        slab(g0, w0, x0, x1);
+    } else {
+        for (uint32_t g = g0; g < g1; g += 2u * SG) {
+            slab(g, w0, x0, x1);
+            if (g + SG < g1) {
+                if constexpr (SG & 1u)
+                    slab(g + SG, w1, x1, x0);
+                else
+                    slab(g + SG, w1, x0, x1);
+            }
         }
     }
     __syncthreads();   // every wave is through with its staging area
@@ -356,12 +421,9 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
             for (int r = 0; r < 4; ++r)
                 meet[wave * PER_WAVE + ((uint32_t)i * 16u + kq * 4u + (uint32_t)r) * COLS + (uint32_t)t * 16u + c16] = acc[i][t][r];
     __syncthreads();
-    constexpr uint32_t OUT = 16u * CT;
-    const uint32_t yst = a.y_stride[seg];
     uint16_t* yo = a.y[seg] + (size_t)m0 * yst;
-    const uint16_t* res = a.res ? a.res + (size_t)m0 * yst : nullptr;
-    const uint16_t* bias = a.bias[seg];
-    for (uint32_t e0 = 0; e0 < M * OUT; e0 += WAVES * kWave) {
+    // One round of outputs; EARLY ones have their operands already.
+    auto outputs = [&](uint32_t e0, auto early, uint32_t bias_bits, uint32_t res_bits) __attribute__((always_inline)) {
         const uint32_t e = e0 + threadIdx.x, m = e / OUT, col = e % OUT, n = blk * OUT + col;
         const bool live = m < M && n < N;
         uint32_t o = 0;
@@ -376,8 +438,8 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
             if constexpr (PAIR) {
                 o = swiglu_bits(s0, s1, a.variant, 1.0f);
             } else {
-                if (bias) s0 += bf16_bits_to_f32(bias[n]);
-                if (res) s0 += bf16_bits_to_f32(res[(size_t)m * yst + n]);
+                if (bias) s0 += bf16_bits_to_f32(decltype(early)::value ? bias_bits : (uint32_t)bias[n]);
+                if (res) s0 += bf16_bits_to_f32(decltype(early)::value ? res_bits : (uint32_t)res[(size_t)m * yst + n]);
                 o = f32_to_bf16_bits(s0);
             }
             yo[(size_t)m * yst + n] = (uint16_t)o;
@@ -388,25 +450,35 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
                 if (m < M && (col & 15u) == 0) a.ssq_out[(size_t)(m0 + m) * a.ssq_n + blk * CT + (col >> 4)] = t;
             }
         }
+    };
+    constexpr uint32_t ROUND = WAVES * kWave;
+    if constexpr (PAIR) {
+        for (uint32_t e0 = 0; e0 < M * OUT; e0 += ROUND) outputs(e0, std::false_type{}, 0u, 0u);
+    } else {
+#pragma unroll
+        for (int k = 0; k < EARLY; ++k)
+            if ((uint32_t)k * ROUND < M * OUT) outputs((uint32_t)k * ROUND, std::true_type{}, e_bias[k], e_res[k]);
+        for (uint32_t e0 = EARLY * ROUND; e0 < M * OUT; e0 += ROUND) outputs(e0, std::false_type{}, 0u, 0u);
     }
 }
 
-template <WKind KIND, bool PAIR, int NT>
+template <WKind KIND, bool PAIR, int NT, bool ONE>
 const void* rows_func(uint32_t mt, uint32_t waves) {
-#define FK_ROWS_CASE(MT)                                                                          \
-    return waves == 8 ? reinterpret_cast<const void*>(&qgemm_rows_kernel<KIND, PAIR, NT, MT, 8>)   \
-                      : reinterpret_cast<const void*>(&qgemm_rows_kernel<KIND, PAIR, NT, MT, 4>)
+#define FK_ROWS_CASE(MT)                                                                               \
+    return waves == 8 ? reinterpret_cast<const void*>(&qgemm_rows_kernel<KIND, PAIR, NT, MT, 8, ONE>)   \
+                      : reinterpret_cast<const void*>(&qgemm_rows_kernel<KIND, PAIR, NT, MT, 4, ONE>)
     switch (mt) {
         case 1: FK_ROWS_CASE(1);
         case 2: FK_ROWS_CASE(2);
         case 3: FK_ROWS_CASE(3);
         default: FK_ROWS_CASE(4);
     }
+#undef FK_ROWS_CASE
 }
-template <WKind KIND>
+template <WKind KIND, bool ONE>
 const void* rows_func(bool pair, bool two, uint32_t mt, uint32_t waves) {
-    if (pair) return rows_func<KIND, true, 2>(mt, waves);
-    return two ? rows_func<KIND, false, 2>(mt, waves) : rows_func<KIND, false, 1>(mt, waves);
+    if (pair) return rows_func<KIND, true, 2, ONE>(mt, waves);
+    return two ? rows_func<KIND, false, 2, ONE>(mt, waves) : rows_func<KIND, false, 1, ONE>(mt, waves);
 }
 
 }  // namespace
@@ -474,8 +546,15 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
         a.blk0[i] = blocks;
         blocks += (a.n[i] + (two ? 31u : 15u)) / (two ? 32u : 16u);
     }
-    out->func = W0->bits == 4 ? rows_func<W_Q4>(rq.pair, two, mt, waves)
-                              : (W0->bits == 8 ? rows_func<W_Q8>(rq.pair, two, mt, waves) : rows_func<W_BF16>(rq.pair, two, mt, waves));
+    // one slab a wave, and rows of at least the four scales that its one request takes
+    const uint32_t groups = K / 64u;
+    const bool one = W0->bits != 16 && (groups + waves - 1u) / waves <= rows_slab_groups(W0->bits) && (groups >> a.gshift) >= 4u;
+    if (W0->bits == 4)
+        out->func = one ? rows_func<W_Q4, true>(rq.pair, two, mt, waves) : rows_func<W_Q4, false>(rq.pair, two, mt, waves);
+    else if (W0->bits == 8)
+        out->func = one ? rows_func<W_Q8, true>(rq.pair, two, mt, waves) : rows_func<W_Q8, false>(rq.pair, two, mt, waves);
+    else
+        out->func = rows_func<W_BF16, false>(rq.pair, two, mt, waves);
     out->grid = dim3(blocks, m_blocks, 1);
     out->block = dim3(waves * kWave, 1, 1);
     out->shmem = rows_lds_bytes(mt, rq.pair || two ? 2u : 1u, waves);

@@ -162,6 +162,41 @@ def test_norm_gate_up_and_swiglu_of_several_rows_in_one_launch(fk, bits, m, hidd
                               variant, fk.DeviceBuffer(2 * 9 * inter))
 
 
+@pytest.mark.parametrize("bits,group,m,n,k", [
+    (4, 64, 37, 162, 256),    # one group a wave, the fewest scales a row may have
+    (4, 64, 3, 145, 320),     # the last wave's scales end the row; waves of one and of two groups
+    (4, 64, 64, 161, 1024),   # four waves, four groups each
+    (4, 64, 7, 136, 2048),    # eight waves, four groups each
+    (4, 64, 48, 4129, 256),   # two tiles of weight rows per block, the last one row deep
+    (8, 64, 20, 146, 512),    # int8: two groups a wave
+    (4, 128, 9, 136, 512),    # four scales a row, two groups to each
+    (4, 128, 8, 167, 896),    # seven: a wave may start inside one
+])
+def test_rows_of_a_short_k_are_requested_in_one_go(fk, bits, group, m, n, k):
+    """At most one slab of K per wave: the straight-line form of the multi-row matmul at the edges of what it takes (the bars
+    of _check: the single-row arithmetic in another order of summation; rows long enough that its share of flipped roundings
+    allows one), with residual, bias, as a pair, and normalised."""
+    W, U = make_qweight(640 + bits, n, k, bits, group=group), make_qweight(641 + bits, n, k, bits, group=group)
+    x, res, bias = normal_bf16(642, (m, k)), normal_bf16(643, (m, n)), normal_bf16(644, n)
+    with_res, with_bias = _run(fk, W, x, res=res), _run(fk, W, x, bias=bias)
+    out, ws = fk.DeviceBuffer(2 * m * n), fk.DeviceBuffer(fk.qgemm_workspace_bytes(m, n, k, group))
+    fk.qgemm_swiglu(to_device(fk, W), to_device(fk, U), _dev(fk, x), m, 1, out, ws)
+    pair = out.to_numpy(np.uint16, (m, n))
+    for r in range(m):
+        acc = oracle.linear_acc(W, x[r])
+        _check(with_res[r], oracle.linear_residual(W, x[r], res[r], None), acc + oracle.bf16_to_f32(res[r]), W, x[r])
+        _check(with_bias[r], oracle.qgemv(W, x[r], bias), acc + oracle.bf16_to_f32(bias), W, x[r])
+        _check_swiglu(pair[r], oracle.gateup_swiglu(x[r], None, 1e-6, W, U, 1), x[r], W, U, 1)
+    if m > 8 or group != 64:
+        return
+    nw, y = normal_bf16(645, k, 0.1, 1.0), fk.DeviceBuffer(2 * m * n)
+    fk.rmsnorm_qkv_rows(_dev(fk, x), m, k, _dev(fk, nw), 1e-6, to_device(fk, W), None, None, y, n)
+    normed = y.to_numpy(np.uint16, (m, n))
+    for r in range(m):
+        xn = oracle.rmsnorm(x[r], nw, 1e-6)
+        _check(normed[r], oracle.qgemv(W, xn, None), oracle.linear_acc(W, xn), W, xn)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("m", [9, 100])
 def test_qgemm_group_128(fk, bits, m):
