@@ -90,7 +90,7 @@ fk_status run_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const uin
 }
 
 fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint16_t* bias, const uint16_t* residual, uint16_t* y,
-                    void* workspace, bool kept_order, hipStream_t s) {
+                    void* workspace, bool kept_order, hipStream_t s, RowsNorm* norm) {
     if (W && W->bits == 16) {  // dense bf16 weights: the plain library GEMM with this library's epilogue
         if (!x || !y || !workspace) return set_error(FK_ERR_INVALID, "fk_qgemm: null activation, output or workspace");
         if (qgemm_takes_rows(m, 16, 0, W->k) && (g_rows_form || !gemm_library_available())) {
@@ -101,12 +101,13 @@ fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uin
             return run_launch(l, s);
         }
         if (!gemm_library_available()) return set_error(FK_ERR_UNSUPPORTED, "fk_qgemm: bf16 weights need rocBLAS (librocblas.so.5 not found)");
-        return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, s);
+        return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, s, norm);
     }
     Launch main, reduce;
     if (!kept_order && !qgemm_takes_library(m)) {
         DmaRequest rq;
         rq.W[0] = W; rq.x = x; rq.M = m; rq.bias[0] = bias; rq.res = residual; rq.y[0] = y; rq.workspace = workspace;
+        rq.norm = norm;
         if (qgemm_takes_dma(rq)) {
             FK_TRY(plan_qgemm_dma(rq, &main, &reduce));
             FK_TRY(run_launch(main, s));
@@ -114,7 +115,7 @@ fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uin
         }
     }
     FK_TRY(plan_qgemm(W, x, m, bias, residual, y, workspace, &main, &reduce));  // validates the arguments for both routes
-    if (qgemm_takes_library(m)) return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, s);
+    if (qgemm_takes_library(m)) return run_qgemm_library(W, nullptr, x, m, bias, residual, 0, y, workspace, s, norm);
     FK_TRY(run_launch(main, s));
     return run_launch(reduce, s);
 }

@@ -178,8 +178,15 @@ bool qgemm_takes_library(uint32_t m, bool pair = false);
 // quantised caches have been filled with (see prompt.hip).
 fk_status run_sdpa_prefill(const uint16_t* q, const uint16_t* cache_k, const uint16_t* cache_v, uint16_t* out, uint32_t rows, uint32_t kv_len,
                            uint32_t n_heads, uint32_t n_kv, uint32_t head_dim, uint32_t capacity, float scale, bool kept_order, hipStream_t s);
+// The RMSNorm of a projection's output rows (with the residual), for the launch that finishes them to form as well where it can.
+struct RowsNorm {
+    const uint16_t* w;
+    uint16_t* y;
+    float eps;
+    bool done = false;   // set: y holds the normalised rows, no launch of its own needed
+};
 fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint16_t* bias, const uint16_t* residual, uint16_t* y,
-                    void* workspace, bool kept_order, hipStream_t s);
+                    void* workspace, bool kept_order, hipStream_t s, RowsNorm* norm = nullptr);
 fk_status run_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const uint16_t* x, uint32_t m, const uint16_t* const* bias,
                            uint16_t* const* y, void* workspace, bool kept_order, hipStream_t s);
 fk_status run_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint16_t* x, uint32_t m, int variant, uint16_t* out,
@@ -228,6 +235,7 @@ struct DmaRequest {
     int variant = 0;
     uint16_t* y[3] = {nullptr, nullptr, nullptr};
     void* workspace = nullptr;
+    RowsNorm* norm = nullptr;          // one matrix, or null
 };
 bool qgemm_takes_dma(const DmaRequest& rq);
 uint32_t qgemm_dma_split(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, bool pair);
@@ -237,9 +245,9 @@ bool gemm_library_available();
 size_t qgemm_library_sums_bytes(uint32_t m, uint32_t n, uint32_t k);
 size_t qgemm_library_workspace_bytes(uint32_t m, uint32_t n, uint32_t k);
 void plan_qgemm_epilogue(const float* p0, const float* p1, const uint16_t* bias, const uint16_t* res, uint16_t* y,
-                         uint32_t M, uint32_t N, uint32_t ksplit, int variant, Launch* out);
+                         uint32_t M, uint32_t N, uint32_t ksplit, int variant, Launch* out, RowsNorm* norm = nullptr);
 fk_status run_qgemm_library(const fk_weight* W0, const fk_weight* W1, const uint16_t* x, uint32_t m, const uint16_t* bias,
-                            const uint16_t* res, int variant, uint16_t* y, void* workspace, hipStream_t s);
+                            const uint16_t* res, int variant, uint16_t* y, void* workspace, hipStream_t s, RowsNorm* norm = nullptr);
 
 // RoPE / per-head RMSNorm / KV-cache store (one wave per head).
 struct RopeArgs {

@@ -4,7 +4,8 @@
 // A pass is some ten launches per layer.  Called one by one through the operator entry points from Python each costs 7..10 us
 // of host time, more than a short prompt's kernels run for; from here a launch costs what the runtime takes (3.7 us), so that
 // the GPU is what a pass waits for.  37 tokens of the 0.5B-class model, whole call: 1378 us from Python, 1055 from here
-// with the norms inside the projections (two launches per layer fewer).
+// with the norms inside the projections (two launches per layer fewer); of 512 tokens of the 4B-class model 7279 us with the
+// norms in launches of their own, 7046 with them in the launches that add split sums up.
 #include <math.h>
 
 #include "fk_host.hpp"
@@ -46,8 +47,8 @@ bool kept_order(const fk_prompt_model& m, const fk_weight& W, uint32_t rows) {
     return m.kv_bits != 0 && rows <= 64 && (W.bits == 16 ? gemm_library_available() : rows > 10);
 }
 fk_status matmul(const fk_prompt_model& m, const fk_weight& W, const uint16_t* x, uint32_t rows, const uint16_t* bias, const uint16_t* res,
-                 uint16_t* y, hipStream_t s) {
-    if (!kept_order(m, W, rows)) return run_qgemm(&W, x, rows, bias, res, y, m.workspace, m.kv_bits != 0, s);
+                 uint16_t* y, hipStream_t s, RowsNorm* norm = nullptr) {
+    if (!kept_order(m, W, rows)) return run_qgemm(&W, x, rows, bias, res, y, m.workspace, m.kv_bits != 0, s, norm);
     if (W.bits == 16) return run_qgemm_library(&W, nullptr, x, rows, bias, res, 0, y, m.workspace, s);
     Launch main, reduce;
     FK_TRY(plan_qgemm(&W, x, rows, bias, res, y, m.workspace, &main, &reduce, true));
@@ -55,33 +56,42 @@ fk_status matmul(const fk_prompt_model& m, const fk_weight& W, const uint16_t* x
     return run_launch(reduce, s);
 }
 
-// One matrix with the residual.  *ssq: whether the sums of squares of its rows are in m.xn afterwards (the normalised rows'
-// place, free between a projection's launch and the next norm).
+// What the launch that wrote a projection's input rows left in m.xn, free between a projection's launch and the next norm.
+enum Left { LEFT_NOTHING, LEFT_SQUARES /* the rows' sums of squares */, LEFT_NORMED /* the normalised rows */ };
+
+// One matrix with the residual; next_norm: the weights of the norm that its rows enter next, or null.
 fk_status residual_rows(const fk_prompt_model& m, const fk_weight& W, const uint16_t* x, uint32_t rows, const uint16_t* res, uint16_t* y,
-                        bool* ssq, hipStream_t s) {
-    *ssq = m.kv_bits == 0 && qgemm_takes_rows(rows, W.bits, W.group, W.k) && W.n % 64u == 0 && ((uintptr_t)m.xn & 15u) == 0;
-    if (!*ssq) return matmul(m, W, x, rows, nullptr, res, y, s);
+                        const uint16_t* next_norm, Left* left, hipStream_t s) {
+    const bool ssq = m.kv_bits == 0 && qgemm_takes_rows(rows, W.bits, W.group, W.k) && W.n % 64u == 0 && ((uintptr_t)m.xn & 15u) == 0;
+    *left = ssq ? LEFT_SQUARES : LEFT_NOTHING;
+    if (!ssq) {
+        RowsNorm norm{next_norm, m.xn, m.eps};
+        FK_TRY(matmul(m, W, x, rows, nullptr, res, y, s, next_norm && m.xn && m.kv_bits == 0 ? &norm : nullptr));
+        if (norm.done) *left = LEFT_NORMED;
+        return FK_OK;
+    }
     RowsRequest rq;
     rq.W[0] = &W; rq.x = x; rq.M = rows; rq.res = res; rq.y[0] = y;
     rq.ssq_out = reinterpret_cast<float*>(m.xn);
     return run_rows(rq, s);
 }
 
-fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* ssq, uint32_t rows, uint32_t pos, fk_stream s) {
+fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, const fk_prompt_layer* next, Left* left, uint32_t rows,
+                     uint32_t pos, fk_stream s) {
     const uint32_t dim = m.head_dim, len = pos + rows;
     const float scale = (float)(1.0 / sqrt((double)dim));
     const bool tiled = dim == 64 || dim == 128;
-    if (m.kv_bits == 0 && l.k.bits == l.q.bits && l.v.bits == l.q.bits && l.k.group == l.q.group && l.v.group == l.q.group &&
+    if (m.kv_bits == 0 && *left != LEFT_NORMED && l.k.bits == l.q.bits && l.v.bits == l.q.bits && l.k.group == l.q.group && l.v.group == l.q.group &&
         takes_norm(l.q, rows, l.q.n + l.k.n + l.v.n, m.x, l.input_norm)) {
         RowsRequest rq;
         rq.W[0] = &l.q; rq.W[1] = &l.k; rq.W[2] = &l.v; rq.n_mats = 3;
         rq.x = m.x; rq.M = rows; rq.norm_w = l.input_norm; rq.eps = m.eps;
-        if (*ssq) rq.ssq_in = reinterpret_cast<const float*>(m.xn);   // (not where the rows come from the embedding)
+        if (*left == LEFT_SQUARES) rq.ssq_in = reinterpret_cast<const float*>(m.xn);   // (not where the rows come from the embedding)
         rq.bias[0] = l.q_bias; rq.bias[1] = l.k_bias; rq.bias[2] = l.v_bias;
         rq.y[0] = m.q; rq.y[1] = m.k; rq.y[2] = m.v;
         FK_TRY(run_rows(rq, (hipStream_t)s));
     } else {
-        FK_TRY(norm_rows(m, m.x, l.input_norm, rows, (hipStream_t)s));
+        if (*left != LEFT_NORMED) FK_TRY(norm_rows(m, m.x, l.input_norm, rows, (hipStream_t)s));
         const fk_weight* W[3] = {&l.q, &l.k, &l.v};
         const uint16_t* bias[3] = {l.q_bias, l.k_bias, l.v_bias};
         uint16_t* y[3] = {m.q, m.k, m.v};
@@ -112,8 +122,8 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* s
             FK_TRY(fk_sdpa_decode_rows(m.q, l.cache_k, l.cache_v, m.att, rows, pos + 1, m.n_heads, m.n_kv, dim, dim, m.capacity, scale,
                                        m.partials, m.counters, s));
     }
-    FK_TRY(residual_rows(m, l.o, m.att, rows, m.x, m.x2, ssq, (hipStream_t)s));
-    if (*ssq && l.gate.bits == l.up.bits && l.gate.group == l.up.group && takes_norm(l.gate, rows, l.gate.n, m.x2, l.post_norm)) {
+    FK_TRY(residual_rows(m, l.o, m.att, rows, m.x, m.x2, l.post_norm, left, (hipStream_t)s));
+    if (*left == LEFT_SQUARES && l.gate.bits == l.up.bits && l.gate.group == l.up.group && takes_norm(l.gate, rows, l.gate.n, m.x2, l.post_norm)) {
         RowsRequest rq;
         rq.W[0] = &l.gate; rq.W[1] = &l.up; rq.n_mats = 2; rq.pair = true;
         rq.x = m.x2; rq.M = rows; rq.norm_w = l.post_norm; rq.eps = m.eps; rq.variant = m.swiglu_variant;
@@ -121,7 +131,7 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* s
         rq.y[0] = m.mid;
         FK_TRY(run_rows(rq, (hipStream_t)s));
     } else {
-        FK_TRY(norm_rows(m, m.x2, l.post_norm, rows, (hipStream_t)s));
+        if (*left != LEFT_NORMED) FK_TRY(norm_rows(m, m.x2, l.post_norm, rows, (hipStream_t)s));
         if (kept_order(m, l.gate, rows) && l.gate.bits == 16) {
             FK_TRY(run_qgemm_library(&l.gate, &l.up, m.xn, rows, nullptr, nullptr, m.swiglu_variant, m.mid, m.workspace, (hipStream_t)s));
         } else if (kept_order(m, l.gate, rows)) {
@@ -134,7 +144,7 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, bool* s
             FK_TRY(run_qgemm_swiglu(&l.gate, &l.up, m.xn, rows, m.swiglu_variant, m.mid, m.workspace, m.kv_bits != 0, (hipStream_t)s));
         }
     }
-    return residual_rows(m, l.down, m.mid, rows, m.x2, m.x, ssq, (hipStream_t)s);
+    return residual_rows(m, l.down, m.mid, rows, m.x2, m.x, next ? next->input_norm : nullptr, left, (hipStream_t)s);
 }
 
 }  // namespace
@@ -155,8 +165,9 @@ extern "C" fk_status fk_prompt_run(const fk_prompt_model* model, const uint32_t*
         FK_HIP(hipMemcpyAsync(m.tokens, tokens + done, (size_t)rows * 4, hipMemcpyHostToDevice, (hipStream_t)s));
         FK_TRY(fk_embed_lookup_rows(&m.embed, m.tokens, rows, m.embed_scale, m.x, s));
         FK_TRY(fk_rope_table_rows(m.rope_tab, m.head_dim, m.theta, pos, rows, s));   // once per pass, for every layer and head
-        bool ssq = false;
-        for (uint32_t i = 0; i < m.n_layers; ++i) FK_TRY(layer_pass(m, m.layers[i], &ssq, rows, pos, s));
+        Left left = LEFT_NOTHING;
+        for (uint32_t i = 0; i < m.n_layers; ++i)
+            FK_TRY(layer_pass(m, m.layers[i], i + 1u < m.n_layers ? &m.layers[i + 1u] : nullptr, &left, rows, pos, s));
     }
     // the last row's hidden state -> logits -> greedy token, and the decode loop's step counter
     FK_TRY(fk_final_rmsnorm_lm_head(m.x + (size_t)(rows - 1) * m.hidden, m.final_norm, m.eps, &m.head, m.logits, s));

@@ -626,6 +626,88 @@ __global__ __launch_bounds__(256) void qgemm_reduce_kernel(const QgemmReduceArgs
     a.y[i] = (uint16_t)f32_to_bf16_bits(s0);
 }
 
+// The second kernel of a residual projection together with the RMSNorm that reads its rows: a block per row, which it holds in
+// registers between the two (P pieces of eight outputs a thread).  The two launches asked memory for the row twice and cost
+// three dependent trips; here it is one.  The additions and the norm's sums are in the order of qgemm_reduce4_kernel and
+// rmsnorm_rows_vec_kernel: the same bits.  Split sums and norm of 2560 columns, two launches / this one, in a prompt pass: 512
+// rows 6.0 + 4.9 / 6.6 us, 256 rows 4.9 + 4.6 / 5.2; 100 rows of 896 columns 4.6 + 2.9 / 4.2.
+struct QgemmReduceNormArgs {
+    const float* p;   // [ksplit, M, N]
+    const uint16_t* res;
+    const uint16_t* w;   // norm weights
+    uint16_t* y;
+    uint16_t* yn;        // the normalised rows
+    uint32_t M, N, ksplit;
+    float eps;
+};
+template <int P>
+__global__ __launch_bounds__(256) void qgemm_reduce_norm_kernel(const QgemmReduceNormArgs a) {
+    __shared__ float scratch[8];
+    const uint32_t n8 = a.N >> 3;
+    const size_t row = (size_t)blockIdx.x * a.N, total = (size_t)a.M * a.N;
+    uint32_t at[P];
+    uint4 rv[P], wv[P];
+    float s[P][8];
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        at[i] = (threadIdx.x + 256u * i < n8 ? threadIdx.x + 256u * i : 0u) * 8u;   // (past the row's end: its first piece, not stored)
+        rv[i] = a.res ? *reinterpret_cast<const uint4*>(a.res + row + at[i]) : make_uint4(0u, 0u, 0u, 0u);
+        wv[i] = *reinterpret_cast<const uint4*>(a.w + at[i]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[i][e] = 0.f;
+    }
+    const float* from = a.p + row;
+    constexpr int AHEAD = P > 2 ? 1 : 4;   // splits requested ahead of their additions
+#pragma unroll AHEAD
+    for (uint32_t ks = 0; ks < a.ksplit; ++ks, from += total) {
+        float4 v[P][2];
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[i][h] = reinterpret_cast<const float4*>(from + at[i])[h];
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                s[i][4 * h] += v[i][h].x; s[i][4 * h + 1] += v[i][h].y; s[i][4 * h + 2] += v[i][h].z; s[i][4 * h + 3] += v[i][h].w;
+            }
+    }
+    uint32_t o[P][4];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const uint32_t r4[4] = {rv[i].x, rv[i].y, rv[i].z, rv[i].w};
+        float q = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float lo = s[i][2 * e], hi = s[i][2 * e + 1];
+            if (a.res) {
+                lo += bf16_lo(r4[e]);
+                hi += bf16_hi(r4[e]);
+            }
+            o[i][e] = f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+            q = fmaf(bf16_hi(o[i][e]), bf16_hi(o[i][e]), fmaf(bf16_lo(o[i][e]), bf16_lo(o[i][e]), q));
+        }
+        if (threadIdx.x + 256u * i < n8) {
+            ss += q;
+            *reinterpret_cast<uint4*>(a.y + row + at[i]) = make_uint4(o[i][0], o[i][1], o[i][2], o[i][3]);
+        }
+    }
+    ss = block_sum<256>(ss, scratch);
+    const float r = 1.0f / sqrtf(ss / (float)a.N + a.eps);
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const uint32_t w4[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
+        uint32_t n[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t t = pack_bf16(bf16_lo(o[i][e]) * r, bf16_hi(o[i][e]) * r);
+            n[e] = pack_bf16(bf16_lo(w4[e]) * bf16_lo(t), bf16_hi(w4[e]) * bf16_hi(t));
+        }
+        if (threadIdx.x + 256u * i < n8) *reinterpret_cast<uint4*>(a.yn + row + at[i]) = make_uint4(n[0], n[1], n[2], n[3]);
+    }
+}
+
 // Split-k sums of a fan-out (rows of n_total columns, the matrices side by side) to the matrices' own outputs; four
 // consecutive columns per thread (every matrix's N is a multiple of 4), additions in split order, then the bias.
 struct QgemmFanReduceArgs {
@@ -778,7 +860,24 @@ fk_status plan_qgemm_main(const DeviceFacts* dev, const fk_weight* W, const uint
 }
 
 void plan_reduce(const float* p0, const float* p1, const uint16_t* bias, const uint16_t* res, uint16_t* y, uint32_t M,
-                 uint32_t N, uint32_t ksplit, int variant, Launch* out) {
+                 uint32_t N, uint32_t ksplit, int variant, Launch* out, RowsNorm* norm = nullptr) {
+    // with the norm that follows, where the norm's own launch would hold the row in registers too (the same sums then)
+    if (norm && !p1 && !bias && N % 8u == 0 && N <= 8u * 256u * 8u &&
+        ((reinterpret_cast<uintptr_t>(p0) | reinterpret_cast<uintptr_t>(res) | reinterpret_cast<uintptr_t>(y) |
+          reinterpret_cast<uintptr_t>(norm->w) | reinterpret_cast<uintptr_t>(norm->y)) & 15u) == 0) {
+        QgemmReduceNormArgs n{p0, res, norm->w, y, norm->y, M, N, ksplit, norm->eps};
+        const uint32_t pieces = (N / 8u + 255u) / 256u;
+        out->func = pieces == 1 ? reinterpret_cast<const void*>(&qgemm_reduce_norm_kernel<1>)
+                  : pieces == 2 ? reinterpret_cast<const void*>(&qgemm_reduce_norm_kernel<2>)
+                  : pieces <= 4 ? reinterpret_cast<const void*>(&qgemm_reduce_norm_kernel<4>)
+                                : reinterpret_cast<const void*>(&qgemm_reduce_norm_kernel<8>);
+        out->grid = dim3(M, 1, 1);
+        out->block = dim3(256, 1, 1);
+        out->shmem = 0;
+        out->set_args(n);
+        norm->done = true;
+        return;
+    }
     QgemmReduceArgs r;
     r.p0 = p0; r.p1 = p1; r.bias = bias; r.res = res; r.y = y;
     r.M = M; r.N = N; r.ksplit = ksplit; r.variant = variant;
@@ -797,15 +896,15 @@ bool g_rows_form = true;
 
 // the epilogue of a product whose fp32 sums are complete (the library route)
 void plan_qgemm_epilogue(const float* p0, const float* p1, const uint16_t* bias, const uint16_t* res, uint16_t* y,
-                         uint32_t M, uint32_t N, uint32_t ksplit, int variant, Launch* out) {
-    plan_reduce(p0, p1, bias, res, y, M, N, ksplit, variant, out);
+                         uint32_t M, uint32_t N, uint32_t ksplit, int variant, Launch* out, RowsNorm* norm) {
+    plan_reduce(p0, p1, bias, res, y, M, N, ksplit, variant, out, norm);
 }
 
 // the second kernel of qgemm_dma.hip's split-k sums
 void plan_qgemm_dma_reduce(const DmaRequest& rq, uint32_t n_total, uint32_t ksplit, Launch* out) {
     const float* p = static_cast<const float*>(rq.workspace);
     if (rq.pair) return plan_reduce(p, p + (size_t)ksplit * rq.M * n_total, nullptr, nullptr, rq.y[0], rq.M, n_total, ksplit, rq.variant, out);
-    if (rq.n_mats == 1) return plan_reduce(p, nullptr, rq.bias[0], rq.res, rq.y[0], rq.M, n_total, ksplit, 0, out);
+    if (rq.n_mats == 1) return plan_reduce(p, nullptr, rq.bias[0], rq.res, rq.y[0], rq.M, n_total, ksplit, 0, out, rq.norm);
     QgemmFanReduceArgs r;
     memset(&r, 0, sizeof(r));
     r.p = p;

@@ -246,7 +246,7 @@ size_t qgemm_library_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
 
 // workspace: [(m x N) fp32 sums per matrix or k slice][N x K bf16 dequantised matrix, reused by the second matrix in stream order]
 fk_status run_qgemm_library(const fk_weight* W0, const fk_weight* W1, const uint16_t* x, uint32_t m, const uint16_t* bias,
-                            const uint16_t* res, int variant, uint16_t* y, void* workspace, hipStream_t s) {
+                            const uint16_t* res, int variant, uint16_t* y, void* workspace, hipStream_t s, RowsNorm* norm) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
     if (!shape_ok(W0, m) || (W1 && !shape_ok(W1, m))) return set_error(FK_ERR_UNSUPPORTED, "qgemm (library route): shape not supported");
@@ -272,7 +272,7 @@ fk_status run_qgemm_library(const fk_weight* W0, const fk_weight* W1, const uint
     if (split > 1) {
         FK_TRY(library_product_split(wb, x, m, W0->n, W0->k, split, p0, s));
         Launch reduce;
-        plan_qgemm_epilogue(p0, nullptr, bias, res, y, m, W0->n, split, 0, &reduce);
+        plan_qgemm_epilogue(p0, nullptr, bias, res, y, m, W0->n, split, 0, &reduce, norm);
         return run_launch(reduce, s);
     }
     if (!W1 && !bias)  // nothing left for an epilogue kernel but the rounding (and the residual)

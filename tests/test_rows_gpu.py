@@ -164,3 +164,50 @@ def test_prefill_with_resident_bf16_weights_is_bit_identical(fk, bits):
     from helpers import host_weight
     want = oracle.f32_to_bf16(oracle.dequantize(host_weight(W.mats[name])))
     assert np.array_equal(b._bf16_weights[name].w.to_numpy(np.uint16, want.shape), want)
+
+
+@pytest.mark.parametrize("bits,hidden,n_heads,n_kv,dim,inter,rows,bias", [
+    (4, 896, 14, 2, 64, 1024, 65, True),      # a piece of the row for under half of a block's threads
+    (4, 2176, 12, 4, 128, 768, 100, False),   # two pieces, the second ragged; few key / value heads
+    (8, 4224, 13, 1, 64, 768, 130, False),    # four, three of them used
+    (4, 8320, 12, 2, 64, 768, 70, True),      # eight, the fifth ragged
+    (16, 832, 6, 2, 128, 4096, 70, False),    # the library's split sums
+])
+def test_prompt_passes_join_launches_without_changing_a_bit(fk, bits, hidden, n_heads, n_kv, dim, inter, rows, bias):
+    """From 65 rows a pass forms the norm of a projection's rows in the launch that adds its split sums up (where it has
+    any): caches and logits of the operators called one by one, bit for bit."""
+    from fusekit_amd.decoder import DecoderConfig, DecoderRuntime, DecoderWeights
+    c = DecoderConfig(n_layers=2, hidden=hidden, n_heads=n_heads, n_kv=n_kv, head_dim=dim, inter=inter, vocab=512, capacity=256,
+                      bits=bits, qk_norm=not bias, qkv_bias=bias, swiglu_variant=1)
+    W = DecoderWeights.random_init(c, seed=45)
+    prompt = rng(46).integers(0, c.vocab, rows).tolist()
+    d = DecoderRuntime(c, W)
+    d.prefill_rows(prompt, rows_per_pass=256)
+
+    new = lambda n: fk.DeviceBuffer(2 * rows * n)
+    x, x2, xn, q, k, v, att, mid = (new(n) for n in (hidden, hidden, hidden, c.n_q, c.n_kvd, c.n_kvd, c.n_q, inter))
+    ck, cv = ([fk.zeros(2 * n_kv * c.capacity * dim) for _ in range(2)] for _ in range(2))
+    group = 0 if bits == 16 else c.group
+    ws = fk.DeviceBuffer(2 * max(fk.qgemm_workspace_bytes(rows, n, kk, group) for n, kk in
+                                 ((c.n_q + 2 * c.n_kvd, hidden), (hidden, c.n_q), (inter, hidden), (hidden, inter))))
+    tab, logits = fk.DeviceBuffer(4 * rows * dim), fk.DeviceBuffer(2 * c.vocab)
+    fk.embed_lookup_rows(W.mats["embed_tokens"], _dev(fk, np.array(prompt, np.uint32)), rows, c.embed_scale, x)
+    fk.rope_table_rows(tab, dim, c.theta, 0, rows)
+    for l in range(c.n_layers):
+        p = f"layers.{l}."
+        m = lambda n: W.mats[p + n]
+        fk.rmsnorm_rows(x, W.vecs[p + "input_layernorm"], c.eps, rows, hidden, xn)
+        fk.qgemm_fanout([m(f"self_attn.{n}_proj") for n in "qkv"], xn, rows,
+                        [W.vecs[p + f"self_attn.{n}_proj.bias"] for n in "qkv"] if bias else None, [q, k, v], ws)
+        norms = [None if bias else W.vecs[p + f"self_attn.{n}_norm"] for n in "qk"]
+        fk.qkv_rope_store_rows(q, k, v, *norms, n_heads, n_kv, dim, dim, c.theta, c.eps, rows, 0, c.capacity, ck[l], cv[l], rope_tab=tab)
+        fk.sdpa_prefill(q, ck[l], cv[l], att, rows, rows, n_heads, n_kv, dim, c.capacity, dim ** -0.5)
+        fk.qgemm(m("self_attn.o_proj"), att, rows, None, x, x2, ws)
+        fk.rmsnorm_rows(x2, W.vecs[p + "post_attention_layernorm"], c.eps, rows, hidden, xn)
+        fk.qgemm_swiglu(m("mlp.gate_proj"), m("mlp.up_proj"), xn, rows, c.swiglu_variant, mid, ws)
+        fk.qgemm(m("mlp.down_proj"), mid, rows, None, x2, x, ws)
+        assert np.array_equal(d.cache_k[l].to_numpy(np.uint16), ck[l].to_numpy(np.uint16)), l
+        assert np.array_equal(d.cache_v[l].to_numpy(np.uint16), cv[l].to_numpy(np.uint16)), l
+    last = fk.DeviceBuffer.from_numpy(x.to_numpy(np.uint16, (rows, hidden))[-1])
+    fk.final_rmsnorm_lm_head(last, W.vecs["final_norm"], c.eps, W.mats.get("lm_head", W.mats["embed_tokens"]), logits)
+    assert np.array_equal(d.logits.to_numpy(np.uint16), logits.to_numpy(np.uint16))
