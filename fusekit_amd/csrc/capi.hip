@@ -121,12 +121,13 @@ fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uin
 }
 
 fk_status run_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const uint16_t* x, uint32_t m, const uint16_t* const* bias,
-                           uint16_t* const* y, void* workspace, bool kept_order, hipStream_t s) {
+                           uint16_t* const* y, void* workspace, bool kept_order, hipStream_t s, FanSums* sums) {
     if (!W || !y || n_mats < 1 || n_mats > 3) return set_error(FK_ERR_INVALID, "fk_qgemm_fanout: one to three matrices");
     if (n_mats > 1 && W[0] && W[0]->bits != 16 && !qgemm_takes_library(m)) {
         Launch main, reduce;
         DmaRequest rq;
         rq.n_mats = n_mats; rq.x = x; rq.M = m; rq.workspace = workspace;
+        rq.sums = sums;
         for (uint32_t i = 0; i < n_mats; ++i) {
             rq.W[i] = W[i];
             rq.bias[i] = bias ? bias[i] : nullptr;

@@ -87,8 +87,15 @@ fk_status plan_rope_table(float* tab, uint32_t rope_dims, float base_log2, uint3
 // pair (d, d + dim/2) sits HL/2 lanes apart and is exchanged as packed bf16, the norm's sum of squares
 // is a butterfly over the HL lanes.  One wave per (head, row) with 2-byte accesses took 92 us for
 // 4096 rows of the 4B-class model; the kernel is bound by its short chains, not by bytes.
-template <int HL>
-__global__ __launch_bounds__(256) void rope_rows_fast_kernel(const RopeArgs a) {
+// SUMS: the rows come as the split sums of the projection (and its bias), which a launch of their own would add up, round and
+// write for this one to read: the same additions and roundings.  In a pass, two launches / one: 100 rows of 1152 columns (seven
+// splits) 4.4 + 3.1 / 5.4 us, 256 rows of 6144 (two) 5.0 + 5.0 / 5.8.
+struct RopeSumsArgs : RopeArgs {
+    FanSums sums;
+    const uint16_t* bias[3];   // of q, k, v, or null
+};
+template <int HL, bool SUMS>
+__global__ __launch_bounds__(256) void rope_rows_fast_kernel(const std::conditional_t<SUMS, RopeSumsArgs, RopeArgs> a) {
     constexpr uint32_t DIM = HL * 8u, HPW = kWave / HL;
     const uint32_t lane = threadIdx.x & (kWave - 1u);
     const uint32_t heads = a.n_q + 2u * a.n_kv, groups = (heads + HPW - 1u) / HPW;
@@ -120,12 +127,40 @@ __global__ __launch_bounds__(256) void rope_rows_fast_kernel(const RopeArgs a) {
         rotate = false;
     }
     // every load is issued before anything is used; lanes without a norm weight read their own row instead
-    const uint4 xv = *reinterpret_cast<const uint4*>(src + p * 8u);
-    const uint4 wv = *reinterpret_cast<const uint4*>((nw ? nw : src) + p * 8u);
+    uint4 xv;
+    if constexpr (!SUMS) xv = *reinterpret_cast<const uint4*>(src + p * 8u);
+    const uint4 wv = *reinterpret_cast<const uint4*>((nw ? nw : SUMS ? a.q : src) + p * 8u);
     const float4* tp = reinterpret_cast<const float4*>(a.rope_tab + (size_t)tr * DIM + 2u * ((p % (HL / 2u)) * 8u));
     const float4 t0 = tp[0], t1 = tp[1], t2 = tp[2], t3 = tp[3];  // (cos, sin) of this lane's eight pairs
     const float cs[8] = {t0.x, t0.z, t1.x, t1.z, t2.x, t2.z, t3.x, t3.z};
     const float sn[8] = {t0.y, t0.w, t1.y, t1.w, t2.y, t2.w, t3.y, t3.w};
+    if constexpr (SUMS) {
+        const uint32_t seg = b < a.n_q ? 0u : (b < a.n_q + a.n_kv ? 1u : 2u), first = seg == 0u ? 0u : (seg == 1u ? a.n_q : a.n_q + a.n_kv);
+        const uint16_t* bias = a.bias[seg];
+        uint2 bv[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) bv[h] = bias ? reinterpret_cast<const uint2*>(bias + (b - first) * DIM + p * 8u)[h] : make_uint2(0u, 0u);
+        const size_t total = (size_t)a.rows * a.sums.cols;
+        const float* from = a.sums.p + (size_t)tr * a.sums.cols + b * DIM + p * 8u;
+        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (uint32_t ks = 0; ks < a.sums.ksplit; ++ks, from += total) {
+            const float4 f0 = reinterpret_cast<const float4*>(from)[0], f1 = reinterpret_cast<const float4*>(from)[1];
+            v[0] += f0.x; v[1] += f0.y; v[2] += f0.z; v[3] += f0.w;
+            v[4] += f1.x; v[5] += f1.y; v[6] += f1.z; v[7] += f1.w;
+        }
+        const uint32_t b4[4] = {bv[0].x, bv[0].y, bv[1].x, bv[1].y};
+        uint32_t x4[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (bias) {
+                v[2 * e] += bf16_lo(b4[e]);
+                v[2 * e + 1] += bf16_hi(b4[e]);
+            }
+            x4[e] = f32_to_bf16_bits(v[2 * e]) | (f32_to_bf16_bits(v[2 * e + 1]) << 16);
+        }
+        xv = make_uint4(x4[0], x4[1], x4[2], x4[3]);
+    }
 
     uint32_t pv[4] = {xv.x, xv.y, xv.z, xv.w};
     const uint32_t wq[4] = {wv.x, wv.y, wv.z, wv.w};
@@ -166,7 +201,20 @@ __global__ __launch_bounds__(256) void rope_rows_fast_kernel(const RopeArgs a) {
     if (live) *reinterpret_cast<uint4*>(dst + p * 8u) = res;
 }
 
-fk_status plan_rope_store(const RopeArgs& in, Launch* out) {
+// Whether a request takes the row form above.
+static bool rope_rows_fast(const RopeArgs& a) {
+    const bool aligned = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) | reinterpret_cast<uintptr_t>(a.v) |
+                           reinterpret_cast<uintptr_t>(a.cache_k) | reinterpret_cast<uintptr_t>(a.cache_v) |
+                           reinterpret_cast<uintptr_t>(a.q_norm) | reinterpret_cast<uintptr_t>(a.k_norm) |
+                           reinterpret_cast<uintptr_t>(a.rope_tab)) & 15u) == 0;
+    const uint32_t dim = a.n_q ? a.head_dim : a.k_dim;
+    return a.rows >= 8 && a.rope_tab && a.rope_on && a.n_q && a.n_kv && (dim == 64 || dim == 128) && a.rope_dims == dim &&
+           a.k_dim == dim && a.v_dim == dim && aligned;
+}
+
+bool rope_takes_sums(const RopeArgs& a) { return rope_rows_fast(a); }
+
+fk_status plan_rope_store(const RopeArgs& in, Launch* out, const FanSums* sums, const uint16_t* const* bias) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
     RopeArgs a = in;
@@ -181,20 +229,25 @@ fk_status plan_rope_store(const RopeArgs& in, Launch* out) {
     if (!a.rows) a.rows = 1;
     if (a.rows > 65535) return set_error(FK_ERR_UNSUPPORTED, "rope: too many rows");
     if (a.n_kv && a.rows > a.capacity) return set_error(FK_ERR_INVALID, "rope: more rows than the cache holds");
-    const bool aligned = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) | reinterpret_cast<uintptr_t>(a.v) |
-                           reinterpret_cast<uintptr_t>(a.cache_k) | reinterpret_cast<uintptr_t>(a.cache_v) |
-                           reinterpret_cast<uintptr_t>(a.q_norm) | reinterpret_cast<uintptr_t>(a.k_norm) |
-                           reinterpret_cast<uintptr_t>(a.rope_tab)) & 15u) == 0;
-    const uint32_t dim = a.n_q ? a.head_dim : a.k_dim;
-    if (a.rows >= 8 && a.rope_tab && a.rope_on && a.n_q && a.n_kv && (dim == 64 || dim == 128) && a.rope_dims == dim &&
-        a.k_dim == dim && a.v_dim == dim && aligned) {
-        const uint32_t hpw = dim == 128 ? 4u : 8u, heads = a.n_q + 2 * a.n_kv;
+    if (sums && !rope_rows_fast(a)) return set_error(FK_ERR_INVALID, "rope: this form takes finished rows");
+    if (rope_rows_fast(a)) {
+        const uint32_t dim = a.head_dim, hpw = dim == 128 ? 4u : 8u, heads = a.n_q + 2 * a.n_kv;
         const uint64_t waves = (uint64_t)a.rows * ((heads + hpw - 1u) / hpw);
-        out->func = dim == 128 ? reinterpret_cast<const void*>(&rope_rows_fast_kernel<16>) : reinterpret_cast<const void*>(&rope_rows_fast_kernel<8>);
         out->grid = dim3((uint32_t)((waves + 3u) / 4u), 1, 1);
         out->block = dim3(256, 1, 1);
         out->shmem = 0;
-        out->set_args(a);
+        if (sums) {
+            RopeSumsArgs r;
+            memset(static_cast<void*>(&r), 0, sizeof(r));
+            static_cast<RopeArgs&>(r) = a;
+            r.sums = *sums;
+            for (int i = 0; i < 3; ++i) r.bias[i] = bias ? bias[i] : nullptr;
+            out->func = dim == 128 ? reinterpret_cast<const void*>(&rope_rows_fast_kernel<16, true>) : reinterpret_cast<const void*>(&rope_rows_fast_kernel<8, true>);
+            out->set_args(r);
+        } else {
+            out->func = dim == 128 ? reinterpret_cast<const void*>(&rope_rows_fast_kernel<16, false>) : reinterpret_cast<const void*>(&rope_rows_fast_kernel<8, false>);
+            out->set_args(a);
+        }
         return FK_OK;
     }
     out->func = reinterpret_cast<const void*>(&rope_store_kernel);

@@ -185,10 +185,15 @@ struct RowsNorm {
     float eps;
     bool done = false;   // set: y holds the normalised rows, no launch of its own needed
 };
+// Sums of a fan-out's k splits, rows of the matrices' columns side by side, left for the launch that reads its outputs to add up.
+struct FanSums {
+    const float* p;   // [ksplit, rows, cols], null: none (the outputs are finished)
+    uint32_t ksplit, cols;
+};
 fk_status run_qgemm(const fk_weight* W, const uint16_t* x, uint32_t m, const uint16_t* bias, const uint16_t* residual, uint16_t* y,
                     void* workspace, bool kept_order, hipStream_t s, RowsNorm* norm = nullptr);
 fk_status run_qgemm_fanout(const fk_weight* const* W, uint32_t n_mats, const uint16_t* x, uint32_t m, const uint16_t* const* bias,
-                           uint16_t* const* y, void* workspace, bool kept_order, hipStream_t s);
+                           uint16_t* const* y, void* workspace, bool kept_order, hipStream_t s, FanSums* sums = nullptr);
 fk_status run_qgemm_swiglu(const fk_weight* Wg, const fk_weight* Wu, const uint16_t* x, uint32_t m, int variant, uint16_t* out,
                            void* workspace, bool kept_order, hipStream_t s);
 // Up to 64 activation rows (qgemm_rows.hip): one launch, epilogue included, no workspace; bits 4 / 8 (group 64 / 128) and
@@ -236,6 +241,7 @@ struct DmaRequest {
     uint16_t* y[3] = {nullptr, nullptr, nullptr};
     void* workspace = nullptr;
     RowsNorm* norm = nullptr;          // one matrix, or null
+    FanSums* sums = nullptr;           // where the caller adds up what a split of k leaves, or null
 };
 bool qgemm_takes_dma(const DmaRequest& rq);
 uint32_t qgemm_dma_split(uint32_t bits, uint32_t M, uint32_t N, uint32_t K, bool pair);
@@ -268,7 +274,9 @@ struct RopeArgs {
     uint32_t rows;     // active token rows (0 = 1): row r is position offset + r and reads q/k/v row r
     const float* rope_tab;  // optional [rows][rope_dims/2] (cos, sin) as plan_rope_table fills it, for position offset + r
 };
-fk_status plan_rope_store(const RopeArgs& in, Launch* out);
+// sums: the rows as their projection's split sums, bias[3] with them (where rope_takes_sums; k and v themselves are not read then).
+fk_status plan_rope_store(const RopeArgs& in, Launch* out, const FanSums* sums = nullptr, const uint16_t* const* bias = nullptr);
+bool rope_takes_sums(const RopeArgs& a);
 // (cos, sin) of every rotary pair at positions offset .. offset + rows - 1: the values the
 // rope/store kernel would compute itself, filled once per prompt pass for all layers and heads.
 fk_status plan_rope_table(float* tab, uint32_t rope_dims, float base_log2, uint32_t offset, uint32_t rows, Launch* out);

@@ -80,6 +80,15 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, const f
                      uint32_t pos, fk_stream s) {
     const uint32_t dim = m.head_dim, len = pos + rows;
     const float scale = (float)(1.0 / sqrt((double)dim));
+    const uint16_t* bias[3] = {l.q_bias, l.k_bias, l.v_bias};
+    RopeArgs rope;
+    memset(&rope, 0, sizeof(rope));
+    rope.q = m.q; rope.k = m.k; rope.v = m.v; rope.q_norm = l.q_norm; rope.k_norm = l.k_norm;
+    rope.n_q = m.n_heads; rope.n_kv = m.n_kv; rope.head_dim = rope.k_dim = rope.v_dim = rope.rope_dims = dim; rope.rope_on = 1;
+    rope.offset_imm = pos; rope.capacity = m.capacity; rope.cache_k = l.cache_k; rope.cache_v = l.cache_v;
+    rope.eps = m.eps; rope.base_log2 = (float)log2((double)m.theta); rope.rows = rows; rope.rope_tab = m.rope_tab;
+    FanSums sums{};   // (one split, or another kernel: finished rows)
+    const bool takes_sums = m.kv_bits == 0 && rope_takes_sums(rope) && l.q.n == m.n_heads * dim && l.k.n == m.n_kv * dim && l.v.n == l.k.n;
     const bool tiled = dim == 64 || dim == 128;
     if (m.kv_bits == 0 && *left != LEFT_NORMED && l.k.bits == l.q.bits && l.v.bits == l.q.bits && l.k.group == l.q.group && l.v.group == l.q.group &&
         takes_norm(l.q, rows, l.q.n + l.k.n + l.v.n, m.x, l.input_norm)) {
@@ -93,12 +102,12 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, const f
     } else {
         if (*left != LEFT_NORMED) FK_TRY(norm_rows(m, m.x, l.input_norm, rows, (hipStream_t)s));
         const fk_weight* W[3] = {&l.q, &l.k, &l.v};
-        const uint16_t* bias[3] = {l.q_bias, l.k_bias, l.v_bias};
         uint16_t* y[3] = {m.q, m.k, m.v};
         if (kept_order(m, l.q, rows))
             for (int i = 0; i < 3; ++i) FK_TRY(matmul(m, *W[i], m.xn, rows, bias[i], nullptr, y[i], (hipStream_t)s));
         else
-            FK_TRY(run_qgemm_fanout(W, 3, m.xn, rows, l.q_bias ? bias : nullptr, y, m.workspace, m.kv_bits != 0, (hipStream_t)s));
+            FK_TRY(run_qgemm_fanout(W, 3, m.xn, rows, l.q_bias ? bias : nullptr, y, m.workspace, m.kv_bits != 0, (hipStream_t)s,
+                                    takes_sums ? &sums : nullptr));
     }
     if (m.kv_bits) {
         FK_TRY(fk_qkv_rope_store_rows(m.q, nullptr, nullptr, l.q_norm, nullptr, m.n_heads, 0, dim, dim, m.theta, m.eps, rows, pos,
@@ -114,8 +123,9 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, const f
                                         m.capacity, m.kv_bits, m.kv_group, scale, m.partials, m.counters, s));
         }
     } else {
-        FK_TRY(fk_qkv_rope_store_rows(m.q, m.k, m.v, l.q_norm, l.k_norm, m.n_heads, m.n_kv, dim, dim, m.theta, m.eps, rows, pos, m.capacity,
-                                      l.cache_k, l.cache_v, m.rope_tab, s));
+        Launch store;
+        FK_TRY(plan_rope_store(rope, &store, sums.p ? &sums : nullptr, l.q_bias ? bias : nullptr));
+        FK_TRY(run_launch(store, (hipStream_t)s));
         if (tiled)
             FK_TRY(fk_sdpa_prefill(m.q, l.cache_k, l.cache_v, m.att, rows, len, m.n_heads, m.n_kv, dim, m.capacity, scale, s));
         else

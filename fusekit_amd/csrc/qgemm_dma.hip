@@ -602,7 +602,8 @@ fk_status plan_qgemm_dma(const DmaRequest& rq, Launch* main, Launch* reduce) {
     FK_TRY(raise_dynamic_lds(main->func, main->shmem));
     main->set_args(a);
     *reduce = Launch();
-    if (a.ksplit > 1u) plan_qgemm_dma_reduce(rq, n_total, a.ksplit, reduce);
+    if (rq.sums) *rq.sums = FanSums{a.ksplit > 1u ? a.partial : nullptr, a.ksplit, n_total};
+    if (a.ksplit > 1u && !rq.sums) plan_qgemm_dma_reduce(rq, n_total, a.ksplit, reduce);
     return FK_OK;
 }
 

@@ -175,7 +175,8 @@ def test_prefill_with_resident_bf16_weights_is_bit_identical(fk, bits):
 ])
 def test_prompt_passes_join_launches_without_changing_a_bit(fk, bits, hidden, n_heads, n_kv, dim, inter, rows, bias):
     """From 65 rows a pass forms the norm of a projection's rows in the launch that adds its split sums up (where it has
-    any): caches and logits of the operators called one by one, bit for bit."""
+    any), and the rotation and the cache store of q, k, v in the one that adds theirs up: caches and logits of the operators
+    called one by one, bit for bit."""
     from fusekit_amd.decoder import DecoderConfig, DecoderRuntime, DecoderWeights
     c = DecoderConfig(n_layers=2, hidden=hidden, n_heads=n_heads, n_kv=n_kv, head_dim=dim, inter=inter, vocab=512, capacity=256,
                       bits=bits, qk_norm=not bias, qkv_bias=bias, swiglu_variant=1)
