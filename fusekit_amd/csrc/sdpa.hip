@@ -171,12 +171,16 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     a.partials = partials;
     a.counters = counters;
 
+    // heads of 128 dims on 16 lanes a row: each lane finishes its own scores (sdpa_block, ROW16)
+    const bool row16 = gt <= 4 && qk_dim == 128 && v_dim == 128 &&
+                       (!kvq || (quant->group == 64 && (((uintptr_t)quant->k_scales | (uintptr_t)quant->k_biases | (uintptr_t)quant->v_scales |
+                                                         (uintptr_t)quant->v_biases) & 3u) == 0));
     const void* func = nullptr;
 #define FK_SDPA_PICK(Q)                                                                         \
     switch (gt) {                                                                               \
-        case 1: func = reinterpret_cast<const void*>(&sdpa_decode_kernel<1, Q>); break;         \
-        case 2: func = reinterpret_cast<const void*>(&sdpa_decode_kernel<2, Q>); break;         \
-        case 4: func = reinterpret_cast<const void*>(&sdpa_decode_kernel<4, Q>); break;         \
+        case 1: func = row16 ? reinterpret_cast<const void*>(&sdpa_decode_kernel<1, Q, true>) : reinterpret_cast<const void*>(&sdpa_decode_kernel<1, Q>); break; \
+        case 2: func = row16 ? reinterpret_cast<const void*>(&sdpa_decode_kernel<2, Q, true>) : reinterpret_cast<const void*>(&sdpa_decode_kernel<2, Q>); break; \
+        case 4: func = row16 ? reinterpret_cast<const void*>(&sdpa_decode_kernel<4, Q, true>) : reinterpret_cast<const void*>(&sdpa_decode_kernel<4, Q>); break; \
         default: func = reinterpret_cast<const void*>(&sdpa_decode_kernel<8, Q>); break;        \
     }
     if (fusion) {
@@ -185,9 +189,9 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
         const bool fast = fusion->rope_tab && fusion->rope_dims == qk_dim && qk_dim <= 128 && !(kvq && fusion->q_norm && qk_dim != 128);
 #define FK_SDPA_FUSED(F, Q)                                                                           \
     switch (gt) {                                                                                     \
-        case 1: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<1, F, Q>); break;        \
-        case 2: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<2, F, Q>); break;        \
-        case 4: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<4, F, Q>); break;        \
+        case 1: func = row16 ? reinterpret_cast<const void*>(&sdpa_rope_store_kernel<1, F, Q, true>) : reinterpret_cast<const void*>(&sdpa_rope_store_kernel<1, F, Q>); break; \
+        case 2: func = row16 ? reinterpret_cast<const void*>(&sdpa_rope_store_kernel<2, F, Q, true>) : reinterpret_cast<const void*>(&sdpa_rope_store_kernel<2, F, Q>); break; \
+        case 4: func = row16 ? reinterpret_cast<const void*>(&sdpa_rope_store_kernel<4, F, Q, true>) : reinterpret_cast<const void*>(&sdpa_rope_store_kernel<4, F, Q>); break; \
         default: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<8, F, Q>); break;       \
     }
 #define FK_SDPA_FUSED_Q(F)              \

@@ -84,6 +84,27 @@ __host__ __device__ inline uint32_t sdpa_lds_floats(uint32_t gt, uint32_t chunk,
            (fused && quant ? sdpa_quant_row_floats(qk_dim, v_dim) : 0);
 }
 
+// f(0), ... f(N - 1) with constant arguments.
+template <int N, typename F, int I = 0>
+__device__ __forceinline__ void each_index(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        each_index<N, F, I + 1>(static_cast<F&&>(f));
+    }
+}
+// Lane J of the caller's 16-lane row (row_newbcast); a value moved as a DPP control says.
+template <int J>
+__device__ __forceinline__ uint32_t row_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + J, 0xF, 0xF, false); }
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false)); }
+// The maximum over the wave's four 16-lane rows, lane by lane.
+__device__ __forceinline__ float rows_max(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 // One (range, kv head, head tile) work item.  Uniform per block; `kv_len` already read.
 // MODE 0: q is already rotated and the new K/V rows are in the cache.  MODE 1: a phase of the
 // whole-token kernel (kv_len known on entry, coherent stores); MODE 2: a kernel of its own.  In
@@ -94,7 +115,9 @@ __host__ __device__ inline uint32_t sdpa_lds_floats(uint32_t gt, uint32_t chunk,
 // the transforms' loads are issued ahead of the cache rows and used after them.
 // NOMERGE: the caller merges the ranges' results itself: every active block writes its (m, l, o) partial with
 // ordinary stores -- also when one range covers the context -- and returns; no arrival counter is touched.
-template <int GT, int MODE, typename ARGS, int KVQ = 0, bool FASTHEAD = false, bool NOMERGE = false>
+// ROW16: heads of 128 dims for keys and values, a row on 16 lanes (a quantised cache: two groups of 64, scale and bias arrays
+// 4-byte aligned).  See the wave-local form below.
+template <int GT, int MODE, typename ARGS, int KVQ = 0, bool FASTHEAD = false, bool NOMERGE = false, bool ROW16 = false>
 __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint32_t split, uint32_t kvh,
                                            uint32_t gz, uint32_t gz_count, float* lds, uint32_t kv_add = 0) {
     // kv_raw + kv_add positions are visible (kv_add: the row's index among several active rows).  The sum is formed
@@ -109,6 +132,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // the ranges of a block need no barrier; the waves meet once, after the last range.
     constexpr bool WAVES = MODE != 1 && GT <= 4;
     constexpr int kSteps = FUSED ? kSdpaStepsFused : kSdpaSteps;
+    static_assert(!ROW16 || (WAVES && kSteps == 4), "");
     static_assert(!(FUSED && KVQ != 0), "the whole-token kernel reads a bf16 cache");
     const uint32_t span = a.chunk_len * a.chunks_per_block;  // cache positions per block
     const uint32_t blk0 = split * span;
@@ -219,8 +243,8 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // ~60 registers that the 64 registers of in-flight rows would otherwise have to share.
     if constexpr (MODE == 1) transform_heads(0);
 
-    const uint32_t lpk = a.lpk, cpk = a.qk_dim >> 3;
-    const uint32_t lpv = a.lpv, cpv = a.v_dim >> 3;
+    const uint32_t lpk = ROW16 ? 16u : a.lpk, cpk = ROW16 ? 16u : a.qk_dim >> 3;
+    const uint32_t lpv = ROW16 ? 16u : a.lpv, cpv = ROW16 ? 16u : a.v_dim >> 3;
     const uint32_t ck = tid & (lpk - 1), kslot = tid / lpk, kslots = kSdpaBlock / lpk;
     const uint32_t cv = tid & (lpv - 1), vslot = tid / lpv, vslots = kSdpaBlock / lpv;
     const bool kcol_ok = ck < cpk, vcol_ok = cv < cpv;
@@ -231,6 +255,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         stat[tid] = -INFINITY;
         stat[8 + tid] = 0.f;
     }
+    float m_own = -INFINITY;     // ROW16: running maximum of the head whose score the lane finishes
     float m_run[GT], l_run[GT];  // wave-local form: running maximum (uniform) and this lane row's share of the sum
 #pragma unroll
     for (int h = 0; h < GT; ++h) {
@@ -292,7 +317,20 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // starts 8.8 us into the launch instead of 13.6; a bf16 cache is bound by the bytes and was 5 % slower with it).
     constexpr bool DEEP = MODE != 1 && WAVES && KVQ != 0;
     uint4 kn_[kSteps], vn_[kSteps], kf_[DEEP ? kSteps : 1], vf_[DEEP ? kSteps : 1];
-    auto request_rows = [&](uint4(&kd)[kSteps], uint4(&vd)[kSteps], uint32_t key0, uint32_t nkeys, bool owner,
+    // ROW16, quantised: lane 4 u + i of a row's 16 lanes holds both groups' entries of key row u in array i (scales and biases
+    // of the keys, of the values), so a range's take a wave ONE request -- two bytes a lane from each array and row they were 16
+    // of its 24, and a CU issues one in 16 .. 20 cycles.
+    constexpr bool META16 = ROW16 && KVQ != 0;
+    uint32_t mc = 0, mn_ = 0, mf_ = 0;
+    // (a global access: chosen among the arguments' pointers as they are, the arguments move to memory and the access is a flat one)
+    typedef const __attribute__((address_space(1))) uint32_t* gmeta;
+    gmeta mbase = nullptr;
+    if constexpr (META16) {
+        const uintptr_t ks = (uintptr_t)a.k_scales, kb = (uintptr_t)a.k_biases, vs = (uintptr_t)a.v_scales, vb = (uintptr_t)a.v_biases;
+        const uintptr_t kk = (lane & 1u) ? kb : ks, vv = (lane & 1u) ? vb : vs;
+        mbase = (gmeta)((lane & 2u) ? vv : kk);
+    }
+    auto request_rows = [&](uint4(&kd)[kSteps], uint4(&vd)[kSteps], uint32_t& md, uint32_t key0, uint32_t nkeys, bool owner,
                             uint32_t jpos) {
         const uint16_t* kbase = a.k + ((size_t)kvh * a.capacity + key0) * a.qk_dim + 8 * ck;
         const uint16_t* vbase = a.v + ((size_t)kvh * a.capacity + key0) * a.v_dim + 8 * cv;
@@ -308,12 +346,16 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
             const size_t kmeta = (size_t)kvh * a.capacity * kg + (8u * kcol) / a.kv_group;
             const size_t vmeta = (size_t)kvh * a.capacity * vg + (8u * vcol) / a.kv_group;
             const uint32_t last = a.capacity - 1;
+            if constexpr (META16) {
+                const uint32_t r0 = key0 + kslot + ((lane >> 2) & 3u) * kslots, r = r0 < last ? r0 : last;
+                md = mbase[(size_t)kvh * a.capacity + r];
+            }
 #pragma unroll
             for (int u = 0; u < kSteps; ++u) {
                 const uint32_t r0 = key0 + kslot + u * kslots, r = r0 < last ? r0 : last;
                 kd[u].x = kp[(size_t)r * kw];
                 kd[u].y = WPL == 2 ? kp[(size_t)r * kw + 1] : 0u;
-                kd[u].z = (uint32_t)a.k_scales[kmeta + (size_t)r * kg] | ((uint32_t)a.k_biases[kmeta + (size_t)r * kg] << 16);
+                kd[u].z = META16 ? 0u : (uint32_t)a.k_scales[kmeta + (size_t)r * kg] | ((uint32_t)a.k_biases[kmeta + (size_t)r * kg] << 16);
                 kd[u].w = 0u;
             }
 #pragma unroll
@@ -321,7 +363,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
                 const uint32_t r0 = key0 + vslot + u * vslots, r = r0 < last ? r0 : last;
                 vd[u].x = vp[(size_t)r * vw];
                 vd[u].y = WPL == 2 ? vp[(size_t)r * vw + 1] : 0u;
-                vd[u].z = (uint32_t)a.v_scales[vmeta + (size_t)r * vg] | ((uint32_t)a.v_biases[vmeta + (size_t)r * vg] << 16);
+                vd[u].z = META16 ? 0u : (uint32_t)a.v_scales[vmeta + (size_t)r * vg] | ((uint32_t)a.v_biases[vmeta + (size_t)r * vg] << 16);
                 vd[u].w = 0u;
             }
             return;
@@ -392,7 +434,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
             settle();
             if (split >= n_active) return;
         }
-        request_rows(kc, vc, blk0, 0, false, 0);
+        request_rows(kc, vc, mc, blk0, 0, false, 0);
         if constexpr (MODE == 0) settle_q();
         if constexpr (MODE == 2 && KVQ == 0)
             vnew = *reinterpret_cast<const uint4*>(a.v_new + (size_t)kvh * a.v_stride + (vcol_ok ? 8 * cv : 0u));
@@ -418,21 +460,35 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     }
 
     if constexpr (DEEP)
-        if (n_chunks > 1) request_rows(kn_, vn_, blk0 + a.chunk_len, 0, false, 0);
+        if (n_chunks > 1) request_rows(kn_, vn_, mn_, blk0 + a.chunk_len, 0, false, 0);
     for (uint32_t c = 0; c < n_chunks; ++c) {
     const uint32_t key0 = blk0 + c * a.chunk_len;
     const uint32_t nkeys = (kv_len - key0) < a.chunk_len ? (kv_len - key0) : a.chunk_len;
     const bool owner = XFORM && pos >= key0 && pos < key0 + nkeys;
     const uint32_t jpos = pos - key0;
     if constexpr (FUSED) {
-        request_rows(kc, vc, key0, nkeys, owner, jpos);
+        request_rows(kc, vc, mc, key0, nkeys, owner, jpos);
     } else if constexpr (DEEP) {
-        if (c + 2 < n_chunks) request_rows(kf_, vf_, key0 + 2 * a.chunk_len, 0, false, 0);
+        if (c + 2 < n_chunks) request_rows(kf_, vf_, mf_, key0 + 2 * a.chunk_len, 0, false, 0);
     } else {
-        if (c + 1 < n_chunks) request_rows(kn_, vn_, key0 + a.chunk_len, 0, false, 0);
+        if (c + 1 < n_chunks) request_rows(kn_, vn_, mn_, key0 + a.chunk_len, 0, false, 0);
     }
 
     FK_SDPA_STAMP(1);
+    uint32_t kz[kSteps], vz[kSteps];   // quantised: scale | bias << 16 of this lane's group of each row
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+        kz[u] = kc[u].z;
+        vz[u] = vc[u].z;
+    }
+    if constexpr (META16) {
+        const uint32_t half = ck >= 8u ? 0x07060302u : 0x05040100u;   // this lane's group
+        each_index<kSteps>([&](auto u) __attribute__((always_inline)) {
+            constexpr int U = decltype(u)::value;
+            kz[U] = __builtin_amdgcn_perm(row_lane<4 * U + 1>(mc), row_lane<4 * U>(mc), half);
+            vz[U] = __builtin_amdgcn_perm(row_lane<4 * U + 3>(mc), row_lane<4 * U + 2>(mc), half);
+        });
+    }
     if constexpr (XFORM) {
         if constexpr (KVQ != 0) {
             if (owner) {
@@ -441,8 +497,16 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
                 const uint32_t *kw = nword + kcol * WPL, *vw = nword + a.qk_dim / 4u + vcol * WPL;
 #pragma unroll
                 for (int u = 0; u < kSteps; ++u) {
-                    if (kslot + u * kslots == jpos) kc[u] = make_uint4(kw[0], kw[WPL - 1u], nmeta[8u * kcol / a.kv_group], 0u);
-                    if (vslot + u * vslots == jpos) vc[u] = make_uint4(vw[0], vw[WPL - 1u], nmeta[a.qk_dim / 32u + 8u * vcol / a.kv_group], 0u);
+                    if (kslot + u * kslots == jpos) {
+                        kc[u].x = kw[0];
+                        kc[u].y = kw[WPL - 1u];
+                        kz[u] = nmeta[8u * kcol / a.kv_group];
+                    }
+                    if (vslot + u * vslots == jpos) {
+                        vc[u].x = vw[0];
+                        vc[u].y = vw[WPL - 1u];
+                        vz[u] = nmeta[a.qk_dim / 32u + 8u * vcol / a.kv_group];
+                    }
                 }
             }
         } else if (owner && kcol_ok) {
@@ -456,14 +520,14 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         float d = 0.f;
         if constexpr (KVQ == 4) {
             d = q4_word_dot(kc[u].x, qf[h], 0.f);
-            d = fmaf(bf16_lo(kc[u].z), d, bf16_hi(kc[u].z) * sq[h]);  // s * sum(q * code) + b * sum(q)
+            d = fmaf(bf16_lo(kz[u]), d, bf16_hi(kz[u]) * sq[h]);  // s * sum(q * code) + b * sum(q)
         } else if constexpr (KVQ == 8) {
             const uint32_t w0 = kc[u].x, w1 = kc[u].y;
             d = dot2_bf16(pack_bf16((float)(w0 & 0xffu), (float)((w0 >> 8) & 0xffu)), qf[h].x, d);
             d = dot2_bf16(pack_bf16((float)((w0 >> 16) & 0xffu), (float)(w0 >> 24)), qf[h].y, d);
             d = dot2_bf16(pack_bf16((float)(w1 & 0xffu), (float)((w1 >> 8) & 0xffu)), qf[h].z, d);
             d = dot2_bf16(pack_bf16((float)((w1 >> 16) & 0xffu), (float)(w1 >> 24)), qf[h].w, d);
-            d = fmaf(bf16_lo(kc[u].z), d, bf16_hi(kc[u].z) * sq[h]);
+            d = fmaf(bf16_lo(kz[u]), d, bf16_hi(kz[u]) * sq[h]);
         } else {
             d = dot2_bf16(kc[u].x, qf[h].x, d);
             d = dot2_bf16(kc[u].y, qf[h].y, d);
@@ -498,8 +562,8 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     auto value = [&](int u, uint32_t j, float(&f)[8], float& vs, float& vb) {
         const bool ok = j < nkeys && vcol_ok;
         if constexpr (KVQ != 0) {
-            vs = ok ? bf16_lo(vc[u].z) : 0.f;
-            vb = ok ? bf16_hi(vc[u].z) : 0.f;
+            vs = ok ? bf16_lo(vz[u]) : 0.f;
+            vb = ok ? bf16_hi(vz[u]) : 0.f;
             if constexpr (KVQ == 4) {
                 const uint32_t even = vc[u].x & 0x0F0F0F0Fu, odd = (vc[u].x >> 4) & 0x0F0F0F0Fu;
                 f[0] = (float)(even & 0xffu); f[2] = (float)((even >> 8) & 0xffu);
@@ -529,9 +593,68 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         // ---------------- wave-local: scores, online softmax and value sums in registers ----------------
         // Scores and running maxima are kept in base-2 units (scale * log2(e) folded into one
         // multiply), so a probability is one v_exp_f32.
-        float pr[kSteps][GT];
-        scores_of(pr);
         const float scale2 = a.scale * 1.44269504088896341f;
+        float pr[kSteps][GT];
+        if constexpr (ROW16) {
+            // A row's 16 lanes each finish ONE of its 4 GT scores (fewer: several the same one): at every step of the butterfly
+            // a lane keeps the half of the sums that its own score is in and hands over the other -- the same additions -- then
+            // scales it and raises it to a probability alone, where every lane did so for all of them (16 exponentials of
+            // a quarter rate for one at four heads), and hands it round.  Score v = u GT + h is that of the lanes with
+            // bits (b0 ^ b2, b1 ^ b2, b2 ^ b3, b3) of v, which the row's half mirror and mirror pair as they need be.
+            // 32 q / 8 kv heads, every lane all scores / this: 32768 positions of a bf16 cache 40.5 / 36.8 us; with the scales'
+            // single request (META16) a token of the 4B-class model behind 12000 positions of an 8-bit cache 1938 / 1807 us.
+            constexpr int LH = GT == 4 ? 2 : (GT == 2 ? 1 : 0), LV = LH + 2;   // log2 of the heads, of the scores
+            const bool sel[4] = {((lane ^ (lane >> 2)) & 1u) != 0, (((lane >> 1) ^ (lane >> 2)) & 1u) != 0, (((lane >> 2) ^ (lane >> 3)) & 1u) != 0, (lane & 8u) != 0};
+            float x[kSteps * GT];
+#pragma unroll
+            for (int u = 0; u < kSteps; ++u)
+#pragma unroll
+                for (int h = 0; h < GT; ++h) x[u * GT + h] = score(u, h);
+            each_index<4>([&](auto step) __attribute__((always_inline)) {
+                constexpr int S = decltype(step)::value, CTRL = S == 0 ? 0xB1 : (S == 1 ? 0x4E : (S == 2 ? 0x141 : 0x140));
+                if constexpr (S < LV) {
+#pragma unroll
+                    for (int i = 0; i < (1 << (LV - 1 - S)); ++i) {   // (kept in place: sums i of the step's 2^(LV - S))
+                        const float keep = sel[S] ? x[2 * i + 1] : x[2 * i], give = sel[S] ? x[2 * i] : x[2 * i + 1];
+                        x[i] = keep + dpp_move<CTRL>(give);
+                    }
+                } else {
+                    x[0] = dpp_add<CTRL>(x[0]);
+                }
+            });
+            uint32_t own = 0;   // this lane's score
+#pragma unroll
+            for (int k = 0; k < LV; ++k) own |= sel[k] ? 1u << k : 0u;
+            const float mine = kslot + (own >> LH) * kslots < nkeys ? x[0] * scale2 : -INFINITY;
+            float mx = mine;   // of the lane's head: over the row's four keys, then the wave's four rows
+            each_index<4>([&](auto step) __attribute__((always_inline)) {
+                constexpr int S = decltype(step)::value, CTRL = S == 0 ? 0xB1 : (S == 1 ? 0x4E : (S == 2 ? 0x141 : 0x140));
+                if constexpr (S >= LH && S < LV) mx = dpp_max<CTRL>(mx);
+            });
+            mx = rows_max(mx);
+            const float m_new = fmaxf(m_own, mx), m_ref = m_new == -INFINITY ? 0.f : m_new;   // no live key yet: every term is 2^-inf = 0
+            const float alpha_own = __builtin_amdgcn_exp2f(m_own - m_ref), p_own = __builtin_amdgcn_exp2f(mine - m_ref);
+            m_own = m_new;
+            each_index<kSteps * GT>([&](auto v) __attribute__((always_inline)) {
+                constexpr int V = decltype(v)::value, B3 = (V >> 3) & 1, B2 = ((V >> 2) & 1) ^ B3, B1 = ((V >> 1) & 1) ^ B2, B0 = (V & 1) ^ B2;
+                pr[V / GT][V % GT] = __int_as_float((int)row_lane<8 * B3 + 4 * B2 + 2 * B1 + B0>((uint32_t)__float_as_int(p_own)));
+            });
+#pragma unroll
+            for (int h = 0; h < GT; ++h) {
+                const int bits = __builtin_amdgcn_readlane(__float_as_int(alpha_own), h);   // (lane h: score h)
+                const float alpha = __int_as_float(bits);
+                float psum = 0.f;
+#pragma unroll
+                for (int u = 0; u < kSteps; ++u) psum += pr[u][h];
+                l_run[h] = fmaf(l_run[h], alpha, psum);
+                if (bits != 0x3F800000) {  // the maximum rose (rare after the first ranges)
+                    accb[h] *= alpha;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) acc[h][i] *= alpha;
+                }
+            }
+        } else {
+        scores_of(pr);
 #pragma unroll
         for (int u = 0; u < kSteps; ++u) {
             const bool live = kslot + u * kslots < nkeys;
@@ -577,6 +700,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
 #pragma unroll
                 for (int i = 0; i < 8; ++i) acc[h][i] *= alpha;
             }
+        }
         }
 #pragma unroll
         for (int u = 0; u < kSteps; ++u) {
@@ -673,6 +797,8 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
                     vn_[u] = vf_[u];
                 }
             }
+            mc = mn_;
+            mn_ = mf_;
         }
     }
     }  // ranges of this block
@@ -687,6 +813,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
 #pragma unroll
         for (int h = 0; h < GT; ++h) {
             const float lw = wave_sum(l_run[h]) * inv_lanes;
+            if constexpr (ROW16) m_run[h] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m_own), h));
             if (lane == 0) {
                 wm[wave * 8 + h] = m_run[h];
                 wl[wave * 8 + h] = lw;
@@ -753,7 +880,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         const uint32_t h = e / a.v_dim, d = e - h * a.v_dim;
         float o = 0.f;
         // sixteen slots are read at once (every bf16 / quantised head of up to 128 dims has 16 or 32): read one by one, each
-        // waits out the LDS (heads of 128: 0.8 us of the launch, see the dispatch notes in sdpa.hip)
+        // waits out the LDS (heads of 128: 0.8 us of the launch)
         uint32_t sl = 0;
         for (; sl + 16 <= vslots; sl += 16) {
             float v[16];
@@ -896,7 +1023,7 @@ __device__ __forceinline__ uint32_t sdpa_load_kv_len(const SdpaArgs& a) {
 #endif
 }
 
-template <int GT, int KVQ = 0>
+template <int GT, int KVQ = 0, bool ROW16 = false>
 __global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_decode_kernel(const SdpaArgs a) {
     extern __shared__ __align__(16) float lds[];
     // One unconditional load (the immediate is read from the kernel-argument segment
@@ -905,7 +1032,7 @@ __global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_decode_kerne
     kernarg_warm<(int)sizeof(SdpaArgs)>();
     const uint32_t kv_len0 = sdpa_load_kv_len(a);
     if (a.rows <= 1) {
-        sdpa_block<GT, false, SdpaArgs, KVQ>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
+        sdpa_block<GT, false, SdpaArgs, KVQ, false, false, ROW16>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
         return;
     }
     // Several active rows (multi-token verification, chunked prefill): grid.z carries
@@ -918,19 +1045,19 @@ __global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_decode_kerne
     r.out = a.out + (size_t)tr * a.n_heads * a.v_dim;
     r.partials = a.partials + (size_t)tr * a.n_heads * a.n_splits * (a.v_dim + 2);
     r.counters = a.counters + (size_t)tr * a.n_kv * gz_count;
-    sdpa_block<GT, false, SdpaArgs, KVQ>(r, kv_len0, blockIdx.x, blockIdx.y, gz, gz_count, lds, tr);
+    sdpa_block<GT, false, SdpaArgs, KVQ, false, false, ROW16>(r, kv_len0, blockIdx.x, blockIdx.y, gz, gz_count, lds, tr);
 }
 
 // RoPE (+ head norm) of q and of the new k row, the cache append and the attention in one
 // launch: a.q / a.k_new / a.v_new are the raw projection outputs of the token at position
 // kv_len - 1, a.k / a.v the cache it is appended to.
 // KVQ: a quantised cache; the new rows are quantised by the block whose range holds them.
-template <int GT, bool FASTHEAD, int KVQ = 0>
+template <int GT, bool FASTHEAD, int KVQ = 0, bool ROW16 = false>
 __global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_rope_store_kernel(const SdpaArgs a) {
     extern __shared__ __align__(16) float lds[];
     kernarg_warm<(int)sizeof(SdpaArgs)>();
     const uint32_t kv_len0 = sdpa_load_kv_len(a);
-    sdpa_block<GT, 2, SdpaArgs, KVQ, FASTHEAD>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
+    sdpa_block<GT, 2, SdpaArgs, KVQ, FASTHEAD, false, ROW16>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
 }
 
 }  // namespace fk

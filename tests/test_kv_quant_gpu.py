@@ -161,6 +161,42 @@ def test_store_then_attend_matches_bf16_cache(fk):
     assert rel_l2(o1.to_numpy(np.uint16), oracle.bf16_to_f32(o2.to_numpy(np.uint16))) <= 2e-2
 
 
+class _Shifted:
+    """A quantised cache whose scale and bias arrays lie two bytes past a multiple of four."""
+
+    def __init__(self, fk, c):
+        self.__dict__.update({n: getattr(c, n) for n in ("n_kv", "capacity", "dim", "bits", "group", "packed")})
+        one = np.zeros(1, np.uint16)
+        self.held = [fk.DeviceBuffer.from_numpy(np.concatenate([one, b.to_numpy(np.uint16)])) for b in (c.scales, c.biases)]
+        self.c = type(c.c)(c.packed.ptr, *(b.ptr + 2 for b in self.held))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("n_heads,n_kv,kv_len,max_len,rows", [
+    (2, 2, 1, 1, 1), (4, 2, 15, 16, 1), (8, 2, 17, 64, 3),          # a head a block, one range
+    (8, 2, 2048, 2048, 1),                                          # several ranges, their merge
+    (4, 4, 2999, 3001, 2), (4, 2, 2113, 2120, 1), (8, 2, 4095, 4100, 1),   # tiles of 1, 2 and 4 heads, ranges that a block walks
+])
+def test_attention_of_128_dims_equals_the_general_form_bit_for_bit(fk, bits, n_heads, n_kv, kv_len, max_len, rows):
+    """Heads of 128 dims with groups of 64: every lane finishes its own scores and a range's scales and biases come with one
+    request; scale arrays that are not 4-byte aligned take the general form.  The same sums in the same order."""
+    dim, cap, group = 128, max_len + rows - 1, 64
+    rows_k, rows_v = normal_bf16(70, (n_kv, cap, dim)), normal_bf16(71, (n_kv, cap, dim))
+    rows_k[:, cap // 3] = 0                                          # a group of one value
+    K, V = _caches(fk, n_kv, cap, dim, bits, group)
+    flat = lambda x: _dev(fk, np.ascontiguousarray(x.transpose(1, 0, 2)).reshape(cap, n_kv * dim))
+    fk.kv_cache_store_quant(flat(rows_k), flat(rows_v), None, n_kv, dim, 0, 1e4, 0.0, None, 0, cap, K, V)
+    q = _dev(fk, normal_bf16(72, (rows, n_heads * dim), 3.0))
+    got = []
+    for k, v in ((K, V), (_Shifted(fk, K), _Shifted(fk, V))):
+        out = fk.DeviceBuffer(2 * rows * n_heads * dim)
+        pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, dim, dim, cap)
+        fk.sdpa_decode_quant(q, k, v, out, None, kv_len, cap, rows, n_heads, dim ** -0.5, fk.DeviceBuffer(max(pb, 4) * rows),
+                             fk.zeros(max(cb, 4) * rows))
+        got.append(out.to_numpy(np.uint16, (rows, n_heads, dim)))
+    assert np.isfinite(oracle.bf16_to_f32(got[0])).all() and np.array_equal(got[0], got[1])
+
+
 def test_rejects_bad_geometry(fk):
     K, V = _caches(fk, 2, 16, 128, 4, 64)
     k = _dev(fk, normal_bf16(1, 256))
