@@ -207,10 +207,8 @@ struct RowsRequest {
     uint32_t M = 0, x_stride = 0;      // x_stride 0: K
     const uint16_t* norm_w = nullptr;  // RMSNorm of the rows on the way in
     float eps = 0.f;
-    const float* ssq_in = nullptr;     // x holds weighted rows T(w * x) as the launch that wrote them left them, with their sums of squares
-    float* ssq_out = nullptr;          // single matrix: leave those of the outputs, rows_ssq_parts(N) floats per row,
-    uint16_t* yw = nullptr;            // and T(yw_w * y), dense rows
-    const uint16_t* yw_w = nullptr;
+    const float* ssq_in = nullptr;     // with norm_w: the rows' sums of squares as the launch that wrote the rows left them
+    float* ssq_out = nullptr;          // single matrix: leave those of the outputs, rows_ssq_parts(N) floats per row
     const uint16_t* bias[3] = {nullptr, nullptr, nullptr};
     const uint16_t* res = nullptr;
     int variant = 0;

@@ -4,7 +4,7 @@
 // A pass is some ten launches per layer.  Called one by one through the operator entry points from Python each costs 7..10 us
 // of host time, more than a short prompt's kernels run for; from here a launch costs what the runtime takes (3.7 us), so that
 // the GPU is what a pass waits for.  37 tokens of the 0.5B-class model, whole call: 1378 us from Python, 1055 from here
-// with the norms inside the projections (two launches per layer fewer), 957 with T(w * x) written beside x; of 512 tokens of the 4B-class model 7279 us with the
+// with the norms inside the projections (two launches per layer fewer); of 512 tokens of the 4B-class model 7279 us with the
 // norms in launches of their own, 7046 with them in the launches that add split sums up.
 #include <math.h>
 
@@ -13,23 +13,16 @@
 namespace fk {
 namespace {
 
-// Up to 64 rows a norm between two projections has no launch of its own and no pass over the rows: the launch that writes the
-// rows x leaves T(w * x) and their sums of squares beside them, the next one multiplies its finished fp32 sums by 1 / rms (one
-// rounding fewer than T(w * T(x / rms)): 1.65e-3 of the product against float64 where that has 2.33e-3).  37 rows of the
-// 0.5B-class model: 998 -> 957 us a prompt; of 41 us a layer it took the norm ahead of the pair (2.7) and what q / k / v spent
-// on theirs (1.2).
-// The rows from the embedding come without: the projection's own launch forms T(w * T(x / rms)) on the way in, every block for
-// all rows, about 0.4 us per million values, or the norm has a launch of its own of some 3.5 us.  (On the way in, 37 rows of
-// K = 896: 1152 outputs, 2.4 million values, 5.4 us against 4.1 + 4.1; a 4864 pair, 10 million, 15.2 against 10.1 + 4.1.)
+// Whether a projection of N outputs takes the form of up to 64 rows AND the RMSNorm ahead of it: the form normalises on the
+// way in (with the sums of squares that the launch which wrote the rows left), but every block does so for all rows, about
+// 0.4 us per million values it normalises, where the norm as a launch of its own costs some 3.5 us.  37 rows of K = 896:
+// 1152 outputs (2.4 million) 5.4 us against 4.1 + 4.1, a 4864 pair (10 million) 15.2 against 10.1 + 4.1; 50 rows of
+// K = 2560, a 9728 pair (78 million) 54 against 30 + 5.
 // (Rows and norm weights that are not 16-byte aligned take the norm's own launch.)
 bool takes_norm(const fk_weight& W, uint32_t rows, uint32_t n_total, const uint16_t* x, const uint16_t* norm_w) {
     return qgemm_takes_rows(rows, W.bits, W.group, W.k) && (uint64_t)rows * W.k * ((n_total + 15u) / 16u) < 8000000ull &&
            (((uintptr_t)x | (uintptr_t)norm_w) & 15u) == 0;
 }
-bool qkv_in_one(const fk_prompt_layer& l) {
-    return l.k.bits == l.q.bits && l.v.bits == l.q.bits && l.k.group == l.q.group && l.v.group == l.q.group;
-}
-bool pair_in_one(const fk_prompt_layer& l) { return l.gate.bits == l.up.bits && l.gate.group == l.up.group; }
 
 fk_status run_rows(const RowsRequest& rq, hipStream_t s) {
     Launch l;
@@ -64,28 +57,23 @@ fk_status matmul(const fk_prompt_model& m, const fk_weight& W, const uint16_t* x
 }
 
 // What the launch that wrote a projection's input rows left in m.xn, free between a projection's launch and the next norm.
-enum Left { LEFT_NOTHING, LEFT_WEIGHTED /* T(w * x), the rows' sums of squares in `parts` */, LEFT_NORMED /* the normalised rows */ };
+enum Left { LEFT_NOTHING, LEFT_SQUARES /* the rows' sums of squares */, LEFT_NORMED /* the normalised rows */ };
 
-// One matrix with the residual.  next: the matrix that its rows enter next, through a norm of the weights next_norm, or null;
-// parts: where their sums of squares may be left (rows of n_q values that nothing reads meanwhile).
+// One matrix with the residual; next_norm: the weights of the norm that its rows enter next, or null.
 fk_status residual_rows(const fk_prompt_model& m, const fk_weight& W, const uint16_t* x, uint32_t rows, const uint16_t* res, uint16_t* y,
-                        const fk_weight* next, const uint16_t* next_norm, uint16_t* parts, Left* left, hipStream_t s) {
-    *left = LEFT_NOTHING;
-    if (m.kv_bits || !next_norm || !m.xn) return matmul(m, W, x, rows, nullptr, res, y, s);
-    if (qgemm_takes_rows(rows, W.bits, W.group, W.k) && W.n % 64u == 0 && ((uintptr_t)m.xn & 15u) == 0) {
-        RowsRequest rq;
-        rq.W[0] = &W; rq.x = x; rq.M = rows; rq.res = res; rq.y[0] = y;
-        if (next && qgemm_takes_rows(rows, next->bits, next->group, next->k) && ((uintptr_t)parts & 15u) == 0 &&
-            rows_ssq_parts(W.n) * sizeof(float) <= (size_t)m.n_heads * m.head_dim * sizeof(uint16_t)) {
-            rq.ssq_out = reinterpret_cast<float*>(parts); rq.yw = m.xn; rq.yw_w = next_norm;
-            *left = LEFT_WEIGHTED;
-        }
-        return run_rows(rq, s);
+                        const uint16_t* next_norm, Left* left, hipStream_t s) {
+    const bool ssq = m.kv_bits == 0 && qgemm_takes_rows(rows, W.bits, W.group, W.k) && W.n % 64u == 0 && ((uintptr_t)m.xn & 15u) == 0;
+    *left = ssq ? LEFT_SQUARES : LEFT_NOTHING;
+    if (!ssq) {
+        RowsNorm norm{next_norm, m.xn, m.eps};
+        FK_TRY(matmul(m, W, x, rows, nullptr, res, y, s, next_norm && m.xn && m.kv_bits == 0 ? &norm : nullptr));
+        if (norm.done) *left = LEFT_NORMED;
+        return FK_OK;
     }
-    RowsNorm norm{next_norm, m.xn, m.eps};
-    FK_TRY(matmul(m, W, x, rows, nullptr, res, y, s, &norm));
-    if (norm.done) *left = LEFT_NORMED;
-    return FK_OK;
+    RowsRequest rq;
+    rq.W[0] = &W; rq.x = x; rq.M = rows; rq.res = res; rq.y[0] = y;
+    rq.ssq_out = reinterpret_cast<float*>(m.xn);
+    return run_rows(rq, s);
 }
 
 fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, const fk_prompt_layer* next, Left* left, uint32_t rows,
@@ -102,18 +90,12 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, const f
     FanSums sums{};   // (one split, or another kernel: finished rows)
     const bool takes_sums = m.kv_bits == 0 && rope_takes_sums(rope) && l.q.n == m.n_heads * dim && l.k.n == m.n_kv * dim && l.v.n == l.k.n;
     const bool tiled = dim == 64 || dim == 128;
-    if (*left == LEFT_WEIGHTED ||
-        (m.kv_bits == 0 && *left == LEFT_NOTHING && qkv_in_one(l) && takes_norm(l.q, rows, l.q.n + l.k.n + l.v.n, m.x, l.input_norm))) {
+    if (m.kv_bits == 0 && *left != LEFT_NORMED && l.k.bits == l.q.bits && l.v.bits == l.q.bits && l.k.group == l.q.group && l.v.group == l.q.group &&
+        takes_norm(l.q, rows, l.q.n + l.k.n + l.v.n, m.x, l.input_norm)) {
         RowsRequest rq;
         rq.W[0] = &l.q; rq.W[1] = &l.k; rq.W[2] = &l.v; rq.n_mats = 3;
-        rq.M = rows; rq.eps = m.eps;
-        if (*left == LEFT_WEIGHTED) {
-            rq.x = m.xn;
-            rq.ssq_in = reinterpret_cast<const float*>(m.att);
-        } else {
-            rq.x = m.x;
-            rq.norm_w = l.input_norm;
-        }
+        rq.x = m.x; rq.M = rows; rq.norm_w = l.input_norm; rq.eps = m.eps;
+        if (*left == LEFT_SQUARES) rq.ssq_in = reinterpret_cast<const float*>(m.xn);   // (not where the rows come from the embedding)
         rq.bias[0] = l.q_bias; rq.bias[1] = l.k_bias; rq.bias[2] = l.v_bias;
         rq.y[0] = m.q; rq.y[1] = m.k; rq.y[2] = m.v;
         FK_TRY(run_rows(rq, (hipStream_t)s));
@@ -150,12 +132,12 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, const f
             FK_TRY(fk_sdpa_decode_rows(m.q, l.cache_k, l.cache_v, m.att, rows, pos + 1, m.n_heads, m.n_kv, dim, dim, m.capacity, scale,
                                        m.partials, m.counters, s));
     }
-    FK_TRY(residual_rows(m, l.o, m.att, rows, m.x, m.x2, pair_in_one(l) ? &l.gate : nullptr, l.post_norm, m.q, left, (hipStream_t)s));
-    if (*left == LEFT_WEIGHTED) {
+    FK_TRY(residual_rows(m, l.o, m.att, rows, m.x, m.x2, l.post_norm, left, (hipStream_t)s));
+    if (*left == LEFT_SQUARES && l.gate.bits == l.up.bits && l.gate.group == l.up.group && takes_norm(l.gate, rows, l.gate.n, m.x2, l.post_norm)) {
         RowsRequest rq;
         rq.W[0] = &l.gate; rq.W[1] = &l.up; rq.n_mats = 2; rq.pair = true;
-        rq.x = m.xn; rq.M = rows; rq.eps = m.eps; rq.variant = m.swiglu_variant;
-        rq.ssq_in = reinterpret_cast<const float*>(m.q);
+        rq.x = m.x2; rq.M = rows; rq.norm_w = l.post_norm; rq.eps = m.eps; rq.variant = m.swiglu_variant;
+        rq.ssq_in = reinterpret_cast<const float*>(m.xn);
         rq.y[0] = m.mid;
         FK_TRY(run_rows(rq, (hipStream_t)s));
     } else {
@@ -172,8 +154,7 @@ fk_status layer_pass(const fk_prompt_model& m, const fk_prompt_layer& l, const f
             FK_TRY(run_qgemm_swiglu(&l.gate, &l.up, m.xn, rows, m.swiglu_variant, m.mid, m.workspace, m.kv_bits != 0, (hipStream_t)s));
         }
     }
-    return residual_rows(m, l.down, m.mid, rows, m.x2, m.x, next && qkv_in_one(*next) ? &next->q : nullptr, next ? next->input_norm : nullptr, m.att, left,
-                         (hipStream_t)s);
+    return residual_rows(m, l.down, m.mid, rows, m.x2, m.x, next ? next->input_norm : nullptr, left, (hipStream_t)s);
 }
 
 }  // namespace

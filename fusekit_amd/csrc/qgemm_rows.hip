@@ -47,12 +47,10 @@ struct QgemmRowsArgs {
     const uint16_t* x;        // M rows of K values, x_stride apart
     const uint16_t* res;      // like y[0], or null (single matrix)
     const uint16_t* norm_w;   // the rows enter as T(w * T(x * r)), r = 1 / rms of the row; null: as they are
-    // Rows that the launch which wrote them left as T(w * x), with sums of squares ssq_in[row * ssq_n + i], i < ssq_n: their r
-    // multiplies the finished sums (or null).  And where this launch leaves those of its outputs (single matrix): yw, yw_w.
+    // sums of squares of the rows, as the launch that wrote them left them (or null: formed here, in one more pass over
+    // the rows): ssq_in[row * ssq_n + i], i < ssq_n; and where this launch leaves those of its outputs (single matrix)
     const float* ssq_in;
     float* ssq_out;
-    uint16_t* yw;
-    const uint16_t* yw_w;
     uint32_t ssq_n;
     float eps;
     uint32_t M, K, n_seg, x_stride;
@@ -163,22 +161,21 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     };
     // ONE: four entries of each row's scales and biases, from the wave's first group or, at a row's end, the row's last four
     [[maybe_unused]] const uint32_t e_first = ONE ? ((g0 >> a.gshift) + 4u <= gpr ? g0 >> a.gshift : gpr - 4u) : 0u;
-    // What the epilogue's first outputs of this thread add.
+    // What the epilogue's first outputs of this thread add (a null operand reads the activations instead and is not used).
     constexpr uint32_t OUT = 16u * CT;
-    constexpr int EARLY = MT * NT > 6 ? 0 : 2;   // (no registers left for them beyond)
+    constexpr int EARLY = 2;
     const uint32_t yst = a.y_stride[seg];
     const uint16_t* res = a.res ? a.res + (size_t)m0 * yst : nullptr;
     const uint16_t* bias = a.bias[seg];
-    [[maybe_unused]] uint32_t e_bias[EARLY + 1] = {}, e_res[EARLY + 1] = {}, e_norm[EARLY + 1] = {};
+    [[maybe_unused]] uint32_t e_bias[EARLY], e_res[EARLY];
     auto fetch_epilogue = [&]() __attribute__((always_inline)) {
         if constexpr (!PAIR) {
 #pragma unroll
             for (int k = 0; k < EARLY; ++k) {
                 const uint32_t e = (uint32_t)k * (WAVES * kWave) + threadIdx.x, m = e / OUT, n = blk * OUT + e % OUT;
                 const uint32_t mc = m < M ? m : M - 1u, nc = n < N ? n : N - 1u;
-                if (bias) e_bias[k] = bias[nc];
-                if (res) e_res[k] = res[(size_t)mc * yst + nc];
-                if (a.yw) e_norm[k] = a.yw_w[nc];
+                e_bias[k] = *(bias ? bias + nc : a.x);
+                e_res[k] = *(res ? res + (size_t)mc * yst + nc : a.x);
             }
         }
     };
@@ -286,10 +283,12 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     fetch_x(g0 + 1u, x1);
     if constexpr (!ONE) fetch_w(g0 + SG, w1);
     fetch_epilogue();
-    float* tot = reinterpret_cast<float*>(reinterpret_cast<char*>(lds_raw) + WAVES * rows_wave_lds(MT, NT));   // [MT * 16] 1 / rms, past the sums' place too
-    if (a.ssq_in) {
-        // sixteen lanes a row, four rows a wave and step, every step's requests made before the first is used; the barriers
-        // before the epilogue are this one's too
+    float rr[MT][2];   // 1 / rms of the rows this lane parks
+#pragma unroll
+    for (int i = 0; i < MT; ++i) rr[i][0] = rr[i][1] = 1.f;
+    if (normed && a.ssq_in) {
+        float* tot = reinterpret_cast<float*>(reinterpret_cast<char*>(lds_raw) + WAVES * rows_wave_lds(MT, NT));   // [MT * 16]
+        // sixteen lanes a row, four rows a wave and step, every step's requests made before the first is used
         constexpr int STEPS = (MT * 16 + 4 * WAVES - 1) / (4 * WAVES);
         float v[STEPS];
 #pragma unroll
@@ -307,11 +306,15 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
             const float t = group_sum(v[i], 16);
             if (c16 == 0 && m < MT * 16u) tot[m] = 1.0f / sqrtf(t / (float)K + a.eps);
         }
-    }
-    float rr[MT][2];   // 1 / rms of the rows this lane parks
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < MT; ++i) rr[i][0] = rr[i][1] = 1.f;
-    if (normed) {
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t m = (uint32_t)i * 16u + r8 + 8u * (uint32_t)h;
+                rr[i][h] = tot[m];
+            }
+    } else if (normed) {
         // the squares of the wave's own columns, the first weights on their way meanwhile; the waves add them up in LDS
         float ss[MT][2];
 #pragma unroll
@@ -420,7 +423,7 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     __syncthreads();
     uint16_t* yo = a.y[seg] + (size_t)m0 * yst;
     // One round of outputs; EARLY ones have their operands already.
-    auto outputs = [&](uint32_t e0, auto early, uint32_t bias_bits, uint32_t res_bits, uint32_t norm_bits) __attribute__((always_inline)) {
+    auto outputs = [&](uint32_t e0, auto early, uint32_t bias_bits, uint32_t res_bits) __attribute__((always_inline)) {
         const uint32_t e = e0 + threadIdx.x, m = e / OUT, col = e % OUT, n = blk * OUT + col;
         const bool live = m < M && n < N;
         uint32_t o = 0;
@@ -432,20 +435,12 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
                 s0 += at[(uint32_t)w * PER_WAVE];
                 if constexpr (PAIR) s1 += at[(uint32_t)w * PER_WAVE + OUT];
             }
-            if (a.ssq_in) {
-                s0 *= tot[m];
-                if constexpr (PAIR) s1 *= tot[m];
-            }
             if constexpr (PAIR) {
                 o = swiglu_bits(s0, s1, a.variant, 1.0f);
             } else {
                 if (bias) s0 += bf16_bits_to_f32(decltype(early)::value ? bias_bits : (uint32_t)bias[n]);
                 if (res) s0 += bf16_bits_to_f32(decltype(early)::value ? res_bits : (uint32_t)res[(size_t)m * yst + n]);
                 o = f32_to_bf16_bits(s0);
-                if (a.yw) {
-                    const uint32_t w = decltype(early)::value ? norm_bits : (uint32_t)a.yw_w[n];
-                    a.yw[(size_t)(m0 + m) * N + n] = (uint16_t)f32_to_bf16_bits(bf16_bits_to_f32(w) * bf16_bits_to_f32(o));
-                }
             }
             yo[(size_t)m * yst + n] = (uint16_t)o;
         }
@@ -458,12 +453,12 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     };
     constexpr uint32_t ROUND = WAVES * kWave;
     if constexpr (PAIR) {
-        for (uint32_t e0 = 0; e0 < M * OUT; e0 += ROUND) outputs(e0, std::false_type{}, 0u, 0u, 0u);
+        for (uint32_t e0 = 0; e0 < M * OUT; e0 += ROUND) outputs(e0, std::false_type{}, 0u, 0u);
     } else {
 #pragma unroll
         for (int k = 0; k < EARLY; ++k)
-            if ((uint32_t)k * ROUND < M * OUT) outputs((uint32_t)k * ROUND, std::true_type{}, e_bias[k], e_res[k], e_norm[k]);
-        for (uint32_t e0 = EARLY * ROUND; e0 < M * OUT; e0 += ROUND) outputs(e0, std::false_type{}, 0u, 0u, 0u);
+            if ((uint32_t)k * ROUND < M * OUT) outputs((uint32_t)k * ROUND, std::true_type{}, e_bias[k], e_res[k]);
+        for (uint32_t e0 = EARLY * ROUND; e0 < M * OUT; e0 += ROUND) outputs(e0, std::false_type{}, 0u, 0u);
     }
 }
 
@@ -526,11 +521,9 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
         if (a.y_stride[i] < W->n) return set_error(FK_ERR_INVALID, "qgemm (rows): output row stride below the matrix's rows");
         b16 += (W->n + 15u) / 16u;
     }
-    if ((rq.ssq_out || rq.yw) && (rq.pair || rq.n_mats != 1 || !rq.ssq_out || !rq.yw || !rq.yw_w))
-        return set_error(FK_ERR_INVALID, "qgemm (rows): weighted rows and their sums of squares come together, from a single matrix");
-    if (rq.ssq_in && rq.norm_w) return set_error(FK_ERR_INVALID, "qgemm (rows): weighted rows take no norm");
+    if (rq.ssq_out && (rq.pair || rq.n_mats != 1)) return set_error(FK_ERR_INVALID, "qgemm (rows): sums of squares come from a single matrix");
     a.x = rq.x; a.res = rq.res; a.norm_w = rq.norm_w; a.eps = rq.eps;
-    a.ssq_in = rq.ssq_in; a.ssq_out = rq.ssq_out; a.yw = rq.yw; a.yw_w = rq.yw_w;
+    a.ssq_in = rq.ssq_in; a.ssq_out = rq.ssq_out;
     a.ssq_n = rq.ssq_out ? rows_ssq_parts(W0->n) : rows_ssq_parts(K);
     a.M = M; a.K = K; a.x_stride = x_stride; a.variant = rq.variant;
     a.n_seg = rq.pair ? 1u : rq.n_mats;
