@@ -108,20 +108,16 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     int gt = !same_lanes ? 8 : (G >= 8 ? 8 : (G >= 4 ? (G == 4 ? 4 : 8) : (G >= 2 ? (G == 2 ? 2 : 4) : 1)));
     // Groups of 2 .. 4 query heads per KV head: smaller tiles mean more blocks with fewer registers each, and the
     // repeated K / V reads of a KV head's tiles hit the L2.  Measured (32 q / 8 kv heads x 128, cold caches), tiles
-    // of 1 / 2 / 4 heads: 512 positions 7.9 / 8.5 / 9.1 us, 4096 16.5 / 14.6 / 16.0, 32768 53.8 / 42.0 / 41.7;
-    // the 4B decode loop at context 64 .. 576: 568 / 566 / 550 tokens/s.
-    // (a quantised cache keeps its larger tile beyond 2048 positions: int4 at 32768 ran 41.4 us with 4 heads, 44.4 with 2)
-    if (same_lanes && G >= 2 && G <= 4) gt = max_len <= 2048 ? 1 : (kvq ? gt : 2);
+    // of 1 / 2 / 4 heads: 512 positions 7.2 / 7.9 / 8.3 us, 4096 12.6 / 13.5 / 14.2, 8192 17.3 / 18.4 / 17.5, 32768 47.8 / 37.8 / 37.6.
+    // (a quantised cache has other kernels and a merge that must stay as it is: its larger tile beyond 2048 positions)
+    if (same_lanes && G >= 2 && G <= 4) gt = max_len <= (kvq ? 2048u : 4096u) ? 1 : (kvq ? gt : 2);
     // Larger groups (the tile of 8 goes through LDS, three block barriers per range).  14 q / 2 kv heads x 64, time of the
     // task alone with tiles of 8 / 4 / 2 / 1 heads: 544 positions 15.8 / 11.9 / 10.7 / 9.8 us, 4096 18.4 / 14.2 / 14.2 /
     // 13.4, 12032 30.6 / 19.1 / 17.7 / 18.6.  (Not over a quantised cache: the two forms differ in the last bit, and what
     // follows from that -- a key whose group takes the other sign of its scale -- stays in the cache.)
     if (same_lanes && G > 4 && !kvq) gt = max_len <= 4096 ? 1 : 2;
-    // Long contexts: a block walks several consecutive ranges (online softmax, the next
-    // range's rows in flight), so that the grid stays near one to two blocks per CU and
-    // the final merge, which costs one memory round trip per 16 partials, stays short.
-    // Measured (32 q / 8 kv heads x 128): 4096 positions are fastest with 32 splits,
-    // 32768 with 64.
+    // Long contexts: a block walks several consecutive ranges (online softmax, the next range's rows in flight), so that the
+    // grid stays near one to two blocks per CU and the final merge, which draws every partial into one CU, stays short.
     // (several active rows multiply the tiles: each row then needs fewer ranges to fill the chip; 8 rows x 16 heads at
     // a capacity of 1024 ran 16 ranges per row and head -- 2048 blocks, most of them past the context -- in 14.4 us; with as
     // many blocks as CUs a block of those walks its ranges alone on its CU, so from four rows on there are two a CU: a layer of
@@ -130,6 +126,15 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     // merge is the last bit of a row)
     const uint32_t tiles = n_kv * ((G + gt - 1) / gt) * rows;
     uint32_t want = (n_chunks > 128 || (rows >= 4 && !kvq) ? 2u : 1u) * (uint32_t)dev->cus / tiles;
+    // Up to 4096 positions, in groups: two blocks a CU where one would walk four ranges or more, up to the 16 that a merge has
+    // from one trip to memory.  Tiles of one head, one a CU (for 2049 positions and more as it was, tiles of two) / this: 32 q / 8 kv x 128,
+    // 2048 positions 10.5 / 10.2 us, 3300 12.9 / 12.1, 4096 13.5 / 12.7; 28 / 4, 4096 14.3 / 12.3; 64 / 8, 1000 10.1 / 9.6, 4096
+    // 22.0 / 16.2.  Where one a CU walks fewer it is the slower: 32 / 8, 1000 positions 8.4 / 8.8; and with a KV head per query
+    // head, whose reads share nothing: 32 / 32, 2048 positions 12.7 / 13.6.
+    if (rows == 1 && same_lanes && !kvq && G >= 2 && max_len <= 4096 && want < 16u && n_chunks > 3u * want) {
+        const uint32_t two = 2u * (uint32_t)dev->cus / tiles;
+        want = two < 16u ? two : 16u;
+    }
     if (want < 1) want = 1;
     if (want > 256) want = 256;
     const uint32_t cpb = (n_chunks + want - 1) / want;
