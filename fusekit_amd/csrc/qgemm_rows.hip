@@ -161,13 +161,14 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     };
     // ONE: four entries of each row's scales and biases, from the wave's first group or, at a row's end, the row's last four
     [[maybe_unused]] const uint32_t e_first = ONE ? ((g0 >> a.gshift) + 4u <= gpr ? g0 >> a.gshift : gpr - 4u) : 0u;
-    // What the epilogue's first outputs of this thread add (a null operand reads the activations instead and is not used).
+    // What the epilogue's first outputs of this thread add (a null operand reads the activations instead and is not used: asked for
+    // under a condition 37 rows of 6144 x 2560 are at 12.4 us instead of 11.9).
     constexpr uint32_t OUT = 16u * CT;
-    constexpr int EARLY = 2;
+    constexpr int EARLY = MT * NT > 6 ? 0 : 2;   // (beyond, no registers are left for them: 64 rows of 6144 x 2560 at 16.7 us instead of 14.9)
     const uint32_t yst = a.y_stride[seg];
     const uint16_t* res = a.res ? a.res + (size_t)m0 * yst : nullptr;
     const uint16_t* bias = a.bias[seg];
-    [[maybe_unused]] uint32_t e_bias[EARLY], e_res[EARLY];
+    [[maybe_unused]] uint32_t e_bias[EARLY + 1] = {}, e_res[EARLY + 1] = {};
     auto fetch_epilogue = [&]() __attribute__((always_inline)) {
         if constexpr (!PAIR) {
 #pragma unroll
