@@ -53,6 +53,38 @@ fk_status sdpa_workspace_bytes(uint32_t n_heads, uint32_t n_kv, uint32_t qk_dim,
     return FK_OK;
 }
 
+namespace {
+
+// The kernels by tile, cache and row form (tiles of 8 heads over a bf16 cache have the general one only).
+template <int GT, int Q>
+const void* decode_func(int row) {
+    if constexpr (GT <= 4 || Q != 0) {
+        if (row == 16) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 16>);
+        if (row == 8) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 8>);
+    }
+    return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 0>);
+}
+template <int GT, bool F, int Q>
+const void* fused_func(int row) {
+    if constexpr (GT <= 4 || Q != 0) {
+        if (row == 16) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 16>);
+        if (row == 8) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 8>);
+    }
+    return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 0>);
+}
+template <int Q>
+const void* decode_func(int gt, int row) {
+    return gt == 1 ? decode_func<1, Q>(row) : (gt == 2 ? decode_func<2, Q>(row) : (gt == 4 ? decode_func<4, Q>(row) : decode_func<8, Q>(row)));
+}
+template <bool F, int Q>
+const void* fused_tile(int gt, int row) {
+    return gt == 1 ? fused_func<1, F, Q>(row) : (gt == 2 ? fused_func<2, F, Q>(row) : (gt == 4 ? fused_func<4, F, Q>(row) : fused_func<8, F, Q>(row)));
+}
+template <int Q>
+const void* fused_func(bool fast, int gt, int row) { return fast ? fused_tile<true, Q>(gt, row) : fused_tile<false, Q>(gt, row); }
+
+}  // namespace
+
 fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* out,
                            const uint32_t* kv_len_ptr, uint32_t kv_len_imm, uint32_t max_len, uint32_t n_heads,
                            uint32_t n_kv, uint32_t qk_dim, uint32_t v_dim, uint32_t capacity, float scale,
@@ -176,52 +208,21 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     a.partials = partials;
     a.counters = counters;
 
-    // heads of 128 dims on 16 lanes a row: each lane finishes its own scores (sdpa_block, ROW16)
-    const bool row16 = gt <= 4 && qk_dim == 128 && v_dim == 128 &&
-                       (!kvq || (quant->group == 64 && (((uintptr_t)quant->k_scales | (uintptr_t)quant->k_biases | (uintptr_t)quant->v_scales |
-                                                         (uintptr_t)quant->v_biases) & 3u) == 0));
+    // heads of 128 (64) dims on 16 (8) lanes a row: each lane finishes its own scores, scales and biases together (sdpa_block, ROW;
+    // the general form / this, 64 dims: 16 q / 4 kv heads, 11308 positions of an int4 cache 19.2 / 16.9 us; 56 / 8, the tile of 8
+    // with the scales alone, 30.1 / 28.2)
+    const bool alike = qk_dim == v_dim && (!kvq || quant->group == 64);
+    const bool words = !kvq || (((uintptr_t)quant->k_scales | (uintptr_t)quant->k_biases | (uintptr_t)quant->v_scales | (uintptr_t)quant->v_biases) & 3u) == 0;
+    const int row = gt > 4 && !kvq ? 0 : (alike && qk_dim == 128 && words ? 16 : (alike && qk_dim == 64 ? 8 : 0));
     const void* func = nullptr;
-#define FK_SDPA_PICK(Q)                                                                         \
-    switch (gt) {                                                                               \
-        case 1: func = row16 ? reinterpret_cast<const void*>(&sdpa_decode_kernel<1, Q, true>) : reinterpret_cast<const void*>(&sdpa_decode_kernel<1, Q>); break; \
-        case 2: func = row16 ? reinterpret_cast<const void*>(&sdpa_decode_kernel<2, Q, true>) : reinterpret_cast<const void*>(&sdpa_decode_kernel<2, Q>); break; \
-        case 4: func = row16 ? reinterpret_cast<const void*>(&sdpa_decode_kernel<4, Q, true>) : reinterpret_cast<const void*>(&sdpa_decode_kernel<4, Q>); break; \
-        default: func = reinterpret_cast<const void*>(&sdpa_decode_kernel<8, Q>); break;        \
-    }
     if (fusion) {
         // whole-width rotation of at most 128 dims with a table: the form whose loads run ahead
         // (heads of fewer than 128 dims add their squares in another order there: a quantised cache keeps the one it has)
         const bool fast = fusion->rope_tab && fusion->rope_dims == qk_dim && qk_dim <= 128 && !(kvq && fusion->q_norm && qk_dim != 128);
-#define FK_SDPA_FUSED(F, Q)                                                                           \
-    switch (gt) {                                                                                     \
-        case 1: func = row16 ? reinterpret_cast<const void*>(&sdpa_rope_store_kernel<1, F, Q, true>) : reinterpret_cast<const void*>(&sdpa_rope_store_kernel<1, F, Q>); break; \
-        case 2: func = row16 ? reinterpret_cast<const void*>(&sdpa_rope_store_kernel<2, F, Q, true>) : reinterpret_cast<const void*>(&sdpa_rope_store_kernel<2, F, Q>); break; \
-        case 4: func = row16 ? reinterpret_cast<const void*>(&sdpa_rope_store_kernel<4, F, Q, true>) : reinterpret_cast<const void*>(&sdpa_rope_store_kernel<4, F, Q>); break; \
-        default: func = reinterpret_cast<const void*>(&sdpa_rope_store_kernel<8, F, Q>); break;       \
-    }
-#define FK_SDPA_FUSED_Q(F)              \
-    if (kvq == 4) {                     \
-        FK_SDPA_FUSED(F, 4)             \
-    } else if (kvq == 8) {              \
-        FK_SDPA_FUSED(F, 8)             \
-    } else {                            \
-        FK_SDPA_FUSED(F, 0)             \
-    }
-        if (fast) {
-            FK_SDPA_FUSED_Q(true)
-        } else {
-            FK_SDPA_FUSED_Q(false)
-        }
-#undef FK_SDPA_FUSED_Q
-#undef FK_SDPA_FUSED
-    } else if (kvq == 4) {
-        FK_SDPA_PICK(4)
-    } else if (kvq == 8) {
-        FK_SDPA_PICK(8)
+        func = kvq == 4 ? fused_func<4>(fast, gt, row) : (kvq == 8 ? fused_func<8>(fast, gt, row) : fused_func<0>(fast, gt, row));
     } else {
-        FK_SDPA_PICK(0)
+        func = kvq == 4 ? decode_func<4>(gt, row) : (kvq == 8 ? decode_func<8>(gt, row) : decode_func<0>(gt, row));
     }
-#undef FK_SDPA_PICK
     out_launch->func = func;
     out_launch->grid = dim3(n_splits, n_kv, ((G + gt - 1) / gt) * rows);
     out_launch->block = dim3(kSdpaBlock, 1, 1);

@@ -95,6 +95,12 @@ __device__ __forceinline__ void each_index(F&& f) {
 // Lane J of the caller's 16-lane row (row_newbcast); a value moved as a DPP control says.
 template <int J>
 __device__ __forceinline__ uint32_t row_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + J, 0xF, 0xF, false); }
+// Lane J of the caller's half of a 16-lane row.
+template <int J>
+__device__ __forceinline__ uint32_t half_row_lane(uint32_t v) {
+    const int low = __builtin_amdgcn_update_dpp(0, (int)v, 0x150 + J, 0xF, 0x3, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp(low, (int)v, 0x158 + J, 0xF, 0xC, false);
+}
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false)); }
 // The maximum over the wave's four 16-lane rows, lane by lane.
@@ -115,9 +121,9 @@ __device__ __forceinline__ float rows_max(float v) {
 // the transforms' loads are issued ahead of the cache rows and used after them.
 // NOMERGE: the caller merges the ranges' results itself: every active block writes its (m, l, o) partial with
 // ordinary stores -- also when one range covers the context -- and returns; no arrival counter is touched.
-// ROW16: heads of 128 dims for keys and values, a row on 16 lanes (a quantised cache: two groups of 64, scale and bias arrays
-// 4-byte aligned).  See the wave-local form below.
-template <int GT, int MODE, typename ARGS, int KVQ = 0, bool FASTHEAD = false, bool NOMERGE = false, bool ROW16 = false>
+// ROW: 16, heads of 128 dims for keys and values, a row on 16 lanes; 8, heads of 64 dims on 8 (a quantised cache: groups of 64,
+// with 128 dims scale and bias arrays 4-byte aligned); else 0.  See the wave-local form below.
+template <int GT, int MODE, typename ARGS, int KVQ = 0, bool FASTHEAD = false, bool NOMERGE = false, int ROW = 0>
 __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint32_t split, uint32_t kvh,
                                            uint32_t gz, uint32_t gz_count, float* lds, uint32_t kv_add = 0) {
     // kv_raw + kv_add positions are visible (kv_add: the row's index among several active rows).  The sum is formed
@@ -132,7 +138,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // the ranges of a block need no barrier; the waves meet once, after the last range.
     constexpr bool WAVES = MODE != 1 && GT <= 4;
     constexpr int kSteps = FUSED ? kSdpaStepsFused : kSdpaSteps;
-    static_assert(!ROW16 || (WAVES && kSteps == 4), "");
+    static_assert(ROW == 0 || (MODE != 1 && kSteps == 4), "");
     static_assert(!(FUSED && KVQ != 0), "the whole-token kernel reads a bf16 cache");
     const uint32_t span = a.chunk_len * a.chunks_per_block;  // cache positions per block
     const uint32_t blk0 = split * span;
@@ -243,8 +249,8 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // ~60 registers that the 64 registers of in-flight rows would otherwise have to share.
     if constexpr (MODE == 1) transform_heads(0);
 
-    const uint32_t lpk = ROW16 ? 16u : a.lpk, cpk = ROW16 ? 16u : a.qk_dim >> 3;
-    const uint32_t lpv = ROW16 ? 16u : a.lpv, cpv = ROW16 ? 16u : a.v_dim >> 3;
+    const uint32_t lpk = ROW ? (uint32_t)ROW : a.lpk, cpk = ROW ? (uint32_t)ROW : a.qk_dim >> 3;
+    const uint32_t lpv = ROW ? (uint32_t)ROW : a.lpv, cpv = ROW ? (uint32_t)ROW : a.v_dim >> 3;
     const uint32_t ck = tid & (lpk - 1), kslot = tid / lpk, kslots = kSdpaBlock / lpk;
     const uint32_t cv = tid & (lpv - 1), vslot = tid / lpv, vslots = kSdpaBlock / lpv;
     const bool kcol_ok = ck < cpk, vcol_ok = cv < cpv;
@@ -255,7 +261,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         stat[tid] = -INFINITY;
         stat[8 + tid] = 0.f;
     }
-    float m_own = -INFINITY;     // ROW16: running maximum of the head whose score the lane finishes
+    float m_own = -INFINITY;     // ROW: running maximum of the head whose score the lane finishes
     float m_run[GT], l_run[GT];  // wave-local form: running maximum (uniform) and this lane row's share of the sum
 #pragma unroll
     for (int h = 0; h < GT; ++h) {
@@ -317,20 +323,30 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // starts 8.8 us into the launch instead of 13.6; a bf16 cache is bound by the bytes and was 5 % slower with it).
     constexpr bool DEEP = MODE != 1 && WAVES && KVQ != 0;
     uint4 kn_[kSteps], vn_[kSteps], kf_[DEEP ? kSteps : 1], vf_[DEEP ? kSteps : 1];
-    // ROW16, quantised: lane 4 u + i of a row's 16 lanes holds both groups' entries of key row u in array i (scales and biases
-    // of the keys, of the values), so a range's take a wave ONE request -- two bytes a lane from each array and row they were 16
+    // Quantised, ROW: scales and biases of a range with one request a wave (128 dims: lane 4 u + i of a row's 16 holds both groups'
+    // entries of key row u in array i: scales and biases of the keys, of the values) or two (64 dims: lane 2 u + i of a row's 8
+    // the scale and the bias of key row u of the keys, of the values) -- two bytes a lane from each array and row they were 16
     // of its 24, and a CU issues one in 16 .. 20 cycles.
-    constexpr bool META16 = ROW16 && KVQ != 0;
-    uint32_t mc = 0, mn_ = 0, mf_ = 0;
-    // (a global access: chosen among the arguments' pointers as they are, the arguments move to memory and the access is a flat one)
-    typedef const __attribute__((address_space(1))) uint32_t* gmeta;
-    gmeta mbase = nullptr;
-    if constexpr (META16) {
+    constexpr bool META = ROW != 0 && KVQ != 0;
+    struct Meta {
+        uint32_t a, b;   // (64 dims: the scale and the bias, put together where they are used: not a wait at the request)
+    };
+    Meta mc = {0u, 0u}, mn_ = {0u, 0u}, mf_ = {0u, 0u};
+    // (global accesses: chosen among the arguments' pointers as they are, the arguments move to memory and the access is a flat one)
+    typedef const __attribute__((address_space(1))) uint32_t* gmeta32;
+    typedef const __attribute__((address_space(1))) uint16_t* gmeta16;
+    uintptr_t mbase = 0, mbase2 = 0;
+    if constexpr (META) {
         const uintptr_t ks = (uintptr_t)a.k_scales, kb = (uintptr_t)a.k_biases, vs = (uintptr_t)a.v_scales, vb = (uintptr_t)a.v_biases;
-        const uintptr_t kk = (lane & 1u) ? kb : ks, vv = (lane & 1u) ? vb : vs;
-        mbase = (gmeta)((lane & 2u) ? vv : kk);
+        if constexpr (ROW == 16) {
+            const uintptr_t kk = (lane & 1u) ? kb : ks, vv = (lane & 1u) ? vb : vs;
+            mbase = (lane & 2u) ? vv : kk;
+        } else {
+            mbase = (lane & 1u) ? vs : ks;
+            mbase2 = (lane & 1u) ? vb : kb;
+        }
     }
-    auto request_rows = [&](uint4(&kd)[kSteps], uint4(&vd)[kSteps], uint32_t& md, uint32_t key0, uint32_t nkeys, bool owner,
+    auto request_rows = [&](uint4(&kd)[kSteps], uint4(&vd)[kSteps], Meta& md, uint32_t key0, uint32_t nkeys, bool owner,
                             uint32_t jpos) {
         const uint16_t* kbase = a.k + ((size_t)kvh * a.capacity + key0) * a.qk_dim + 8 * ck;
         const uint16_t* vbase = a.v + ((size_t)kvh * a.capacity + key0) * a.v_dim + 8 * cv;
@@ -346,16 +362,22 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
             const size_t kmeta = (size_t)kvh * a.capacity * kg + (8u * kcol) / a.kv_group;
             const size_t vmeta = (size_t)kvh * a.capacity * vg + (8u * vcol) / a.kv_group;
             const uint32_t last = a.capacity - 1;
-            if constexpr (META16) {
-                const uint32_t r0 = key0 + kslot + ((lane >> 2) & 3u) * kslots, r = r0 < last ? r0 : last;
-                md = mbase[(size_t)kvh * a.capacity + r];
+            if constexpr (META) {
+                const uint32_t r0 = key0 + kslot + (ROW == 16 ? (lane >> 2) & 3u : (lane >> 1) & 3u) * kslots, r = r0 < last ? r0 : last;
+                const size_t at = (size_t)kvh * a.capacity + r;
+                if constexpr (ROW == 16) {
+                    md.a = ((gmeta32)mbase)[at];
+                } else {
+                    md.a = ((gmeta16)mbase)[at];
+                    md.b = ((gmeta16)mbase2)[at];
+                }
             }
 #pragma unroll
             for (int u = 0; u < kSteps; ++u) {
                 const uint32_t r0 = key0 + kslot + u * kslots, r = r0 < last ? r0 : last;
                 kd[u].x = kp[(size_t)r * kw];
                 kd[u].y = WPL == 2 ? kp[(size_t)r * kw + 1] : 0u;
-                kd[u].z = META16 ? 0u : (uint32_t)a.k_scales[kmeta + (size_t)r * kg] | ((uint32_t)a.k_biases[kmeta + (size_t)r * kg] << 16);
+                kd[u].z = META ? 0u : (uint32_t)a.k_scales[kmeta + (size_t)r * kg] | ((uint32_t)a.k_biases[kmeta + (size_t)r * kg] << 16);
                 kd[u].w = 0u;
             }
 #pragma unroll
@@ -363,7 +385,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
                 const uint32_t r0 = key0 + vslot + u * vslots, r = r0 < last ? r0 : last;
                 vd[u].x = vp[(size_t)r * vw];
                 vd[u].y = WPL == 2 ? vp[(size_t)r * vw + 1] : 0u;
-                vd[u].z = META16 ? 0u : (uint32_t)a.v_scales[vmeta + (size_t)r * vg] | ((uint32_t)a.v_biases[vmeta + (size_t)r * vg] << 16);
+                vd[u].z = META ? 0u : (uint32_t)a.v_scales[vmeta + (size_t)r * vg] | ((uint32_t)a.v_biases[vmeta + (size_t)r * vg] << 16);
                 vd[u].w = 0u;
             }
             return;
@@ -481,12 +503,18 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         kz[u] = kc[u].z;
         vz[u] = vc[u].z;
     }
-    if constexpr (META16) {
+    if constexpr (META) {
         const uint32_t half = ck >= 8u ? 0x07060302u : 0x05040100u;   // this lane's group
+        const uint32_t both = ROW == 16 ? mc.a : mc.a | (mc.b << 16);
         each_index<kSteps>([&](auto u) __attribute__((always_inline)) {
             constexpr int U = decltype(u)::value;
-            kz[U] = __builtin_amdgcn_perm(row_lane<4 * U + 1>(mc), row_lane<4 * U>(mc), half);
-            vz[U] = __builtin_amdgcn_perm(row_lane<4 * U + 3>(mc), row_lane<4 * U + 2>(mc), half);
+            if constexpr (ROW == 16) {
+                kz[U] = __builtin_amdgcn_perm(row_lane<4 * U + 1>(both), row_lane<4 * U>(both), half);
+                vz[U] = __builtin_amdgcn_perm(row_lane<4 * U + 3>(both), row_lane<4 * U + 2>(both), half);
+            } else {
+                kz[U] = half_row_lane<2 * U>(both);
+                vz[U] = half_row_lane<2 * U + 1>(both);
+            }
         });
     }
     if constexpr (XFORM) {
@@ -595,26 +623,30 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
         // multiply), so a probability is one v_exp_f32.
         const float scale2 = a.scale * 1.44269504088896341f;
         float pr[kSteps][GT];
-        if constexpr (ROW16) {
-            // A row's 16 lanes each finish ONE of its 4 GT scores (fewer: several the same one): at every step of the butterfly
-            // a lane keeps the half of the sums that its own score is in and hands over the other -- the same additions -- then
-            // scales it and raises it to a probability alone, where every lane did so for all of them (16 exponentials of
-            // a quarter rate for one at four heads), and hands it round.  Score v = u GT + h is that of the lanes with
-            // bits (b0 ^ b2, b1 ^ b2, b2 ^ b3, b3) of v, which the row's half mirror and mirror pair as they need be.
-            // 32 q / 8 kv heads, every lane all scores / this: 32768 positions of a bf16 cache 40.5 / 36.8 us; with the scales'
-            // single request (META16) a token of the 4B-class model behind 12000 positions of an 8-bit cache 1938 / 1807 us.
-            constexpr int LH = GT == 4 ? 2 : (GT == 2 ? 1 : 0), LV = LH + 2;   // log2 of the heads, of the scores
-            const bool sel[4] = {((lane ^ (lane >> 2)) & 1u) != 0, (((lane >> 1) ^ (lane >> 2)) & 1u) != 0, (((lane >> 2) ^ (lane >> 3)) & 1u) != 0, (lane & 8u) != 0};
+        if constexpr (ROW != 0) {
+            // A row's lanes each finish ONE of its 4 GT scores (64 dims and four heads: two; fewer scores than lanes: several the
+            // same one): at every step of the butterfly a lane keeps the half of the sums that its own score is in and hands over
+            // the other -- the same additions -- then scales it and raises it to a probability alone, where every lane did so for
+            // all of them (16 exponentials of a quarter rate for one at four heads), and hands it round.  Score v = u GT + h is
+            // that of the lanes with bits (b0 ^ b2, b1 ^ b2, b2 ^ b3, b3) of v, which the row's half mirror and mirror pair as
+            // they need be (8 lanes: (b0 ^ b2, b1 ^ b2, b2)).
+            // 32 q / 8 kv heads x 128, every lane all scores / this: 32768 positions of a bf16 cache 40.5 / 36.8 us; with the
+            // scales' single request a token of the 4B-class model behind 12000 positions of an 8-bit cache 1938 / 1807 us.
+            constexpr int LR = ROW == 16 ? 4 : 3;                                                      // log2 of the lanes,
+            constexpr int LH = GT == 4 ? 2 : (GT == 2 ? 1 : 0), LV = LH + 2 < LR ? LH + 2 : LR;        // the heads, the scores by lane
+            constexpr int R = (kSteps * GT) >> LV;                                                     // scores a lane finishes
+            const bool sel[4] = {((lane ^ (lane >> 2)) & 1u) != 0, (((lane >> 1) ^ (lane >> 2)) & 1u) != 0,
+                                 ROW == 16 ? (((lane >> 2) ^ (lane >> 3)) & 1u) != 0 : (lane & 4u) != 0, (lane & 8u) != 0};
             float x[kSteps * GT];
 #pragma unroll
             for (int u = 0; u < kSteps; ++u)
 #pragma unroll
                 for (int h = 0; h < GT; ++h) x[u * GT + h] = score(u, h);
-            each_index<4>([&](auto step) __attribute__((always_inline)) {
+            each_index<LR>([&](auto step) __attribute__((always_inline)) {
                 constexpr int S = decltype(step)::value, CTRL = S == 0 ? 0xB1 : (S == 1 ? 0x4E : (S == 2 ? 0x141 : 0x140));
                 if constexpr (S < LV) {
 #pragma unroll
-                    for (int i = 0; i < (1 << (LV - 1 - S)); ++i) {   // (kept in place: sums i of the step's 2^(LV - S))
+                    for (int i = 0; i < ((kSteps * GT) >> (S + 1)); ++i) {   // (in place: the step leaves half as many sums)
                         const float keep = sel[S] ? x[2 * i + 1] : x[2 * i], give = sel[S] ? x[2 * i] : x[2 * i + 1];
                         x[i] = keep + dpp_move<CTRL>(give);
                     }
@@ -622,22 +654,32 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
                     x[0] = dpp_add<CTRL>(x[0]);
                 }
             });
-            uint32_t own = 0;   // this lane's score
+            uint32_t own = 0;   // this lane's score, the first
 #pragma unroll
             for (int k = 0; k < LV; ++k) own |= sel[k] ? 1u << k : 0u;
-            const float mine = kslot + (own >> LH) * kslots < nkeys ? x[0] * scale2 : -INFINITY;
-            float mx = mine;   // of the lane's head: over the row's four keys, then the wave's four rows
+            float mine[R], mx = -INFINITY;   // mx of the lane's head: over the row's four keys, then the wave's rows
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                mine[i] = kslot + ((own + ((uint32_t)i << LV)) >> LH) * kslots < nkeys ? x[i] * scale2 : -INFINITY;
+                mx = fmaxf(mx, mine[i]);
+            }
             each_index<4>([&](auto step) __attribute__((always_inline)) {
                 constexpr int S = decltype(step)::value, CTRL = S == 0 ? 0xB1 : (S == 1 ? 0x4E : (S == 2 ? 0x141 : 0x140));
-                if constexpr (S >= LH && S < LV) mx = dpp_max<CTRL>(mx);
+                if constexpr ((S >= LH && S < LV) || S >= LR) mx = dpp_max<CTRL>(mx);   // (8 lanes: the neighbouring row's too)
             });
             mx = rows_max(mx);
             const float m_new = fmaxf(m_own, mx), m_ref = m_new == -INFINITY ? 0.f : m_new;   // no live key yet: every term is 2^-inf = 0
-            const float alpha_own = __builtin_amdgcn_exp2f(m_own - m_ref), p_own = __builtin_amdgcn_exp2f(mine - m_ref);
+            const float alpha_own = __builtin_amdgcn_exp2f(m_own - m_ref);
+            float p_own[R];
+#pragma unroll
+            for (int i = 0; i < R; ++i) p_own[i] = __builtin_amdgcn_exp2f(mine[i] - m_ref);
             m_own = m_new;
             each_index<kSteps * GT>([&](auto v) __attribute__((always_inline)) {
-                constexpr int V = decltype(v)::value, B3 = (V >> 3) & 1, B2 = ((V >> 2) & 1) ^ B3, B1 = ((V >> 1) & 1) ^ B2, B0 = (V & 1) ^ B2;
-                pr[V / GT][V % GT] = __int_as_float((int)row_lane<8 * B3 + 4 * B2 + 2 * B1 + B0>((uint32_t)__float_as_int(p_own)));
+                constexpr int V = decltype(v)::value, W = V & ((1 << LV) - 1);
+                constexpr int B3 = ROW == 16 ? (W >> 3) & 1 : 0, B2 = ((W >> 2) & 1) ^ B3, B1 = ((W >> 1) & 1) ^ B2, B0 = (W & 1) ^ B2;
+                constexpr int FROM = 8 * B3 + 4 * B2 + 2 * B1 + B0;
+                const uint32_t p = (uint32_t)__float_as_int(p_own[V >> LV]);
+                pr[V / GT][V % GT] = __int_as_float((int)(ROW == 16 ? row_lane<FROM>(p) : half_row_lane<FROM & 7>(p)));
             });
 #pragma unroll
             for (int h = 0; h < GT; ++h) {
@@ -813,7 +855,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
 #pragma unroll
         for (int h = 0; h < GT; ++h) {
             const float lw = wave_sum(l_run[h]) * inv_lanes;
-            if constexpr (ROW16) m_run[h] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m_own), h));
+            if constexpr (ROW != 0) m_run[h] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m_own), h));
             if (lane == 0) {
                 wm[wave * 8 + h] = m_run[h];
                 wl[wave * 8 + h] = lw;
@@ -1023,7 +1065,7 @@ __device__ __forceinline__ uint32_t sdpa_load_kv_len(const SdpaArgs& a) {
 #endif
 }
 
-template <int GT, int KVQ = 0, bool ROW16 = false>
+template <int GT, int KVQ = 0, int ROW = 0>
 __global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_decode_kernel(const SdpaArgs a) {
     extern __shared__ __align__(16) float lds[];
     // One unconditional load (the immediate is read from the kernel-argument segment
@@ -1032,7 +1074,7 @@ __global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_decode_kerne
     kernarg_warm<(int)sizeof(SdpaArgs)>();
     const uint32_t kv_len0 = sdpa_load_kv_len(a);
     if (a.rows <= 1) {
-        sdpa_block<GT, false, SdpaArgs, KVQ, false, false, ROW16>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
+        sdpa_block<GT, false, SdpaArgs, KVQ, false, false, ROW>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
         return;
     }
     // Several active rows (multi-token verification, chunked prefill): grid.z carries
@@ -1045,19 +1087,19 @@ __global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_decode_kerne
     r.out = a.out + (size_t)tr * a.n_heads * a.v_dim;
     r.partials = a.partials + (size_t)tr * a.n_heads * a.n_splits * (a.v_dim + 2);
     r.counters = a.counters + (size_t)tr * a.n_kv * gz_count;
-    sdpa_block<GT, false, SdpaArgs, KVQ, false, false, ROW16>(r, kv_len0, blockIdx.x, blockIdx.y, gz, gz_count, lds, tr);
+    sdpa_block<GT, false, SdpaArgs, KVQ, false, false, ROW>(r, kv_len0, blockIdx.x, blockIdx.y, gz, gz_count, lds, tr);
 }
 
 // RoPE (+ head norm) of q and of the new k row, the cache append and the attention in one
 // launch: a.q / a.k_new / a.v_new are the raw projection outputs of the token at position
 // kv_len - 1, a.k / a.v the cache it is appended to.
 // KVQ: a quantised cache; the new rows are quantised by the block whose range holds them.
-template <int GT, bool FASTHEAD, int KVQ = 0, bool ROW16 = false>
+template <int GT, bool FASTHEAD, int KVQ = 0, int ROW = 0>
 __global__ __launch_bounds__(kSdpaBlock, GT == 8 ? 1 : 2) void sdpa_rope_store_kernel(const SdpaArgs a) {
     extern __shared__ __align__(16) float lds[];
     kernarg_warm<(int)sizeof(SdpaArgs)>();
     const uint32_t kv_len0 = sdpa_load_kv_len(a);
-    sdpa_block<GT, 2, SdpaArgs, KVQ, FASTHEAD, false, ROW16>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
+    sdpa_block<GT, 2, SdpaArgs, KVQ, FASTHEAD, false, ROW>(a, kv_len0, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, lds);
 }
 
 }  // namespace fk

@@ -173,6 +173,7 @@ class _Shifted:
 
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("n_heads,n_kv,kv_len,max_len,rows", [
+    (7, 1, 130, 140, 2), (6, 1, 3000, 3000, 1),                     # the tile of 8, which goes through LDS
     (2, 2, 1, 1, 1), (4, 2, 15, 16, 1), (8, 2, 17, 64, 3),          # a head a block, one range
     (8, 2, 2048, 2048, 1),                                          # several ranges, their merge
     (4, 4, 2999, 3001, 2), (4, 2, 2113, 2120, 1), (8, 2, 4095, 4100, 1),   # tiles of 1, 2 and 4 heads, ranges that a block walks
