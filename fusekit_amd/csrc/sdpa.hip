@@ -167,6 +167,10 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
         const uint32_t two = 2u * (uint32_t)dev->cus / tiles;
         want = two < 16u ? two : 16u;
     }
+    // Up to three ranges of a bf16 cache: one block walks them.  A range more in the same block costs 1.04 us, the partials of two
+    // blocks, their count and their merge 2.5: 14 q / 2 kv heads x 64, split / walked, 256 positions 6.2 / 4.7 us, 384 6.4 / 5.7, 512
+    // 6.5 / 6.7; 32 / 8 x 128, 128 positions 6.2 / 4.7, 256 6.5 / 6.8.  (Over a quantised cache the two differ in the last bit.)
+    if (!kvq && n_chunks <= 3u) want = 1;
     if (want < 1) want = 1;
     if (want > 256) want = 256;
     const uint32_t cpb = (n_chunks + want - 1) / want;
