@@ -16,9 +16,9 @@
 // values, a group's dot product is accumulated from zero in fp32 and folded as s * dot + b * Sx; Sx, the group's activation
 // sum, is one more matrix instruction per step against a B operand of ones, which leaves it in the very registers the fold
 // needs.
-// 37 rows of int4, one call in a chain, before (32 x 32 x 16 tiles, split-k sums, second kernel) / now: 896 x 896 12.8 / 5.0
-// us, 4864 x 896 pair 26.3 / 10.1, 896 x 4864 17.8 / 12.5, 2560 x 4096 19.8 / 11.2, 9728 x 2560 pair 53.0 / 27.7; 8 rows (a
-// form of its own for 2..10 rows) 896 x 896 4.65 / 3.94, 2560 x 4096 8.80 / 7.06, 2560 x 9728 14.4 / 12.7.
+// 37 rows of int4, one call in a chain, before (32 x 32 x 16 tiles, split-k sums, second kernel) / now: 896 x 896 12.8 / 3.4
+// us, 4864 x 896 pair 26.3 / 8.5, 896 x 4864 17.8 / 7.1, 2560 x 4096 19.8 / 9.9, 9728 x 2560 pair 53.0 / 27.7; 8 rows (a
+// form of its own for 2..10 rows) 896 x 896 4.65 / 3.34, 2560 x 4096 8.80 / 6.2, 2560 x 9728 14.4 / 12.7.
 #include "fk_host.hpp"
 #include "gemv_kernel.hpp"
 
