@@ -55,7 +55,8 @@ fk_status sdpa_workspace_bytes(uint32_t n_heads, uint32_t n_kv, uint32_t qk_dim,
 
 namespace {
 
-// The kernels by tile, cache and row form (tiles of 8 heads over a bf16 cache have the general one only).
+// The kernels by tile, cache and row form.  A bf16 cache has tiles of 1 and 2 heads and, where keys and values differ too much in width,
+// of 8 in the general form; tiles of 4 belong to quantised caches.
 template <int GT, int Q>
 const void* decode_func(int row) {
     if constexpr (GT <= 4 || Q != 0) {
@@ -74,11 +75,15 @@ const void* fused_func(int row) {
 }
 template <int Q>
 const void* decode_func(int gt, int row) {
-    return gt == 1 ? decode_func<1, Q>(row) : (gt == 2 ? decode_func<2, Q>(row) : (gt == 4 ? decode_func<4, Q>(row) : decode_func<8, Q>(row)));
+    if constexpr (Q != 0)
+        if (gt == 4) return decode_func<4, Q>(row);
+    return gt == 1 ? decode_func<1, Q>(row) : (gt == 2 ? decode_func<2, Q>(row) : decode_func<8, Q>(row));
 }
 template <bool F, int Q>
 const void* fused_tile(int gt, int row) {
-    return gt == 1 ? fused_func<1, F, Q>(row) : (gt == 2 ? fused_func<2, F, Q>(row) : (gt == 4 ? fused_func<4, F, Q>(row) : fused_func<8, F, Q>(row)));
+    if constexpr (Q != 0)
+        if (gt == 4) return fused_func<4, F, Q>(row);
+    return gt == 1 ? fused_func<1, F, Q>(row) : (gt == 2 ? fused_func<2, F, Q>(row) : fused_func<8, F, Q>(row));
 }
 template <int Q>
 const void* fused_func(bool fast, int gt, int row) { return fast ? fused_tile<true, Q>(gt, row) : fused_tile<false, Q>(gt, row); }

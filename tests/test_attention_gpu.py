@@ -141,6 +141,15 @@ def test_sdpa_split_invariance(fk):
     assert ulps <= 1.0 and frac <= 0.02
 
 
+@pytest.mark.parametrize("n_heads,n_kv,dim,kv_len", [
+    (2, 2, 64, 129), (14, 2, 64, 384), (14, 2, 64, 385), (32, 8, 128, 192), (32, 8, 128, 193),   # up to three ranges: one block
+    (64, 8, 128, 1025), (32, 8, 128, 1601), (32, 8, 128, 4096), (4, 2, 64, 4097), (32, 8, 128, 4097),   # 16 ranges, tiles of one and two
+    (2, 2, 128, 1024), (2, 2, 128, 1025), (2, 2, 128, 2049), (2, 2, 128, 4096), (2, 2, 128, 4097),   # merges of 16, 17, 33, 64 and 65 partials
+])
+def test_sdpa_at_the_edges_of_its_ranges_and_merge(fk, n_heads, n_kv, dim, kv_len):
+    _sdpa_case(fk, n_heads, n_kv, dim, dim, kv_len, kv_len)
+
+
 @pytest.mark.parametrize("bits", [16, 4, 8])
 def test_embed_lookup(fk, bits):
     vocab, hidden = 1000, 896
