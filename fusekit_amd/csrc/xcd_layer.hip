@@ -217,8 +217,8 @@ __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, 
         const uint32_t gz = sync.slot % G, split = sync.slot / G;
         if (split < a.sdpa.n_splits) {
             using Args = std::remove_cv_t<std::remove_reference_t<decltype((a.sdpa))>>;
-            // (uniform; each lane its own score, the same bits: 24 tokens at context 480 of the 4B class 26.94 / 26.70 ms, general form /
-            // this, of a 12-layer model with heads of 64 dims 7.76 / 7.63, 2500 positions 8.33 / 8.15)
+            // (uniform; each lane its own score, the same bits: general form / this, 64 tokens at context 480 of the 4B class 73.1 / 72.7
+            // ms, 24 tokens of a 12-layer model with heads of 64 dims 7.76 / 7.63, behind 2500 positions 8.33 / 8.15)
             if (a.sdpa.qk_dim == 128)
                 sdpa_block<1, 2, Args, 0, true, true, 16>(a.sdpa, kv_len0, split, sync.xcd, gz, G, work);
             else if (a.sdpa.qk_dim == 64)
