@@ -16,6 +16,7 @@
 // activation sum (computed once per block).
 #pragma once
 #include "fk_device.hpp"
+#include "gemv_tiling.hpp"
 
 // Hook for timing probes: a build may define FK_GEMV_STAMP(i) to record a clock at
 // phase boundary i; the library build leaves it empty.
@@ -24,12 +25,6 @@
 #endif
 
 namespace fk {
-
-enum WKind : int { W_Q4 = 0, W_Q8 = 1, W_BF16 = 2 };
-
-constexpr int kGemvBlock = 256;
-constexpr int kGemvUnroll = 4;  // 16-byte loads in flight per lane and batch
-constexpr int kMaxMats = 3;
 
 struct GemvArgs {
     const uint4* w[kMaxMats];
@@ -55,29 +50,6 @@ struct GemvArgs {
     int swiglu_variant;
     float y_scale;  // SwiGLU variant 1 only: multiplies the fp32 product before the final round
 };
-
-template <WKind KIND>
-struct ChunkTraits;
-template <>
-struct ChunkTraits<W_Q4> {
-    static constexpr int kValues = 32, kPieces = 4;
-};
-template <>
-struct ChunkTraits<W_Q8> {
-    static constexpr int kValues = 16, kPieces = 4;
-};
-template <>
-struct ChunkTraits<W_BF16> {
-    static constexpr int kValues = 8, kPieces = 1;
-};
-
-// LDS bytes the kernel needs: staged activations + per-chunk sums + partials + scratch.
-template <WKind KIND>
-__host__ __device__ inline uint32_t gemv_lds_bytes(uint32_t cpr, uint32_t seg_chunks, uint32_t nseg) {
-    const uint32_t pos = kGemvBlock * (kGemvUnroll / nseg);
-    const uint32_t seg_pad = (seg_chunks + pos - 1) / pos * pos;
-    return ChunkTraits<KIND>::kPieces * cpr * 16u + cpr * 4u + nseg * seg_pad * 4u + 64u;
-}
 
 __device__ __forceinline__ float q8_word_dot(uint32_t w, uint4 xf, float d) {
     d = fmaf((float)(w & 0xffu), __uint_as_float(xf.x), d);

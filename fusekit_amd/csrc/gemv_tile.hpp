@@ -9,7 +9,7 @@
 //     LDS as (scale | bias << 16), instead of two 2-byte requests for every 16-byte chunk of weights;
 //   * the activations are asked for as often as the row is long, the norm weight only where there is one;
 //   * projection bias and residual are asked for in front of the weights' use, not behind the row sums;
-//   * the tile height follows the launch: a few chunks a thread on as many CUs as there are (gemv_tile_choice in gemv.hip).
+//   * the tile height follows the launch: a few chunks a thread on as many CUs as there are (gemv_tile_choice in gemv_tiling.hpp).
 // int4, launch to launch over cold weights, gemv_stream_kernel -> this: 896 x 896 3.8 -> 2.75 us, 4864 x 896 4.2 -> 3.35, its gate / up
 // pair 5.9 -> 4.7, 2560 x 4096 5.5 -> 4.2, 2560 x 9728 8.0 -> 6.2, pair of 9728 x 2560 10.9 -> 9.2, of 14336 x 4096 19.1 -> 16.8.
 // Every partial, the order in which a row's partials are added and the epilogue are those of gemv_run, bit for bit.
@@ -19,17 +19,6 @@
 namespace fk {
 
 typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));  // four 16-bit entries at any of their addresses
-
-constexpr uint32_t kTileGroups = 4u * kGemvBlock;  // quantisation groups of a tile and matrix: four a thread
-
-// Entries of a matrix's scale / bias words in LDS.
-__host__ __device__ inline uint32_t gemv_tile_meta(uint32_t rows, uint32_t gpr) { return (rows * gpr + 3u) & ~3u; }
-
-template <WKind KIND>
-__host__ __device__ inline uint32_t gemv_tile_lds_bytes(uint32_t cpr, uint32_t rows, uint32_t gpr, uint32_t nl, uint32_t nseg) {
-    return ChunkTraits<KIND>::kPieces * cpr * 16u + cpr * 4u + nseg * nl * kGemvBlock * 4u +
-           (KIND == W_BF16 ? 0u : nseg * gemv_tile_meta(rows, gpr) * 4u) + 64u;
-}
 
 // NL: 16-byte chunks of each matrix per thread.  AHEAD of them go out in front of the staging (a wave cannot stage before it
 // has issued what stands in front of it; pair of 9728 x 2560, 12 a thread: 1 / 2 / 4 / 6 ahead 9.5 / 9.3 / 9.1 / 9.6 us; 6144 x 2560, 3 a

@@ -117,6 +117,26 @@ def test_one_tile_form_at_its_edges(fk, n, k, bits, group):
         assert rel_l2(d.to_numpy(np.uint16), oracle.bf16_to_f32(oracle.qgemv(w, ny, bias))) <= REL_L2_BAR
 
 
+@pytest.mark.parametrize("n,k,pair,groups", [(9728, 2560, True, (64, 32, 128)), (2560, 9728, False, (64, 32, 128)), (4864, 896, True, (128, 32, 64)),
+                                             (1, 128, False, (32, 128, 64)), (1, 128, True, (32, 64, 128)), (515, 256, False, (32, 128, 64))])
+def test_group_sizes_of_one_shape_in_turn(fk, n, k, pair, groups):
+    """One int4 shape with one group size after the other, and all again: each call is tiled for its own groups."""
+    x, g = normal_bf16(3, k, 2.0), normal_bf16(4, k, 0.1, 1.0)
+    dx, dg, dy = fk.DeviceBuffer.from_numpy(x), fk.DeviceBuffer.from_numpy(g), fk.DeviceBuffer(2 * n)
+    calls = []
+    for group in groups:
+        W = [make_qweight(700 + group + i, n, k, 4, group) for i in range(2 if pair else 1)]
+        calls.append(([to_device(fk, w) for w in W], oracle.gateup_swiglu(x, g, 1e-6, *W, 1) if pair else oracle.qgemv(W[0], x)))
+    for dW, ref in calls + calls:
+        if pair:
+            fk.gateup_swiglu(dx, dg, 1e-6, *dW, 1, dy)
+        else:
+            fk.qgemv(dW[0], dx, None, dy)
+        got = dy.to_numpy(np.uint16)
+        assert rel_l2(got, oracle.bf16_to_f32(ref)) <= REL_L2_BAR
+        assert bf16_mismatch(got, ref)[0] <= FLIP_FRACTION_BAR + 1.0 / n
+
+
 def test_qgemv_vocab_sized_matches_oracle(fk):
     """The 219 MB shape whose streaming rate the kernel bench reports (1536 blocks, many tiles per block)."""
     n, k = 151936, 2560
