@@ -141,7 +141,8 @@ inline TileChoice gemv_tile_choice(const GemvShape& s, uint32_t lr, uint32_t cus
     const uint32_t K = s.K, cpr = s.cpr(), gpr = s.gpr(), nseg = s.nseg;
     TileChoice best{0, 0};
     uint64_t best_cost = ~0ull, best_per_cu = 0;
-    if (s.kind != W_BF16 && gpr < 4) return best;  // a tile's scales are fetched in whole runs of four
+    // a tile's scales are fetched in whole runs of four, and as whole groups a row (K = 576 with groups of 128 has 4.5)
+    if (s.kind != W_BF16 && (gpr < 4 || K % s.group != 0)) return best;
     for (uint32_t nl : {1u, 2u, 3u, 4u, 6u, 8u}) {
         uint32_t r = nl * kGemvBlock / cpr;
         if (r > kGemvBlock / lr) r = kGemvBlock / lr;

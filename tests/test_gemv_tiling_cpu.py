@@ -27,7 +27,7 @@ static int call(const GemvShape& s) {
     const bool same = t->rows == fresh.rows && t->blocks == fresh.blocks && t->lr == fresh.lr && t->chunks == fresh.chunks;
     const bool fits = !t->chunks || (t->rows >= 1 && t->rows * cpr <= t->chunks * kGemvBlock && t->rows * t->lr <= (uint32_t)kGemvBlock &&
                                      t->blocks == s.tiles(t->rows) && s.tile_lds(t->rows, t->chunks) <= kMaxLds &&
-                                     (s.kind == W_BF16 || (gpr >= 4 && t->rows * gpr <= kTileGroups)));
+                                     (s.kind == W_BF16 || (gpr >= 4 && s.K % s.group == 0 && t->rows * gpr <= kTileGroups)));
     if (same && fits) return 0;
     printf("kind %d nseg %u n %u K %u group %u: rows %u (%u groups) chunks %u%s\n", s.kind, s.nseg, s.n[0], s.K, s.group, t->rows,
            t->rows * gpr, t->chunks, same ? "" : ", another launch's");
@@ -53,8 +53,7 @@ int main() {
             for (uint32_t nseg : {1u, 2u})
                 for (WKind kind : {W_Q4, W_Q8, W_BF16})
                     for (uint32_t group : {64u, 32u, 128u, 64u, 128u, 32u})
-                        if (kind != W_BF16 && K % group == 0) bad += call(shape(kind, nseg, n, K, group));
-                        else if (kind == W_BF16) bad += call(shape(kind, nseg, n, K, 0));
+                        bad += call(shape(kind, nseg, n, K, kind == W_BF16 ? 0 : group));
     // a fan-out of the same first matrix, and a policy, are other launches too
     GemvShape s = shape(W_Q4, 1, 2560, 2560, 64);
     bad += call(s);
