@@ -223,7 +223,7 @@ bool qgemm_takes_rows(uint32_t M, uint32_t bits, uint32_t group, uint32_t K);
 fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out);
 // Routed projections of several tokens, each expert's weights read once for all of its routes (same arguments as
 // plan_routed_gemv); the rule that says which calls take it.
-bool qgemm_takes_routed(const fk_weight* W, uint32_t n_experts, uint32_t n_x_rows, uint32_t n_routes);
+bool qgemm_takes_routed(const fk_weight* W, bool pair, uint32_t n_experts, uint32_t n_x_rows, uint32_t n_routes);
 fk_status plan_qgemm_routed(const uint16_t* x, uint32_t n_x_rows, const fk_weight* Wa, const fk_weight* Wb, uint32_t n_experts,
                             const uint32_t* row_idx, const uint32_t* expert_idx, const uint16_t* route_weight, uint32_t n_routes,
                             uint16_t* y, Launch* out);

@@ -12,6 +12,7 @@
 // piece while this one is finished.
 #include "fk_host.hpp"
 #include "gemv_kernel.hpp"
+#include "routed_rule.hpp"
 
 #include "fk_probe.hpp"
 FK_PROBE_DEFINE(routed, 1024, 8)
@@ -26,8 +27,7 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));   // 16 bytes of an operand at any of its addresses
 
-constexpr uint32_t kRtThreads = 256, kRtWaves = 4, kRtMaxRoutes = 1024, kRtMaxExperts = 256, kRtLine = 9,
-                   kRtRows = 16;   // routes of an expert served together: one tile
+constexpr uint32_t kRtThreads = kRtWaves * kWave, kRtMaxRoutes = 1024, kRtMaxExperts = 256, kRtLine = 9;
 
 struct QgemmRoutedArgs {
     const unsigned char* w[2];   // stacks of n_experts matrices: one, or gate and up
@@ -43,7 +43,6 @@ struct QgemmRoutedArgs {
     uint32_t tiles;               // pieces of one expert
 };
 
-__host__ __device__ constexpr uint32_t rt_slab_groups(uint32_t bits) { return bits == 4 ? 4u : 2u; }
 // The sorted list: row << 16 | route by expert; routes of an expert (then their first place); the pieces' experts, first
 // places and counts.
 struct RtList {
@@ -181,8 +180,7 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
     if (blockIdx.x >= pieces) return;
     const uint32_t g0 = wave * G / kRtWaves, g1 = (wave + 1u) * G / kRtWaves;
     const uint32_t gl = g1 > g0 ? g1 - 1u : (g0 < G ? g0 : G - 1u);
-    // slabs of a piece, the same for every wave and even: the next piece's first slab takes the first set of registers again
-    const uint32_t per_wave = (G + kRtWaves - 1u) / kRtWaves, slabs = ((per_wave + SG - 1u) / SG + 1u) & ~1u;
+    const uint32_t slabs = rt_slabs(K, BITS);
 
     // A piece: uniform bases, 32-bit lane offsets (rows past the matrix repeat its last one and are not stored).
     struct Piece {
@@ -356,16 +354,13 @@ const void* routed_func(bool pair) {
 
 }  // namespace
 
-// From three quarters of a route per expert: below that hardly an expert is named twice and the route-by-route stream, which
-// has no list to sort, is ahead.  64 experts of 2 x 1408 x 2048 + 2048 x 1408 int4, uniform routes, a layer of the model, us, route by
-// route / this form: 24 routes 113 / 116, 36 125 / 126, 48 133.5 / 132, 60 156 / 151, 72 168 / 158, 96 182 / 166, 144 226 / 190, 288 333 / 211,
-// 576 590 / 303.
-bool qgemm_takes_routed(const fk_weight* W, uint32_t n_experts, uint32_t n_x_rows, uint32_t n_routes) {
-    if (4u * (uint64_t)n_routes < 3u * (uint64_t)n_experts) return false;
+bool qgemm_takes_routed(const fk_weight* W, bool pair, uint32_t n_experts, uint32_t n_x_rows, uint32_t n_routes) {
     if (n_x_rows < 2 || n_x_rows > 0xffffu || n_routes > kRtMaxRoutes || n_experts > kRtMaxExperts) return false;
     if ((W->bits != 4 && W->bits != 8) || (W->group != 64 && !(W->group == 128 && W->k % 128u == 0)) || W->k < 64u || W->k % 64u) return false;
     // 32-bit offsets: into the activations, into a tile's rows
-    return (uint64_t)n_x_rows * W->k * 2u <= 0xffffffffull && (uint64_t)32u * W->k <= 0xffffffffull && (uint64_t)n_experts * W->n <= 0x7fffffffull;
+    if ((uint64_t)n_x_rows * W->k * 2u > 0xffffffffull || (uint64_t)32u * W->k > 0xffffffffull || (uint64_t)n_experts * W->n > 0x7fffffffull) return false;
+    const DeviceFacts* dev;
+    return device_facts(&dev) == FK_OK && routes_served_together(n_experts, n_routes, W->n, W->k, W->bits, pair, (uint32_t)dev->cus);
 }
 
 fk_status plan_qgemm_routed(const uint16_t* x, uint32_t n_x_rows, const fk_weight* Wa, const fk_weight* Wb, uint32_t n_experts,
@@ -397,7 +392,7 @@ fk_status plan_qgemm_routed(const uint16_t* x, uint32_t n_x_rows, const fk_weigh
     a.n_routes = n_routes;
     a.n_experts = n_experts;
     a.n_x_rows = n_x_rows;
-    a.tiles = pair ? (a.N + 15u) / 16u : (a.N + 31u) / 32u;
+    a.tiles = rt_pieces_of_an_expert(a.N, pair);
     const uint64_t most = (uint64_t)(n_routes < n_experts ? n_routes : n_experts + n_routes / kRtRows) * a.tiles;
     const uint32_t resident = 3u * (uint32_t)dev->cus;   // by LDS four; two were 1 %, four 0 .. 1 % slower
     out->func = Wa->bits == 4 ? routed_func<W_Q4>(pair) : routed_func<W_Q8>(pair);

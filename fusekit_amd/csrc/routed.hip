@@ -419,7 +419,7 @@ fk_status plan_routed_gemv(const uint16_t* x, uint32_t n_x_rows, const fk_weight
     if (n_routes > 65536) return set_error(FK_ERR_UNSUPPORTED, "routed: at most 65536 routes per launch");
     if (!w_a) return set_error(FK_ERR_INVALID, "routed: null weight");
     const bool swiglu = w_b != nullptr;
-    if (!rk && !sh_a && !order && qgemm_takes_routed(w_a, n_experts, n_x_rows, n_routes))
+    if (!rk && !sh_a && !order && qgemm_takes_routed(w_a, swiglu, n_experts, n_x_rows, n_routes))
         return plan_qgemm_routed(x, n_x_rows, w_a, w_b, n_experts, row_idx, expert_idx, route_weight, n_routes, y, out);
 
     GemvRequest rq;

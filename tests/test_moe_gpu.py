@@ -10,6 +10,7 @@ import pytest
 import oracle
 from helpers import bf16_mismatch, make_qweight, normal_bf16, rel_l2, rng, to_device
 from test_gemv_gpu import FLIP_FRACTION_BAR, REL_L2_BAR, _check_swiglu
+from test_routed_rule_cpu import TOGETHER
 
 pytestmark = pytest.mark.gpu
 
@@ -256,16 +257,15 @@ def test_routed_reduce_tokens_and_row_idx(fk):
     assert frac <= FLIP_FRACTION_BAR and ulps <= 2.0, (frac, ulps)
 
 
-# (experts, outputs, K, tokens, top-k, bits, group): the fewest routes that are served together; outputs no multiple of 16; K of 11 and
-# of 3 groups (waves with more and fewer, and with none); a group of 128; more experts than a wave; 1024 routes, the most
-TOGETHER = [(8, 40, 704, 3, 2, 4, 64), (4, 333, 192, 40, 4, 4, 64), (16, 48, 256, 30, 6, 8, 64), (16, 32, 384, 17, 3, 8, 128),
-            (100, 16, 128, 64, 4, 4, 64), (5, 16, 64, 512, 2, 4, 64)]
+# As TOGETHER, in sizes so small that they are served route by route, however many routes an expert has.
+ROUTE_BY_ROUTE = [(8, 40, 704, 3, 2, 4, 64), (4, 333, 192, 40, 4, 4, 64), (16, 48, 256, 30, 6, 8, 64), (16, 32, 384, 17, 3, 8, 128),
+                  (100, 16, 128, 64, 4, 4, 64), (5, 16, 64, 512, 2, 4, 64)]
 
 
-@pytest.mark.parametrize("E,O,K,tokens,top_k,bits,group", TOGETHER)
+@pytest.mark.parametrize("E,O,K,tokens,top_k,bits,group", ROUTE_BY_ROUTE + TOGETHER)
 def test_routes_of_an_expert_served_together(fk, E, O, K, tokens, top_k, bits, group):
-    """Three quarters of a route per expert and more: pair and single matrix against the oracle, by the bars of the other
-    routed tests; half of the routes go to one expert (several chunks of 16), one expert index and one row index lie beyond
+    """Three quarters of a route per expert and more, in both forms: pair and single matrix against the oracle, by the bars of the
+    other routed tests; half of the routes go to one expert (several chunks of 16), one expert index and one row index lie beyond
     the range, and nothing is written past the outputs."""
     n = tokens * top_k
     stack = lambda seed: oracle.StackedWeight([make_qweight(seed + e, O, K, bits, group) for e in range(E)])
