@@ -185,7 +185,13 @@ fk_status fk_gateup_swiglu_rows(const uint16_t *x, uint32_t rows, const uint16_t
  *     Route r reads activation row min(row_idx[r], n_x_rows-1) (row_idx NULL: row r)
  *     and expert min(expert_idx[r], n_experts-1);
  *     out0[r, o] = T(((sigmoid(g) * g) * u) * route_weight[r]) with g, u = T(acc)
- *     (route_weight NULL: factor 1). */
+ *     (route_weight NULL: factor 1).
+ *     Several rows (no order, no shared pair; 4- or 8-bit, group 64, or 128 that divides k; up to 1024 routes of up to 256
+ *     experts): where a call's shape makes it cheaper, an expert's weights are read once for all of its routes.  The
+ *     choice goes by the numbers of routes and experts, n, k and bits alone.  The arithmetic is as wide (exact codes, fp32
+ *     sums), but a dot product is then added up group by group in another order, so a route's output may differ in its
+ *     last bit from what the same route gives in a call with fewer routes; fk_routed_qmv_reduce likewise.  A call
+ *     with `order` (below), or of one row, does not change with the number of routes in this way. */
 fk_status fk_routed_qmv_swiglu(const uint16_t *x, uint32_t n_x_rows, const fk_weight *Wg, const fk_weight *Wu,
                                uint32_t n_experts, const uint32_t *row_idx, const uint32_t *expert_idx,
                                const uint16_t *route_weight, uint32_t n_routes, uint16_t *out0, fk_stream s);
