@@ -221,10 +221,8 @@ __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, 
             // ms, 24 tokens of a 12-layer model with heads of 64 dims 7.76 / 7.63, behind 2500 positions 8.33 / 8.15)
             if (a.sdpa.qk_dim == 128)
                 sdpa_block<1, 2, Args, 0, true, true, 16>(a.sdpa, kv_len0, split, sync.xcd, gz, G, work);
-            else if (a.sdpa.qk_dim == 64)
+            else  // 64: xcd_layer_supported admits no other
                 sdpa_block<1, 2, Args, 0, true, true, 8>(a.sdpa, kv_len0, split, sync.xcd, gz, G, work);
-            else
-                sdpa_block<1, 2, Args, 0, true, true>(a.sdpa, kv_len0, split, sync.xcd, gz, G, work);
         }
     }
     FK_XCD_STAMP(0, 8);
