@@ -290,6 +290,39 @@ def test_routes_of_an_expert_served_together(fk, E, O, K, tokens, top_k, bits, g
     assert rel_l2(got, oracle.bf16_to_f32(ref)) <= REL_L2_BAR and bf16_mismatch(got, ref)[0] <= FLIP_FRACTION_BAR
 
 
+def _dequantized64(W):
+    """code * scale + bias in 64 bits."""
+    codes = (W.w[..., None] >> np.arange(0, 32, W.bits, dtype=np.uint32)) & np.uint32((1 << W.bits) - 1)
+    s, b = (oracle.bf16_to_f32(a).astype(np.float64).reshape(W.n, -1, 1) for a in (W.scales, W.biases))
+    return (codes.reshape(W.n, -1, W.group) * s + b).reshape(W.n, W.k)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("mean", [0.0, 1.0, 4.0])
+def test_routes_served_together_are_as_exact_as_one_by_one(fk, bits, mean):
+    """128 routes over 16 experts are served together, in expert order one by one: against the products in 64 bits the first rounds
+    no more outputs to the wrong side than the second.  Either's count is a sum of rare independent events, so equal rates differ
+    by less than four standard deviations; activations far from zero mean are where a fold that cancels shows."""
+    E, O, K, routes = 16, 1024, 2048, 128
+    W = _stack(6500, E, O, K, bits)
+    h = normal_bf16(90, (routes, K), 1.0, mean)
+    expert_idx = rng(91).integers(0, E, routes).astype(np.uint32)
+    out, ws, order = fk.DeviceBuffer(2 * routes * O), fk.DeviceBuffer(fk.routed_reduce_workspace_bytes(routes, 1, O)), fk.zeros(4 * routes)
+    d_h, d_W, d_e = _dev(fk, h), to_device(fk, W), _dev(fk, expert_idx)
+    fk.route_order(d_e, routes, E, order)
+    exact = np.empty((routes, O))
+    for e in range(E):
+        exact[expert_idx == e] = oracle.bf16_to_f32(h[expert_idx == e]).astype(np.float64) @ _dequantized64(W.expert(e)).T
+    right = oracle.f32_to_bf16(exact.astype(np.float32))   # (a second rounding of 2^-24 changes hardly any)
+
+    def wrong(call, *order_arg):
+        call(d_h, routes, d_W, E, None, d_e, None, None, None, None, routes, 1, *order_arg, out, ws)
+        return int((out.to_numpy(np.uint16, (routes, O)) != right).sum())
+
+    together, one_by_one = wrong(fk.routed_qmv_reduce), wrong(fk.routed_qmv_reduce_ordered, order)
+    assert together <= one_by_one + 4.0 * (together + one_by_one) ** 0.5, (together, one_by_one)
+
+
 def test_routes_served_in_expert_order_give_the_same_bits(fk):
     """Several tokens whose routes share experts (config-5 widths, 8 tokens x top-6 over 16 experts): fk_route_order
     is numpy's stable sort by (clamped) expert, and the routed launches served in that order -- an expert's slice

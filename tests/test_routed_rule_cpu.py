@@ -15,7 +15,7 @@ TOGETHER = [(8, 2005, 704, 24, 2, 4, 64), (4, 2189, 192, 40, 4, 4, 64), (16, 731
 MEASURED = [(64, 36, 1408, 2048, 4, 1, 0), (64, 48, 1408, 2048, 4, 1, 1), (64, 48, 1408, 2048, 8, 1, 1), (64, 48, 2048, 1408, 4, 0, 0),
             (64, 60, 2048, 1408, 4, 0, 1), (64, 576, 2048, 1408, 4, 0, 1), (128, 192, 2048, 768, 4, 0, 0), (128, 384, 2048, 768, 4, 0, 1),
             (128, 96, 2048, 768, 8, 0, 1), (256, 384, 2048, 512, 4, 0, 0), (32, 24, 1024, 1024, 4, 1, 0), (32, 96, 1024, 1024, 4, 1, 1),
-            (2, 8, 512, 512, 4, 1, 0), (8, 6, 2048, 3584, 4, 0, 0), (8, 32, 2048, 3584, 4, 0, 1)]
+            (16, 128, 1024, 2048, 4, 0, 1), (16, 128, 1024, 2048, 8, 0, 1), (2, 8, 512, 512, 4, 1, 0), (8, 6, 2048, 3584, 4, 0, 0), (8, 32, 2048, 3584, 4, 0, 1)]
 
 PROGRAM = r"""
 #include <cstdio>
