@@ -176,12 +176,18 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     // blocks, their count and their merge 2.5: 14 q / 2 kv heads x 64, split / walked, 256 positions 6.2 / 4.7 us, 384 6.4 / 5.7, 512
     // 6.5 / 6.7; 32 / 8 x 128, 128 positions 6.2 / 4.7, 256 6.5 / 6.8.  (Over a quantised cache the two differ in the last bit.)
     if (!kvq && n_chunks <= 3u) want = 1;
+    // No workspace: one block walks the context, for callers whose heads and rows fill the chip that way (at one block a CU, tiles of
+    // two heads from 2049 positions on); where they do not a null workspace is taken for an oversight.
+    if (n_chunks > 1u && (!partials || !counters)) {
+        const uint32_t pair = same_lanes && !kvq && G >= 2 && G <= 4 && max_len > 2048 ? 2u : (uint32_t)gt;
+        if ((n_chunks > 128 ? 2u : 1u) * (uint32_t)dev->cus / (n_kv * ((G + pair - 1) / pair) * rows) > 1u)
+            return set_error(FK_ERR_INVALID, "sdpa: workspace required when the context spans several ranges");
+        want = 1;
+    }
     if (want < 1) want = 1;
     if (want > 256) want = 256;
     const uint32_t cpb = (n_chunks + want - 1) / want;
     const uint32_t n_splits = (n_chunks + cpb - 1) / cpb;
-    if (n_splits > 1 && (!partials || !counters))
-        return set_error(FK_ERR_INVALID, "sdpa: workspace required when the context spans several ranges");
 
     SdpaArgs a;
     memset(&a, 0, sizeof(a));

@@ -150,6 +150,32 @@ def test_sdpa_at_the_edges_of_its_ranges_and_merge(fk, n_heads, n_kv, dim, kv_le
     _sdpa_case(fk, n_heads, n_kv, dim, dim, kv_len, kv_len)
 
 
+@pytest.mark.parametrize("n_heads,n_kv,dim,kv_len,rows,taken", [
+    (32, 8, 128, 64, 1, True), (14, 2, 64, 128, 1, True),             # one range
+    (32, 8, 128, 65, 1, False), (14, 2, 64, 383, 2, False),           # two and three ranges, far from a block a CU
+    (32, 8, 128, 400, 8, True), (128, 128, 128, 300, 2, True),        # 256 tiles
+    (32, 8, 128, 400, 4, False), (2, 2, 64, 400, 63, False),
+    (32, 8, 128, 3000, 9, True), (16, 8, 128, 3000, 9, False),        # tiles of two heads from 2049 positions on
+])
+def test_sdpa_without_a_workspace(fk, n_heads, n_kv, dim, kv_len, rows, taken):
+    """A null workspace is taken where the context is one range or a block per tile and row fills the chip of 256 CUs, and
+    refused elsewhere, however the launch would be cut with one."""
+    cap = kv_len + rows - 1
+    q, ck, cv = normal_bf16(1, (rows, n_heads * dim)), normal_bf16(2, n_kv * cap * dim), normal_bf16(3, n_kv * cap * dim)
+    dq, dk, dv = (fk.DeviceBuffer.from_numpy(a) for a in (q, ck, cv))
+    out = fk.DeviceBuffer(2 * rows * n_heads * dim)
+    call = lambda part, cnt: fk.sdpa_decode_rows(dq, dk, dv, out, rows, kv_len, n_heads, n_kv, dim, dim, cap, dim ** -0.5, part, cnt)
+    if not taken:
+        with pytest.raises(fk.InvalidArgument):
+            call(None, None)
+        return
+    call(None, None)
+    got = out.to_numpy(np.uint16, (rows, n_heads * dim))
+    for r in (0, rows - 1):
+        ref = oracle.sdpa_decode(q[r], ck, cv, n_heads, n_kv, dim, dim, kv_len + r, cap, dim ** -0.5)
+        assert rel_l2(got[r], oracle.bf16_to_f32(ref)) <= REL_L2_BAR
+
+
 @pytest.mark.parametrize("bits", [16, 4, 8])
 def test_embed_lookup(fk, bits):
     vocab, hidden = 1000, 896
