@@ -154,7 +154,7 @@ class DeviceWeight:
 
     assigned = 0   # how often a buffer of any matrix has been assigned: unchanged, no matrix has been given another buffer
 
-    _c = None      # the struct last handed out and the addresses it holds
+    _c = None      # the operators' struct and the addresses it holds
 
     def __setattr__(self, name: str, value) -> None:
         object.__setattr__(self, name, value)
@@ -170,14 +170,9 @@ class DeviceWeight:
 
     @property
     def c(self) -> Weight:
-        """fk_weight: made when an attribute has been set or a buffer's address is another (a call copies what it needs)."""
+        """fk_weight, the caller's own."""
         scales, biases = self.scales, self.biases
-        at = (self.w.ptr, scales.ptr if scales else None, biases.ptr if biases else None)
-        kept = self._c
-        if kept is None or kept[0] != at:
-            kept = (at, Weight(*at, self.n, self.k, self.bits, self.group))
-            self.__dict__["_c"] = kept
-        return kept[1]
+        return Weight(self.w.ptr, scales.ptr if scales else None, biases.ptr if biases else None, self.n, self.k, self.bits, self.group)
 
     @property
     def nbytes(self) -> int:
@@ -191,6 +186,20 @@ def _addr(b):
     return b.ptr if isinstance(b, DeviceBuffer) else int(b)
 
 
+def _w(W):
+    """An fk_weight operand (a call copies what it needs): of a DeviceWeight made when an attribute has been set or a buffer's address is
+    another.  Nothing else holds that one: what a caller does with W.c must not change the next call."""
+    if W.__class__ is not DeviceWeight:
+        return W.c
+    scales, biases = W.scales, W.biases
+    at = (W.w.ptr, scales.ptr if scales else None, biases.ptr if biases else None)
+    kept = W._c
+    if kept is None or kept[0] != at:
+        kept = (at, Weight(*at, W.n, W.k, W.bits, W.group))
+        W.__dict__["_c"] = kept
+    return kept[1]
+
+
 def _ptr(b) -> C.c_void_p:
     if b is None:
         return C.c_void_p(None)
@@ -202,56 +211,56 @@ def _ptr(b) -> C.c_void_p:
 # ---------------------------------------------------------------- operators
 
 def qgemv(W: DeviceWeight, x, bias, y, stream=None) -> None:
-    check(lib.fk_qgemv(W.c, _addr(x), _addr(bias), _addr(y), _addr(stream)))
+    check(lib.fk_qgemv(_w(W), _addr(x), _addr(bias), _addr(y), _addr(stream)))
 
 
 def linear_residual(W: DeviceWeight, x, res, res2, y, stream=None) -> None:
-    check(lib.fk_linear_residual(W.c, _addr(x), _addr(res), _addr(res2), _addr(y), _addr(stream)))
+    check(lib.fk_linear_residual(_w(W), _addr(x), _addr(res), _addr(res2), _addr(y), _addr(stream)))
 
 
 def rmsnorm_qkv(x, norm_w, eps, Wq, Wk, Wv, bq, bk, bv, q, k, v, stream=None) -> None:
-    check(lib.fk_rmsnorm_qkv(_addr(x), _addr(norm_w), eps, Wq.c, Wk.c, Wv.c, _addr(bq), _addr(bk), _addr(bv), _addr(q),
+    check(lib.fk_rmsnorm_qkv(_addr(x), _addr(norm_w), eps, _w(Wq), _w(Wk), _w(Wv), _addr(bq), _addr(bk), _addr(bv), _addr(q),
                              _addr(k), _addr(v), _addr(stream)))
 
 
 def gateup_swiglu_rows(x, rows, norm_w, eps, Wg, Wu, variant, out, stream=None) -> None:
     """fk_gateup_swiglu_rows: RMSNorm + gate / up + SwiGLU of 2..8 token rows in one launch."""
-    check(lib.fk_gateup_swiglu_rows(_addr(x), rows, _addr(norm_w), eps, Wg.c, Wu.c, variant, _addr(out), _addr(stream)))
+    check(lib.fk_gateup_swiglu_rows(_addr(x), rows, _addr(norm_w), eps, _w(Wg), _w(Wu), variant, _addr(out), _addr(stream)))
 
 
 def rmsnorm_qkv_rows(x, rows, x_row_stride, norm_w, eps, Wq, Wk, Wv, q, q_row_stride, k=None, k_row_stride=0, v=None,
                      v_row_stride=0, stream=None) -> None:
     """fk_rmsnorm_qkv_rows: RMSNorm + one to three projections of 2..8 token rows in one launch."""
-    wk = Wk.c if Wk is not None else None
-    wv = Wv.c if Wv is not None else None
-    check(lib.fk_rmsnorm_qkv_rows(_addr(x), rows, x_row_stride, _addr(norm_w), eps, Wq.c, wk, wv, _addr(q), q_row_stride,
+    wk = _w(Wk) if Wk is not None else None
+    wv = _w(Wv) if Wv is not None else None
+    check(lib.fk_rmsnorm_qkv_rows(_addr(x), rows, x_row_stride, _addr(norm_w), eps, _w(Wq), wk, wv, _addr(q), q_row_stride,
                                   _addr(k), k_row_stride, _addr(v), v_row_stride, _addr(stream)))
 
 
 def gateup_swiglu(x, norm_w, eps, Wg, Wu, variant, out, stream=None) -> None:
-    check(lib.fk_gateup_swiglu(_addr(x), _addr(norm_w), eps, Wg.c, Wu.c, variant, _addr(out), _addr(stream)))
+    check(lib.fk_gateup_swiglu(_addr(x), _addr(norm_w), eps, _w(Wg), _w(Wu), variant, _addr(out), _addr(stream)))
 
 
 def routed_qmv_swiglu(x, n_x_rows, Wg, Wu, n_experts, row_idx, expert_idx, route_weight, n_routes, out0,
                       stream=None) -> None:
     """Wg / Wu: DeviceWeight whose arrays are stacked [E, n, ...] and whose n, k describe one expert."""
-    check(lib.fk_routed_qmv_swiglu(_addr(x), n_x_rows, Wg.c, Wu.c, n_experts, _addr(row_idx), _addr(expert_idx),
+    check(lib.fk_routed_qmv_swiglu(_addr(x), n_x_rows, _w(Wg), _w(Wu), n_experts, _addr(row_idx), _addr(expert_idx),
                                    _addr(route_weight), n_routes, _addr(out0), _addr(stream)))
 
 
 def routed_qmv_swiglu_shared(x, Wg, Wu, n_experts, expert_idx, route_weight, n_routes, out0, Sg, Su, shared_out,
                              stream=None) -> None:
     """One token: the routed gate/up + SwiGLU with the shared experts' pair as further routes of the same launch."""
-    check(lib.fk_routed_qmv_swiglu_shared(_addr(x), Wg.c, Wu.c, n_experts, _addr(expert_idx), _addr(route_weight), n_routes,
-                                          _addr(out0), Sg.c, Su.c, _addr(shared_out), _addr(stream)))
+    check(lib.fk_routed_qmv_swiglu_shared(_addr(x), _w(Wg), _w(Wu), n_experts, _addr(expert_idx), _addr(route_weight), n_routes,
+                                          _addr(out0), _w(Sg), _w(Su), _addr(shared_out), _addr(stream)))
 
 
 def routed_qmv_swiglu_routing(x, Wg, Wu, n_experts, logits, scale, top_k, apply_weight, idx_out, weight_out, out0, Sg=None,
                               Su=None, shared_out=None, stream=None) -> None:
     """One token: the routed (+ shared) gate/up launch ranking the router logits itself (fk_routed_qmv_swiglu_routing)."""
-    check(lib.fk_routed_qmv_swiglu_routing(_addr(x), Wg.c, Wu.c, n_experts, _addr(logits), _addr(scale), top_k,
+    check(lib.fk_routed_qmv_swiglu_routing(_addr(x), _w(Wg), _w(Wu), n_experts, _addr(logits), _addr(scale), top_k,
                                            int(apply_weight), _addr(idx_out), _addr(weight_out), _addr(out0),
-                                           Sg.c if Sg is not None else None, Su.c if Su is not None else None,
+                                           _w(Sg) if Sg is not None else None, _w(Su) if Su is not None else None,
                                            _addr(shared_out), _addr(stream)))
 
 
@@ -269,22 +278,22 @@ def routed_reduce_workspace_bytes(n_tokens, top_k, out_dim, shared_k=0, group=64
 
 def routed_qmv_reduce(h, n_h_rows, Wd, n_experts, row_idx, expert_idx, route_weight, shared_x, W_shared,
                       residual_extra, n_tokens, top_k, out, workspace, stream=None) -> None:
-    check(lib.fk_routed_qmv_reduce(_addr(h), n_h_rows, Wd.c, n_experts, _addr(row_idx), _addr(expert_idx),
-                                   _addr(route_weight), _addr(shared_x), W_shared.c if W_shared is not None else None,
+    check(lib.fk_routed_qmv_reduce(_addr(h), n_h_rows, _w(Wd), n_experts, _addr(row_idx), _addr(expert_idx),
+                                   _addr(route_weight), _addr(shared_x), _w(W_shared) if W_shared is not None else None,
                                    _addr(residual_extra), n_tokens, top_k, _addr(out), _addr(workspace), _addr(stream)))
 
 
 def routed_qmv_swiglu_ordered(x, n_x_rows, Wg, Wu, n_experts, row_idx, expert_idx, route_weight, n_routes, order, out0,
                               stream=None) -> None:
     """fk_routed_qmv_swiglu with the routes served in `order` (fk_route_order): same results, shared slices read once."""
-    check(lib.fk_routed_qmv_swiglu_ordered(_addr(x), n_x_rows, Wg.c, Wu.c, n_experts, _addr(row_idx), _addr(expert_idx),
+    check(lib.fk_routed_qmv_swiglu_ordered(_addr(x), n_x_rows, _w(Wg), _w(Wu), n_experts, _addr(row_idx), _addr(expert_idx),
                                            _addr(route_weight), n_routes, _addr(order), _addr(out0), _addr(stream)))
 
 
 def routed_qmv_reduce_ordered(h, n_h_rows, Wd, n_experts, row_idx, expert_idx, route_weight, shared_x, W_shared,
                               residual_extra, n_tokens, top_k, order, out, workspace, stream=None) -> None:
-    check(lib.fk_routed_qmv_reduce_ordered(_addr(h), n_h_rows, Wd.c, n_experts, _addr(row_idx), _addr(expert_idx),
-                                           _addr(route_weight), _addr(shared_x), W_shared.c if W_shared is not None else None,
+    check(lib.fk_routed_qmv_reduce_ordered(_addr(h), n_h_rows, _w(Wd), n_experts, _addr(row_idx), _addr(expert_idx),
+                                           _addr(route_weight), _addr(shared_x), _w(W_shared) if W_shared is not None else None,
                                            _addr(residual_extra), n_tokens, top_k, _addr(order), _addr(out), _addr(workspace),
                                            _addr(stream)))
 
@@ -300,7 +309,7 @@ def qgemm_workspace_bytes(m, n, k, group=64) -> int:
 
 
 def qgemm(W, x, m, bias, residual, y, workspace, stream=None) -> None:
-    check(lib.fk_qgemm(W.c, _addr(x), m, _addr(bias), _addr(residual), _addr(y), _addr(workspace), _addr(stream)))
+    check(lib.fk_qgemm(_w(W), _addr(x), m, _addr(bias), _addr(residual), _addr(y), _addr(workspace), _addr(stream)))
 
 
 def qgemm_fanout(Ws, x, m, biases, ys, workspace, stream=None) -> None:
@@ -314,11 +323,11 @@ def qgemm_fanout(Ws, x, m, biases, ys, workspace, stream=None) -> None:
 
 
 def qgemm_swiglu(Wg, Wu, x, m, variant, out, workspace, stream=None) -> None:
-    check(lib.fk_qgemm_swiglu(Wg.c, Wu.c, _addr(x), m, variant, _addr(out), _addr(workspace), _addr(stream)))
+    check(lib.fk_qgemm_swiglu(_w(Wg), _w(Wu), _addr(x), m, variant, _addr(out), _addr(workspace), _addr(stream)))
 
 
 def final_rmsnorm_lm_head(x, norm_w, eps, W, logits, stream=None) -> None:
-    check(lib.fk_final_rmsnorm_lm_head(_addr(x), _addr(norm_w), eps, W.c, _addr(logits), _addr(stream)))
+    check(lib.fk_final_rmsnorm_lm_head(_addr(x), _addr(norm_w), eps, _w(W), _addr(logits), _addr(stream)))
 
 
 HEAD_ARGMAX_WORKSPACE_BYTES = 32776
@@ -327,7 +336,7 @@ HEAD_ARGMAX_WORKSPACE_BYTES = 32776
 def final_rmsnorm_lm_head_argmax(x, norm_w, eps, W, logits, next_token, history, hist_counter, hist_capacity, workspace,
                                  stream=None) -> None:
     """The LM head that also selects the greedy token (one launch); UnsupportedError unless gemv_form(...) == 1."""
-    check(lib.fk_final_rmsnorm_lm_head_argmax(_addr(x), _addr(norm_w), eps, W.c, _addr(logits), _addr(next_token),
+    check(lib.fk_final_rmsnorm_lm_head_argmax(_addr(x), _addr(norm_w), eps, _w(W), _addr(logits), _addr(next_token),
                                               _addr(history), _addr(hist_counter), hist_capacity, _addr(workspace),
                                               _addr(stream)))
 
@@ -459,7 +468,7 @@ def rmsnorm_rows(x, w, eps, rows, hidden, y, stream=None):
 
 
 def embed_lookup_rows(E, d_tokens, rows, out_scale, x, stream=None):
-    check(lib.fk_embed_lookup_rows(E.c, _addr(d_tokens), rows, out_scale, _addr(x), _addr(stream)))
+    check(lib.fk_embed_lookup_rows(_w(E), _addr(d_tokens), rows, out_scale, _addr(x), _addr(stream)))
 
 
 def qkv_rope_store_rows(q, k, v, q_norm, k_norm, n_heads, n_kv, head_dim, rope_dims, theta, eps, rows, offset,
@@ -521,7 +530,7 @@ def dequantize_bf16(W: DeviceWeight, stream=None) -> DeviceWeight:
     D = DeviceWeight.__new__(DeviceWeight)
     D.n, D.k, D.bits, D.group, D.scales, D.biases = W.n, W.k, 16, 0, None, None
     D.w = DeviceBuffer(W.n * W.k * 2)
-    check(lib.fk_dequantize_bf16(W.c, _addr(D.w), _addr(stream)))
+    check(lib.fk_dequantize_bf16(_w(W), _addr(D.w), _addr(stream)))
     return D
 
 
@@ -534,7 +543,7 @@ def set_gemm_library_rows(rows: int):
 
 
 def embed_lookup_decode(E, d_token, token, out_scale, x, stream=None):
-    check(lib.fk_embed_lookup_decode(E.c, _addr(d_token), token, out_scale, _addr(x), _addr(stream)))
+    check(lib.fk_embed_lookup_decode(_w(E), _addr(d_token), token, out_scale, _addr(x), _addr(stream)))
 
 
 ARGMAX_WORKSPACE_BYTES = 1288
