@@ -198,6 +198,41 @@ def test_attention_of_128_dims_equals_the_general_form_bit_for_bit(fk, bits, n_h
     assert np.isfinite(oracle.bf16_to_f32(got[0])).all() and np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("n_heads,n_kv,kv_len,max_len,rows", [
+    (2, 2, 1, 1, 1), (6, 2, 131, 200, 3),                              # a head a block, one range and the second's first keys
+    (4, 4, 2999, 3001, 2), (4, 2, 2113, 2120, 1),                      # tiles of 1 and 2 heads, ranges that a block walks
+    (6, 2, 2201, 2300, 1), (16, 4, 2049, 4096, 1), (16, 4, 4095, 4100, 2),   # tiles of 4, two scores a lane: three heads of four, all
+    (7, 1, 130, 140, 2), (12, 2, 3000, 3000, 1),                       # the tile of 8, which goes through LDS
+])
+def test_attention_of_64_dims_against_the_oracle_and_the_general_form(fk, bits, n_heads, n_kv, kv_len, max_len, rows):
+    """Heads of 64 dims with one group to a row, 8 lanes a row, every lane its own scores: the oracle's rows, and bit for bit those of
+    the general form, which takes the same cache written as groups of 32 with a group's scale and bias twice."""
+    dim, cap = 64, max_len + rows - 1
+    rs = rng(bits * 100 + kv_len)
+    whole, halves = ([oracle.QuantCache(n_kv, cap, dim, bits, g) for _ in range(2)] for g in (64, 32))
+    for w, h in zip(whole, halves):
+        w.packed[:] = rs.integers(0, 2 ** 32, w.packed.shape, dtype=np.uint32)
+        w.scales[:] = oracle.f32_to_bf16((rs.standard_normal(w.scales.shape) * 0.02 + (0.1 if bits == 4 else 0.008)).astype(np.float32))
+        w.biases[:] = oracle.f32_to_bf16((rs.standard_normal(w.biases.shape) * 0.3 - (0.7 if bits == 4 else 1.0)).astype(np.float32))
+        h.packed[:], h.scales[:], h.biases[:] = w.packed, w.scales.repeat(2, axis=-1), w.biases.repeat(2, axis=-1)
+    q = normal_bf16(73, (rows, n_heads * dim), 2.0)
+    got = []
+    for host, group in ((whole, 64), (halves, 32)):
+        K, V = _caches(fk, n_kv, cap, dim, bits, group)
+        _upload(fk, host[0], K), _upload(fk, host[1], V)
+        out = fk.DeviceBuffer(2 * rows * n_heads * dim)
+        pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, dim, dim, cap)
+        fk.sdpa_decode_quant(_dev(fk, q), K, V, out, None, kv_len, cap, rows, n_heads, dim ** -0.5, fk.DeviceBuffer(max(pb, 4) * rows),
+                             fk.zeros(max(cb, 4) * rows))
+        got.append(out.to_numpy(np.uint16, (rows, n_heads * dim)))
+    assert np.array_equal(got[0], got[1])
+    for r in range(rows):
+        want = oracle.bf16_to_f32(oracle.sdpa_decode_quant(q[r], *whole, n_heads, kv_len + r, dim ** -0.5))
+        assert rel_l2(got[0][r], want) <= 1e-2
+        assert np.max(np.abs(oracle.bf16_to_f32(got[0][r]) - want)) <= 2.0 ** -6 * np.max(np.abs(want))
+
+
 def test_rejects_bad_geometry(fk):
     K, V = _caches(fk, 2, 16, 128, 4, 64)
     k = _dev(fk, normal_bf16(1, 256))
