@@ -55,34 +55,35 @@ fk_status sdpa_workspace_bytes(uint32_t n_heads, uint32_t n_kv, uint32_t qk_dim,
 
 namespace {
 
-// The kernels by tile, cache and row form.  A bf16 cache has tiles of 1 and 2 heads; those of 4 and of 8 belong to quantised caches.
+// The kernels by tile, cache and row form.  A bf16 cache has tiles of 1 and 2 heads and, where keys and values differ too much in width,
+// of 8 in the general form; tiles of 4 belong to quantised caches.
 template <int GT, int Q>
 const void* decode_func(int row) {
-    if (row == 16) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 16>);
-    if (row == 8) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 8>);
+    if constexpr (GT <= 4 || Q != 0) {
+        if (row == 16) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 16>);
+        if (row == 8) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 8>);
+    }
     return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 0>);
 }
 template <int GT, bool F, int Q>
 const void* fused_func(int row) {
-    if (row == 16) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 16>);
-    if (row == 8) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 8>);
+    if constexpr (GT <= 4 || Q != 0) {
+        if (row == 16) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 16>);
+        if (row == 8) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 8>);
+    }
     return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 0>);
 }
 template <int Q>
 const void* decode_func(int gt, int row) {
-    if constexpr (Q != 0) {
+    if constexpr (Q != 0)
         if (gt == 4) return decode_func<4, Q>(row);
-        if (gt == 8) return decode_func<8, Q>(row);
-    }
-    return gt == 1 ? decode_func<1, Q>(row) : decode_func<2, Q>(row);
+    return gt == 1 ? decode_func<1, Q>(row) : (gt == 2 ? decode_func<2, Q>(row) : decode_func<8, Q>(row));
 }
 template <bool F, int Q>
 const void* fused_tile(int gt, int row) {
-    if constexpr (Q != 0) {
+    if constexpr (Q != 0)
         if (gt == 4) return fused_func<4, F, Q>(row);
-        if (gt == 8) return fused_func<8, F, Q>(row);
-    }
-    return gt == 1 ? fused_func<1, F, Q>(row) : fused_func<2, F, Q>(row);
+    return gt == 1 ? fused_func<1, F, Q>(row) : (gt == 2 ? fused_func<2, F, Q>(row) : fused_func<8, F, Q>(row));
 }
 template <int Q>
 const void* fused_func(bool fast, int gt, int row) { return fast ? fused_tile<true, Q>(gt, row) : fused_tile<false, Q>(gt, row); }
@@ -136,10 +137,11 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     const uint32_t n_chunks = (max_len + chunk - 1) / chunk;
     const uint32_t G = n_heads / n_kv;
     // Tiles of 1, 2 or 4 heads run the wave-local form, which needs a key row and its value row on
-    // the same lanes.  Rows of different widths (192 / 128) both take the lane count of the wider one -- the spare
-    // lanes of the narrower row idle; a row of 512 dims still fits a wave --, of a quantised cache the tile of 8, which goes through LDS.
+    // the same lanes (equal lanes per row); other shapes take the tile of 8, which goes through LDS.
+    // Rows of different widths (192 / 128) both take the lane count of the wider one -- the spare
+    // lanes of the narrower row idle -- as long as a row fits a wave; bf16 caches only.
     const uint32_t lpk0 = pow2_ceil(qk_dim / 8), lpv0 = pow2_ceil(v_dim / 8), lp_wide = lpk0 > lpv0 ? lpk0 : lpv0;
-    const bool same_lanes = lpk0 == lpv0 || !kvq;
+    const bool same_lanes = lpk0 == lpv0 || (!kvq && lp_wide <= (uint32_t)kWave);
     int gt = !same_lanes ? 8 : (G >= 8 ? 8 : (G >= 4 ? (G == 4 ? 4 : 8) : (G >= 2 ? (G == 2 ? 2 : 4) : 1)));
     // Groups of 2 .. 4 query heads per KV head: smaller tiles mean more blocks with fewer registers each, and the
     // repeated K / V reads of a KV head's tiles hit the L2.  Measured (32 q / 8 kv heads x 128, cold caches), tiles
@@ -150,7 +152,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     // task alone with tiles of 8 / 4 / 2 / 1 heads: 544 positions 15.8 / 11.9 / 10.7 / 9.8 us, 4096 18.4 / 14.2 / 14.2 /
     // 13.4, 12032 30.6 / 19.1 / 17.7 / 18.6.  (Not over a quantised cache: the two forms differ in the last bit, and what
     // follows from that -- a key whose group takes the other sign of its scale -- stays in the cache.)
-    if (!kvq && G > 4) gt = max_len <= 4096 ? 1 : 2;
+    if (same_lanes && G > 4 && !kvq) gt = max_len <= 4096 ? 1 : 2;
     // Long contexts: a block walks several consecutive ranges (online softmax, the next range's rows in flight), so that the
     // grid stays near one to two blocks per CU and the final merge, which draws every partial into one CU, stays short.
     // (several active rows multiply the tiles: each row then needs fewer ranges to fill the chip; 8 rows x 16 heads at
@@ -166,7 +168,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     // 2048 positions 10.5 / 10.2 us, 3300 12.9 / 12.1, 4096 13.5 / 12.7; 28 / 4, 4096 14.3 / 12.3; 64 / 8, 1000 10.1 / 9.6, 4096
     // 22.0 / 16.2.  Where one a CU walks fewer it is the slower: 32 / 8, 1000 positions 8.4 / 8.8; and with a KV head per query
     // head, whose reads share nothing: 32 / 32, 2048 positions 12.7 / 13.6.
-    if (rows == 1 && !kvq && G >= 2 && max_len <= 4096 && want < 16u && n_chunks > 3u * want) {
+    if (rows == 1 && same_lanes && !kvq && G >= 2 && max_len <= 4096 && want < 16u && n_chunks > 3u * want) {
         const uint32_t two = 2u * (uint32_t)dev->cus / tiles;
         want = two < 16u ? two : 16u;
     }
@@ -177,7 +179,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     // No workspace: one block walks the context, for callers whose heads and rows fill the chip that way (at one block a CU, tiles of
     // two heads from 2049 positions on); where they do not a null workspace is taken for an oversight.
     if (n_chunks > 1u && (!partials || !counters)) {
-        const uint32_t pair = !kvq && G >= 2 && G <= 4 && max_len > 2048 ? 2u : (uint32_t)gt;
+        const uint32_t pair = same_lanes && !kvq && G >= 2 && G <= 4 && max_len > 2048 ? 2u : (uint32_t)gt;
         if ((n_chunks > 128 ? 2u : 1u) * (uint32_t)dev->cus / (n_kv * ((G + pair - 1) / pair) * rows) > 1u)
             return set_error(FK_ERR_INVALID, "sdpa: workspace required when the context spans several ranges");
         want = 1;
@@ -226,7 +228,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     // with the scales alone, 30.1 / 28.2)
     const bool alike = qk_dim == v_dim && (!kvq || quant->group == 64);
     const bool words = !kvq || (((uintptr_t)quant->k_scales | (uintptr_t)quant->k_biases | (uintptr_t)quant->v_scales | (uintptr_t)quant->v_biases) & 3u) == 0;
-    const int row = alike && qk_dim == 128 && words ? 16 : (alike && qk_dim == 64 ? 8 : 0);
+    const int row = gt > 4 && !kvq ? 0 : (alike && qk_dim == 128 && words ? 16 : (alike && qk_dim == 64 ? 8 : 0));
     const void* func = nullptr;
     if (fusion) {
         // whole-width rotation of at most 128 dims with a table: the form whose loads run ahead
