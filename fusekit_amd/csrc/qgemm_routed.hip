@@ -232,8 +232,6 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
 #pragma unroll
         for (int h = 0; h < 2; ++h) s.x[h] = *reinterpret_cast<const u32x4_any_t*>(xbase + (q.xoff + gc * 128u + 16u * (uint32_t)h));
     };
-    const uint4 ones4 = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
-    const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, ones4);
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     f32x4_t acc[NT];
     // A group's product is formed about the codes' middle: the matrix instructions start from -MID * Sx and the fold adds
@@ -241,22 +239,23 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
     // with activations whose mean is not zero what is lost there is more than the route-by-route form loses, whose terms have
     // half the length.  Outputs rounded to the wrong side, of a million, route by route / uncentred / this: 64 experts of
     // 1408 x 2048 int4, activations of mean 0 104 / 136 / 82, mean 1 281 / 514 / 148, mean 4 27 / 529 / 21; 16 of 1024 x 2048, 8
-    // bits, 117 / 160 / 85, 206 / 795 / 146, 90 / 627 / 111.  Uncentred / this, us: pair of 1408 x 2048 int4, 48 routes 29.5 / 30.4, 96
-    // 43.1 / 44.6, 576 61.5 / 61.6; 8 bits, 96 routes 66.4 / 67.4.
+    // bits, 117 / 160 / 85, 206 / 795 / 146, 90 / 627 / 111.  Uncentred / this, us: pair of 1408 x 2048 int4, 48 routes 28.6 / 29.2, 96
+    // 42.6 / 43.9, 576 60.9 / 61.3; 8 bits, 96 routes 65.7 / 66.2.
     // HALVES: each half of a group starts from its own Sx.  8-bit codes need it: from the whole group's, what the first half has
     // not yet made up for is 128 times the other half's sum (309 of a million at mean 1).
     constexpr float MID = KIND == W_Q4 ? 8.f : 128.f;
+    constexpr uint32_t MID2 = KIND == W_Q4 ? 0xC100C100u : 0xC300C300u;   // -MID as two bf16 values
     constexpr bool HALVES = KIND == W_Q8;
+    const bf16x8_t mids = __builtin_bit_cast(bf16x8_t, make_uint4(MID2, MID2, MID2, MID2));
     auto consume = [&](uint32_t u, const Acts& x) __attribute__((always_inline)) {   // group u of the parked slab
         const bf16x8_t xa0 = __builtin_bit_cast(bf16x8_t, x.x[0]), xa1 = __builtin_bit_cast(bf16x8_t, x.x[1]);
-        const f32x4_t s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa0, ones, zero, 0, 0, 0);
-        const f32x4_t s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa1, ones, HALVES ? zero : s0, 0, 0, 0);
-        f32x4_t sx, from0, from1;
+        // -MID * Sx, as the instructions take it (a power of two: exactly MID times what Sx would be)
+        const f32x4_t m0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa0, mids, zero, 0, 0, 0);
+        const f32x4_t m1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa1, mids, HALVES ? zero : m0, 0, 0, 0);
+        f32x4_t mx = m1;
+        if constexpr (HALVES) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            sx[r] = HALVES ? s0[r] + s1[r] : s1[r];
-            from0[r] = -MID * (HALVES ? s0[r] : s1[r]);
-            from1[r] = HALVES ? -MID * s1[r] : 0.f;
+            for (int r = 0; r < 4; ++r) mx[r] += m0[r];
         }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -272,11 +271,11 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
                 b1 = rt_unpack<KIND>(v.z, v.w);
             }
             const uint32_t sb = ml[((uint32_t)t * 16u + c16) * 4u + u];
-            const float sf = bf16_lo(sb), bm = fmaf(MID, sf, bf16_hi(sb));
-            f32x4_t c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa0, b0, from0, 0, 0, 0);
-            const f32x4_t c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa1, b1, HALVES ? from1 : c, 0, 0, 0);
+            const float sf = bf16_lo(sb), bm = fmaf(bf16_hi(sb), -1.f / MID, -sf);   // (b + MID s) / -MID
+            f32x4_t c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa0, b0, HALVES ? m0 : mx, 0, 0, 0);
+            const f32x4_t c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa1, b1, HALVES ? m1 : c, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[t][r] += fmaf(sf, HALVES ? c[r] + c1[r] : c1[r], bm * sx[r]);
+            for (int r = 0; r < 4; ++r) acc[t][r] += fmaf(sf, HALVES ? c[r] + c1[r] : c1[r], bm * mx[r]);
         }
     };
 
