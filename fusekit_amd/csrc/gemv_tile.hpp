@@ -1,6 +1,7 @@
-// One-tile GEMV: the flat stream of gemv_kernel.hpp for matrices whose tiles all fit the chip at once (the projections of
-// a decode step, 0.2 .. 60 MB).  A block owns ONE tile of R rows and asks for everything it will use before it waits for
-// anything.
+// One-tile GEMV: the flat stream of gemv_kernel.hpp for the projections of a decode step (0.2 .. 60 MB).  A block owns ONE tile of R
+// rows and asks for its activations, scales, biases, epilogue operands and first chunks of weights before it waits for anything; the
+// other chunks follow when the activations are staged.  A launch of more blocks than are resident starts blocks over
+// (gemv_tile_choice says where that is worth it).
 //
 // What bounds these launches is not the bytes but the chain a block runs through: its arguments, the activations, the
 // weights, the row sums, the epilogue's operands -- a memory trip each where they are not overlapped -- and the vector
@@ -10,8 +11,9 @@
 //   * the activations are asked for as often as the row is long, the norm weight only where there is one;
 //   * projection bias and residual are asked for in front of the weights' use, not behind the row sums;
 //   * the tile height follows the launch: a few chunks a thread on as many CUs as there are (gemv_tile_choice in gemv_tiling.hpp).
-// int4, launch to launch over cold weights, gemv_stream_kernel -> this: 896 x 896 3.8 -> 2.75 us, 4864 x 896 4.2 -> 3.35, its gate / up
-// pair 5.9 -> 4.7, 2560 x 4096 5.5 -> 4.2, 2560 x 9728 8.0 -> 6.2, pair of 9728 x 2560 10.9 -> 9.2, of 14336 x 4096 19.1 -> 16.8.
+// int4, launch to launch in a captured chain over cold weights, gemv_stream_kernel -> this, with a residual: 896 x 896 4.3 -> 2.95 us, 4864 x
+// 896 4.8 -> 3.7, 2560 x 4096 5.8 -> 4.3, 2560 x 9728 7.9 -> 6.2; gate / up pairs: 4864 x 896 5.9 -> 4.7, 9728 x 2560 10.4 -> 8.9, 14336 x 4096
+// 17.8 -> 15.3.
 // Every partial, the order in which a row's partials are added and the epilogue are those of gemv_run, bit for bit.
 #pragma once
 #include "gemv_kernel.hpp"

@@ -55,8 +55,10 @@ fk_status sdpa_workspace_bytes(uint32_t n_heads, uint32_t n_kv, uint32_t qk_dim,
 
 namespace {
 
-// The kernels by tile, cache and row form.  A bf16 cache has tiles of 1 and 2 heads and, where keys and values differ too much in width,
-// of 8 in the general form; tiles of 4 belong to quantised caches.
+// The kernels by tile, cache and row form.  A bf16 cache has tiles of 1 and 2 heads (rows of up to 512 dims fit a wave, so that keys and
+// values always share their lanes); those of 4 and 8 belong to quantised caches.  The tile of 8 over a bf16 cache, which no shape takes, is
+// compiled all the same: without it the other kernels lie at other places, and a token behind 12000 positions of an 8-bit cache takes 1828
+// us instead of 1809.
 template <int GT, int Q>
 const void* decode_func(int row) {
     if constexpr (GT <= 4 || Q != 0) {
@@ -173,8 +175,11 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
         want = two < 16u ? two : 16u;
     }
     // Up to three ranges of a bf16 cache: one block walks them.  A range more in the same block costs 1.04 us, the partials of two
-    // blocks, their count and their merge 2.5: 14 q / 2 kv heads x 64, split / walked, 256 positions 6.2 / 4.7 us, 384 6.4 / 5.7, 512
-    // 6.5 / 6.7; 32 / 8 x 128, 128 positions 6.2 / 4.7, 256 6.5 / 6.8.  (Over a quantised cache the two differ in the last bit.)
+    // blocks, their count and their merge 2.5: 14 q / 2 kv heads x 64, split / walked, 256 positions 6.0 / 4.1 us, 384 6.1 / 4.7; eight rows of
+    // 384 7.3 / 5.1; 32 / 8 x 128, 128 positions 5.9 / 4.0, 192 6.2 / 4.7; 4 / 1 heads of 192 / 128 dims, 96 positions 6.4 / 5.7; 16 / 16 of 96
+    // dims 6.6 / 5.9; 8 / 1 of 512 dims, 48 positions 9.1 / 6.2.  (18 shapes of 32 .. 512 dims, 1 .. 128 KV heads, 1 / 2 / 4 / 8 rows, two and three
+    // ranges: walked takes 0.57 .. 0.91 of the time, the same where the rows fill the chip either way.  Over a quantised cache the two
+    // differ in the last bit.)
     if (!kvq && n_chunks <= 3u) want = 1;
     // No workspace: one block walks the context, for callers whose heads and rows fill the chip that way (at one block a CU, tiles of
     // two heads from 2049 positions on); where they do not a null workspace is taken for an oversight.

@@ -285,7 +285,8 @@ def routed_qmv_reduce(h, n_h_rows, Wd, n_experts, row_idx, expert_idx, route_wei
 
 def routed_qmv_swiglu_ordered(x, n_x_rows, Wg, Wu, n_experts, row_idx, expert_idx, route_weight, n_routes, order, out0,
                               stream=None) -> None:
-    """fk_routed_qmv_swiglu with the routes served in `order` (fk_route_order): same results, shared slices read once."""
+    """fk_routed_qmv_swiglu with the routes served one by one in `order` (fk_route_order): the same products, a dot product added up
+    as the listed launch of few routes does it (a call whose routes are served together may differ in the last bit)."""
     check(lib.fk_routed_qmv_swiglu_ordered(_addr(x), n_x_rows, _w(Wg), _w(Wu), n_experts, _addr(row_idx), _addr(expert_idx),
                                            _addr(route_weight), n_routes, _addr(order), _addr(out0), _addr(stream)))
 

@@ -326,7 +326,7 @@ def test_routes_served_together_are_as_exact_as_one_by_one(fk, bits, mean):
 def test_routes_served_in_expert_order_give_the_same_bits(fk):
     """Several tokens whose routes share experts (config-5 widths, 8 tokens x top-6 over 16 experts): fk_route_order
     is numpy's stable sort by (clamped) expert, and the routed launches served in that order -- an expert's slice
-    then comes from HBM once -- give the listed order's results (to rounding-edge flips: the tiles differ) and the
+    then comes from HBM once -- give the listed call's results (to rounding-edge flips: it serves them together) and the
     oracle's, for M1 and for M2 with a shared expert and a residual.  The launches that rank the routes themselves
     (no order array) give the bits of the launches that read the array."""
     E, O, K, tokens, top_k = 16, 1408, 2048, 8, 6
@@ -350,8 +350,8 @@ def test_routes_served_in_expert_order_give_the_same_bits(fk):
     fk.routed_qmv_swiglu_ordered(dx, tokens, dWg, dWu, E, dr, d_e, None, routes, order, h1)
     fk.sync()
     a, b = h0.to_numpy(np.uint16, (routes, O)), h1.to_numpy(np.uint16, (routes, O))
-    # same chunks, same products; the tile geometry follows the blocks a route gets (a multiple of eight when
-    # served in order), and with it the order in which a row's partial sums are added: rounding-edge flips only
+    # the listed call serves an expert's routes together on the matrix cores, the ordered one route by route: the same products
+    # added up in another order, so rounding-edge flips only
     frac, ulps = bf16_mismatch(b, a)
     print("ordered against listed: %.4f of the outputs differ, by at most %.1f ulp" % (frac, ulps))
     assert frac <= FLIP_FRACTION_BAR, (frac, ulps)
