@@ -315,3 +315,61 @@ def test_rope_store_sdpa_rejects_bad_arguments(fk):
         fk.rope_store_sdpa_decode(b, b, b, None, None, b, b, b, None, 17, 16, 8, 2, 64, 64, 1e4, 1e-6, 16, 0.1, None, b, b)
     with pytest.raises(fk.FusekitError):      # table requested with rope_dims 0
         fk.step_init_rope(b, b, b, b, 0, 1e4)
+
+
+@pytest.mark.parametrize("n_heads,n_kv,qk,vd,rows,kv_len", [
+    (8, 8, 64, 64, 1, 193), (6, 2, 64, 64, 1, 256), (10, 2, 64, 64, 1, 257), (24, 2, 64, 64, 1, 769),       # groups of 1, 3, 5 and 12; round edges
+    (32, 8, 128, 128, 1, 255), (3, 1, 128, 128, 1, 512), (7, 1, 128, 128, 1, 513), (16, 1, 128, 128, 1, 4097),
+    (2, 1, 64, 64, 1, 9000), (5, 1, 128, 128, 1, 33000),                                                      # merges of up to 64 partials
+    (14, 2, 64, 64, 3, 200), (32, 8, 128, 128, 2, 223), (64, 2, 64, 64, 13, 500), (128, 8, 128, 128, 17, 300),  # tiles of 8 and of 16, last ones not full
+    (16, 16, 192, 128, 2, 30), (16, 16, 192, 128, 8, 225), (4, 2, 192, 128, 9, 700), (64, 64, 192, 128, 33, 128),
+])
+def test_sdpa_on_the_matrix_cores_at_the_edges_of_its_tiles(fk, n_heads, n_kv, qk, vd, rows, kv_len):
+    """Rows of a group against the oracle, element by element: products and probabilities are exact, sums fp32, so an output is within one
+    rounding of the float64 one, or where the value sums cancel within an fp32 sum's error of the typical output.  The cache ends with the
+    context, and what lies behind every row's own context never reaches it: infinities and NaN there."""
+    cap, scale = kv_len + rows - 1, qk ** -0.5
+    q = normal_bf16(21, (rows, n_heads * qk))
+    ck, cv = normal_bf16(22, n_kv * cap * qk).reshape(n_kv, cap, qk), normal_bf16(23, n_kv * cap * vd).reshape(n_kv, cap, vd)
+    pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, qk, vd, cap)
+    part, cnt = fk.DeviceBuffer(max(pb, 16) * rows), fk.zeros(max(cb, 16) * rows)
+    dq, dk, dv, out = (fk.DeviceBuffer.from_numpy(a) for a in (q, ck, cv, np.zeros(rows * n_heads * vd, np.uint16)))
+    run = lambda: fk.sdpa_decode_rows(dq, dk, dv, out, rows, kv_len, n_heads, n_kv, qk, vd, cap, scale, part, cnt)
+    run()
+    got = out.to_numpy(np.uint16, (rows, n_heads * vd))
+    for r in sorted({0, rows // 2, rows - 1}):
+        ref = oracle.bf16_to_f32(oracle.sdpa_decode(q[r], ck.ravel(), cv.ravel(), n_heads, n_kv, qk, vd, kv_len + r, cap, scale)).astype(np.float64)
+        g = oracle.bf16_to_f32(got[r]).astype(np.float64)
+        assert np.all(np.abs(g - ref) <= 2.0 ** -7 * np.abs(ref) + 1e-4 * np.sqrt(np.mean(ref * ref))), r
+    assert not cnt.to_numpy(np.uint32).any()
+    run()
+    assert np.array_equal(out.to_numpy(np.uint16, (rows, n_heads * vd)), got)     # (merged in range order)
+    if rows > 1:
+        ck2, cv2 = ck.copy(), cv.copy()
+        ck2[:, kv_len:], cv2[:, kv_len:, ::2], cv2[:, kv_len:, 1::2] = 0x7F80, 0x7FC0, 0xFF80
+        dk, dv = fk.DeviceBuffer.from_numpy(ck2), fk.DeviceBuffer.from_numpy(cv2)
+        run()
+        first = out.to_numpy(np.uint16, (rows, n_heads * vd))
+        assert np.array_equal(first[0], got[0])
+        assert np.isnan(oracle.bf16_to_f32(first[-1])).all()
+
+
+@pytest.mark.parametrize("n_heads,n_kv,dim", [(14, 2, 64), (32, 8, 128), (4, 4, 64)])
+@pytest.mark.parametrize("length,given", [(1, 1), (33, 33), (700, 700), (2000, 2000), (0, 1), (5000, 2000)])
+def test_sdpa_length_on_the_device_of_a_longer_plan(fk, n_heads, n_kv, dim, length, given):
+    """A launch planned for 2000 positions: any shorter context, and lengths outside the plan taken as its ends; the rows behind the context
+    hold NaN, an infinite value of a row inside it gives an infinity."""
+    cap, scale = 2000, dim ** -0.5
+    q = normal_bf16(31, n_heads * dim)
+    ck, cv = normal_bf16(32, n_kv * cap * dim).reshape(n_kv, cap, dim), normal_bf16(33, n_kv * cap * dim).reshape(n_kv, cap, dim)
+    ck[:, given:], cv[:, given:] = 0x7FC0, 0x7FC0
+    ref = oracle.sdpa_decode(q, ck.ravel(), cv.ravel(), n_heads, n_kv, dim, dim, given, cap, scale)
+    cv[:, given // 2, 5] = 0x7F80
+    pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, dim, dim, cap)
+    out = fk.DeviceBuffer(2 * n_heads * dim)
+    fk.sdpa_decode(*(fk.DeviceBuffer.from_numpy(a) for a in (q, ck, cv)), out, _u32(fk, length), 0, cap, n_heads, n_kv, dim, dim, cap, scale,
+                   fk.DeviceBuffer(pb), fk.zeros(cb))
+    got = out.to_numpy(np.uint16).reshape(n_heads, dim)
+    assert (got[:, 5] == 0x7F80).all()
+    keep = np.arange(dim) != 5
+    assert rel_l2(got[:, keep].ravel(), oracle.bf16_to_f32(ref.reshape(n_heads, dim)[:, keep].ravel())) <= 3e-3
