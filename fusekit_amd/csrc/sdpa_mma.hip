@@ -9,16 +9,17 @@
 // query and four keys of each 16; its softmax reference moves only when a step's maximum outgrows it by 2^8.
 //
 // A wave owns its steps of 32 keys: K and V rows go from memory into its own part of LDS (global_load_lds, 16-byte pieces XOR-swizzled by
-// the row, so that the fragment reads meet all banks), 128 KB of them on their way per CU, so that no barrier and no wait for another wave
-// stands in its loop; V^T is read with ds_read_b64_tr_b16.  The waves meet once, after their last step; blocks that share a context leave
-// (m, l, o) partials in 16-byte pieces, and the one that arrives last merges them in range order, all of a head requested together.
+// the row, so that the fragment reads meet all banks); the next step's keys are requested as soon as this one's are in registers, its
+// values behind the second product.  No barrier and no wait for another wave stands in a wave's loop; V^T is read with ds_read_b64_tr_b16.
+// The waves meet once, after their last step; blocks that share a context leave (m, l, o) partials in 16-byte pieces, and the one that
+// arrives last merges them in range order, all of a head requested together.
 //
 // The form on vector instructions (sdpa_kernel.hpp: quantised caches, other widths, short contexts) spends about 110 of them on a lane's 8
 // dims of a key for 4 heads; here the products cost none and a step's softmax about 100 for 32 keys of a whole tile, so that what remains is
-// the bytes (one block alone draws 90 bytes a ns), the start and, where blocks share a context, 2.2 us for partials, count and merge.
-// That form -> this, us, launch to launch in a graph, cold caches: 32 / 8 heads x 128 at 512 positions 7.4 -> 6.6, 4096 12.2 -> 9.2, 12000
-// 21.1 -> 14.5, 32768 37 -> 28.3 (134 MB: 4.7 TB/s of the 5.8 that a plain read reaches); 14 / 2 x 64 at 544 6.9 -> 5.7, 12000 12.4 -> 8.2;
-// 64 rows of 32 / 8 x 128 at 500 31 -> 8.4; 16 heads of 192 / 128, 8 rows at 480 12.0 -> 8.8, 96 rows at 1500 137 -> 15.4.
+// the bytes, the start and, where blocks share a context, the 2.2 us of partials, count and merge.  That form -> this, us, launch to launch
+// in a graph, caches from memory: 32 / 8 heads x 128 at 512 positions 7.6 -> 7.4, 1024 8.9 -> 7.8, 4096 13.3 -> 9.9, 12000 21.3 -> 14.6, 32768 37 ->
+// 28.1 (134 MB: 4.8 TB/s of the 5.8 that a plain read reaches); 14 / 2 x 64 at 544 6.9 -> 5.5, 4096 10.0 -> 6.9, 12000 13.0 -> 8.4; 64 rows of
+// 32 / 8 x 128 at 500 33 -> 9.6; 16 heads of 192 / 128, 8 rows at 480 12.6 -> 10.8, 96 rows at 1500 141 -> 19.4.
 #include "dma_device.hpp"
 #include "fk_host.hpp"
 #include "rope_device.hpp"
@@ -65,8 +66,8 @@ constexpr uint32_t mma_input_bytes(uint32_t qk, uint32_t qt, bool fused) {
     return raw + (fused ? ((qt + 1u) * (qk * 2u + 16u) + 1023u) / 1024u * 1024u : 0u);
 }
 constexpr uint32_t mma_stage_bytes(uint32_t qk, uint32_t vd) { return kMmaStep * (qk + vd) * 2u; }
-constexpr uint32_t mma_lds_bytes(uint32_t qk, uint32_t vd, uint32_t qt, uint32_t nw, uint32_t nbuf, bool fused) {
-    const uint32_t stages = nw * nbuf * mma_stage_bytes(qk, vd), meet = nw * qt * (vd + 4u) * 4u + 2u * nw * qt * 4u + 64u;
+constexpr uint32_t mma_lds_bytes(uint32_t qk, uint32_t vd, uint32_t qt, uint32_t nw, bool fused) {
+    const uint32_t stages = nw * mma_stage_bytes(qk, vd), meet = nw * qt * (vd + 4u) * 4u + 2u * nw * qt * 4u + 64u;
     return mma_input_bytes(qk, qt, fused) + (stages > meet ? stages : meet);
 }
 
@@ -87,8 +88,8 @@ __device__ __forceinline__ float mma_dpp(float v) { return __int_as_float(__buil
 // what another block of this launch wrote, or is to read, moves past every cache that the two do not share (sc1)
 constexpr int kShared = 16;
 
-// QT queries of a KV head a block, NW waves, NBUF steps of a wave in flight.
-template <int QK, int VD, int QT, int NW, int NBUF, bool FUSED>
+// QT queries of a KV head a block, NW waves.
+template <int QK, int VD, int QT, int NW, bool FUSED>
 __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs a) {
     constexpr uint32_t KROW = QK * 2u, VROW = VD * 2u, KP = QK / 8u, VP = VD / 8u;      // bytes and 16-byte pieces of a row
     constexpr uint32_t KT = kMmaStep * KROW, STAGE = mma_stage_bytes(QK, VD);
@@ -97,7 +98,6 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
     constexpr int PARTS = QT == 4 ? 1 : (QT == 8 ? 2 : 3);                              // matrix instructions for the probabilities' parts
     constexpr uint32_t IN = mma_input_bytes(QK, QT, FUSED), ROUND = NW * kMmaStep;
     static_assert(!FUSED || QK == VD, "");
-    static_assert(NBUF == 1 || NBUF == 2, "");
     extern __shared__ uint4 mma_lds[];
     unsigned char* const lds = reinterpret_cast<unsigned char*>(mma_lds);
     kernarg_warm<(int)sizeof(SdpaMmaArgs)>();
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
     // ---- K and V of a step into this wave's stage ----
     const unsigned char* kbase = reinterpret_cast<const unsigned char*>(a.k + (size_t)kvh * a.capacity * QK);
     const unsigned char* vbase = reinterpret_cast<const unsigned char*>(a.v + (size_t)kvh * a.capacity * VD);
-    const uint32_t my_stages = IN + wave * (NBUF * STAGE);
+    const uint32_t my_stage = IN + wave * STAGE;
     uint32_t koff[KREQ], voff[VREQ];
 #pragma unroll
     for (int i = 0; i < KREQ; ++i) {
@@ -150,33 +150,31 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
         voff[i] = row * VROW + ((flat % VP) ^ v_swizzle(row)) * 16u;
     }
     // (rows past the allocation repeat its last row: they are masked)
-    auto issue_k = [&](uint32_t kv0, uint32_t buf) {
+    auto issue_k = [&](uint32_t kv0) {
         const uint32_t at = kv0 < a.capacity ? kv0 : a.capacity - 1u, more = a.capacity - 1u - at;
         const unsigned char* base = kbase + (size_t)at * KROW;
-        const uint32_t to = my_stages + buf * STAGE;
         if (__builtin_expect(more >= kMmaStep - 1u, 1)) {
 #pragma unroll
-            for (int i = 0; i < KREQ; ++i) dma16(to + (uint32_t)i * 1024u, koff[i], base);
+            for (int i = 0; i < KREQ; ++i) dma16(my_stage + (uint32_t)i * 1024u, koff[i], base);
         } else {
 #pragma unroll
             for (int i = 0; i < KREQ; ++i) {
                 const uint32_t row = ((uint32_t)i * 64u + lane) / KP, over = row > more ? row - more : 0u;
-                dma16(to + (uint32_t)i * 1024u, koff[i] - over * KROW, base);
+                dma16(my_stage + (uint32_t)i * 1024u, koff[i] - over * KROW, base);
             }
         }
     };
-    auto issue_v = [&](uint32_t kv0, uint32_t buf) {
+    auto issue_v = [&](uint32_t kv0) {
         const uint32_t at = kv0 < a.capacity ? kv0 : a.capacity - 1u, more = a.capacity - 1u - at;
         const unsigned char* base = vbase + (size_t)at * VROW;
-        const uint32_t to = my_stages + buf * STAGE + KT;
         if (__builtin_expect(more >= kMmaStep - 1u, 1)) {
 #pragma unroll
-            for (int i = 0; i < VREQ; ++i) dma16(to + (uint32_t)i * 1024u, voff[i], base);
+            for (int i = 0; i < VREQ; ++i) dma16(my_stage + KT + (uint32_t)i * 1024u, voff[i], base);
         } else {
 #pragma unroll
             for (int i = 0; i < VREQ; ++i) {
                 const uint32_t row = ((uint32_t)i * 64u + lane) / VP, over = row > more ? row - more : 0u;
-                dma16(to + (uint32_t)i * 1024u, voff[i] - over * VROW, base);
+                dma16(my_stage + KT + (uint32_t)i * 1024u, voff[i] - over * VROW, base);
             }
         }
     };
@@ -185,7 +183,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
     const uint32_t covered = a.n_splits * a.span < a.capacity ? a.n_splits * a.span : a.capacity;
     // the first range's keys are requested ahead of the length (its values are not: a short context would wait for what it does not need)
     const bool ahead = split == 0 && first < covered;
-    if (ahead) issue_k(first, 0);
+    if (ahead) issue_k(first);
     uint32_t kv_raw = a.kv_len_imm;
     if (a.kv_len_ptr) kv_raw = *(const __attribute__((address_space(4))) uint32_t*)(uintptr_t)a.kv_len_ptr;
     auto limit_of = [&](uint32_t row) {
@@ -201,14 +199,10 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
     const uint32_t end = lim_hi - blk0 < a.span ? lim_hi : blk0 + a.span;
     const uint32_t n_steps = end > first ? (end - first + ROUND - 1u) / ROUND : 0u;
     if (n_steps != 0) {
-        if (!ahead) issue_k(first, 0);
-        issue_v(first, 0);
+        if (!ahead) issue_k(first);
+        issue_v(first);
     }
-    if (NBUF == 2 && n_steps > 1u) {
-        issue_k(first + ROUND, 1);
-        issue_v(first + ROUND, 1);
-        wait_loads<NBUF == 2 ? 2 * REQ : 0>();
-    } else if (n_steps != 0) {
+    if (n_steps != 0) {
         wait_loads<REQ>();
     } else if (ahead) {
         wait_loads<KREQ>();
@@ -258,12 +252,11 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
     const uint32_t part = n / QT;   // QT 4, 8: which part of the probabilities this column multiplies
 
     for (uint32_t j = 0; j < n_steps; ++j) {
-        const uint32_t kv0 = first + j * ROUND, buf = NBUF == 2 ? j & 1u : 0u;
-        unsigned char* const ks = lds + my_stages + buf * STAGE;
+        const uint32_t kv0 = first + j * ROUND;
+        unsigned char* const ks = lds + my_stage;
         unsigned char* const vs = ks + KT;
         const bool more = j + 1u < n_steps;
-        if (NBUF == 2 && more) wait_loads<NBUF == 2 ? REQ + VREQ : 0>();
-        else wait_loads<VREQ>();
+        wait_loads<VREQ>();
         const bool has_new = FUSED && pos >= kv0 && pos < kv0 + kMmaStep;
         if constexpr (FUSED) {
             if (has_new) {   // the new key, not yet cached
@@ -286,10 +279,8 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[t * 4 + i] = s4[i] * scale2;
         }
-        if constexpr (NBUF == 1) {   // the keys are in registers: their place takes the next step's
-            __builtin_amdgcn_sched_barrier(0);
-            if (more) issue_k(kv0 + ROUND, 0);
-        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) issue_k(kv0 + ROUND);   // the keys are in registers: their place takes the next step's
         if (kv0 + kMmaStep > lim_lo) {
 #pragma unroll
             for (int i = 0; i < 8; ++i)
@@ -341,7 +332,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
                 }
             }
         }
-        if (more) wait_loads<NBUF == 2 ? REQ : KREQ>();
+        if (more) wait_loads<KREQ>();
         else wait_loads<0>();
         bool repeat = false;
         if (kv0 + kMmaStep > lim_lo || has_new) {
@@ -407,14 +398,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (NBUF == 2) {
-            if (j + 2u < n_steps) {
-                issue_k(kv0 + 2u * ROUND, buf);
-                issue_v(kv0 + 2u * ROUND, buf);
-            }
-        } else {
-            if (more) issue_v(kv0 + ROUND, 0);
-        }
+        if (more) issue_v(kv0 + ROUND);
     }
     wait_loads<0>();   // (a first step that no key of the context lies in)
 
@@ -535,11 +519,11 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
 
 namespace {
 
-template <int QK, int VD, int QT, int NW, int NBUF, bool FUSED>
+template <int QK, int VD, int QT, int NW, bool FUSED>
 fk_status fill(Launch* l) {
-    l->func = reinterpret_cast<const void*>(&sdpa_mma_kernel<QK, VD, QT, NW, NBUF, FUSED>);
+    l->func = reinterpret_cast<const void*>(&sdpa_mma_kernel<QK, VD, QT, NW, FUSED>);
     l->block = dim3(NW * 64, 1, 1);
-    l->shmem = mma_lds_bytes(QK, VD, QT, NW, NBUF, FUSED);
+    l->shmem = mma_lds_bytes(QK, VD, QT, NW, FUSED);
     return raise_dynamic_lds(l->func, l->shmem);
 }
 
@@ -557,8 +541,9 @@ bool sdpa_takes_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v, con
     }
     if (a & 15u) return false;
     // Short contexts of few rows: the form on vector instructions has less to set up (us, that / this: 32 / 8 heads x 128, 64 positions 4.0 / 4.7, 128
-    // 4.7 / 4.8, 256 6.6 / 5.4, 8 rows at 100 4.3 / 6.6, 64 rows at 100 14.7 / 8.1; 14 / 2 x 64, 128 positions 4.1 / 4.1, 256 4.9 / 4.5).
-    if (qk_dim <= 128 && max_len <= 192 && (uint64_t)n_heads * rows <= 512u) return false;
+    // 4.9 / 4.9, 256 6.8 / 6.6, 8 rows at 100 4.3 / 6.6, 64 rows at 100 14.7 / 8.1; 14 / 2 x 64, 128 positions 4.1 / 4.1, 256 5.1 / 4.5; 16 heads of
+    // 192 / 128, 8 rows at 30 5.4 / 6.1, 2 rows at 100 7.6 / 6.2).
+    if (max_len <= (qk_dim == 192 ? 64u : 192u) && (uint64_t)n_heads * rows <= 512u) return false;
     // (partials are addressed with 32 bits)
     return (uint64_t)rows * n_heads * kMmaMaxSplits * (v_dim + 2u) * 4u < 0x7fffffffull;
 }
@@ -584,36 +569,40 @@ fk_status plan_sdpa_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v,
     // 7.0, 64 rows 13.7 / 8.4, 128 rows -- 512 tiles -- 12.4 / 15.1; 16 heads of 192 / 128, 32 rows at 480 positions 10.9 / 8.8).
     const uint32_t queries = rows * a.group;
     const uint32_t qt = queries <= 4u ? 4u : (queries <= 8u || fusion || (uint64_t)n_kv * ((queries + 7u) / 8u) <= (uint64_t)dev->cus ? 8u : 16u);
-    // Waves, and the rounds of theirs that one block walks rather than leave partials: a round more takes 0.5 .. 1.3 us, the partials, their count
-    // and their merge 2.2 (one block / several, us: 64 dims, 256 positions a round, 768 6.2 / 6.4, 1024 6.8 / 6.4; 128 dims, 512 6.7 / 7.6, 768 7.7 /
-    // 7.4; 192 / 128, 224 a round, 8 rows at 480 8.8 / 9.6).  128 dims, 4 waves of two steps in flight instead of 8 of one: 256 positions 6.1 for
-    // 5.4, 4096 9.9 for 9.2; 64 dims, 16 of one instead of 8 of two: 544 5.9 for 5.7, 4096 7.7 for 6.5.
-    uint32_t nw = 8, alone = 2;
+    // Waves, and the rounds of theirs that one block walks rather than leave partials.  A block draws 90 bytes a ns where its rows lie in the
+    // L2, half of that where they come from memory; partials, their count and their merge take 2.2 us.  Cold caches, us: 64 dims (256
+    // positions a round), one block / several, 544 positions 5.5 / 6.2, 1024 6.5 / 6.5 (16 / 8 heads 6.4 / 6.4, 8.1 / 6.5).  One row of 128 dims: at
+    // 256 positions one round of 8 waves 6.6, two of 4 7.4; beyond, 32 KB a wave in fewer CUs is the slower, until the rounds are many:
+    // 8 / 4 waves, 512 8.5 / 7.4, 1024 8.6 / 7.8, 2048 8.9 / 8.5, 4096 9.9 / 10.1, 12000 14.6 / 14.9.  Several rows share what is drawn: 8 of them
+    // at 500 positions, 8 waves in one block 8.6, 4 in four 9.2.  (Two steps of a wave in flight at half the waves: 64 dims 544 5.8, 12000 8.5.)
+    uint32_t nw = 8, alone = rows > 1 ? 2u : 1u;
     if (qk_dim == 64) {
         alone = 3;
-        if (fusion) FK_TRY(qt == 4 ? (fill<64, 64, 4, 8, 2, true>(l)) : (fill<64, 64, 8, 8, 2, true>(l)));
-        else FK_TRY(qt == 4 ? (fill<64, 64, 4, 8, 2, false>(l)) : (qt == 8 ? fill<64, 64, 8, 8, 2, false>(l) : fill<64, 64, 16, 8, 2, false>(l)));
+        if (fusion) FK_TRY(qt == 4 ? (fill<64, 64, 4, 8, true>(l)) : (fill<64, 64, 8, 8, true>(l)));
+        else FK_TRY(qt == 4 ? (fill<64, 64, 4, 8, false>(l)) : (qt == 8 ? fill<64, 64, 8, 8, false>(l) : fill<64, 64, 16, 8, false>(l)));
     } else if (qk_dim == 128) {
-        if (fusion) {
-            FK_TRY(qt == 4 ? (fill<128, 128, 4, 8, 1, true>(l)) : (fill<128, 128, 8, 8, 1, true>(l)));
-        } else if (qt <= 8) {
-            FK_TRY(qt == 4 ? (fill<128, 128, 4, 8, 1, false>(l)) : (fill<128, 128, 8, 8, 1, false>(l)));
-        } else {
+        if (qt == 16) {
             nw = 4;
             alone = 4;
-            FK_TRY((fill<128, 128, 16, 4, 2, false>(l)));
+            FK_TRY((fill<128, 128, 16, 4, false>(l)));
+        } else if (rows == 1 && max_len > 256u && max_len <= 3072u) {
+            nw = 4;
+            if (fusion) FK_TRY(qt == 4 ? (fill<128, 128, 4, 4, true>(l)) : (fill<128, 128, 8, 4, true>(l)));
+            else FK_TRY(qt == 4 ? (fill<128, 128, 4, 4, false>(l)) : (fill<128, 128, 8, 4, false>(l)));
+        } else {
+            if (fusion) FK_TRY(qt == 4 ? (fill<128, 128, 4, 8, true>(l)) : (fill<128, 128, 8, 8, true>(l)));
+            else FK_TRY(qt == 4 ? (fill<128, 128, 4, 8, false>(l)) : (fill<128, 128, 8, 8, false>(l)));
         }
     } else if (qt <= 8) {
-        nw = 7;
+        nw = 7;   // (160 KB)
         alone = 3;
-        FK_TRY(qt == 4 ? (fill<192, 128, 4, 7, 1, false>(l)) : (fill<192, 128, 8, 7, 1, false>(l)));
+        FK_TRY(qt == 4 ? (fill<192, 128, 4, 7, false>(l)) : (fill<192, 128, 8, 7, false>(l)));
     } else {
         nw = 4;
         alone = 4;
-        FK_TRY((fill<192, 128, 16, 4, 1, false>(l)));
+        FK_TRY((fill<192, 128, 16, 4, false>(l)));
     }
-    // Beyond that a block a CU, but no shorter than two rounds where there would be more than the 16 partials that a merge has soonest
-    // (32 / 8 heads x 128, 4096 positions: 8 blocks a KV head 9.2, 16 9.3).
+    // Beyond that a block a CU, but no shorter than two rounds where there would be more than the 16 partials that a merge has soonest.
     const uint32_t tiles = (queries + qt - 1u) / qt, round = nw * kMmaStep, rounds = (max_len + round - 1u) / round;
     uint32_t want = (uint32_t)dev->cus / (n_kv * tiles), many = (rounds + 1u) / 2u;
     many = many < 16u ? 16u : (many > kMmaMaxSplits ? kMmaMaxSplits : many);
