@@ -457,12 +457,23 @@ __device__ __forceinline__ void meta_store(const MetaRegs& r, uint32_t ti, uint3
     }
 }
 
-// One fp32 partial per chunk into part[pos]; positions past the tile land in the padding of `part` (it holds whole
-// passes) and read group 0's scale and bias.
+// A wave's lanes hold consecutive chunks of a row, so the partials of 2^part_shift adjacent lanes (as many as divide the row, at most
+// 8, of 4-bit weights 4) are added where they are, in registers, and the row sums read one word for them.  The row sums are a phase in
+// which no memory request of the block's can be used: 4B-class layers, us a token, every partial through LDS / this: bf16 (12160 partials a
+// gate / up tile, 1.5 .. 3.3 us of row sums at each of the four projections) 2053 / 1897, 8 bits 1580 / 1506, 4 bits 1107 / 1095, the
+// mixture of experts 1100 / 1060.  (4 bits: by pairs 1104, by eights 1098, by sixteens 1094; mixture of experts 1061 / 1073 / 1083.  bf16: by
+// fours 1909, by sixteens 1902.)
+template <WKind KIND>
+__device__ __forceinline__ uint32_t part_shift(uint32_t cs) {
+    return (uint32_t)__builtin_ctz(cs | (KIND == W_Q4 ? 4u : 8u));
+}
+// One fp32 partial per 2^part_shift chunks into part[pos >> shift]; positions past the tile land in the padding of `part` (it holds
+// whole passes) and read group 0's scale and bias.
 template <WKind KIND, int NL, int SN, typename MAT>
 __device__ __forceinline__ void tile_partials(const MAT& m, const Tile& t, const TilePos<NL>& p, const TileRegs<NL>& r,
                                               const uint4* xs, const float* sx, const uint32_t* meta, float* part) {
-    const uint32_t total = t.rows * t.cs;
+    const uint32_t total = t.rows * t.cs, shift = part_shift<KIND>(t.cs);
+    float v[NL];
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
         const uint32_t pos = p.p0 + j * SN;
@@ -472,8 +483,27 @@ __device__ __forceinline__ void tile_partials(const MAT& m, const Tile& t, const
             sb = mw & 0xffffu;
             bb = mw >> 16;
         }
-        part[pos] = chunk_partial<KIND>(r.w[j], sb, bb, xs, sx, p.col[j], t.cs);
+        v[j] = chunk_partial<KIND>(r.w[j], sb, bb, xs, sx, p.col[j], t.cs);
         __builtin_amdgcn_sched_barrier(0);
+    }
+    // (a wave-uniform test for all of the pass's partials, not one for each)
+    if (shift >= 1u) {
+#pragma unroll
+        for (int j = 0; j < NL; ++j) v[j] = dpp_add<0xB1>(v[j]);
+    }
+    if (shift >= 2u) {
+#pragma unroll
+        for (int j = 0; j < NL; ++j) v[j] = dpp_add<0x4E>(v[j]);
+    }
+    if constexpr (KIND != W_Q4) {
+        if (shift >= 3u) {
+#pragma unroll
+            for (int j = 0; j < NL; ++j) v[j] = dpp_add<0x141>(v[j]);
+        }
+    }
+    if ((p.p0 & ((1u << shift) - 1u)) == 0u) {
+#pragma unroll
+        for (int j = 0; j < NL; ++j) part[(p.p0 + j * SN) >> shift] = v[j];
     }
 }
 
@@ -563,73 +593,59 @@ __device__ __forceinline__ void tile_run_pair(const MAT& ma, const MAT& mb, cons
     }
 }
 
-// Lanes that share a row in the row-sum phase: about four to eight partials per lane, at most 16 lanes (so that
-// the cross-lane sum stays inside a 16-lane row of the wave).
-__device__ __forceinline__ uint32_t lanes_per_row(uint32_t cs) {
-    uint32_t lr = 1;
-    while (lr < 16 && lr * 8 <= cs) lr <<= 1;
-    return lr;
-}
-
-// Adds each row's partials in a fixed order; f(row, sum0, sum1) runs in one lane per row.
-// ONCE (the one-pass flavour): when a row group of 16, 8, ... lanes covers every row of the tile in ONE round and a lane
-// then holds at most ten partials per matrix, all its LDS reads go out first (clamped positions) and a row's epilogue
-// runs once -- instead of rounds of a read-wait-add loop (gate / up rows of the 4B-class MLP launch: two rounds of
-// sixteen lanes and five dependent LDS trips each took 1.65 us; one round of eight lanes 1.1).
-template <bool TWO, bool ONCE = false, typename F>
+// Adds each row's partials (what tile_partials left of them) in a fixed order; f(row, sum0, sum1) runs in one lane per row.  The widest
+// group of lanes a row (at most 16, no more than it has partials) with which all rows fit one round; a lane's one to ten LDS
+// reads go out together (clamped positions, masked additions).  Tiles of other shapes take rounds of a read-wait-add loop.
+template <WKind KIND, bool TWO, typename F>
 __device__ __forceinline__ void tile_rows(const Tile& t, const float* part, const float* part1, F f) {
-    if constexpr (ONCE) {
-        // the widest row group (at most 16 lanes) with which every row of the tile fits one round
-        uint32_t lr1 = 16;
-        while (lr1 > 1 && t.rows * lr1 > (uint32_t)kBlock) lr1 >>= 1;
-        if (t.rows * lr1 <= (uint32_t)kBlock && t.cs <= 10u * lr1) {
-            const uint32_t lane1 = threadIdx.x & (lr1 - 1), rr = threadIdx.x / lr1;
-            const bool ok = rr < t.rows;
-            const uint32_t base = (ok ? rr : 0u) * t.cs;
-            float v0[10], v1[10];
+    const uint32_t cs = t.cs >> part_shift<KIND>(t.cs);
+    uint32_t lr = 16;
+    while (lr > 1 && (t.rows * lr > (uint32_t)kBlock || lr >= 2u * cs)) lr >>= 1;
+    const uint32_t lane = threadIdx.x & (lr - 1);
+    if (t.rows * lr <= (uint32_t)kBlock && cs <= 10u * lr) {
+        const uint32_t rr = threadIdx.x / lr;
+        const bool ok = rr < t.rows;
+        const uint32_t base = (ok ? rr : 0u) * cs;
+        float s0 = 0.f, s1 = 0.f;
+        auto read = [&](auto count) {
+            constexpr int N = decltype(count)::value;
+            float v0[N], v1[N];
 #pragma unroll
-            for (int k = 0; k < 10; ++k) {
-                const uint32_t i = lane1 + lr1 * k;
-                const uint32_t at = base + (i < t.cs ? i : 0u);
+            for (int k = 0; k < N; ++k) {
+                const uint32_t i = lane + lr * k;
+                const uint32_t at = base + (i < cs ? i : 0u);
                 v0[k] = part[at];
                 if constexpr (TWO) v1[k] = part1[at];
             }
-            float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-            for (int k = 0; k < 10; ++k) {
-                const bool in = lane1 + lr1 * k < t.cs;
+            for (int k = 0; k < N; ++k) {
+                const bool in = lane + lr * k < cs;
                 s0 += in ? v0[k] : 0.f;
                 if constexpr (TWO) s1 += in ? v1[k] : 0.f;
             }
-            s0 = group_sum(s0, lr1);
-            if constexpr (TWO) s1 = group_sum(s1, lr1);
-            if (ok && lane1 == 0) f(rr, s0, s1);
-            return;
-        }
+        };
+        if (cs <= lr) read(std::integral_constant<int, 1>{});
+        else if (cs <= 3u * lr) read(std::integral_constant<int, 3>{});
+        else if (cs <= 5u * lr) read(std::integral_constant<int, 5>{});
+        else read(std::integral_constant<int, 10>{});
+        s0 = group_sum(s0, lr);
+        if constexpr (TWO) s1 = group_sum(s1, lr);
+        if (ok && lane == 0) f(rr, s0, s1);
+        return;
     }
-    const uint32_t lr = lanes_per_row(t.cs), lane = threadIdx.x & (lr - 1);
     const uint32_t step = kBlock / lr, rows_up = (t.rows + step - 1) / step * step;
-    auto one = [&](uint32_t rr) {
+    for (uint32_t rr = threadIdx.x / lr; rr < rows_up; rr += step) {
         const bool ok = rr < t.rows;
         float s0 = 0.f, s1 = 0.f;
         if (ok)
-            for (uint32_t i = lane; i < t.cs; i += lr) {
-                s0 += part[rr * t.cs + i];
-                if constexpr (TWO) s1 += part1[rr * t.cs + i];
+            for (uint32_t i = lane; i < cs; i += lr) {
+                s0 += part[rr * cs + i];
+                if constexpr (TWO) s1 += part1[rr * cs + i];
             }
         s0 = group_sum(s0, lr);
         if constexpr (TWO) s1 = group_sum(s1, lr);
         if (ok && lane == 0) f(rr, s0, s1);
-    };
-    // Up to two rounds (the 4B-class tiles) run straight-line: f stores to memory, and in front of a LOOP with
-    // stores in it the compiler waits for every request still in flight -- here the next projection's weights,
-    // requested just before, whose trip to memory the row sums and the hand-over are meant to cover.
-    if (rows_up <= 2 * step) {
-        one(threadIdx.x / lr);
-        if (rows_up > step) one(threadIdx.x / lr + step);
-        return;
     }
-    for (uint32_t rr = threadIdx.x / lr; rr < rows_up; rr += step) one(rr);
 }
 
 // An empty tile (a block without work in this projection) still issues its loads, clamped to the tile's

@@ -91,7 +91,7 @@ __device__ __forceinline__ void xcd_mlp_phase(const ARGS& a, const LEAD& lead, I
     if (streams && gu_n) {
         uint16_t* mid = a.mid + (size_t)sync.xcd * per_xcd + gu0;
         const int variant = a.swiglu_variant;
-        tile_rows<true, ONE>(tg, work, work + seg,
+        tile_rows<KIND, true>(tg, work, work + seg,
                         [&](uint32_t r, float s0, float s1) { mid[r] = (uint16_t)swiglu_bits(s0, s1, variant, 1.0f); });
 
     }
@@ -111,7 +111,7 @@ __device__ __forceinline__ void xcd_mlp_phase(const ARGS& a, const LEAD& lead, I
     if (streams && d_n && ok) {
         long long* out = a.out_sums;
         XcdControl* ctl = sync.ctl;
-        tile_rows<false, ONE>(td, work, work, [&](uint32_t r, float s0, float) { xcd_sum_add(out, d0 + r, s0, ctl); });
+        tile_rows<KIND, false>(td, work, work, [&](uint32_t r, float s0, float) { xcd_sum_add(out, d0 + r, s0, ctl); });
     }
     FK_XCD_STAMP(1, 11);
 }
@@ -203,7 +203,7 @@ __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, 
     FK_XCD_STAMP(0, 15);
     if (pr_n) {
         uint16_t* dst = (part_id == 0 ? a.q : (part_id == 1 ? a.k : a.v)) + (size_t)sync.xcd * part_rows + pr0;
-        tile_rows<false, ONE>(tq, work, work, [&](uint32_t r, float s0, float) { dst[r] = (uint16_t)f32_to_bf16_bits(s0); });
+        tile_rows<KIND, false>(tq, work, work, [&](uint32_t r, float s0, float) { dst[r] = (uint16_t)f32_to_bf16_bits(s0); });
     }
     FK_XCD_STAMP(0, 6);
     uint32_t* okw = reinterpret_cast<uint32_t*>(red) + 8;
@@ -272,8 +272,7 @@ __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, 
     if (o_n && ok2) {
         long long* out = a.out_sums;
         XcdControl* ctl = sync.ctl;
-        // (the one-round form was slower here: 835 against 837 tok/s; the o_proj slice has 16 chunks per row)
-        tile_rows<false>(to, work, work, [&](uint32_t r, float s0, float) { xcd_sum_add(out, o0 + r, s0, ctl); });
+        tile_rows<KIND, false>(to, work, work, [&](uint32_t r, float s0, float) { xcd_sum_add(out, o0 + r, s0, ctl); });
     }
     FK_XCD_STAMP(0, 12);
 }

@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kBlock, 2) void xcd_mla_kernel(const long long* sum
     __syncthreads();
     if (pr_n) {
         uint16_t* dst = is_q ? a.q + (size_t)xcd * a.q_rows + pr0 : a.kva + (size_t)xcd * a.a_rows + pr0;
-        tile_rows<false, true>(ta, work, work, [&](uint32_t r, float s0, float) { dst[r] = (uint16_t)f32_to_bf16_bits(s0); });
+        tile_rows<KIND, false>(ta, work, work, [&](uint32_t r, float s0, float) { dst[r] = (uint16_t)f32_to_bf16_bits(s0); });
     }
     FK_XCD_STAMP(0, 3);
     meta_store<KIND, kBlock, true>(mb, tid, meta + MW);
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(kBlock, 2) void xcd_mla_kernel(const long long* sum
             uint16_t* ck = a.sdpa.cache_k_w;
             uint16_t* cv = a.sdpa.cache_v_w;
             const uint32_t head0 = xcd * a.hl;
-            tile_rows<false, true>(tb, work, work, [&](uint32_t r, float s0, float) {
+            tile_rows<KIND, false>(tb, work, work, [&](uint32_t r, float s0, float) {
                 const uint16_t v16 = (uint16_t)f32_to_bf16_bits(s0);
                 dst[r] = v16;
                 const uint32_t rr_ = b0 + r, hl_ = rr_ / packed, w = rr_ - hl_ * packed;
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kBlock, 2) void xcd_mla_kernel(const long long* sum
     if (o_n && ok) {
         long long* out = a.out_sums;
         XcdControl* ctl = sync.ctl;
-        tile_rows<false, true>(to, work, work, [&](uint32_t r, float s0, float) { xcd_sum_add(out, o0 + r, s0, ctl); });
+        tile_rows<KIND, false>(to, work, work, [&](uint32_t r, float s0, float) { xcd_sum_add(out, o0 + r, s0, ctl); });
     }
     FK_XCD_STAMP(0, 11);
     xcd_mark_placement(sync, a.mark_placement);

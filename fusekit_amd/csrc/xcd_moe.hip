@@ -264,7 +264,7 @@ __global__ __launch_bounds__(kBlock, 2) void xcd_moe_kernel(const long long* sum
     FK_XCD_STAMP(0, 5);
     __syncthreads();
     if (!idle)
-        tile_rows<true, true>(tg, work, work + seg,
+        tile_rows<KIND, true>(tg, work, work + seg,
                               [&](uint32_t r, float s0, float s1) { mid[gu0 + r] = (uint16_t)swiglu_bits(s0, s1, variant, 1.0f); });
     FK_XCD_STAMP(0, 6);
     meta_store<KIND, kBlock, false>(md, tid, meta + 2 * MW);
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kBlock, 2) void xcd_moe_kernel(const long long* sum
         XcdControl* ctl = sync.ctl;
         // a route's full dot product is rounded to T before it is weighted and summed (routed_qmv_reduce.rs:236-322);
         // a shared unit contributes its K-slice of the shared expert's dot product as it is
-        tile_rows<false, true>(td, work, work, [&](uint32_t r, float s0, float) {
+        tile_rows<KIND, false>(td, work, work, [&](uint32_t r, float s0, float) {
             xcd_sum_add(out, out0 + r, routed ? __fmul_rn(route_w, round_bf16(s0)) : s0, ctl);
         });
     }
