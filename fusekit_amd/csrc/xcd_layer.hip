@@ -468,21 +468,64 @@ struct PassDepth {
 constexpr PassDepth depth_of(WKind k) {
     return k == W_Q8 ? PassDepth{9, 5, kNlGu, kNlDown} : PassDepth{kNlQkv, kNlO, kNlGu, kNlDown};
 }
-inline PassDepth depth_of_bits(uint32_t bits) { return depth_of(bits == 4 ? W_Q4 : (bits == 8 ? W_Q8 : W_BF16)); }
+inline WKind kind_of_bits(uint32_t bits) { return bits == 4 ? W_Q4 : (bits == 8 ? W_Q8 : W_BF16); }
+inline PassDepth depth_of_bits(uint32_t bits) { return depth_of(kind_of_bits(bits)); }
 
 
 
-template <WKind KIND>
-const void* mlp_func(bool one) {
-    constexpr PassDepth d = depth_of(KIND);  // the deeper passes only where they make the launch one pass
-    return one ? reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, d.gu, d.down, true>)
-               : reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, kNlGu, kNlDown, false>);
+// The requests a pass of a launch's two projections has.  Every request of a pass is made and multiplied whether the tile reaches it or
+// not (straight-line code; one more is 0.3 us of dequantisation), so a launch takes the shallowest one-pass flavour that holds its tiles,
+// and of the passes of 6 (3) and 5 those that end nearer the tile's last request.  us a token behind 480 positions: 12 layers of hidden 1024,
+// intermediate 3072, 16 / 8 heads x 64 (one request each, all in the deepest flavour / this) 306 / 241; the 4B class (attention 4 + 3 of 5 + 3)
+// 1095 / 1092; hidden 4096, intermediate 14336 (attention one pass of 6 + 4 for two of 5 + 3, MLP 14 requests in 15 for 18) 886 / 843.
+struct Depth {
+    uint32_t a, b;
+};
+Depth mlp_depth(WKind k, bool one, uint32_t gu, uint32_t down) {
+    if (!one) return ceil_div(gu, 5) * 5 < ceil_div(gu, kNlGu) * kNlGu ? Depth{5, 5} : Depth{kNlGu, kNlDown};
+    if (gu <= 1 && down <= 1) return Depth{1, 1};
+    if (gu <= 3 && down <= 3) return Depth{3, 3};
+    return Depth{(uint32_t)depth_of(k).gu, (uint32_t)depth_of(k).down};
+}
+// One pass: at most these (4 bits: the attention launch alone also takes hidden 4096 in one).
+Depth attn_one_pass(WKind k) { return k == W_Q4 ? Depth{6, 4} : Depth{(uint32_t)depth_of(k).qkv, (uint32_t)depth_of(k).o}; }
+Depth attn_depth(WKind k, bool one, uint32_t qkv, uint32_t o) {
+    const Depth d = {(uint32_t)depth_of(k).qkv, (uint32_t)depth_of(k).o};
+    if (!one) return ceil_div(o, 5) * 5 < ceil_div(o, kNlO) * kNlO ? Depth{kNlQkv, 5} : Depth{kNlQkv, kNlO};
+    if (qkv <= 1 && o <= 1) return Depth{1, 1};
+    if (qkv <= 2 && o <= 1) return Depth{2, 1};
+    if (qkv < d.a && o <= d.b) return Depth{d.a - 1, d.b};
+    return qkv <= d.a && o <= d.b ? d : attn_one_pass(k);
 }
 template <WKind KIND>
-const void* attn_func(bool one) {
+const void* mlp_func(bool one, Depth n) {
     constexpr PassDepth d = depth_of(KIND);
-    return one ? reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, d.qkv, d.o, true>)
-               : reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, kNlQkv, kNlO, false>);
+    if (!one) return n.a == 5 ? reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, 5, 5, false>)
+                              : reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, kNlGu, kNlDown, false>);
+    if (n.a == 1) return reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, 1, 1, true>);
+    if (n.a == 3) return reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, 3, 3, true>);
+    return reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, d.gu, d.down, true>);
+}
+template <WKind KIND>
+const void* attn_func(bool one, Depth n) {
+    constexpr PassDepth d = depth_of(KIND);
+    if (!one) return n.b == 5 ? reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, kNlQkv, 5, false>)
+                              : reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, kNlQkv, kNlO, false>);
+    if (n.a == 1) return reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, 1, 1, true>);
+    if (n.a == 2) return reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, 2, 1, true>);
+    if constexpr (KIND == W_Q4)
+        if (n.a == 6) return reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, 6, 4, true>);
+    return n.a < (uint32_t)d.qkv ? reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, d.qkv - 1, d.o, true>)
+                                 : reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, d.qkv, d.o, true>);
+}
+// Are these one-pass flavours whose tiles the whole-layer launch (both phases at the deepest one) holds?
+template <WKind KIND>
+bool one_pass(const void* attn, const void* mlp) {
+    constexpr PassDepth d = depth_of(KIND);
+    bool a = false, m = false;
+    for (uint32_t n : {1u, 2u, (uint32_t)d.qkv - 1u, (uint32_t)d.qkv}) a |= attn == attn_func<KIND>(true, Depth{n, (uint32_t)d.o});
+    for (uint32_t n : {1u, 3u, (uint32_t)d.gu}) m |= mlp == mlp_func<KIND>(true, Depth{n, n});
+    return a && m;
 }
 
 template <WKind KIND>
@@ -519,13 +562,16 @@ MlpGeometry mlp_geometry(const XcdLayerShape& s, bool for_token) {
     const PassDepth deep = depth_of_bits(s.bits);
     // every tile within one pass (the 4B-class shapes): the flavour compiled without the pass loop
     g.one = !for_token && g.gu_rows * g.gate_cpr <= (uint32_t)deep.gu * kBlock && g.down_rows * g.down_cs <= (uint32_t)deep.down * kBlock;
-    const PassDepth depth = for_token ? PassDepth{kNlQkv, kNlO, kNlGuToken, kNlDown} : (g.one ? deep : PassDepth{kNlQkv, kNlO, kNlGu, kNlDown});
-    const uint32_t gu = 2 * padded(g.gu_rows * g.gate_cpr, depth.gu), dn = padded(g.down_rows * g.down_cs, depth.down);
+    const uint32_t gu_n = ceil_div(g.gu_rows * g.gate_cpr, kBlock), down_n = ceil_div(g.down_rows * g.down_cs, kBlock);
+    const WKind kind = kind_of_bits(s.bits);
+    const Depth depth = for_token ? Depth{kNlGuToken, kNlDown} : mlp_depth(kind, g.one, gu_n, down_n);
+    // partials padded to whole passes (one pass: to the deepest, which the whole-layer launch makes)
+    const uint32_t gu = 2 * padded(g.gu_rows * g.gate_cpr, g.one ? deep.gu : (int)depth.a), dn = padded(g.down_rows * g.down_cs, g.one ? deep.down : (int)depth.b);
     g.lp.work_floats = gu > dn ? gu : dn;
     g.lp.att_elems = 0;
     g.lp.meta_words = g.one ? kMetaWords : kMetaWordsBig;
     g.lds = lds_for(s.bits, g.lp);
-    g.func = s.bits == 4 ? mlp_func<W_Q4>(g.one) : (s.bits == 8 ? mlp_func<W_Q8>(g.one) : mlp_func<W_BF16>(g.one));
+    g.func = s.bits == 4 ? mlp_func<W_Q4>(g.one, depth) : (s.bits == 8 ? mlp_func<W_Q8>(g.one, depth) : mlp_func<W_BF16>(g.one, depth));
     return g;
 }
 
@@ -561,19 +607,24 @@ AttnGeometry attn_geometry(const XcdLayerShape& s, bool for_token = false) {
     auto padded = [](uint32_t chunks, int nl) { return ceil_div(chunks, nl * kAttnStream) * nl * kAttnStream; };
     g.lp.cs_max = g.wq_cpr > g.o_cs ? g.wq_cpr : g.o_cs;
     // partial rows padded to whole passes: of this launch's depths and of the whole-token launch's (it shares this plan)
-    const PassDepth deep = depth_of_bits(s.bits);
-    g.one = !for_token && R * g.wq_cpr <= (uint32_t)deep.qkv * kAttnStream && g.o_rows * g.o_cs <= (uint32_t)deep.o * kAttnStream;
-    const PassDepth depth = g.one ? deep : PassDepth{kNlQkv, kNlO, kNlGu, kNlDown};
     auto larger = [](uint32_t x, uint32_t y) { return x > y ? x : y; };
-    uint32_t wf = larger(padded(R * g.wq_cpr, depth.qkv), padded(R * g.wq_cpr, kNlQkv));
-    const uint32_t wo_ = larger(padded(g.o_rows * g.o_cs, depth.o), padded(g.o_rows * g.o_cs, kNlO));
+    const uint32_t qkv_n = ceil_div(R * g.wq_cpr, kAttnStream), o_n = ceil_div(g.o_rows * g.o_cs, kAttnStream);
+    const WKind kind = kind_of_bits(s.bits);
+    const PassDepth deep = depth_of(kind);
+    const Depth most = attn_one_pass(kind);
+    const uint32_t groups = s.bits == 16 ? 0u : larger(R * (s.hidden / s.group), g.o_rows * (G * s.head_dim / s.group));
+    const bool held = qkv_n <= (uint32_t)deep.qkv && o_n <= (uint32_t)deep.o;   // (whatever its groups: more than the flavour fetches are refused)
+    g.one = !for_token && (held || (qkv_n <= most.a && o_n <= most.b && groups <= kMetaWords));
+    const Depth depth = for_token ? Depth{kNlQkv, kNlO} : attn_depth(kind, g.one, qkv_n, o_n);
+    uint32_t wf = larger(padded(R * g.wq_cpr, depth.a), padded(R * g.wq_cpr, kNlQkv));
+    const uint32_t wo_ = larger(padded(g.o_rows * g.o_cs, depth.b), padded(g.o_rows * g.o_cs, kNlO));
     wf = wf > wo_ ? wf : wo_;
     const uint32_t sf = sdpa_lds_floats(1, g.chunk_len, s.head_dim, s.head_dim, true);
     g.lp.work_floats = wf > sf ? wf : sf;
     g.lp.att_elems = G * s.head_dim;
     g.lp.meta_words = g.one ? kMetaWords : kMetaWordsBig;   // the whole-token launch runs the flavour with the pass loop
     g.lds = lds_for(s.bits, g.lp);
-    g.func = s.bits == 4 ? attn_func<W_Q4>(g.one) : (s.bits == 8 ? attn_func<W_Q8>(g.one) : attn_func<W_BF16>(g.one));
+    g.func = s.bits == 4 ? attn_func<W_Q4>(g.one, depth) : (s.bits == 8 ? attn_func<W_Q8>(g.one, depth) : attn_func<W_BF16>(g.one, depth));
     return g;
 }
 
@@ -799,9 +850,9 @@ fk_status plan_xcd_layer(const Launch& la, const Launch& lm, Launch* out) {
     memcpy(&t.attn, la.args, sizeof(XcdAttnArgs));
     memcpy(&t.mlp, lm.args, sizeof(XcdMlpArgs));
     const void* func = nullptr;
-    if (la.func == attn_func<W_Q4>(true) && lm.func == mlp_func<W_Q4>(true)) func = layer_func<W_Q4>();
-    if (la.func == attn_func<W_Q8>(true) && lm.func == mlp_func<W_Q8>(true)) func = layer_func<W_Q8>();
-    if (la.func == attn_func<W_BF16>(true) && lm.func == mlp_func<W_BF16>(true)) func = layer_func<W_BF16>();
+    if (one_pass<W_Q4>(la.func, lm.func)) func = layer_func<W_Q4>();
+    if (one_pass<W_Q8>(la.func, lm.func)) func = layer_func<W_Q8>();
+    if (one_pass<W_BF16>(la.func, lm.func)) func = layer_func<W_BF16>();
     if (!func) return set_error(FK_ERR_UNSUPPORTED, "xcd layer launch: both launches must take their one-pass flavour, same weight kind");
     if (t.attn.ctl != t.mlp.ctl) return set_error(FK_ERR_INVALID, "xcd layer launch: the two launches use different control blocks");
     if (!t.mlp.in.sums || t.mlp.in.sums != t.attn.out_sums || t.mlp.in.residual != t.attn.in.x_out ||

@@ -14,6 +14,8 @@ FK_PROBE_DEFINE(xcd_mla, 512, 16)
 
 namespace fk {
 
+// The deepest passes, and the flavour's with the benchmark architecture's depths: a request more is made and multiplied whether a tile
+// reaches it or not (0.3 us; 16 heads of 192 / 128, latent 512, hidden 2048: 4 + 1 + 1 requests for 5 + 2 + 3, a token of 27 layers 1061 -> 1048 us).
 constexpr int kMlaNlA = 5;   // 16-byte requests per thread: a q / kv_a tile holds at most 5 * 256 chunks
 constexpr int kMlaNlB = 2;   // ... a kv_b tile
 constexpr int kMlaNlO = 3;   // ... an o_proj tile
@@ -107,11 +109,10 @@ __device__ __forceinline__ void mla_clear2(long long* row, uint32_t row_elems) {
 
 }  // namespace
 
-template <WKind KIND>
+template <WKind KIND, int NLA, int NLB, int NLO>
 __global__ __launch_bounds__(kBlock, 2) void xcd_mla_kernel(const long long* sums, const uint16_t* residual, const uint16_t* norm_w,
                                                             uint32_t hidden, const XcdMlaArgs a) {
     extern __shared__ uint4 lds_raw[];
-    constexpr int NLA = kMlaNlA, NLB = kMlaNlB, NLO = kMlaNlO;
     const XcdInputLead lead{sums, residual, norm_w, hidden};
     InputRegs inr;
     InputRegs2 inr2;
@@ -347,6 +348,7 @@ struct MlaGeometry {
     uint32_t chunk_len, chunks_per_block, n_splits, lp;
     LdsPlan lp_;
     uint32_t lds;
+    const void* func;
 };
 MlaGeometry mla_geometry(const XcdMlaShape& s) {
     MlaGeometry g;
@@ -390,6 +392,9 @@ MlaGeometry mla_geometry(const XcdMlaShape& s) {
     g.lp_.att_elems = g.hl * s.v_dim;
     g.lp_.meta_words = kMetaWords;
     g.lds = xcd_lds_bytes<W_Q4>(g.lp_);
+    const bool shallow = g.R * wq_cpr <= 4u * kBlock && g.b_rows * wb_cpr <= (uint32_t)kBlock && g.o_rows * g.o_cs <= (uint32_t)kBlock;
+    g.func = shallow ? reinterpret_cast<const void*>(&xcd_mla_kernel<W_Q4, 4, 1, 1>)
+                     : reinterpret_cast<const void*>(&xcd_mla_kernel<W_Q4, kMlaNlA, kMlaNlB, kMlaNlO>);
     return g;
 }
 
@@ -425,7 +430,7 @@ fk_status xcd_mla_supported(const XcdMlaShape& s) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
     if (dev->cus != (int)(kXcds * 32)) return set_error(FK_ERR_UNSUPPORTED, "xcd mla: needs 8 XCDs of 32 CUs");
-    return require_two_blocks_per_cu(reinterpret_cast<const void*>(&xcd_mla_kernel<W_Q4>), g.lds, "low-rank attention");
+    return require_two_blocks_per_cu(g.func, g.lds, "low-rank attention");
 }
 
 size_t xcd_mla_partials_bytes(const XcdMlaShape& s) { return (size_t)s.n_heads * kXcdMaxRanges * (s.v_dim + 2) * sizeof(float); }
@@ -514,7 +519,7 @@ fk_status plan_xcd_mla(const XcdMlaRequest& rq, Launch* out) {
     a.work_floats = g.lp_.work_floats;
     a.att_elems = g.lp_.att_elems;
     a.mark_placement = rq.mark_placement ? 1u : 0u;
-    out->func = reinterpret_cast<const void*>(&xcd_mla_kernel<W_Q4>);
+    out->func = g.func;
     FK_TRY(require_two_blocks_per_cu(out->func, g.lds, "low-rank attention"));
     out->grid = dim3(kXcdGrid, 1, 1);
     out->block = dim3(kBlock, 1, 1);
