@@ -18,7 +18,8 @@ constexpr int kMlpBlock = kBlock;
 // the residual row in LDS (token kernel only).
 // EARLY: the caller has already issued input_request into `inr` (the stand-alone launch does so before anything
 // else, from its leading parameters).
-template <WKind KIND, int NLA, int NLB, bool TOKEN, bool EARLY, bool ONE = false, typename ARGS, typename LEAD>
+// BIG: tiles of up to 2048 quantisation groups (else 768).
+template <WKind KIND, int NLA, int NLB, bool TOKEN, bool EARLY, bool ONE = false, bool BIG = !ONE, typename ARGS, typename LEAD>
 __device__ __forceinline__ void xcd_mlp_phase(const ARGS& a, const LEAD& lead, InputRegs& inr, XcdSync& sync, uint4* lds_raw,
                                               const uint4* xres_in, uint4* xres_out) {
     const uint32_t cs_max = a.cs_max, work_floats = a.work_floats;
@@ -26,7 +27,7 @@ __device__ __forceinline__ void xcd_mlp_phase(const ARGS& a, const LEAD& lead, I
     uint4* xs = lds_raw;
     float* sx = reinterpret_cast<float*>(xs + PIECES * cs_max);
     float* work = sx + cs_max;
-    constexpr uint32_t MW = meta_words<ONE>();
+    constexpr uint32_t MW = meta_words<!BIG>();
     uint32_t* meta = reinterpret_cast<uint32_t*>(work + work_floats);  // [3][MW]
     float* red = reinterpret_cast<float*>(meta + 3 * MW);              // [16]
     const uint32_t tid = threadIdx.x;
@@ -52,8 +53,8 @@ __device__ __forceinline__ void xcd_mlp_phase(const ARGS& a, const LEAD& lead, I
     if constexpr (!EARLY) input_request<TOKEN>(lead, inr, xres_in);
     tile_pos_init<NLA, kBlock>(a.gate, tg, tid, pg);
     tile_pos_init<NLB, kBlock>(a.down, td, tid, pd);
-    meta_fetch<KIND, kBlock, true, !ONE>(a.gate, tg, tid, mg);
-    meta_fetch<KIND, kBlock, true, !ONE>(a.up, tg, tid, mu);
+    meta_fetch<KIND, kBlock, true, BIG>(a.gate, tg, tid, mg);
+    meta_fetch<KIND, kBlock, true, BIG>(a.up, tg, tid, mu);
     // Only kGuAhead requests of the gate matrix go out ahead of the input's staging, the rest of the pass and the up
     // matrix's behind it: a wave cannot stage before it has ISSUED what stands in front, issue stalls once the CU's
     // request queue is full, and the block's staging waits for its slowest wave.  With all twelve in front the
@@ -69,9 +70,9 @@ __device__ __forceinline__ void xcd_mlp_phase(const ARGS& a, const LEAD& lead, I
     tile_load<KIND, NLA, kBlock>(a.up, tg, pg, ru);
     FK_XCD_STAMP(1, 5);
     input_clear<TOKEN>(a.in);
-    meta_store<KIND, kBlock, true, !ONE>(mg, tid, meta);
-    meta_store<KIND, kBlock, true, !ONE>(mu, tid, meta + MW);
-    meta_fetch<KIND, kBlock, true, !ONE>(a.down, td, tid, md, sync.xcd);  // not needed before the hand-over: kept off the start-up path
+    meta_store<KIND, kBlock, true, BIG>(mg, tid, meta);
+    meta_store<KIND, kBlock, true, BIG>(mu, tid, meta + MW);
+    meta_fetch<KIND, kBlock, true, BIG>(a.down, td, tid, md, sync.xcd);  // not needed before the hand-over: kept off the start-up path
     __syncthreads();
 
     // ---- gate / up rows of this XCD's slice, SwiGLU ----
@@ -85,7 +86,7 @@ __device__ __forceinline__ void xcd_mlp_phase(const ARGS& a, const LEAD& lead, I
             request_down();
     }
     FK_XCD_STAMP(1, 6);
-    meta_store<KIND, kBlock, true, !ONE>(md, tid, meta + 2 * MW);
+    meta_store<KIND, kBlock, true, BIG>(md, tid, meta + 2 * MW);
     __syncthreads();
     FK_XCD_STAMP(1, 12);
     if (streams && gu_n) {
@@ -116,7 +117,7 @@ __device__ __forceinline__ void xcd_mlp_phase(const ARGS& a, const LEAD& lead, I
     FK_XCD_STAMP(1, 11);
 }
 
-template <WKind KIND, int NLA, int NLB, bool ONE>
+template <WKind KIND, int NLA, int NLB, bool ONE, bool BIG = !ONE>
 __global__ __launch_bounds__(kMlpBlock, 2) void xcd_mlp_kernel(const long long* sums, const uint16_t* residual,
                                                                const uint16_t* norm_w, uint32_t hidden, const XcdMlpArgs a) {
     extern __shared__ uint4 lds_raw[];
@@ -126,7 +127,7 @@ __global__ __launch_bounds__(kMlpBlock, 2) void xcd_mlp_kernel(const long long* 
     input_request<false>(lead, inr, nullptr);
     kernarg_warm<32 + (int)sizeof(XcdMlpArgs)>();
     XcdSync sync = xcd_sync_init(a.ctl, a.spin_limit);
-    xcd_mlp_phase<KIND, NLA, NLB, false, true, ONE>(a, lead, inr, sync, lds_raw, nullptr, nullptr);
+    xcd_mlp_phase<KIND, NLA, NLB, false, true, ONE, BIG>(a, lead, inr, sync, lds_raw, nullptr, nullptr);
     xcd_mark_placement(sync, a.mark_placement);
 }
 
@@ -485,6 +486,7 @@ Depth mlp_depth(WKind k, bool one, uint32_t gu, uint32_t down) {
     if (!one) return ceil_div(gu, 5) * 5 < ceil_div(gu, kNlGu) * kNlGu ? Depth{5, 5} : Depth{kNlGu, kNlDown};
     if (gu <= 1 && down <= 1) return Depth{1, 1};
     if (gu <= 3 && down <= 3) return Depth{3, 3};
+    if (gu > (uint32_t)depth_of(k).gu || down > (uint32_t)depth_of(k).down) return gu <= 12 && down <= 12 ? Depth{12, 12} : Depth{14, 14};
     return Depth{(uint32_t)depth_of(k).gu, (uint32_t)depth_of(k).down};
 }
 // One pass: at most these (4 bits: the attention launch alone also takes hidden 4096 in one).
@@ -502,6 +504,10 @@ const void* mlp_func(bool one, Depth n) {
     constexpr PassDepth d = depth_of(KIND);
     if (!one) return n.a == 5 ? reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, 5, 5, false>)
                               : reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, kNlGu, kNlDown, false>);
+    if constexpr (KIND != W_BF16) {
+        if (n.a == 12) return reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, 12, 12, true, true>);
+        if (n.a == 14) return reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, 14, 14, true, true>);
+    }
     if (n.a == 1) return reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, 1, 1, true>);
     if (n.a == 3) return reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, 3, 3, true>);
     return reinterpret_cast<const void*>(&xcd_mlp_kernel<KIND, d.gu, d.down, true>);
@@ -561,15 +567,16 @@ MlpGeometry mlp_geometry(const XcdLayerShape& s, bool for_token) {
     g.lp.cs_max = g.gate_cpr > g.down_cs ? g.gate_cpr : g.down_cs;
     const PassDepth deep = depth_of_bits(s.bits);
     // every tile within one pass (the 4B-class shapes): the flavour compiled without the pass loop
-    g.one = !for_token && g.gu_rows * g.gate_cpr <= (uint32_t)deep.gu * kBlock && g.down_rows * g.down_cs <= (uint32_t)deep.down * kBlock;
     const uint32_t gu_n = ceil_div(g.gu_rows * g.gate_cpr, kBlock), down_n = ceil_div(g.down_rows * g.down_cs, kBlock);
     const WKind kind = kind_of_bits(s.bits);
+    const bool held = gu_n <= (uint32_t)deep.gu && down_n <= (uint32_t)deep.down;
+    g.one = !for_token && (held || (kind != W_BF16 && gu_n <= 14u && down_n <= 14u));
     const Depth depth = for_token ? Depth{kNlGuToken, kNlDown} : mlp_depth(kind, g.one, gu_n, down_n);
     // partials padded to whole passes (one pass: to the deepest, which the whole-layer launch makes)
-    const uint32_t gu = 2 * padded(g.gu_rows * g.gate_cpr, g.one ? deep.gu : (int)depth.a), dn = padded(g.down_rows * g.down_cs, g.one ? deep.down : (int)depth.b);
+    const uint32_t gu = 2 * padded(g.gu_rows * g.gate_cpr, held && g.one ? deep.gu : (int)depth.a), dn = padded(g.down_rows * g.down_cs, held && g.one ? deep.down : (int)depth.b);
     g.lp.work_floats = gu > dn ? gu : dn;
     g.lp.att_elems = 0;
-    g.lp.meta_words = g.one ? kMetaWords : kMetaWordsBig;
+    g.lp.meta_words = g.one && held ? kMetaWords : kMetaWordsBig;
     g.lds = lds_for(s.bits, g.lp);
     g.func = s.bits == 4 ? mlp_func<W_Q4>(g.one, depth) : (s.bits == 8 ? mlp_func<W_Q8>(g.one, depth) : mlp_func<W_BF16>(g.one, depth));
     return g;
