@@ -388,11 +388,42 @@ __device__ __forceinline__ void tile_pos_next(const MAT& m, const Tile& t, uint3
     }
 }
 
+// A tile of whole rows that may run on from the end of one matrix into the next (the q, k and v rows of an XCD as one list: 768 rows of the
+// 4B class are 12 a block; cut matrix by matrix 13, 8 % more requests than the tile's depth holds).  From chunk `split` (group
+// `gsplit`) of the tile on, the second matrix, its pointers moved so that the first one's indices run on.
+// (Addresses as numbers, turned into global pointers where they are used: a generic pointer would make the requests flat ones.)
+struct XcdMat2 {
+    uintptr_t w, w2, sc, sc2, bi, bi2;
+    uint32_t rows, cpr, gshift, split, gsplit;
+};
+template <typename MAT>
+__device__ __forceinline__ uint4 mat_chunk(const MAT& m, uint32_t, uint32_t at) { return m.w[at]; }
+__device__ __forceinline__ uint4 mat_chunk(const XcdMat2& m, uint32_t pos, uint32_t at) {
+    typedef const __attribute__((address_space(1))) fk_u32x4_t* gptr;
+    const fk_u32x4_t v = ((gptr)(pos < m.split ? m.w : m.w2))[at];
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <typename MAT>
+__device__ __forceinline__ void mat_groups(const MAT& m, uint32_t, size_t e, uint2& sv, uint2& bv) {
+    sv = *reinterpret_cast<const uint2*>(m.sc + e);
+    bv = *reinterpret_cast<const uint2*>(m.bi + e);
+}
+__device__ __forceinline__ void mat_groups(const XcdMat2& m, uint32_t gi, size_t e, uint2& sv, uint2& bv) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef const __attribute__((address_space(1))) u32x2* gptr;
+    const bool second = gi >= m.gsplit;
+    const u32x2 s = *(gptr)((second ? m.sc2 : m.sc) + 2u * e), b = *(gptr)((second ? m.bi2 : m.bi) + 2u * e);
+    sv = make_uint2(s.x, s.y);
+    bv = make_uint2(b.x, b.y);
+}
 template <WKind KIND, int NL, int SN, int J0 = 0, int J1 = NL, typename MAT>
 __device__ __forceinline__ void tile_load(const MAT& m, const Tile& t, const TilePos<NL>& p, TileRegs<NL>& r) {
     const uint32_t total = t.rows * t.cs, first = t.row0 * m.cpr + t.col0;
 #pragma unroll
-    for (int j = J0; j < J1; ++j) r.w[j] = m.w[p.p0 + j * SN < total ? p.gidx[j] : first];
+    for (int j = J0; j < J1; ++j) {
+        const uint32_t pos = p.p0 + j * SN;
+        r.w[j] = mat_chunk(m, pos < total ? pos : 0u, pos < total ? p.gidx[j] : first);
+    }
 }
 
 // Group gi of the tile = (row gi / gpr, group gi % gpr of the row's slice), gpr groups per row slice.
@@ -410,16 +441,16 @@ __device__ __forceinline__ void meta_fetch(const MAT& m, const Tile& t, uint32_t
         if constexpr (RUN) {
             // kMetaRegs * SN groups at most: lane ti takes groups 4 ti .. 4 ti + 3 (s[0..1] / b[0..1] hold them)
             const uint32_t gi = 4u * ti;
-            const size_t e = gi < total ? g0 + gi : g0;
-            const uint2 sv = *reinterpret_cast<const uint2*>(m.sc + e), bv = *reinterpret_cast<const uint2*>(m.bi + e);
+            uint2 sv, bv;
+            mat_groups(m, gi < total ? gi : 0u, gi < total ? g0 + gi : g0, sv, bv);
             r.s[0] = sv.x;
             r.s[1] = sv.y;
             r.b[0] = bv.x;
             r.b[1] = bv.y;
             if constexpr (BIG) {  // straight-line: a lane past the tile's groups repeats the first entries
                 const uint32_t gi2 = 4u * (ti + (uint32_t)SN);
-                const size_t e2 = gi2 < total ? g0 + gi2 : g0;
-                const uint2 sv2 = *reinterpret_cast<const uint2*>(m.sc + e2), bv2 = *reinterpret_cast<const uint2*>(m.bi + e2);
+                uint2 sv2, bv2;
+                mat_groups(m, gi2 < total ? gi2 : 0u, gi2 < total ? g0 + gi2 : g0, sv2, bv2);
                 r.s[2] = sv2.x;
                 r.s[3] = sv2.y;
                 r.b[2] = bv2.x;

@@ -134,7 +134,8 @@ __global__ __launch_bounds__(kMlpBlock, 2) void xcd_mlp_kernel(const long long* 
 // =============================================================================================== attention launch
 constexpr int kAttnStream = kBlock;
 
-template <WKind KIND, int NLA, int NLB, bool TOKEN, bool EARLY, bool ONE = false, typename ARGS, typename LEAD>
+// SPLIT: a q / k / v tile may reach into two matrices (else the planner has seen that none does).
+template <WKind KIND, int NLA, int NLB, bool TOKEN, bool EARLY, bool ONE = false, bool SPLIT = true, typename ARGS, typename LEAD>
 __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, InputRegs& inr, XcdSync& sync, uint4* lds_raw,
                                                const uint4* xres_in, uint4* xres_out) {
     const uint32_t cs_max = a.cs_max, work_floats = a.work_floats, att_elems = a.att_elems;
@@ -155,16 +156,39 @@ __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, 
     float* red = reinterpret_cast<float*>(att + ((att_elems + 7u) & ~7u));  // [16]
 
     FK_XCD_STAMP(0, 0);
-    // tile of the q / k / v projections: the XCD's q rows first, then its k rows, then its v rows
-    const uint32_t R = a.qkv_tile_rows, tix = sync.slot;
-    const bool has_tile = tix < a.q_tiles + 2 * a.kv_tiles;
-    const uint32_t part_id = tix < a.q_tiles ? 0u : (tix < a.q_tiles + a.kv_tiles ? 1u : 2u);
-    const uint32_t tl = part_id == 0 ? tix : (part_id == 1 ? tix - a.q_tiles : tix - a.q_tiles - a.kv_tiles);
-    const uint32_t part_rows = part_id == 0 ? a.q_rows : a.kv_rows;
-    const uint32_t pr0 = tl * R;
-    const uint32_t pr_n = has_tile ? ((part_rows - pr0) < R ? (part_rows - pr0) : R) : 0u;
-    const auto& mq = part_id == 0 ? a.wq : (part_id == 1 ? a.wk : a.wv);
+    // tile of the q / k / v projections: rows of the list of the XCD's q rows, its k rows, its v rows (a tile reaches into two of them at most)
+    const uint32_t R = a.qkv_tile_rows, kv_rows = a.kv_rows, k_first = a.q_rows, v_first = k_first + kv_rows, l0 = sync.slot * R;
+    const uint32_t l_n = v_first + kv_rows, pr_n = l0 < l_n ? (l_n - l0 < R ? l_n - l0 : R) : 0u;
+    const uint32_t part_id = l0 < k_first ? 0u : (l0 < v_first ? 1u : 2u);
+    const uint32_t part_end = part_id == 0 ? k_first : (part_id == 1 ? v_first : l_n), part_rows = part_id == 0 ? a.q_rows : kv_rows;
+    const uint32_t pr0 = pr_n ? l0 - (part_id == 0 ? 0u : (part_id == 1 ? k_first : v_first)) : 0u;
+    const uint32_t n1 = pr_n && part_end - l0 < pr_n ? part_end - l0 : pr_n;   // rows of the first of the two matrices
     const Tile tq = make_tile(sync.xcd * part_rows + pr0, pr_n, 0, a.wq.cpr);
+    std::conditional_t<SPLIT, XcdMat2, XcdMat> mq;
+    mq.rows = part_rows;
+    mq.cpr = a.wq.cpr;
+    mq.gshift = a.wq.gshift;
+    if constexpr (SPLIT) {
+        // the second matrix's first row of this XCD stands where row n1 of the tile would stand in the first
+        const int ahead_c = ((int)(sync.xcd * kv_rows) - (int)(tq.row0 + n1)) * (int)a.wq.cpr, ahead_g = ahead_c >> a.wq.gshift;
+        // (every matrix's pointers first, then the choice: chosen among the arguments' places it is a load behind a load, three times over:
+        // 0.4 us of the launch)
+        uintptr_t qw = (uintptr_t)a.wq.w, kw = (uintptr_t)a.wk.w, vw = (uintptr_t)a.wv.w, qs = (uintptr_t)a.wq.sc, ks = (uintptr_t)a.wk.sc,
+                  vs = (uintptr_t)a.wv.sc, qb = (uintptr_t)a.wq.bi, kb = (uintptr_t)a.wk.bi, vb = (uintptr_t)a.wv.bi;
+        asm volatile("" : "+s"(qw), "+s"(kw), "+s"(vw), "+s"(qs), "+s"(ks), "+s"(vs), "+s"(qb), "+s"(kb), "+s"(vb));
+        mq.w = part_id == 0 ? qw : (part_id == 1 ? kw : vw);
+        mq.sc = part_id == 0 ? qs : (part_id == 1 ? ks : vs);
+        mq.bi = part_id == 0 ? qb : (part_id == 1 ? kb : vb);
+        mq.w2 = (part_id == 0 ? kw : vw) + (intptr_t)ahead_c * 16;
+        mq.sc2 = (part_id == 0 ? ks : vs) + (intptr_t)ahead_g * 2;
+        mq.bi2 = (part_id == 0 ? kb : vb) + (intptr_t)ahead_g * 2;
+        mq.split = n1 * a.wq.cpr;
+        mq.gsplit = n1 * (a.wq.cpr >> a.wq.gshift);
+    } else {
+        mq.w = part_id == 0 ? a.wq.w : (part_id == 1 ? a.wk.w : a.wv.w);
+        mq.sc = part_id == 0 ? a.wq.sc : (part_id == 1 ? a.wk.sc : a.wv.sc);
+        mq.bi = part_id == 0 ? a.wq.bi : (part_id == 1 ? a.wk.bi : a.wv.bi);
+    }
     const uint32_t o0 = sync.slot * a.o_rows;
     const uint32_t o_n = o0 < a.in.hidden ? ((a.in.hidden - o0) < a.o_rows ? (a.in.hidden - o0) : a.o_rows) : 0u;
     const Tile to = make_tile(o0, o_n, sync.xcd * a.o_cs, a.o_cs);
@@ -204,7 +228,8 @@ __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, 
     FK_XCD_STAMP(0, 15);
     if (pr_n) {
         uint16_t* dst = (part_id == 0 ? a.q : (part_id == 1 ? a.k : a.v)) + (size_t)sync.xcd * part_rows + pr0;
-        tile_rows<KIND, false>(tq, work, work, [&](uint32_t r, float s0, float) { dst[r] = (uint16_t)f32_to_bf16_bits(s0); });
+        uint16_t* dst2 = (part_id == 0 ? a.k : a.v) + (size_t)sync.xcd * kv_rows;
+        tile_rows<KIND, false>(tq, work, work, [&](uint32_t r, float s0, float) { *(!SPLIT || r < n1 ? dst + r : dst2 + (r - n1)) = (uint16_t)f32_to_bf16_bits(s0); });
     }
     FK_XCD_STAMP(0, 6);
     uint32_t* okw = reinterpret_cast<uint32_t*>(red) + 8;
@@ -278,7 +303,7 @@ __device__ __forceinline__ void xcd_attn_phase(const ARGS& a, const LEAD& lead, 
     FK_XCD_STAMP(0, 12);
 }
 
-template <WKind KIND, int NLA, int NLB, bool ONE>
+template <WKind KIND, int NLA, int NLB, bool ONE, bool SPLIT = true>
 __global__ __launch_bounds__(kBlock, 2) void xcd_attn_kernel(const long long* sums, const uint16_t* residual,
                                                              const uint16_t* norm_w, uint32_t hidden, const XcdAttnArgs a) {
     extern __shared__ uint4 lds_raw[];
@@ -287,7 +312,7 @@ __global__ __launch_bounds__(kBlock, 2) void xcd_attn_kernel(const long long* su
     input_request<false>(lead, inr, nullptr);
     kernarg_warm<32 + (int)sizeof(XcdAttnArgs)>();
     XcdSync sync = xcd_sync_init(a.ctl, a.spin_limit);
-    xcd_attn_phase<KIND, NLA, NLB, false, true, ONE>(a, lead, inr, sync, lds_raw, nullptr, nullptr);
+    xcd_attn_phase<KIND, NLA, NLB, false, true, ONE, SPLIT>(a, lead, inr, sync, lds_raw, nullptr, nullptr);
     xcd_mark_placement(sync, a.mark_placement);
 }
 
@@ -491,11 +516,12 @@ Depth mlp_depth(WKind k, bool one, uint32_t gu, uint32_t down) {
 }
 // One pass: at most these (4 bits: the attention launch alone also takes hidden 4096 in one).
 Depth attn_one_pass(WKind k) { return k == W_Q4 ? Depth{6, 4} : Depth{(uint32_t)depth_of(k).qkv, (uint32_t)depth_of(k).o}; }
-Depth attn_depth(WKind k, bool one, uint32_t qkv, uint32_t o) {
+Depth attn_depth(WKind k, bool one, bool split, uint32_t qkv, uint32_t o) {
     const Depth d = {(uint32_t)depth_of(k).qkv, (uint32_t)depth_of(k).o};
     if (!one) return ceil_div(o, 5) * 5 < ceil_div(o, kNlO) * kNlO ? Depth{kNlQkv, 5} : Depth{kNlQkv, kNlO};
-    if (qkv <= 1 && o <= 1) return Depth{1, 1};
-    if (qkv <= 2 && o <= 1) return Depth{2, 1};
+    // (the shallowest come without the second matrix of a tile: 0.3 us of their 9)
+    if (!split && qkv <= 1 && o <= 1) return Depth{1, 1};
+    if (!split && qkv <= 2 && o <= 1) return Depth{2, 1};
     if (qkv < d.a && o <= d.b) return Depth{d.a - 1, d.b};
     return qkv <= d.a && o <= d.b ? d : attn_one_pass(k);
 }
@@ -517,8 +543,8 @@ const void* attn_func(bool one, Depth n) {
     constexpr PassDepth d = depth_of(KIND);
     if (!one) return n.b == 5 ? reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, kNlQkv, 5, false>)
                               : reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, kNlQkv, kNlO, false>);
-    if (n.a == 1) return reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, 1, 1, true>);
-    if (n.a == 2) return reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, 2, 1, true>);
+    if (n.a == 1) return reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, 1, 1, true, false>);
+    if (n.a == 2) return reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, 2, 1, true, false>);
     if constexpr (KIND == W_Q4)
         if (n.a == 6) return reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, 6, 4, true>);
     return n.a < (uint32_t)d.qkv ? reinterpret_cast<const void*>(&xcd_attn_kernel<KIND, d.qkv - 1, d.o, true>)
@@ -583,7 +609,7 @@ MlpGeometry mlp_geometry(const XcdLayerShape& s, bool for_token) {
 }
 
 struct AttnGeometry {
-    uint32_t wq_cpr, wo_cpr, q_rows, kv_rows, R, q_tiles, kv_tiles, o_rows, o_cs;
+    uint32_t wq_cpr, wo_cpr, q_rows, kv_rows, R, o_rows, o_cs;
     uint32_t chunk_len, chunks_per_block, n_splits;
     bool one;
     LdsPlan lp;
@@ -597,11 +623,8 @@ AttnGeometry attn_geometry(const XcdLayerShape& s, bool for_token = false) {
     g.wo_cpr = s.n_heads * s.head_dim / cv;
     g.q_rows = G * s.head_dim;
     g.kv_rows = s.head_dim;
-    uint32_t R = 1;
-    while (ceil_div(g.q_rows, R) + 2 * ceil_div(g.kv_rows, R) > kXcdSlots) ++R;
+    const uint32_t R = ceil_div(g.q_rows + 2 * g.kv_rows, kXcdSlots);   // (at most (8 + 2) * 128 / 64: fewer than a matrix has rows)
     g.R = R;
-    g.q_tiles = ceil_div(g.q_rows, R);
-    g.kv_tiles = ceil_div(g.kv_rows, R);
     g.o_rows = ceil_div(s.hidden, kXcdSlots);
     g.o_cs = g.wo_cpr / kXcds;
     // attention of one KV head per XCD: blocks = (query head of the group) x (key range)
@@ -617,12 +640,10 @@ AttnGeometry attn_geometry(const XcdLayerShape& s, bool for_token = false) {
     auto larger = [](uint32_t x, uint32_t y) { return x > y ? x : y; };
     const uint32_t qkv_n = ceil_div(R * g.wq_cpr, kAttnStream), o_n = ceil_div(g.o_rows * g.o_cs, kAttnStream);
     const WKind kind = kind_of_bits(s.bits);
-    const PassDepth deep = depth_of(kind);
     const Depth most = attn_one_pass(kind);
     const uint32_t groups = s.bits == 16 ? 0u : larger(R * (s.hidden / s.group), g.o_rows * (G * s.head_dim / s.group));
-    const bool held = qkv_n <= (uint32_t)deep.qkv && o_n <= (uint32_t)deep.o;   // (whatever its groups: more than the flavour fetches are refused)
-    g.one = !for_token && (held || (qkv_n <= most.a && o_n <= most.b && groups <= kMetaWords));
-    const Depth depth = for_token ? Depth{kNlQkv, kNlO} : attn_depth(kind, g.one, qkv_n, o_n);
+    g.one = !for_token && qkv_n <= most.a && o_n <= most.b && groups <= kMetaWords;
+    const Depth depth = for_token ? Depth{kNlQkv, kNlO} : attn_depth(kind, g.one, g.q_rows % R != 0 || g.kv_rows % R != 0, qkv_n, o_n);
     uint32_t wf = larger(padded(R * g.wq_cpr, depth.a), padded(R * g.wq_cpr, kNlQkv));
     const uint32_t wo_ = larger(padded(g.o_rows * g.o_cs, depth.b), padded(g.o_rows * g.o_cs, kNlO));
     wf = wf > wo_ ? wf : wo_;
@@ -657,12 +678,14 @@ fk_status xcd_layer_supported(const XcdLayerShape& s) {
     const MlpGeometry mg = mlp_geometry(s, false);
     const AttnGeometry ag = attn_geometry(s);
     if (s.bits != 16) {
-        // a tile's quantisation groups are fetched once per block: 768 per matrix in the one-pass flavour, 2048 in the
-        // flavour with the pass loop
-        const uint32_t n_q = s.n_heads * s.head_dim;
-        const uint32_t budget_a = ag.lp.meta_words, budget_m = mg.lp.meta_words;
+        // a tile's quantisation groups are fetched once per block: 768 per matrix in one pass, 2048 with the pass loop.  (The attention
+        // launch's tiles counted matrix by matrix and against the pass that such tiles would take: shapes that its list of rows would
+        // bring within the limits run the five launches, as they did.)
+        const uint32_t n_q = s.n_heads * s.head_dim, deep_qkv = (uint32_t)depth_of_bits(s.bits).qkv, deep_o = (uint32_t)depth_of_bits(s.bits).o;
         uint32_t R = 1;
         while (ceil_div(G * s.head_dim, R) + 2 * ceil_div(s.head_dim, R) > kXcdSlots) ++R;
+        const bool one = R * ag.wq_cpr <= deep_qkv * kAttnStream && ag.o_rows * ag.o_cs <= deep_o * kAttnStream;
+        const uint32_t budget_a = one ? kMetaWords : kMetaWordsBig, budget_m = mg.lp.meta_words;
         if (R * (s.hidden / s.group) > budget_a || ceil_div(s.hidden, kXcdSlots) * (n_q / kXcds / s.group) > budget_a ||
             ceil_div(s.inter / kXcds, kXcdSlots) * (s.hidden / s.group) > budget_m ||
             ceil_div(s.hidden, kXcdSlots) * (s.inter / kXcds / s.group) > budget_m)
@@ -783,8 +806,6 @@ fk_status plan_xcd_attn(const XcdAttnRequest& rq, Launch* out) {
     a.q_rows = g.q_rows;
     a.kv_rows = g.kv_rows;
     a.qkv_tile_rows = g.R;
-    a.q_tiles = g.q_tiles;
-    a.kv_tiles = g.kv_tiles;
     a.o_rows = g.o_rows;
     a.o_cs = g.o_cs;
     a.q = rq.q;

@@ -135,8 +135,7 @@ struct XcdAttnArgs {
     XcdInput in;
     XcdMat wq, wk, wv, wo;
     uint32_t q_rows, kv_rows;   // rows of q / of k (= of v) one XCD owns: G * head_dim, head_dim
-    uint32_t qkv_tile_rows;     // rows per block tile of the q / k / v projections
-    uint32_t q_tiles, kv_tiles; // tiles of the q part, of the k part (= of the v part)
+    uint32_t qkv_tile_rows;     // rows per block tile of the q / k / v projections, the XCD's q, k and v rows one list
     uint32_t o_rows;            // o_proj output rows per block
     uint32_t o_cs;              // chunks of one XCD's K-slice of an o_proj row
     uint16_t* q;                // [n_heads * head_dim] raw projection outputs (every XCD its heads)
