@@ -267,6 +267,12 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     Slab w0;
     [[maybe_unused]] Slab w1;
     Acts x0, x1;
+    // One slab and one tile of rows: all four of the slab's groups of activations are in flight, not two, a trip to the L2 less.  Two / four,
+    // us: 37 rows of 896 x 896 3.70 / 3.59, 8 rows of 3072 x 2048 4.85 / 4.73, of 2048 x 2048 4.60 / 4.43, 16 of the 4864 x 896 pair 5.53 /
+    // 5.38.  More tiles and several slabs keep two: 37 rows of that pair 8.54 / 8.83, 24 rows of 3072 x 2048 5.80 / 6.02 (registers), 8
+    // rows of 2560 x 4096 6.36 / 6.75 (what is asked for past a wave's range).
+    constexpr bool ALL_X = ONE && MT == 1 && SG == 4u;
+    [[maybe_unused]] Acts x2, x3;
     [[maybe_unused]] u32x2_any_t meta;
     [[maybe_unused]] u32x4_t norms;
     if constexpr (ONE) {
@@ -282,6 +288,10 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
     fetch_w(g0, w0);
     fetch_x(g0, x0);
     fetch_x(g0 + 1u, x1);
+    if constexpr (ALL_X) {
+        fetch_x(g0 + 2u, x2);
+        fetch_x(g0 + 3u, x3);
+    }
     if constexpr (!ONE) fetch_w(g0 + SG, w1);
     fetch_epilogue();
     float rr[MT][2];   // 1 / rms of the rows this lane parks
@@ -328,11 +338,18 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
 #pragma unroll
                     for (int e = 0; e < 4; ++e) ss[i][h] = dot2_bf16(x.x[i][h][e], x.x[i][h][e], ss[i][h]);
         };
-        for (uint32_t g = g0; g < g1; g += 2u) {
+        if constexpr (ALL_X) {
             squares(x0);
-            fetch_x(g + 2u < g1 ? g + 2u : g0, x0);
-            if (g + 1u < g1) squares(x1);
-            fetch_x(g + 3u < g1 ? g + 3u : g0 + 1u, x1);
+            if (g0 + 1u < g1) squares(x1);
+            if (g0 + 2u < g1) squares(x2);
+            if (g0 + 3u < g1) squares(x3);
+        } else {
+            for (uint32_t g = g0; g < g1; g += 2u) {
+                squares(x0);
+                fetch_x(g + 2u < g1 ? g + 2u : g0, x0);
+                if (g + 1u < g1) squares(x1);
+                fetch_x(g + 3u < g1 ? g + 3u : g0 + 1u, x1);
+            }
         }
         float* part = reinterpret_cast<float*>(reinterpret_cast<char*>(lds_raw) + WAVES * rows_wave_lds(MT, NT));   // [WAVES][MT * 16]
 #pragma unroll
@@ -371,7 +388,7 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
                 }
                 xs[((uint32_t)i * 16u + r8 + 8u * (uint32_t)h) * kRowsLine + l8] = v;
             }
-        if (!ONE || u + 2u < SG) fetch_x(g + u + 2u, x);
+        if (!ONE || (!ALL_X && u + 2u < SG)) fetch_x(g + u + 2u, x);
         __builtin_amdgcn_wave_barrier();
         if (g + u < g1) consume(u);   // wave-uniform
         __builtin_amdgcn_wave_barrier();
@@ -391,7 +408,10 @@ __global__ __launch_bounds__(WAVES* kWave, 2) void qgemm_rows_kernel(const Qgemm
         }
         step(g, 0u, xa);
         if constexpr (SG > 1) step(g, 1u, xb);
-        if constexpr (SG > 2) {
+        if constexpr (ALL_X) {
+            step(g, 2u, x2);
+            step(g, 3u, x3);
+        } else if constexpr (SG > 2) {
             step(g, 2u, xa);
             step(g, 3u, xb);
         }
