@@ -25,6 +25,7 @@ namespace {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));   // 16 bytes of an operand at any of its addresses
 
 constexpr uint32_t kRtThreads = kRtWaves * kWave, kRtMaxRoutes = 1024, kRtMaxExperts = 256, kRtLine = 9;
@@ -51,7 +52,8 @@ struct RtList {
     uint32_t chunk_expert[kRtMaxExperts + kRtMaxRoutes / kRtRows], chunk_at[kRtMaxExperts + kRtMaxRoutes / kRtRows];
     uint32_t chunks, several;   // several: an expert has more than one chunk
 };
-constexpr uint32_t kRtWaveLds = 2u * 16u * kRtLine * 16u + 2u * 16u * 4u * 4u;   // weight lines, (scale, bias) pairs
+constexpr uint32_t kRtMeta = 12u;   // (scale, bias) pairs of a row in LDS: eight, behind three at most that a clamped request begins early
+constexpr uint32_t kRtWaveLds = 2u * 16u * kRtLine * 16u + 2u * 16u * kRtMeta * 4u;   // weight lines, (scale, bias) pairs
 constexpr uint32_t kRtMeetLds = kRtWaves * 2u * 256u * 4u;
 constexpr uint32_t kRtLds = kRtWaves * kRtWaveLds + kRtMeetLds + (uint32_t)((sizeof(RtList) + 15u) & ~15u);
 
@@ -168,7 +170,7 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
     const uint32_t c16 = lane & 15u, kq = lane >> 4, l8 = lane & 7u, r8 = lane >> 3;
     char* lds = reinterpret_cast<char*>(lds_raw);
     u32x4_t* wl = reinterpret_cast<u32x4_t*>(lds + wave * kRtWaveLds);                      // [NT * 16][kRtLine]
-    uint32_t* ml = reinterpret_cast<uint32_t*>(wl + NT * 16 * kRtLine);                        // [NT * 16][4]
+    uint32_t* ml = reinterpret_cast<uint32_t*>(wl + NT * 16 * kRtLine);                        // [NT * 16][kRtMeta]
     float* meet = reinterpret_cast<float*>(lds + kRtWaves * kRtWaveLds);                  // [waves][16][NT * 16]
     RtList& L = *reinterpret_cast<RtList*>(lds + kRtWaves * kRtWaveLds + kRtMeetLds);
     FK_RT_STAMP(0);
@@ -184,8 +186,9 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
 
     // A piece: uniform bases, 32-bit lane offsets (rows past the matrix repeat its last one and are not stored).
     struct Piece {
-        const unsigned char *w[NT], *s[NT], *b[NT];
-        uint32_t woff[NT][2], soff[NT], xoff, n0, first, count;
+        const unsigned char *w[NT], *s, *b;   // s, b: of this lane's tile
+        uint32_t woff[NT][2], xoff, n0, first, count;
+        int soff, slast;
     };
     auto open = [&](uint32_t p, Piece& q) __attribute__((always_inline)) {
         const uint32_t chunk = p / a.tiles, tile = p - chunk * a.tiles, at = L.chunk_at[chunk];
@@ -198,18 +201,29 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
             const uint32_t mat = PAIR ? (uint32_t)t : 0u, n0 = q.n0 + (PAIR ? 0u : (uint32_t)t * 16u), f = n0 < N ? n0 : N - 1u;
             const size_t row = (size_t)ex * N + f;
             q.w[t] = a.w[mat] + row * row_bytes;
-            q.s[t] = a.sc[mat] + row * gpr * 2u;
-            q.b[t] = a.bi[mat] + row * gpr * 2u;
             auto clamp = [&](uint32_t r) { return f + r < N ? r : N - 1u - f; };
 #pragma unroll
             for (int h = 0; h < 2; ++h) q.woff[t][h] = clamp(r8 + 8u * (uint32_t)h) * row_bytes;
-            q.soff[t] = clamp(lane >> 2) * gpr * 2u;
+            if (t == 0 || lane >= 32u) {   // scales and biases: tile lane / 32, row lane / 2 % 16
+                q.s = a.sc[mat] + row * gpr * 2u;
+                q.b = a.bi[mat] + row * gpr * 2u;
+                q.soff = (int)(clamp((lane >> 1) & 15u) * gpr);
+                const int64_t last = (int64_t)((size_t)a.n_experts * N - row) * gpr - 4;   // where the stack's last four begin
+                q.slast = last < 0x3fffffff ? (int)last : 0x3fffffff;
+            }
         }
         q.xoff = ((L.route[q.first + (c16 < q.count ? c16 : q.count - 1u)] >> 16) * K + kq * 16u) * 2u;
     };
     struct Slab {
         u32x4_t w[NT][2];
-        uint32_t sc[NT], bi[NT];
+    };
+    // Scales and biases of two slabs with one request each: lane 2 r + h of a tile's 32 holds four of row r's from the 4 h-th on (or the
+    // stack's last four), at + i the i-th one's place in the row's line.  Two bytes a lane and tile, four requests a slab, they were a
+    // quarter of all requests and a CU issues one in 16 .. 20 cycles: 64 experts, pair of 1408 x 2048 int4, 48 routes 32.2 / 31.6 us, 96
+    // 43.8 / 42.7, 192 52.3 / 50.4, 576 64.1 / 60.9.
+    struct Meta {
+        u32x2_any_t s, b;
+        uint32_t at;
     };
     struct Acts {   // sixteen of the row's values, straight from memory: the rows are few and stay in the caches
         u32x4_t x[2];
@@ -218,14 +232,18 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
     // Straight-line requests: what lies past the wave's range is clamped to its last piece and never used.
     auto fetch_w = [&](const Piece& q, uint32_t slab, Slab& s) __attribute__((always_inline)) {
         const uint32_t g = g0 + slab * SG, gp = g + l8 / PPG, gc = gp < gl ? gp : gl, at = (gc * PPG + l8 % PPG) * 16u;
-        const uint32_t gm = g + (lane & 3u), gmc = (gm < gl ? gm : gl) >> a.gshift;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) s.w[t][h] = *reinterpret_cast<const u32x4_any_t*>(q.w[t] + (q.woff[t][h] + at));
-            s.sc[t] = *reinterpret_cast<const uint16_t*>(q.s[t] + (q.soff[t] + gmc * 2u));
-            s.bi[t] = *reinterpret_cast<const uint16_t*>(q.b[t] + (q.soff[t] + gmc * 2u));
         }
+    };
+    auto first_meta = [&](uint32_t slab) { return (g0 + slab * SG < gl ? g0 + slab * SG : gl) >> a.gshift; };   // of the two slabs from `slab` on
+    auto fetch_m = [&](const Piece& q, uint32_t slab, Meta& m) __attribute__((always_inline)) {
+        const int from = q.soff + (int)first_meta(slab), want = from + 4 * (int)(lane & 1u), at = want < q.slast ? want : q.slast;
+        m.s = *reinterpret_cast<const u32x2_any_t*>(q.s + at * 2);
+        m.b = *reinterpret_cast<const u32x2_any_t*>(q.b + at * 2);
+        m.at = (uint32_t)(4 + at - from);
     };
     auto fetch_x = [&](const Piece& q, uint32_t u, Acts& s) __attribute__((always_inline)) {   // the wave's u-th group
         const uint32_t g = g0 + u, gc = g < gl ? g : gl;
@@ -247,7 +265,7 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
     constexpr uint32_t MID2 = KIND == W_Q4 ? 0xC100C100u : 0xC300C300u;   // -MID as two bf16 values
     constexpr bool HALVES = KIND == W_Q8;
     const bf16x8_t mids = __builtin_bit_cast(bf16x8_t, make_uint4(MID2, MID2, MID2, MID2));
-    auto consume = [&](uint32_t u, const Acts& x) __attribute__((always_inline)) {   // group u of the parked slab
+    auto consume = [&](uint32_t u, uint32_t entry, const Acts& x) __attribute__((always_inline)) {   // group u of the parked slab, its pair
         const bf16x8_t xa0 = __builtin_bit_cast(bf16x8_t, x.x[0]), xa1 = __builtin_bit_cast(bf16x8_t, x.x[1]);
         // -MID * Sx, as the instructions take it (a power of two: exactly MID times what Sx would be)
         const f32x4_t m0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa0, mids, zero, 0, 0, 0);
@@ -270,7 +288,7 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
                 b0 = rt_unpack<KIND>(v.x, v.y);
                 b1 = rt_unpack<KIND>(v.z, v.w);
             }
-            const uint32_t sb = ml[((uint32_t)t * 16u + c16) * 4u + u];
+            const uint32_t sb = ml[((uint32_t)t * 16u + c16) * kRtMeta + entry];
             const float sf = bf16_lo(sb), bm = fmaf(bf16_hi(sb), -1.f / MID, -sf);   // (b + MID s) / -MID
             f32x4_t c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa0, b0, HALVES ? m0 : mx, 0, 0, 0);
             const f32x4_t c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa1, b1, HALVES ? m1 : c, 0, 0, 0);
@@ -282,13 +300,24 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
     Piece now, next;
     Slab w0, w1;
     Acts x0, x1;
+    Meta meta;
     uint32_t p = blockIdx.x;
     open(p, now);
+    fetch_m(now, 0u, meta);
     fetch_w(now, 0u, w0);
     fetch_x(now, 0u, x0);
     fetch_x(now, 1u, x1);
     fetch_w(now, 1u, w1);
+    // The waves of a CU's three workgroups go first in turn, a piece each: left to their age the third one's first piece was done 5 us
+    // after the first one's and its last so much later, the others' memory idle meanwhile (8 rows x 6 routes, below: 31.6 / 31.4 us; 96 rows
+    // 60.9 / 60.0).
+    uint32_t turn = blockIdx.x >> 8;
     while (true) {
+        switch (turn++ % 3u) {   // uniform
+            case 0: __builtin_amdgcn_s_setprio(0); break;
+            case 1: __builtin_amdgcn_s_setprio(1); break;
+            default: __builtin_amdgcn_s_setprio(2);
+        }
         const uint32_t pn = p + gridDim.x;
         const bool more = pn < pieces;   // uniform
         open(more ? pn : p, next);       // (the last piece asks for its own first slabs again)
@@ -302,7 +331,17 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
             for (int t = 0; t < NT; ++t) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) wl[((uint32_t)t * 16u + r8 + 8u * (uint32_t)h) * kRtLine + l8] = w.w[t][h];
-                ml[(uint32_t)t * 64u + lane] = w.sc[t] | (w.bi[t] << 16);
+            }
+            if constexpr (!SECOND) {
+                uint32_t* line = ml + (lane >> 1) * kRtMeta + meta.at;
+                line[0] = __builtin_amdgcn_perm(meta.b[0], meta.s[0], 0x05040100u);
+                line[1] = __builtin_amdgcn_perm(meta.b[0], meta.s[0], 0x07060302u);
+                line[2] = __builtin_amdgcn_perm(meta.b[1], meta.s[1], 0x05040100u);
+                line[3] = __builtin_amdgcn_perm(meta.b[1], meta.s[1], 0x07060302u);
+                if constexpr (LAST)
+                    fetch_m(next, 0u, meta);
+                else
+                    fetch_m(now, s + 2u, meta);
             }
             if constexpr (LAST)
                 fetch_w(next, SECOND ? 1u : 0u, w);
@@ -313,7 +352,7 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
             for (uint32_t j = 0; j < SG; ++j) {
                 const uint32_t u = s * SG + j;
                 Acts& x = j & 1u ? x1 : x0;
-                if (g0 + u < g1) consume(j, x);   // wave-uniform
+                if (g0 + u < g1) consume(j, 4u + ((g0 + u) >> a.gshift) - first_meta(SECOND ? s - 1u : s), x);   // wave-uniform
                 if (LAST && SECOND && j + 2u >= SG)
                     fetch_x(next, j + 2u - SG, x);
                 else
@@ -376,6 +415,7 @@ bool qgemm_takes_routed(const fk_weight* W, bool pair, uint32_t n_experts, uint3
     if ((W->bits != 4 && W->bits != 8) || (W->group != 64 && !(W->group == 128 && W->k % 128u == 0)) || W->k < 64u || W->k % 64u) return false;
     // 32-bit offsets: into the activations, into a tile's rows
     if ((uint64_t)n_x_rows * W->k * 2u > 0xffffffffull || (uint64_t)32u * W->k > 0xffffffffull || (uint64_t)n_experts * W->n > 0x7fffffffull) return false;
+    if ((uint64_t)n_experts * W->n * (W->k / W->group) < 4u) return false;   // four scales are asked for at a time
     const DeviceFacts* dev;
     return device_facts(&dev) == FK_OK && routes_served_together(n_experts, n_routes, W->n, W->k, W->bits, pair, (uint32_t)dev->cus);
 }

@@ -31,7 +31,8 @@ constexpr uint32_t rt_pieces_of_an_expert(uint32_t N, bool pair) { return pair ?
 //   2 experts, pair 512 x 512 int4:    2 .. 8 routes 5.5 .. 5.6 / 6.0 .. 6.3
 // Over 424 such points (2 .. 256 experts, K 256 .. 4096, both widths) the rule's choice was 0.6 % behind the better of the two on
 // average, 9 % at the worst that it sends together and 19 % (17 us) at the worst that it leaves; three quarters of a route per expert
-// alone: 4 % and 54 %.  (Timed before the products were centred, qgemm_routed.hip, which costs the form 0 .. 3 % near the line.)
+// alone: 4 % and 54 %.  (Timed before the products were centred, qgemm_routed.hip, which costs the form
+// 0 .. 3 % near the line, and before its scales came with fewer requests, which gives it 2 .. 6 %.)
 inline bool routes_served_together(uint32_t n_experts, uint32_t n_routes, uint32_t N, uint32_t K, uint32_t bits, bool pair, uint32_t cus) {
     if (4u * (uint64_t)n_routes < 3u * (uint64_t)n_experts) return false;
     const double touched = n_experts * (1.0 - exp(-(double)n_routes / n_experts));

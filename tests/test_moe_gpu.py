@@ -290,6 +290,13 @@ def test_routes_of_an_expert_served_together(fk, E, O, K, tokens, top_k, bits, g
     assert rel_l2(got, oracle.bf16_to_f32(ref)) <= REL_L2_BAR and bf16_mismatch(got, ref)[0] <= FLIP_FRACTION_BAR
 
 
+@pytest.mark.parametrize("E,O,K,tokens,top_k,bits,group", [(5, 1025, 64, 512, 2, 4, 64), (4, 2049, 128, 256, 4, 8, 128), (3, 1026, 128, 512, 2, 4, 64)])
+def test_routes_served_together_at_the_end_of_the_scales(fk, E, O, K, tokens, top_k, bits, group):
+    """The last tile of the last expert has one row or two, with one or two scales each: the four that are asked for at a time begin
+    before the tile."""
+    test_routes_of_an_expert_served_together(fk, E, O, K, tokens, top_k, bits, group)
+
+
 def _dequantized64(W):
     """code * scale + bias in 64 bits."""
     codes = (W.w[..., None] >> np.arange(0, 32, W.bits, dtype=np.uint32)) & np.uint32((1 << W.bits) - 1)
