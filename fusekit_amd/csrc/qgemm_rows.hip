@@ -16,8 +16,8 @@
 // values, a group's dot product is accumulated from zero in fp32 and folded as s * dot + b * Sx; Sx, the group's activation
 // sum, is one more matrix instruction per step against a B operand of ones, which leaves it in the very registers the fold
 // needs.
-// 37 rows of int4, one call in a chain, before (32 x 32 x 16 tiles, split-k sums, second kernel) / now: 896 x 896 12.8 / 3.4
-// us, 4864 x 896 pair 26.3 / 8.5, 896 x 4864 17.8 / 7.1, 2560 x 4096 19.8 / 9.9, 9728 x 2560 pair 53.0 / 27.7; 8 rows (a
+// 37 rows of int4, one call in a chain, before (32 x 32 x 16 tiles, split-k sums, second kernel) / now: 896 x 896 12.8 / 3.6
+// us, 4864 x 896 pair 26.3 / 6.9, 896 x 4864 17.8 / 7.0, 2560 x 4096 19.8 / 9.5, 9728 x 2560 pair 53.0 / 24.6; 8 rows (a
 // form of its own for 2..10 rows) 896 x 896 4.65 / 3.34, 2560 x 4096 8.80 / 6.2, 2560 x 9728 14.4 / 12.7.
 #include "fk_host.hpp"
 #include "gemv_kernel.hpp"
@@ -549,11 +549,7 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
     a.M = M; a.K = K; a.x_stride = x_stride; a.variant = rq.variant;
     a.n_seg = rq.pair ? 1u : rq.n_mats;
     a.gshift = W0->bits != 16 && W0->group == 128 ? 1u : 0u;
-    // Few blocks: the tiles of 16 activation rows go to blocks of their own (their weights come from the L2), which shortens
-    // what one block does (37 rows: 896 x 4864 12.5 -> 8.0 us, 896 x 896 5.0 -> 4.0, 2048 x 2048 7.6 -> 6.7).
     const uint32_t cus = (uint32_t)dev->cus, tiles = (M + 15u) / 16u;
-    const uint32_t m_blocks = tiles > 1u && b16 * tiles <= cus ? tiles : (tiles > 2u && b16 * 2u <= cus ? 2u : 1u);
-    const uint32_t mt = (tiles + m_blocks - 1u) / m_blocks;
     // Eight waves per block where the blocks do not fill the chip and K is deep enough for them; else four, of which two
     // blocks share a CU and cover each other's start (37 rows of int4, eight / four waves: 896 x 4864 12.1 / 13.3 us,
     // 2560 x 4096 11.1 / 12.1, 896 x 896 5.7 / 5.2, 4864 x 896 pair 14.0 / 9.7, 6144 x 2560 17.6 / 14.0).
@@ -561,7 +557,36 @@ fk_status plan_qgemm_rows(const RowsRequest& rq, Launch* out) {
     // Two tiles of weight rows per block -- half the blocks, each of which reads all activation rows -- once three or four
     // tiles of those make that traffic count (9728 x 2560: 37 rows 20.3 / 18.2 us with one / two, 12 rows 11.1 / 11.7; 64
     // rows of 6144 x 2560 17.0 / 15.5, but of 9728 x 2560 25.1 / 27.8: registers).  A pair has two tiles as it is.
-    const bool two = !rq.pair && b16 > cus && (mt == 3u || (mt == 4u && b16 <= 2u * cus));
+    auto two_of = [&](uint32_t mt) { return !rq.pair && b16 > cus && (mt == 3u || (mt == 4u && b16 <= 2u * cus)); };
+    auto blocks_of = [&](bool two) {
+        uint32_t n = 0;
+        for (uint32_t i = 0; i < a.n_seg; ++i) n += (a.n[i] + (two ? 31u : 15u)) / (two ? 32u : 16u);
+        return n;
+    };
+    // How many of the tiles of 16 activation rows a block takes (the other tiles' blocks read the weights again, from the L2): least work of
+    // the fullest CU, its blocks times a block's products and what its start takes of one (bf16 weights, which are not unpacked, as long as
+    // one; int4 something under half), and another half for each further reading of weights that the L2s do not hold.  All tiles in one
+    // block / this, us, int4: 37 rows of 896 x 4864 11.4 / 7.0, of 2560 x 9728 19.6 / 17.3, of 2560 x 4096 10.3 / 9.5, of the 4864 x 896 pair
+    // 8.6 / 6.9, 64 rows of it 10.1 / 7.7, of the 9728 x 2560 pair 29.4 / 25.8, of 6144 x 2560 16.6 / 13.8; int8, 64 rows of 6144 x 2560 19.1 /
+    // 14.1, 32 13.1 / 12.3 (17, the same tiles, 11.7 / 12.2), 37 of the 4864 x 896 pair 9.9 / 9.4.  On the line's other side, one block / more:
+    // 24 rows of the 9728 x 2560 pair 18.4 / 19.9, 37 of the 2816 x 2048 pair 8.7 / 9.3, 24 of 2560 x 4096 8.3 / 9.2; int8, 64 of 3072 x 2048
+    // 9.1 / 9.3; bf16, 64 of 3072 x 2048 8.6 / 9.2, 17 of 6144 x 2560 9.7 / 10.7.
+    const uint64_t weight_bytes = (uint64_t)b16 * 16u * (rq.pair ? 2u : 1u) * K / 8u * W0->bits;
+    const float reread = weight_bytes > (16ull << 20) ? 0.5f : 0.f, start = W0->bits == 4 ? 0.45f : (W0->bits == 8 ? 0.52f : 1.0f);
+    uint32_t mt = tiles, m_blocks = 1u;
+    float least = 1e30f;
+    for (uint32_t t = tiles; t >= 1u; --t) {
+        const uint32_t mb = (tiles + t - 1u) / t;   // (every block has rows)
+        const bool tw = two_of(t);
+        const float per_cu = (float)((blocks_of(tw) * mb + cus - 1u) / cus);
+        const float work = per_cu * ((float)(t * (tw ? 2u : 1u)) + start) + (float)(mb - 1u) * reread;
+        if (work < least) {
+            least = work;
+            mt = t;
+            m_blocks = mb;
+        }
+    }
+    const bool two = two_of(mt);
     uint32_t blocks = 0;
     for (uint32_t i = 0; i < a.n_seg; ++i) {
         a.blk0[i] = blocks;

@@ -197,6 +197,17 @@ def test_rows_of_a_short_k_are_requested_in_one_go(fk, bits, group, m, n, k):
         _check(normed[r], oracle.qgemv(W, xn, None), oracle.linear_acc(W, xn), W, xn)
 
 
+@pytest.mark.parametrize("bits,m,n", [
+    (4, 33, 4865),   # a block for each tile of 16 rows, the last one row deep, of either dimension
+    (4, 48, 6140),   # all rows in a block, of two tiles of weight rows (as a pair too)
+    (8, 64, 6140),   # two blocks of two tiles of rows
+    (4, 49, 6129),   # the same, the second with seventeen rows
+])
+def test_tiles_of_rows_that_share_a_block_or_not(fk, bits, m, n):
+    """More blocks than CUs: how many tiles of activation rows a block takes depends on what the fullest CU gets, the outputs do not."""
+    test_rows_of_a_short_k_are_requested_in_one_go(fk, bits, 64, m, n, 256)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("m", [9, 100])
 def test_qgemm_group_128(fk, bits, m):
