@@ -56,36 +56,30 @@ fk_status sdpa_workspace_bytes(uint32_t n_heads, uint32_t n_kv, uint32_t qk_dim,
 namespace {
 
 // The kernels by tile, cache and row form.  A bf16 cache has tiles of 1 and 2 heads (rows of up to 512 dims fit a wave, so that keys and
-// values always share their lanes); those of 4 and 8 belong to quantised caches.  The tile of 8 over a bf16 cache, which no shape takes, is
-// compiled all the same: without it the other kernels lie at other places, and a token behind 12000 positions of an 8-bit cache takes 1828
-// us instead of 1809.
+// values always share their lanes); those of 4 and 8 belong to quantised caches.
 template <int GT, int Q>
 const void* decode_func(int row) {
-    if constexpr (GT <= 4 || Q != 0) {
-        if (row == 16) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 16>);
-        if (row == 8) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 8>);
-    }
+    if (row == 16) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 16>);
+    if (row == 8) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 8>);
     return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 0>);
 }
 template <int GT, bool F, int Q>
 const void* fused_func(int row) {
-    if constexpr (GT <= 4 || Q != 0) {
-        if (row == 16) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 16>);
-        if (row == 8) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 8>);
-    }
+    if (row == 16) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 16>);
+    if (row == 8) return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 8>);
     return reinterpret_cast<const void*>(&sdpa_rope_store_kernel<GT, F, Q, 0>);
 }
 template <int Q>
 const void* decode_func(int gt, int row) {
     if constexpr (Q != 0)
-        if (gt == 4) return decode_func<4, Q>(row);
-    return gt == 1 ? decode_func<1, Q>(row) : (gt == 2 ? decode_func<2, Q>(row) : decode_func<8, Q>(row));
+        if (gt >= 4) return gt == 4 ? decode_func<4, Q>(row) : decode_func<8, Q>(row);
+    return gt == 1 ? decode_func<1, Q>(row) : decode_func<2, Q>(row);
 }
 template <bool F, int Q>
 const void* fused_tile(int gt, int row) {
     if constexpr (Q != 0)
-        if (gt == 4) return fused_func<4, F, Q>(row);
-    return gt == 1 ? fused_func<1, F, Q>(row) : (gt == 2 ? fused_func<2, F, Q>(row) : fused_func<8, F, Q>(row));
+        if (gt >= 4) return gt == 4 ? fused_func<4, F, Q>(row) : fused_func<8, F, Q>(row);
+    return gt == 1 ? fused_func<1, F, Q>(row) : fused_func<2, F, Q>(row);
 }
 template <int Q>
 const void* fused_func(bool fast, int gt, int row) { return fast ? fused_tile<true, Q>(gt, row) : fused_tile<false, Q>(gt, row); }
@@ -236,7 +230,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     // with the scales alone, 30.1 / 28.2)
     const bool alike = qk_dim == v_dim && (!kvq || quant->group == 64);
     const bool words = !kvq || (((uintptr_t)quant->k_scales | (uintptr_t)quant->k_biases | (uintptr_t)quant->v_scales | (uintptr_t)quant->v_biases) & 3u) == 0;
-    const int row = gt > 4 && !kvq ? 0 : (alike && qk_dim == 128 && words ? 16 : (alike && qk_dim == 64 ? 8 : 0));
+    const int row = alike && qk_dim == 128 && words ? 16 : (alike && qk_dim == 64 ? 8 : 0);
     const void* func = nullptr;
     if (fusion) {
         // whole-width rotation of at most 128 dims with a table: the form whose loads run ahead

@@ -978,6 +978,83 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // (the head is the same for the whole wave, which the compiler has to be told: the rows' addresses then are scalars)
     for (uint32_t h = __builtin_amdgcn_readfirstlane(wave); h < gcount; h += kSdpaWaves) {
         const float* ph = a.partials + (size_t)(h0 + h) * a.n_splits * row;
+        if constexpr (ROW != 0 && MODE != 1) {
+            // Heads of 128 (64) dims: sixteen (eight) bytes a lane, two ranges a load -- half the loads, of which a CU issues one in 16 .. 20
+            // cycles --, which the half-waves then exchange: lanes l and l + 32 hold dims 4 l, 4 l + 1 and 4 l + 2, 4 l + 3 (both 2 l, 2 l + 1) of
+            // every range.  The same additions in the same order.  8-bit caches, us, one range a load / two: 32 q / 8 kv heads x 128, 480
+            // positions 11.5 / 10.5, 12000 24.5 / 23.2; 14 / 2 x 128, 480 17.5 / 14.3, 32000 67 / 49.
+            constexpr uint32_t VD = ROW * 8u, LINE = (VD + 2u) * 4u, WL = ROW == 16 ? 4u : 2u;   // dims, bytes of a partial, words of a lane
+            const __amdgpu_buffer_rsrc_t parts = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ph), 0, (int)(a.n_splits * LINE), 0x27000);
+            typedef uint32_t words2 __attribute__((ext_vector_type(2)));
+            typedef uint32_t words __attribute__((ext_vector_type(WL)));
+            constexpr int kPast = 1 << 4;   // sc1: past every cache that blocks do not share
+            const uint32_t own = 8u + (lane & 31u) * (4u * WL);
+            float M = -INFINITY, L = 0.f, o0 = 0.f, o1 = 0.f;
+            auto fetch = [&](uint32_t base, words2& ml, words(&po)[kBatch / 2]) {
+                const uint32_t first = base < ranges ? base : 0u, mine = base + (lane & (kBatch - 1));
+                ml = __builtin_bit_cast(words2, __builtin_amdgcn_raw_buffer_load_b64(parts, (int)((mine < ranges ? mine : first) * LINE), 0, kPast));
+#pragma unroll
+                for (uint32_t i = 0; i < kBatch / 2; ++i) {
+                    const uint32_t r = base + 2u * i + (lane >> 5);
+                    const int at = (int)((r < ranges ? r : first) * LINE + own);
+                    if constexpr (ROW == 16)
+                        po[i] = __builtin_bit_cast(words, __builtin_amdgcn_raw_buffer_load_b128(parts, at, 0, kPast));
+                    else
+                        po[i] = __builtin_bit_cast(words, __builtin_amdgcn_raw_buffer_load_b64(parts, at, 0, kPast));
+                }
+            };
+            auto fold = [&](uint32_t base, const words2& ml, const words(&po)[kBatch / 2]) {
+                const float m_mine = __uint_as_float(ml[0]);
+                float mx = dpp_max<0xB1>(m_mine);
+                mx = dpp_max<0x4E>(mx);
+                mx = dpp_max<0x141>(mx);
+                mx = dpp_max<0x140>(mx);
+                const float mn = fmaxf(M, mx);
+                const float w_mine = base + (lane & (kBatch - 1)) < ranges ? expf(m_mine - mn) : 0.f;
+                const float alpha = base ? expf(M - mn) : 0.f;
+                L *= alpha;
+                o0 *= alpha;
+                o1 *= alpha;
+#pragma unroll
+                for (uint32_t i = 0; i < kBatch; i += 2) {
+                    const auto x0 = __builtin_amdgcn_permlane32_swap(po[i / 2][0], po[i / 2][WL - 2u], false, false);
+                    const auto x1 = __builtin_amdgcn_permlane32_swap(po[i / 2][1], po[i / 2][WL - 1u], false, false);
+#pragma unroll
+                    for (uint32_t e = 0; e < 2; ++e) {
+                        const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_mine), i + e));
+                        const float pl = __int_as_float(__builtin_amdgcn_readlane((int)ml[1], i + e));
+                        L = fmaf(pl, w, L);
+                        o0 = fmaf(__uint_as_float(x0[e]), w, o0);
+                        o1 = fmaf(__uint_as_float(x1[e]), w, o1);
+                    }
+                }
+                M = mn;
+            };
+            auto merge = [&](auto n_const, uint32_t base) {
+                constexpr uint32_t N = decltype(n_const)::value;
+                words2 ml[N];
+                words po[N][kBatch / 2];
+#pragma unroll
+                for (uint32_t b = 0; b < N; ++b) fetch(base + b * kBatch, ml[b], po[b]);
+#pragma unroll
+                for (uint32_t b = 0; b < N; ++b)
+                    if (base + b * kBatch < ranges) fold(base + b * kBatch, ml[b], po[b]);
+            };
+            if (ranges <= kBatch) {
+                merge(std::integral_constant<uint32_t, 1>{}, 0u);
+            } else if (ranges <= 2 * kBatch) {
+                merge(std::integral_constant<uint32_t, 2>{}, 0u);
+            } else {
+                for (uint32_t base = 0; base < ranges; base += 4 * kBatch) merge(std::integral_constant<uint32_t, 4>{}, base);
+            }
+            const float inv_l = 1.0f / L;
+            if (ROW == 16 || lane < 32u) {
+                uint16_t* dst = a.out + (size_t)(h0 + h) * VD + (ROW == 16 ? 4u * (lane & 31u) + 2u * (lane >> 5) : 2u * lane);
+                st_u16<FUSED>(dst, f32_to_bf16_bits(o0 * inv_l));
+                st_u16<FUSED>(dst + 1, f32_to_bf16_bits(o1 * inv_l));
+            }
+            continue;
+        }
         for (uint32_t d2 = lane; d2 < ((a.v_dim >> 1) + kWave - 1) / kWave * kWave; d2 += kWave) {
             const bool live = d2 < (a.v_dim >> 1);
             const uint32_t at = 2u + 2u * (live ? d2 : 0u);

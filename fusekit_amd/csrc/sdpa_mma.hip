@@ -544,6 +544,12 @@ bool sdpa_takes_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v, con
     // 4.9 / 4.9, 256 6.8 / 6.6, 8 rows at 100 4.3 / 6.6, 64 rows at 100 14.7 / 8.1; 14 / 2 x 64, 128 positions 4.1 / 4.1, 256 5.1 / 4.5; 16 heads of
     // 192 / 128, 8 rows at 30 5.4 / 6.1, 2 rows at 100 7.6 / 6.2).
     if (max_len <= (qk_dim == 192 ? 64u : 192u) && (uint64_t)n_heads * rows <= 512u) return false;
+    // One row of 128 dims beyond the one round of a block: the partials' count and merge come with either form, and groups of more than four heads
+    // (tiles of 8) or few heads leave this one the longer chain until some 700 positions (warm, that / this: 14 / 2 heads, 300 7.5 / 7.8, 480
+    // 7.8 / 8.2, 1000 9.0 / 8.5; 28 / 4, 480 8.0 / 8.3, 1000 8.8 / 8.6; 56 / 8, 300 7.9 / 8.2, 480 8.4 / 8.4; 8 / 1, 1000 7.9 / 8.5; 8 / 2, 300 7.1 / 7.6, 480
+    // 7.3 / 7.3, 1000 7.9 / 7.6; 16 / 4, 300 7.4 / 7.8, 480 7.9 / 7.4).
+    const uint32_t group = n_heads / n_kv, chain = group > 4u ? (n_heads <= 8u ? 1152u : (n_heads <= 32u ? 704u : 416u)) : (n_heads < 16u ? 704u : (n_heads == 16u ? 384u : 256u));
+    if (qk_dim == 128 && rows == 1 && max_len > 256u && max_len <= chain) return false;
     // (partials are addressed with 32 bits)
     return (uint64_t)rows * n_heads * kMmaMaxSplits * (v_dim + 2u) * 4u < 0x7fffffffull;
 }
@@ -573,7 +579,8 @@ fk_status plan_sdpa_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v,
     // L2, half of that where they come from memory; partials, their count and their merge take 2.2 us.  Cold caches, us: 64 dims (256
     // positions a round), one block / several, 544 positions 5.5 / 6.2, 1024 6.5 / 6.5 (16 / 8 heads 6.4 / 6.4, 8.1 / 6.5).  One row of 128 dims: at
     // 256 positions one round of 8 waves 6.6, two of 4 7.4; beyond, 32 KB a wave in fewer CUs is the slower, until the rounds are many:
-    // 8 / 4 waves, 512 8.5 / 7.4, 1024 8.6 / 7.8, 2048 8.9 / 8.5, 4096 9.9 / 10.1, 12000 14.6 / 14.9.  Several rows share what is drawn: 8 of them
+    // 8 / 4 waves, 512 8.5 / 7.4, 1024 8.6 / 7.8, 2048 8.9 / 8.5, 4096 9.9 / 10.1, 12000 14.6 / 14.9; tiles of 8 are the slower with 4 at every
+    // length (warm, 14 / 2 heads, 480 8.2 / 9.7, 2500 8.5 / 10.7).  Several rows share what is drawn: 8 of them
     // at 500 positions, 8 waves in one block 8.6, 4 in four 9.2.  (Two steps of a wave in flight at half the waves: 64 dims 544 5.8, 12000 8.5.)
     uint32_t nw = 8, alone = rows > 1 ? 2u : 1u;
     if (qk_dim == 64) {
@@ -585,10 +592,9 @@ fk_status plan_sdpa_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v,
             nw = 4;
             alone = 4;
             FK_TRY((fill<128, 128, 16, 4, false>(l)));
-        } else if (rows == 1 && max_len > 256u && max_len <= 3072u) {
+        } else if (rows == 1 && qt == 4u && max_len > 256u && max_len <= 3072u) {
             nw = 4;
-            if (fusion) FK_TRY(qt == 4 ? (fill<128, 128, 4, 4, true>(l)) : (fill<128, 128, 8, 4, true>(l)));
-            else FK_TRY(qt == 4 ? (fill<128, 128, 4, 4, false>(l)) : (fill<128, 128, 8, 4, false>(l)));
+            FK_TRY(fusion ? (fill<128, 128, 4, 4, true>(l)) : (fill<128, 128, 4, 4, false>(l)));
         } else {
             if (fusion) FK_TRY(qt == 4 ? (fill<128, 128, 4, 8, true>(l)) : (fill<128, 128, 8, 8, true>(l)));
             else FK_TRY(qt == 4 ? (fill<128, 128, 4, 8, false>(l)) : (fill<128, 128, 8, 8, false>(l)));
