@@ -233,6 +233,14 @@ def test_attention_of_64_dims_against_the_oracle_and_the_general_form(fk, bits, 
         assert np.max(np.abs(oracle.bf16_to_f32(got[0][r]) - want)) <= 2.0 ** -6 * np.max(np.abs(want))
 
 
+@pytest.mark.parametrize("ranges", [2, 16, 17, 32, 33, 64, 65])
+def test_merge_of_any_number_of_ranges(fk, ranges):
+    """One head, a range a block: odd and even numbers of partials, at the edges of the sixteens and of the sixty-four that the merge asks
+    for together; the last range holds one key."""
+    test_attention_of_128_dims_equals_the_general_form_bit_for_bit(fk, 8, 1, 1, 64 * (ranges - 1) + 1, 64 * ranges, 1)
+    test_attention_of_64_dims_against_the_oracle_and_the_general_form(fk, 4, 1, 1, 128 * (ranges - 1) + 1, 128 * ranges, 1)
+
+
 def test_rejects_bad_geometry(fk):
     K, V = _caches(fk, 2, 16, 128, 4, 64)
     k = _dev(fk, normal_bf16(1, 256))
