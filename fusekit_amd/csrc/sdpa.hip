@@ -1,5 +1,7 @@
-// GQA scaled-dot-product attention for one new token over a bf16 KV cache
-// (split-K "flash decoding"), gfx950.
+// GQA scaled-dot-product attention for one new token over a KV cache
+// (split-K "flash decoding"), gfx950, on vector instructions: quantised caches, and bf16
+// caches where sdpa_mma.hip's form, which plan_sdpa_decode asks first, does not serve them
+// (short contexts, widths other than 64, 128 and 192 / 128, rows that are not 16-byte aligned).
 //
 // Grid (splits, kv heads, head tiles).  A block owns one KV head, one range of
 // `chunk_len` cache positions and up to GT query heads of that KV head's group,
