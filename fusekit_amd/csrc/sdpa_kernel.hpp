@@ -978,7 +978,7 @@ __device__ __forceinline__ void sdpa_block(const ARGS& a, uint32_t kv_raw, uint3
     // (the head is the same for the whole wave, which the compiler has to be told: the rows' addresses then are scalars)
     for (uint32_t h = __builtin_amdgcn_readfirstlane(wave); h < gcount; h += kSdpaWaves) {
         const float* ph = a.partials + (size_t)(h0 + h) * a.n_splits * row;
-        if constexpr (ROW != 0 && MODE != 1) {
+        if constexpr ((KVQ != 0 ? ROW != 0 : ROW == 16) && MODE != 1) {
             // Heads of 128 (64) dims: sixteen (eight) bytes a lane, two ranges a load -- half the loads, of which a CU issues one in 16 .. 20
             // cycles --, which the half-waves then exchange: lanes l and l + 32 hold dims 4 l, 4 l + 1 and 4 l + 2, 4 l + 3 (both 2 l, 2 l + 1) of
             // every range.  The same additions in the same order.  8-bit caches, us, one range a load / two: 32 q / 8 kv heads x 128, 480

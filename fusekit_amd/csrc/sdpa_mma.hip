@@ -17,7 +17,7 @@
 // The form on vector instructions (sdpa_kernel.hpp: quantised caches, other widths, short contexts) spends about 110 of them on a lane's 8
 // dims of a key for 4 heads; here the products cost none and a step's softmax about 100 for 32 keys of a whole tile, so that what remains is
 // the bytes, the start and, where blocks share a context, the 2.2 us of partials, count and merge.  That form -> this, us, launch to launch
-// in a graph, caches from memory: 32 / 8 heads x 128 at 512 positions 7.6 -> 7.4, 1024 8.9 -> 7.8, 4096 13.3 -> 9.9, 12000 21.3 -> 14.6, 32768 37 ->
+// in a graph, caches from memory: 32 / 8 heads x 128 at 1024 positions 8.9 -> 7.8, 4096 13.3 -> 9.9, 12000 21.3 -> 14.6, 32768 37 ->
 // 28.1 (134 MB: 4.8 TB/s of the 5.8 that a plain read reaches); 14 / 2 x 64 at 544 6.9 -> 5.5, 4096 10.0 -> 6.9, 12000 13.0 -> 8.4; 64 rows of
 // 32 / 8 x 128 at 500 33 -> 9.6; 16 heads of 192 / 128, 8 rows at 480 12.6 -> 10.8, 96 rows at 1500 141 -> 19.4.
 #include "dma_device.hpp"
@@ -566,12 +566,14 @@ bool sdpa_takes_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v, con
     // 4.9 / 4.9, 256 6.8 / 6.6, 8 rows at 100 4.3 / 6.6, 64 rows at 100 14.7 / 8.1; 14 / 2 x 64, 128 positions 4.1 / 4.1, 256 5.1 / 4.5; 16 heads of
     // 192 / 128, 8 rows at 30 5.4 / 6.1, 2 rows at 100 7.6 / 6.2).
     if (max_len <= (qk_dim == 192 ? 64u : 192u) && (uint64_t)n_heads * rows <= 512u) return false;
-    // One row of 128 dims beyond the one round of a block: the partials' count and merge come with either form, and groups of more than four heads
-    // (tiles of 8) or few heads leave this one the longer chain until some 700 positions (warm, that / this: 14 / 2 heads, 300 7.5 / 7.8, 480
-    // 7.8 / 8.2, 1000 9.0 / 8.5; 28 / 4, 480 8.0 / 8.3, 1000 8.8 / 8.6; 56 / 8, 300 7.9 / 8.2, 480 8.4 / 8.4; 8 / 1, 1000 7.9 / 8.5; 8 / 2, 300 7.1 / 7.6, 480
-    // 7.3 / 7.3, 1000 7.9 / 7.6; 16 / 4, 300 7.4 / 7.8, 480 7.9 / 7.4).
-    const uint32_t group = n_heads / n_kv, chain = group > 4u ? (n_heads <= 8u ? 1152u : (n_heads <= 32u ? 704u : 416u)) : (n_heads < 16u ? 704u : (n_heads == 16u ? 384u : 256u));
-    if (qk_dim == 128 && rows == 1 && max_len > 256u && max_len <= chain) return false;
+    // One row of 128 dims beyond the one round of a block: the partials, their count and their merge come with either form, and the vector form's
+    // blocks, four times as many, have the shorter way until a block of it walks two or three ranges (caches from memory, that / this: 32 / 8
+    // heads, 300 positions 5.5 / 6.5, 700 6.9 / 7.0, 900 7.4 / 7.2; 16 / 4, 600 6.4 / 6.5, 700 6.6 / 6.5; 8 / 2, 900 6.0 / 6.4, 1500 7.0 / 6.4; a head a
+    // KV head, 8, 1100 7.0 / 7.2, 1500 7.8 / 7.5; groups of more than four, whose tiles of 8 this form fills in part: 14 / 2, 1500 7.4 / 7.9, 2100 9.0 / 8.7;
+    // 32 / 4, 1500 8.5 / 9.0, 2100 9.5 / 9.1; 56 / 8, 1100 8.9 / 9.0, 1500 9.6 / 9.1).
+    const uint32_t group = n_heads / n_kv;
+    const uint32_t line = group > 4u ? (n_heads <= 32u ? 1792u : 1088u) : (group == 1u ? 1280u : (n_heads <= 8u ? 1024u : 704u));
+    if (qk_dim == 128 && rows == 1 && max_len > 256u && max_len <= line) return false;
     // (partials are addressed with 32 bits)
     return (uint64_t)rows * n_heads * kMmaMaxSplits * (v_dim + 2u) * 4u < 0x7fffffffull;
 }
