@@ -320,6 +320,7 @@ def test_rope_store_sdpa_rejects_bad_arguments(fk):
 @pytest.mark.parametrize("n_heads,n_kv,qk,vd,rows,kv_len", [
     (8, 8, 64, 64, 1, 193), (6, 2, 64, 64, 1, 256), (10, 2, 64, 64, 1, 257), (24, 2, 64, 64, 1, 769),       # groups of 1, 3, 5 and 12; round edges
     (32, 8, 128, 128, 1, 255), (3, 1, 128, 128, 1, 512), (7, 1, 128, 128, 1, 513), (16, 1, 128, 128, 1, 4097),
+    (32, 8, 128, 128, 1, 705), (3, 1, 128, 128, 1, 1025), (7, 1, 128, 128, 1, 1793), (56, 8, 128, 128, 1, 1089),   # one past the vector form's lines
     (2, 1, 64, 64, 1, 9000), (5, 1, 128, 128, 1, 33000),                                                      # merges of up to 64 partials
     (14, 2, 64, 64, 3, 200), (32, 8, 128, 128, 2, 223), (64, 2, 64, 64, 13, 500), (128, 8, 128, 128, 17, 300),  # tiles of 8 and of 16, last ones not full
     (16, 16, 192, 128, 2, 30), (16, 16, 192, 128, 8, 225), (4, 2, 192, 128, 9, 700), (64, 64, 192, 128, 33, 128),
