@@ -608,9 +608,10 @@ fk_status plan_sdpa_d(const Dispatch& d, Launch* l, SlotRW* rw) {
     FK_TRY(need_bytes(d, 6, cb * rows));
     rw->reads = {0, 1, 2, 3, 5, 6};
     rw->writes = {4, 5, 6};
+    // (token: a member of the whole-token kernel, whose attention phase is the form on vector instructions)
     return plan_sdpa_decode(arg_ptr<const uint16_t>(d, 0), arg_ptr<const uint16_t>(d, 1), arg_ptr<const uint16_t>(d, 2),
                             arg_ptr<uint16_t>(d, 4), arg_ptr<const uint32_t>(d, 3), 0, max_len, n_heads, n_kv, qk, vd,
-                            capacity, scale, arg_ptr<float>(d, 5), arg_ptr<uint32_t>(d, 6), l, rows);
+                            capacity, scale, arg_ptr<float>(d, 5), arg_ptr<uint32_t>(d, 6), l, rows, nullptr, nullptr, d.u("token", 0) != 0);
 }
 
 // Q, K, V, out: causal attention of `rows` token rows (sdpa_prefill.rs:11-21).  The reference binds
@@ -1603,6 +1604,15 @@ fk_status plan_dispatch(const Dispatch& d, Launch* l, SlotRW* rw) {
     return f->plan(d, l, rw);
 }
 
+// The argument block a member of a fused run or of the whole-token kernel contributes to its device tables: the dispatch planned
+// once more with the parameter `token` (the one launch sizes some tiles differently, and has one form of the attention).
+fk_status plan_for_token(const Dispatch& d, Launch* l) {
+    Dispatch t = d;
+    t.params.emplace_back("token", 1.0);
+    SlotRW rw;
+    return plan_dispatch(t, l, &rw);
+}
+
 fk_status copy_dispatch(const fk_dispatch& in, Dispatch* out) {
     if (!in.kernel) return set_error(FK_ERR_INVALID, "dispatch without a kernel name");
     if ((in.n_args && !in.args) || (in.n_params && !in.params)) return set_error(FK_ERR_INVALID, "null args / params");
@@ -1803,11 +1813,6 @@ bool is_family(const Node& n, const char* prefix) {
     return f && strcmp(f->prefix, prefix) == 0;
 }
 
-template <typename T>
-const T& blob(const Node& n) {
-    return *reinterpret_cast<const T*>(n.launch.args);
-}
-
 fk_status build_token_kernel(std::vector<Node>& nodes, uint32_t spin_limit, Graph* g) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
@@ -1876,13 +1881,20 @@ fk_status build_token_kernel(std::vector<Node>& nodes, uint32_t spin_limit, Grap
     if (layers.empty()) return bad("no layers");
     const uint32_t bits = nodes[layers[0].qkv].d.u("bits", 4);
     const int kind = bits == 4 ? W_Q4 : (bits == 8 ? W_Q8 : W_BF16);
-    const SdpaArgs& s0 = blob<SdpaArgs>(nodes[layers[0].sdpa]);
+    std::vector<SdpaArgs> sdpa(layers.size());
+    for (size_t li = 0; li < layers.size(); ++li) {
+        Launch l;
+        FK_TRY(plan_for_token(nodes[layers[li].sdpa].d, &l));
+        const SdpaArgs* s = l.args_as<SdpaArgs>();
+        if (!s) return bad("an attention that the kernel has no phase for");
+        sdpa[li] = *s;
+    }
+    const SdpaArgs s0 = sdpa[0];
     const uint32_t G = s0.n_heads / s0.n_kv;
     const int gt = G >= 8 ? 8 : (G >= 4 ? (G == 4 ? 4 : 8) : (G >= 2 ? (G == 2 ? 2 : 4) : 1));
     if (gt == 1) return bad("one query head per kv head");
 
     std::vector<GemvArgs> gemv(4 * layers.size() + 1);
-    std::vector<SdpaArgs> sdpa(layers.size());
     uint32_t grid = (uint32_t)dev->cus * 4, lds_max = 0;
     for (int pass = 0; pass < 3; ++pass) {
         t_gemv_grid_override = grid;
@@ -1893,7 +1905,8 @@ fk_status build_token_kernel(std::vector<Node>& nodes, uint32_t spin_limit, Grap
             SlotRW rw;
             fk_status r = plan_dispatch(nodes[node].d, &l, &rw);
             if (r != FK_OK) return r;
-            *out = *reinterpret_cast<const GemvArgs*>(l.args);
+            if (!l.args_as<GemvArgs>()) return bad("a projection that the kernel has no phase for");
+            *out = *l.args_as<GemvArgs>();
             lds_max = std::max(lds_max, l.shmem);
             return FK_OK;
         };
@@ -1927,12 +1940,14 @@ fk_status build_token_kernel(std::vector<Node>& nodes, uint32_t spin_limit, Grap
 
     for (size_t li = 0; li < layers.size(); ++li) {
         const LayerIdx& L = layers[li];
-        SdpaArgs s = blob<SdpaArgs>(nodes[L.sdpa]);
+        SdpaArgs& s = sdpa[li];
         if (s.kv_len_ptr != t.kv_len) return bad("sdpa does not read the step counter's kv_len");
         if (s.n_heads / s.n_kv != G || s.qk_dim != s0.qk_dim || s.v_dim != s0.v_dim) return bad("layers differ in head layout");
         if (s.qk_dim != s.v_dim) return bad("qk_dim != v_dim");
-        const RopeArgs& r0 = blob<RopeArgs>(nodes[L.rope0]);
-        const RopeArgs& r1 = blob<RopeArgs>(nodes[L.rope1]);
+        if (!nodes[L.rope0].launch.args_as<RopeArgs>() || !nodes[L.rope1].launch.args_as<RopeArgs>())
+            return bad("a rope / KV-store task that the kernel has no phase for");
+        const RopeArgs& r0 = *nodes[L.rope0].launch.args_as<RopeArgs>();
+        const RopeArgs& r1 = *nodes[L.rope1].launch.args_as<RopeArgs>();
         if (r0.offset_ptr != t.offset || r1.offset_ptr != t.offset) return bad("rope does not read the step counter's offset");
         if (r1.write_offset_ptr && r1.write_offset_ptr != t.offset) return bad("cache row is not the rope position");
         if (r0.q != s.q) return bad("sdpa does not read the rope task's q");
@@ -1956,7 +1971,6 @@ fk_status build_token_kernel(std::vector<Node>& nodes, uint32_t spin_limit, Grap
         s.rope_dims = r0.rope_dims;
         s.eps = r0.eps;
         s.base_log2 = r0.base_log2;
-        sdpa[li] = s;
     }
 
     // Private activation arena: every layer gets its own x / q / k / v / att / mid
@@ -2208,15 +2222,6 @@ fk_status fk_plan_geometry(fk_handle h, const fk_dispatch* d, fk_launch_geometry
     for (uint32_t s : rw.reads) out->slot_access[s] |= 1;
     for (uint32_t s : rw.writes) out->slot_access[s] |= 2;
     return FK_OK;
-}
-
-// The argument block a member of a fused run contributes to the run's device tables: the dispatch planned once
-// more with the parameter `token` (the one launch sizes some tiles differently).
-fk_status plan_for_token(const Dispatch& d, Launch* l) {
-    Dispatch t = d;
-    t.params.emplace_back("token", 1.0);
-    SlotRW rw;
-    return plan_dispatch(t, l, &rw);
 }
 
 bool is_family(const Dispatch& d, const char* fam) {

@@ -13,11 +13,15 @@
 
 namespace fk {
 
+template <typename T>
+inline char kArgsType = 0;   // its address names T
+
 struct Launch {
     const void* func = nullptr;
     dim3 grid{1, 1, 1}, block{1, 1, 1};
     uint32_t shmem = 0;
     size_t args_size = 0;
+    const void* args_type = nullptr;   // which struct `args` holds
     alignas(16) unsigned char args[896];
     // Kernels that complete the same operation and must run after this one, in
     // order (a split-k reduction, a routed reduction).  run_launch and the graph
@@ -36,6 +40,12 @@ struct Launch {
         static_assert(sizeof(T) <= sizeof(args), "argument block too large");
         memcpy(args, &a, sizeof(T));
         args_size = sizeof(T);
+        args_type = &kArgsType<T>;
+    }
+    // The argument block as a T, or null where this launch holds another struct: one dispatch may be planned onto several kernels.
+    template <typename T>
+    const T* args_as() const {
+        return args_type == &kArgsType<T> ? reinterpret_cast<const T*>(args) : nullptr;
     }
     template <typename T>
     void add_lead(T v) {
@@ -361,7 +371,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
                            const uint32_t* kv_len_ptr, uint32_t kv_len_imm, uint32_t max_len, uint32_t n_heads,
                            uint32_t n_kv, uint32_t qk_dim, uint32_t v_dim, uint32_t capacity, float scale,
                            float* partials, uint32_t* counters, Launch* out_launch, uint32_t rows = 1,
-                           const KvQuant* quant = nullptr, const SdpaFusion* fusion = nullptr);
+                           const KvQuant* quant = nullptr, const SdpaFusion* fusion = nullptr, bool vector_form = false);
 // The matrix-core form of it (sdpa_mma.hip): the shapes and pointers that it takes, and its launch.
 bool sdpa_takes_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* out, uint32_t n_heads, uint32_t n_kv,
                     uint32_t qk_dim, uint32_t v_dim, uint32_t max_len, uint32_t rows, const float* partials, const uint32_t* counters,

@@ -256,6 +256,16 @@ def test_persistent_kernel_tokens_match_oracle(fk, bits, qk_norm, bias, fuse, he
         assert g == r, f"step {i}: gpu {g} oracle {r} (oracle margin {margins[i]})"
 
 
+@pytest.mark.parametrize("capacity,head_dim", [(192, 64), (193, 64), (256, 64), (1024, 64), (256, 128), (512, 128), (1024, 128)])
+def test_persistent_kernel_at_the_capacities_that_decode_uses(fk, capacity, head_dim):
+    """The kernel has one form of the attention at every capacity; the task list's own launch has another one beyond some lines."""
+    cfg = _small_cfg(bits=4, qk_norm=True, capacity=capacity, head_dim=head_dim, hidden=4 * head_dim, n_layers=2)
+    got, ref, margins, rt = _run_pair(fk, cfg, seed=4, persistent=True)
+    assert rt.d.graph_launch_shape(rt.graph)[0]
+    for i, (g, r) in enumerate(zip(got, ref)):
+        assert g == r, f"step {i}: gpu {g} oracle {r} (oracle margin {margins[i]})"
+
+
 def test_persistent_kernel_matches_task_graph_state(fk):
     """Same tokens, same KV-cache contents and same logits as the one-node-per-task graph."""
     from fusekit_amd.decoder import DecoderRuntime, DecoderWeights
