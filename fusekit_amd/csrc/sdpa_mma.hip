@@ -186,8 +186,9 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
     if (ahead) issue_k(first);
     uint32_t kv_raw = a.kv_len_imm;
     if (a.kv_len_ptr) kv_raw = *(const __attribute__((address_space(4))) uint32_t*)(uintptr_t)a.kv_len_ptr;
+    const uint32_t kv0_len = kv_raw > covered ? covered : kv_raw;   // (before a row is added: a tile's rows stay in order whatever was read)
     auto limit_of = [&](uint32_t row) {
-        const uint32_t l = kv_raw + row;
+        const uint32_t l = kv0_len + row;
         return l < 1u ? 1u : (l > covered ? covered : l);
     };
     const uint32_t lim_hi = limit_of(row_hi), lim_lo = limit_of(row_lo), q_limit = limit_of((e0 + mine) / G);

@@ -374,3 +374,21 @@ def test_sdpa_length_on_the_device_of_a_longer_plan(fk, n_heads, n_kv, dim, leng
     assert (got[:, 5] == 0x7F80).all()
     keep = np.arange(dim) != 5
     assert rel_l2(got[:, keep].ravel(), oracle.bf16_to_f32(ref.reshape(n_heads, dim)[:, keep].ravel())) <= 3e-3
+
+
+@pytest.mark.parametrize("given", [0xFFFFFFFF, 0xFFFFFFFE, 5000])
+def test_sdpa_rows_with_a_length_on_the_device_beyond_the_plan(fk, given):
+    """Rows of a group and a device length beyond the plan, up to the last of 32 bits: every row takes the plan's end."""
+    from fusekit_amd.runtime import Dispatch, Dispatcher, arg
+    rows, n_heads, n_kv, dim, cap = 3, 14, 2, 64, 700
+    q = np.repeat(normal_bf16(41, (1, n_heads * dim)), rows, 0)
+    ck, cv = normal_bf16(42, n_kv * cap * dim), normal_bf16(43, n_kv * cap * dim)
+    pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, dim, dim, cap)
+    bufs = [fk.DeviceBuffer.from_numpy(a) for a in (q, ck, cv, np.array([given], np.uint32))]
+    out, part, cnt = fk.DeviceBuffer(q.nbytes), fk.DeviceBuffer(pb * rows), fk.zeros(cb * rows)
+    Dispatcher().dispatch_kernel(Dispatch("fusekit_sdpa_decode_f0", [arg(b) for b in bufs + [out, part, cnt]],
+                                          {"n_heads": n_heads, "n_kv": n_kv, "head_dim": dim, "capacity": cap, "rows": rows}))
+    got = out.to_numpy(np.uint16, (rows, n_heads * dim))
+    ref = oracle.sdpa_decode(q[0], ck, cv, n_heads, n_kv, dim, dim, cap, cap, dim ** -0.5)
+    assert rel_l2(got[0], oracle.bf16_to_f32(ref)) <= 3e-3
+    assert np.array_equal(got[1], got[0]) and np.array_equal(got[2], got[0])
