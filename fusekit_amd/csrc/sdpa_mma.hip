@@ -6,7 +6,9 @@
 //
 // Probabilities are fp32 and stay so: p = hi + mid + lo, three bf16 values that add up to it exactly, are columns (tiles of 4 queries:
 // 12 of the 16) or matrix instructions of their own (8 queries: two, 16: three); products are exact, sums fp32 as before.  A lane owns one
-// query and four keys of each 16; its softmax reference moves only when a step's maximum outgrows it by 2^8.
+// query and four keys of each 16; its softmax reference moves only when a step's maximum outgrows it by 2^8, and a probability carries
+// the factor 2^-8 all the way (sums, too: it cancels), so that none is above 1 and values up to bf16's largest are summed as they
+// would be behind the true maximum.
 //
 // A wave owns its steps of 32 keys: K and V rows go from memory into its own part of LDS (global_load_lds, 16-byte pieces XOR-swizzled by
 // the row, so that the fragment reads meet all banks); the next step's keys are requested as soon as this one's are in registers, its
@@ -58,6 +60,7 @@ struct SdpaMmaArgs {
 
 constexpr uint32_t kMmaStep = 32;   // keys of a wave's step
 constexpr uint32_t kMmaMaxSplits = 64;
+constexpr float kLagLog2 = 8.0f, kLag = 1.0f / 256.0f;   // how far a step's maximum may lie above the softmax reference
 
 // LDS of a block: what the first barrier hands over, then the waves' stages (the meeting reuses them).
 constexpr uint32_t mma_input_bytes(uint32_t qk, uint32_t qt, bool fused) {
@@ -305,9 +308,9 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
         float mx = x[0];
 #pragma unroll
         for (int i = 1; i < 8; ++i) mx = fmaxf(mx, x[i]);
-        if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.0f) != 0) {   // rare after the first steps
+        if (__builtin_amdgcn_ballot_w64(mx > m_run + kLagLog2) != 0) {   // rare after the first steps
             mx = mma_rows_max(mx);
-            const bool grow = mx > m_run + 8.0f;
+            const bool grow = mx > m_run + kLagLog2;
             const float alpha = grow ? __builtin_amdgcn_exp2f(m_run - mx) : 1.0f;
             m_run = grow ? mx : m_run;
             l_run *= alpha;
@@ -327,7 +330,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
         mma_u32x4_t pb[PARTS];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            float p0 = __builtin_amdgcn_exp2f(ex[2 * i]), p1 = __builtin_amdgcn_exp2f(ex[2 * i + 1]);
+            float p0 = __builtin_amdgcn_exp2f(ex[2 * i]) * kLag, p1 = __builtin_amdgcn_exp2f(ex[2 * i + 1]) * kLag;
             l_run += p0 + p1;
             const uint32_t hi = pack_bf16(p0, p1);
             if constexpr (QT == 4) {

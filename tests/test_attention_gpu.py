@@ -392,3 +392,25 @@ def test_sdpa_rows_with_a_length_on_the_device_beyond_the_plan(fk, given):
     ref = oracle.sdpa_decode(q[0], ck, cv, n_heads, n_kv, dim, dim, cap, cap, dim ** -0.5)
     assert rel_l2(got[0], oracle.bf16_to_f32(ref)) <= 3e-3
     assert np.array_equal(got[1], got[0]) and np.array_equal(got[2], got[0])
+
+
+@pytest.mark.parametrize("n_heads,n_kv,dim,cap", [(14, 2, 64, 700), (4, 2, 64, 1500), (32, 8, 128, 1100), (7, 1, 128, 4500), (12, 1, 64, 700)])
+def test_sdpa_of_values_near_the_largest(fk, n_heads, n_kv, dim, cap):
+    """Values of 2^124, and one key, met after others, whose score stands 7.9 above theirs in powers of two: the softmax's mean is a finite
+    number, and no sum on the way to it overflows."""
+    q = np.full(n_heads * dim, 0x3F80, np.uint16)                                  # ones
+    k = np.zeros((n_kv, cap, dim), np.uint16)
+    k[:, cap - 120] = oracle.f32_to_bf16(np.full(dim, 7.9 * np.log(2.0) / np.sqrt(dim), np.float32))
+    sign = np.where(np.arange(cap) % 3 == 0, -1.0, 1.0).astype(np.float32)
+    v = np.ldexp(np.repeat(sign[:, None], dim, 1), 124).astype(np.float32)
+    cv = np.repeat(oracle.f32_to_bf16(v)[None], n_kv, 0)
+    pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, dim, dim, cap)
+    out = fk.DeviceBuffer(2 * n_heads * dim)
+    fk.sdpa_decode(*(fk.DeviceBuffer.from_numpy(a) for a in (q, k, cv)), out, None, cap, cap, n_heads, n_kv, dim, dim, cap, dim ** -0.5,
+                   fk.DeviceBuffer(pb), fk.zeros(cb))
+    score = oracle.bf16_to_f32(k[0]).astype(np.float64).sum(1) * dim ** -0.5
+    p = np.exp(score)
+    want = float((p * sign).sum() / p.sum())                                       # in units of 2^124
+    got = np.ldexp(oracle.bf16_to_f32(out.to_numpy(np.uint16)).astype(np.float64), -124)
+    assert np.isfinite(got).all()
+    assert np.max(np.abs(got - want)) <= 2.0 ** -7 * abs(want) + 1e-4
