@@ -374,8 +374,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
                            const KvQuant* quant = nullptr, const SdpaFusion* fusion = nullptr, bool vector_form = false);
 // The matrix-core form of it (sdpa_mma.hip): the shapes and pointers that it takes, and its launch.
 bool sdpa_takes_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* out, uint32_t n_heads, uint32_t n_kv,
-                    uint32_t qk_dim, uint32_t v_dim, uint32_t max_len, uint32_t rows, const float* partials, const uint32_t* counters,
-                    const SdpaFusion* fusion);
+                    uint32_t qk_dim, uint32_t v_dim, uint32_t max_len, uint32_t rows, const float* partials, const uint32_t* counters);
 fk_status plan_sdpa_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* out, const uint32_t* kv_len_ptr, uint32_t kv_len_imm,
                         uint32_t max_len, uint32_t n_heads, uint32_t n_kv, uint32_t qk_dim, uint32_t v_dim, uint32_t capacity, float scale,
                         float* partials, uint32_t* counters, uint32_t rows, const SdpaFusion* fusion, Launch* l);

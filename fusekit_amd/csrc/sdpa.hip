@@ -131,7 +131,7 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
         return set_error(FK_ERR_INVALID, "sdpa: the last row's kv length exceeds max_len");
     if (!kv_len_ptr && (kv_len_imm == 0 || kv_len_imm > max_len))
         return set_error(FK_ERR_INVALID, "sdpa: kv_len outside (0, max_len]");
-    if (!kvq && !vector_form && sdpa_takes_mma(q, k, v, out, n_heads, n_kv, qk_dim, v_dim, max_len, rows, partials, counters, fusion))
+    if (!kvq && !vector_form && sdpa_takes_mma(q, k, v, out, n_heads, n_kv, qk_dim, v_dim, max_len, rows, partials, counters))
         return plan_sdpa_mma(q, k, v, out, kv_len_ptr, kv_len_imm, max_len, n_heads, n_kv, qk_dim, v_dim, capacity, scale, partials, counters,
                              rows, fusion, out_launch);
     const uint32_t chunk = sdpa_chunk_len(qk_dim, v_dim, false);

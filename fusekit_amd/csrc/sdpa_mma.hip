@@ -57,6 +57,14 @@ struct SdpaMmaArgs {
     float eps, base_log2;
     const float* rope_tab;
 };
+// MMA_STAGED: the token's rows, norms and table are copied value by value (any address; heads of two parts, as SdpaArgs has them), so
+// that such a launch takes the form that the pair it stands for takes.  Against the form on vector instructions, us, that / this: 14 / 2 heads x 64,
+// 256 positions 5.2 / 5.6, 544 7.1 / 6.6, 4096 9.7 / 7.6; 32 / 8 x 128, 256 6.1 / 6.3, 1024 8.2 / 8.7, 4096 12.2 / 10.4.
+// (A block of its own: 32 bytes more in every launch's took 0.15 us where ranges are merged, 14 / 2 heads x 64, 4096 positions 6.82 / 6.97.)
+struct SdpaMmaStagedArgs : SdpaMmaArgs {
+    const uint16_t* k1_new;
+    uint32_t q0_dim, k0_stride, v_stride, k1_heads, traditional;
+};
 
 constexpr uint32_t kMmaStep = 32;   // keys of a wave's step
 constexpr uint32_t kMmaMaxSplits = 64;
@@ -91,9 +99,11 @@ __device__ __forceinline__ float mma_dpp(float v) { return __int_as_float(__buil
 // what another block of this launch wrote, or is to read, moves past every cache that the two do not share (sc1)
 constexpr int kShared = 16;
 
-// QT queries of a KV head a block, NW waves.
-template <int QK, int VD, int QT, int NW, bool FUSED>
-__global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs a) {
+// QT queries of a KV head a block, NW waves.  FORM: what the launch does ahead of the attention.
+enum MmaForm { MMA_PLAIN, MMA_FUSED, MMA_STAGED };   // nothing; rotation and append; the same with its inputs copied value by value
+template <int QK, int VD, int QT, int NW, MmaForm FORM>
+__global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const std::conditional_t<FORM == MMA_STAGED, SdpaMmaStagedArgs, SdpaMmaArgs> a) {
+    constexpr bool FUSED = FORM != MMA_PLAIN, STAGED = FORM == MMA_STAGED;
     constexpr uint32_t KROW = QK * 2u, VROW = VD * 2u, KP = QK / 8u, VP = VD / 8u;      // bytes and 16-byte pieces of a row
     constexpr uint32_t KT = kMmaStep * KROW, STAGE = mma_stage_bytes(QK, VD);
     constexpr int KREQ = (int)(KT / 1024u), VREQ = (int)(kMmaStep * VROW / 1024u), REQ = KREQ + VREQ;   // requests of a step
@@ -103,7 +113,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
     static_assert(!FUSED || QK == VD, "");
     extern __shared__ uint4 mma_lds[];
     unsigned char* const lds = reinterpret_cast<unsigned char*>(mma_lds);
-    kernarg_warm<(int)sizeof(SdpaMmaArgs)>();
+    kernarg_warm<(int)sizeof(a)>();
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15u, g = lane >> 4;
     const uint32_t split = blockIdx.x, kvh = blockIdx.y, tile = blockIdx.z, blk0 = split * a.span;
@@ -119,7 +129,39 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
     // FUSED: q heads | k | v | q norm | k norm | table
     constexpr uint32_t AT_K = QT * KP, AT_V = AT_K + KP, AT_QN = AT_V + VP, AT_KN = AT_QN + KP, AT_TAB = AT_KN + KP, PIECES = AT_TAB + QK / 4u;
     constexpr uint32_t RAW = FUSED ? (PIECES * 16u + 1023u) / 1024u : (QT * KROW + 1023u) / 1024u;   // requests
-    for (uint32_t i = wave; i < RAW; i += NW) {
+    if constexpr (STAGED) {
+        const uint32_t d0 = a.q0_dim ? a.q0_dim : (uint32_t)QK;
+        const uint16_t* k0 = a.k_new + (size_t)kvh * a.k0_stride;
+        const uint16_t* k1 = a.q0_dim ? a.k1_new + (size_t)(a.k1_heads == 1u ? 0u : kvh) * (QK - d0) : k0;
+        static_assert(PIECES <= NW * 64u, "a piece a thread");
+        if (const uint32_t p = tid; p < PIECES) {
+            // eight values: from `src`, from the cut-th on from `src2`, none from the last-th on
+            const uint16_t *src = a.q + (size_t)(kvh * G + e0 + (p / KP < nq ? p / KP : 0u)) * QK + (p % KP) * 8u, *src2 = k0;
+            uint32_t cut = 8u, last = 8u;
+            if (p >= AT_K && p < AT_V) {
+                const uint32_t e = (p - AT_K) * 8u;
+                cut = d0 > e ? (d0 - e < 8u ? d0 - e : 8u) : 0u;
+                src = k0 + e;
+                src2 = k1 + ((ptrdiff_t)e - (ptrdiff_t)d0);
+            }
+            if (p >= AT_V && p < AT_QN) src = a.v_new + (size_t)kvh * a.v_stride + (p - AT_V) * 8u;
+            if (p >= AT_QN && p < AT_KN) src = a.q_norm + (p - AT_QN) * 8u;
+            if (p >= AT_KN && p < AT_TAB) src = a.k_norm + (p - AT_KN) * 8u;
+            if (p >= AT_QN && p < AT_TAB && !a.q_norm) last = 0u;
+            if (p >= AT_TAB) {
+                const uint32_t at = (p - AT_TAB) * 8u, n = a.rope_tab ? a.rope_dims * 2u : 0u;   // (halves of floats)
+                src = reinterpret_cast<const uint16_t*>(a.rope_tab) + at;
+                last = n > at ? (n - at < 8u ? n - at : 8u) : 0u;
+            }
+            uint32_t x[8];   // (where nothing stands behind a value, q's first is read)
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) x[j] = *(j < last ? (j < cut ? src : src2) + j : a.q);
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) x[j] = j < last ? x[j] : 0u;
+            *reinterpret_cast<uint4*>(lds + p * 16u) = make_uint4(x[0] | x[1] << 16, x[2] | x[3] << 16, x[4] | x[5] << 16, x[6] | x[7] << 16);
+        }
+    }
+    for (uint32_t i = wave; i < (STAGED ? 0u : RAW); i += NW) {
         const uint32_t p = i * 64u + lane;
         const unsigned char* src;
         if constexpr (FUSED) {
@@ -228,6 +270,12 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
             const uint16_t* src = raw + (key ? AT_K * 8u : h * QK);
             uint16_t* dst = qn + (key ? (uint32_t)QT : h) * QN;
             const uint16_t* nw = raw + (key ? AT_KN : AT_QN) * 8u;
+            if constexpr (STAGED) {
+                if (a.q0_dim) {
+                    split_head_transform(src, src + a.q0_dim, dst, a.q0_dim, QK - a.q0_dim, a.rope_dims, a.traditional != 0, pos, a.base_log2, lane, tab);
+                    continue;
+                }
+            }
             if (fast) {
                 const HeadPair p = head_pair_fetch(src, nw, tab, QK / 2u, lane);
                 head_pair_apply(p, dst, norm, QK / 2u, a.eps, lane, true);
@@ -545,27 +593,26 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const SdpaMmaArgs 
 
 namespace {
 
-template <int QK, int VD, int QT, int NW, bool FUSED>
+template <int QK, int VD, int QT, int NW, MmaForm FORM = MMA_PLAIN>
 fk_status fill(Launch* l) {
-    l->func = reinterpret_cast<const void*>(&sdpa_mma_kernel<QK, VD, QT, NW, FUSED>);
+    l->func = reinterpret_cast<const void*>(&sdpa_mma_kernel<QK, VD, QT, NW, FORM>);
     l->block = dim3(NW * 64, 1, 1);
-    l->shmem = mma_lds_bytes(QK, VD, QT, NW, FUSED);
+    l->shmem = mma_lds_bytes(QK, VD, QT, NW, FORM != MMA_PLAIN);
     return raise_dynamic_lds(l->func, l->shmem);
+}
+template <int DIM, int QT, int NW>
+fk_status fill(Launch* l, MmaForm form) {
+    return form == MMA_PLAIN ? fill<DIM, DIM, QT, NW>(l) : (form == MMA_FUSED ? fill<DIM, DIM, QT, NW, MMA_FUSED>(l) : fill<DIM, DIM, QT, NW, MMA_STAGED>(l));
 }
 
 }  // namespace
 
 bool sdpa_takes_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* out, uint32_t n_heads, uint32_t n_kv,
-                    uint32_t qk_dim, uint32_t v_dim, uint32_t max_len, uint32_t rows, const float* partials, const uint32_t* counters,
-                    const SdpaFusion* fusion) {
+                    uint32_t qk_dim, uint32_t v_dim, uint32_t max_len, uint32_t rows, const float* partials, const uint32_t* counters) {
     if (!((qk_dim == v_dim && (qk_dim == 64 || qk_dim == 128)) || (qk_dim == 192 && v_dim == 128 && rows > 1))) return false;
     if (!partials || !counters) return false;
-    uintptr_t a = (uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)partials;
-    if (fusion) {
-        if (fusion->q0_dim || (fusion->rope_tab && fusion->rope_dims % 4u)) return false;
-        a |= (uintptr_t)fusion->k_new | (uintptr_t)fusion->v_new | (uintptr_t)fusion->q_norm | (uintptr_t)fusion->k_norm | (uintptr_t)fusion->rope_tab;
-    }
-    if (a & 15u) return false;
+    // (by what a launch with the rotation and the append shares with the launch pair that it equals bit for bit, and nothing else)
+    if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)partials) & 15u) return false;
     // Short contexts of few rows: the form on vector instructions has less to set up (us, that / this: 32 / 8 heads x 128, 64 positions 4.0 / 4.7, 128
     // 4.9 / 4.9, 256 6.8 / 6.6, 8 rows at 100 4.3 / 6.6, 64 rows at 100 14.7 / 8.1; 14 / 2 x 64, 128 positions 4.1 / 4.1, 256 5.1 / 4.5; 16 heads of
     // 192 / 128, 8 rows at 30 5.4 / 6.1, 2 rows at 100 7.6 / 6.2).
@@ -587,22 +634,29 @@ fk_status plan_sdpa_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v,
                         float* partials, uint32_t* counters, uint32_t rows, const SdpaFusion* fusion, Launch* l) {
     const DeviceFacts* dev;
     FK_TRY(device_facts(&dev));
-    SdpaMmaArgs a;
+    SdpaMmaStagedArgs a;
     memset(&a, 0, sizeof(a));
     a.q = q; a.k = k; a.v = v; a.out = out;
     a.kv_len_ptr = kv_len_ptr; a.kv_len_imm = kv_len_imm;
     a.n_heads = n_heads; a.group = n_heads / n_kv; a.capacity = capacity;
     a.rows = rows; a.scale = scale; a.partials = partials; a.counters = counters;
+    MmaForm form = MMA_PLAIN;
     if (fusion) {
         a.k_new = fusion->k_new; a.v_new = fusion->v_new; a.q_norm = fusion->q_norm; a.k_norm = fusion->k_norm;
         a.cache_k_w = const_cast<uint16_t*>(k); a.cache_v_w = const_cast<uint16_t*>(v);
         a.rope_dims = fusion->rope_dims; a.eps = fusion->eps; a.base_log2 = fusion->base_log2; a.rope_tab = fusion->rope_tab;
+        a.k1_new = fusion->k1_new; a.q0_dim = fusion->q0_dim; a.k1_heads = fusion->k1_heads; a.traditional = fusion->traditional;
+        a.k0_stride = fusion->q0_dim ? fusion->k0_stride : qk_dim;
+        a.v_stride = fusion->q0_dim ? fusion->v_stride : v_dim;
+        // requests of sixteen bytes take whole heads, a table of whole pieces and aligned addresses
+        const uintptr_t at = (uintptr_t)a.k_new | (uintptr_t)a.v_new | (uintptr_t)a.q_norm | (uintptr_t)a.k_norm | (uintptr_t)a.rope_tab;
+        form = (at & 15u) || a.q0_dim || (a.rope_tab && a.rope_dims % 4u) ? MMA_STAGED : MMA_FUSED;
     }
     // Tiles of 4 queries put the three parts of the probabilities into one matrix instruction's columns, of 8 into two instructions, of 16
     // into three.  More than 8 queries: tiles of 8 while there is a CU for each (of 16 / 8, us: 32 / 8 heads x 128, 3 rows at 500 positions 10.2 /
     // 7.0, 64 rows 13.7 / 8.4, 128 rows -- 512 tiles -- 12.4 / 15.1; 16 heads of 192 / 128, 32 rows at 480 positions 10.9 / 8.8).
     const uint32_t queries = rows * a.group;
-    const uint32_t qt = queries <= 4u ? 4u : (queries <= 8u || fusion || (uint64_t)n_kv * ((queries + 7u) / 8u) <= (uint64_t)dev->cus ? 8u : 16u);
+    const uint32_t qt = queries <= 4u ? 4u : (queries <= 8u || rows == 1u || (uint64_t)n_kv * ((queries + 7u) / 8u) <= (uint64_t)dev->cus ? 8u : 16u);
     // Waves, and the rounds of theirs that one block walks rather than leave partials.  A block draws 90 bytes a ns where its rows lie in the
     // L2, half of that where they come from memory; partials, their count and their merge take 2.2 us.  Cold caches, us: 64 dims (256
     // positions a round), one block / several, 544 positions 5.5 / 6.2, 1024 6.5 / 6.5 (16 / 8 heads 6.4 / 6.4, 8.1 / 6.5).  One row of 128 dims: at
@@ -613,28 +667,26 @@ fk_status plan_sdpa_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v,
     uint32_t nw = 8, alone = rows > 1 ? 2u : 1u;
     if (qk_dim == 64) {
         alone = 3;
-        if (fusion) FK_TRY(qt == 4 ? (fill<64, 64, 4, 8, true>(l)) : (fill<64, 64, 8, 8, true>(l)));
-        else FK_TRY(qt == 4 ? (fill<64, 64, 4, 8, false>(l)) : (qt == 8 ? fill<64, 64, 8, 8, false>(l) : fill<64, 64, 16, 8, false>(l)));
+        FK_TRY(qt == 4 ? (fill<64, 4, 8>(l, form)) : (qt == 8 ? fill<64, 8, 8>(l, form) : fill<64, 64, 16, 8>(l)));
     } else if (qk_dim == 128) {
         if (qt == 16) {
             nw = 4;
             alone = 4;
-            FK_TRY((fill<128, 128, 16, 4, false>(l)));
+            FK_TRY((fill<128, 128, 16, 4>(l)));
         } else if (rows == 1 && qt == 4u && max_len > 256u && max_len <= 3072u) {
             nw = 4;
-            FK_TRY(fusion ? (fill<128, 128, 4, 4, true>(l)) : (fill<128, 128, 4, 4, false>(l)));
+            FK_TRY((fill<128, 4, 4>(l, form)));
         } else {
-            if (fusion) FK_TRY(qt == 4 ? (fill<128, 128, 4, 8, true>(l)) : (fill<128, 128, 8, 8, true>(l)));
-            else FK_TRY(qt == 4 ? (fill<128, 128, 4, 8, false>(l)) : (fill<128, 128, 8, 8, false>(l)));
+            FK_TRY(qt == 4 ? (fill<128, 4, 8>(l, form)) : (fill<128, 8, 8>(l, form)));
         }
     } else if (qt <= 8) {
         nw = 7;   // (160 KB)
         alone = 3;
-        FK_TRY(qt == 4 ? (fill<192, 128, 4, 7, false>(l)) : (fill<192, 128, 8, 7, false>(l)));
+        FK_TRY(qt == 4 ? (fill<192, 128, 4, 7>(l)) : (fill<192, 128, 8, 7>(l)));
     } else {
         nw = 4;
         alone = 4;
-        FK_TRY((fill<192, 128, 16, 4, false>(l)));
+        FK_TRY((fill<192, 128, 16, 4>(l)));
     }
     // Beyond that a block a CU, but no shorter than two rounds where there would be more than the 16 partials that a merge has soonest.
     const uint32_t tiles = (queries + qt - 1u) / qt, round = nw * kMmaStep, rounds = (max_len + round - 1u) / round;
@@ -646,7 +698,8 @@ fk_status plan_sdpa_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v,
     a.span = per * round;
     a.n_splits = (max_len + a.span - 1u) / a.span;
     l->grid = dim3(a.n_splits, n_kv, tiles);
-    l->set_args(a);
+    if (form == MMA_STAGED) l->set_args(a);
+    else l->set_args(static_cast<const SdpaMmaArgs&>(a));
     return FK_OK;
 }
 

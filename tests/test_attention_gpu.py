@@ -414,3 +414,52 @@ def test_sdpa_of_values_near_the_largest(fk, n_heads, n_kv, dim, cap):
     got = np.ldexp(oracle.bf16_to_f32(out.to_numpy(np.uint16)).astype(np.float64), -124)
     assert np.isfinite(got).all()
     assert np.max(np.abs(got - want)) <= 2.0 ** -7 * abs(want) + 1e-4
+
+
+class _At:
+    """A copy of an array that starts `offset` bytes into its device buffer."""
+    def __init__(self, fk, a, offset):
+        self.buf = fk.DeviceBuffer(a.nbytes + 16)
+        self.buf.upload(a, offset)
+        self.ptr = self.buf.ptr + offset
+
+    def __int__(self):
+        return self.ptr
+
+
+@pytest.mark.parametrize("norm,table,offset", [(False, True, 0), (True, True, 0), (True, False, 2), (True, True, 4), (False, True, 8)])
+@pytest.mark.parametrize("n_heads,n_kv,dim,rope_dims,cap,kv_len", [
+    (14, 2, 64, 62, 1024, 300), (8, 8, 64, 64, 512, 512), (32, 2, 64, 32, 1024, 700),         # groups of 7, 1 and 16: tiles of 8 and 4, two tiles
+    (32, 8, 128, 126, 1024, 1000), (56, 8, 128, 64, 2048, 2048), (7, 1, 128, 128, 2304, 1), (16, 1, 128, 66, 4096, 3000),
+])
+def test_rope_store_sdpa_takes_the_form_of_the_pair(fk, norm, table, offset, n_heads, n_kv, dim, rope_dims, cap, kv_len):
+    """The one launch against fk_qkv_rope_store_decode and fk_sdpa_decode, bit for bit: rotations of part of a head, tables of no whole
+    pieces of sixteen bytes, and rows, norms and tables at any address (offset in bytes)."""
+    theta, eps, scale, pos = 1e6, 1e-6, dim ** -0.5, kv_len - 1
+    q, k, v = normal_bf16(1, n_heads * dim), normal_bf16(2, n_kv * dim), normal_bf16(3, n_kv * dim)
+    ck, cv = normal_bf16(6, n_kv * cap * dim), normal_bf16(7, n_kv * cap * dim)
+    dev = lambda a: fk.DeviceBuffer.from_numpy(a)
+    qw, kw = (normal_bf16(4, dim, 0.1, 1.0), normal_bf16(5, dim, 0.1, 1.0)) if norm else (None, None)
+    pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, dim, dim, cap)
+    part, cnt = fk.DeviceBuffer(max(pb, 16)), fk.zeros(max(cb, 16))
+    dq, ck1, cv1, out1 = dev(q), dev(ck), dev(cv), fk.DeviceBuffer(n_heads * dim * 2)
+    fk.qkv_rope_store_decode(dq, dev(k), dev(v), dev(qw) if norm else None, dev(kw) if norm else None, n_heads, n_kv, dim, rope_dims, theta,
+                             eps, _u32(fk, pos), 0, cap, ck1, cv1)
+    fk.sdpa_decode(dq, ck1, cv1, out1, _u32(fk, kv_len), 0, cap, n_heads, n_kv, dim, dim, cap, scale, part, cnt)
+    at = lambda a: _At(fk, a, offset)
+    tab = None
+    if table:
+        made = fk.DeviceBuffer(rope_dims * 4)
+        fk.step_init_rope(_u32(fk, pos), fk.zeros(4), fk.zeros(4), made, rope_dims, theta)
+        tab = _At(fk, made.to_numpy(np.uint32), offset // 4 * 4)
+    ins = [at(a) if a is not None else None for a in (k, v, qw, kw)]
+    ck2, cv2, out2 = dev(ck), dev(cv), fk.DeviceBuffer(n_heads * dim * 2)
+    fk.rope_store_sdpa_decode(dev(q), *ins, ck2, cv2, out2, _u32(fk, kv_len), 0, cap, n_heads, n_kv, dim, rope_dims, theta, eps, cap, scale,
+                              tab, part, cnt)
+    assert np.array_equal(ck2.to_numpy(np.uint16), ck1.to_numpy(np.uint16))
+    assert np.array_equal(cv2.to_numpy(np.uint16), cv1.to_numpy(np.uint16))
+    assert np.array_equal(out2.to_numpy(np.uint16), out1.to_numpy(np.uint16))
+    ref = oracle.sdpa_decode(dq.to_numpy(np.uint16), ck1.to_numpy(np.uint16), cv1.to_numpy(np.uint16), n_heads, n_kv,
+                             dim, dim, kv_len, cap, scale)
+    assert rel_l2(out2.to_numpy(np.uint16), oracle.bf16_to_f32(ref)) <= REL_L2_BAR
+    assert not cnt.to_numpy(np.uint32).any()

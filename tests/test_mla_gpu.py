@@ -132,6 +132,17 @@ def test_split_store_and_attention_in_one_launch(fk, n_heads, k0d, k1d, vd, rope
     assert np.array_equal(f_q.to_numpy(np.uint16), q.reshape(-1))
 
 
+@pytest.mark.parametrize("traditional,table", [(True, True), (False, False), (True, False)])
+@pytest.mark.parametrize("n_heads,k0d,k1d,vd,rope,kv_len,cap", [
+    (4, 48, 16, 64, 16, 300, 512), (4, 40, 24, 64, 22, 513, 1024),       # 64 dims, parts of no whole pieces, a table of no whole pieces
+    (8, 64, 64, 128, 64, 1200, 2048), (2, 96, 32, 128, 14, 2048, 2048),  # 128 dims, the cache not full and exactly full
+    (8, 64, 64, 128, 64, 1, 2048), (4, 48, 16, 64, 16, 192, 192),        # the first token of a long plan; the last plan of the other form
+])
+def test_split_store_and_attention_in_one_launch_of_square_heads(fk, n_heads, k0d, k1d, vd, rope, kv_len, cap, traditional, table):
+    """Heads whose two parts make the widths that the attention has a matrix-core form for: the launch and the pair take the same form."""
+    test_split_store_and_attention_in_one_launch(fk, n_heads, k0d, k1d, vd, rope, kv_len, cap, traditional, table)
+
+
 @pytest.mark.parametrize("rows,row_n,top_k,per_route", [(1, 64, 6, False), (8, 64, 6, True), (3, 256, 32, False),
                                                         (5, 2, 1, False), (2, 128, 8, True)])
 def test_softmax_topk_route(fk, rows, row_n, top_k, per_route):
