@@ -125,6 +125,10 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const std::conditi
     auto v_swizzle = [](uint32_t row) { return VP == 16u ? (row & 7u) << 1 : ((row >> 1) & 3u) << 1; };
     auto k_at = [&](uint32_t row, uint32_t piece) { return row * KROW + ((KP == 24u ? (piece & ~7u) | ((piece ^ k_swizzle(row)) & 7u) : piece ^ k_swizzle(row)) * 16u); };
 
+    uint32_t kv_raw = a.kv_len_imm;
+    if (a.kv_len_ptr) kv_raw = *(const __attribute__((address_space(4))) uint32_t*)(uintptr_t)a.kv_len_ptr;
+    __builtin_amdgcn_sched_barrier(0);
+
     // ---- what the first barrier hands over: one request a wave (plain: the query rows; else see the order below) ----
     // FUSED: q heads | k | v | q norm | k norm | table
     constexpr uint32_t AT_K = QT * KP, AT_V = AT_K + KP, AT_QN = AT_V + VP, AT_KN = AT_QN + KP, AT_TAB = AT_KN + KP, PIECES = AT_TAB + QK / 4u;
@@ -226,11 +230,13 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const std::conditi
     const uint32_t first = blk0 + wave * kMmaStep;
     // a device scalar is not trusted: a length beyond what the launch was sized for would leave ranges without a block
     const uint32_t covered = a.n_splits * a.span < a.capacity ? a.n_splits * a.span : a.capacity;
-    // the first range's keys are requested ahead of the length (its values are not: a short context would wait for what it does not need)
-    const bool ahead = split == 0 && first < covered;
+    // The first range's keys are requested ahead of a length on the device (its values are not: a short context would wait for what it does not
+    // need), of rows of 128 dims and more the first two waves' only, and the length in front of everything.  All waves' keys, then the
+    // length / this, us: 32 / 8 heads x 128, contexts of 50 in plans of 256 4.9 / 4.5, of 1024 4.5 / 4.4, of 4096 4.9 / 4.5, 150 in 256 5.4 / 5.0; 8 rows,
+    // 30 in 1024 6.1 / 5.8; 16 heads of 192 / 128, 8 rows, 30 in 256 7.1 / 6.3; whole plans the same.  (64 dims: 14 / 2 heads, 50 in 1024
+    // 3.9 / 3.8, but three rounds in one block, 544, 5.7 / 5.8.)
+    const bool ahead = split == 0 && first < covered && (QK == 64 || !a.kv_len_ptr || wave < 2u);
     if (ahead) issue_k(first);
-    uint32_t kv_raw = a.kv_len_imm;
-    if (a.kv_len_ptr) kv_raw = *(const __attribute__((address_space(4))) uint32_t*)(uintptr_t)a.kv_len_ptr;
     const uint32_t kv0_len = kv_raw > covered ? covered : kv_raw;   // (before a row is added: a tile's rows stay in order whatever was read)
     auto limit_of = [&](uint32_t row) {
         const uint32_t l = kv0_len + row;
@@ -613,6 +619,12 @@ bool sdpa_takes_mma(const uint16_t* q, const uint16_t* k, const uint16_t* v, con
     if (!partials || !counters) return false;
     // (by what a launch with the rotation and the append shares with the launch pair that it equals bit for bit, and nothing else)
     if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)partials) & 15u) return false;
+    // The lines are in the length that the launch is planned for, which the host knows; in a graph that is the capacity, and shorter contexts come
+    // along.  Those of one range of the vector form (64 positions of 128 dims, 128 of 64) are the slower for it, longer ones the faster, us, that
+    // / this: plans of 256, 32 / 8 heads x 128, 50 positions 3.2 / 4.5, 100 5.8 / 4.7, 150 6.1 / 5.0, 256 6.3 / 5.3; of 1024, 50 3.2 / 4.4, 100 4.1 / 4.5,
+    // 600 7.6 / 6.9, 1024 8.4 / 7.3; of 4096, 50 3.8 / 4.5, 1000 10.0 / 7.8; 14 / 2 x 64, of 1024, 50 3.2 / 3.9, 300 6.1 / 5.8, 1024 6.9 / 6.3; of 12000, 200
+    // 4.8 / 4.1; 8 rows of 32 / 8 x 128, of 1024, 30 4.2 / 5.8, 300 8.0 / 7.9, 1000 15.1 / 10.0.  A cache that fills meets the first for 64 (128)
+    // tokens of its hundreds and more.
     // Short contexts of few rows: the form on vector instructions has less to set up (us, that / this: 32 / 8 heads x 128, 64 positions 4.0 / 4.7, 128
     // 4.9 / 4.9, 256 6.8 / 6.6, 8 rows at 100 4.3 / 6.6, 64 rows at 100 14.7 / 8.1; 14 / 2 x 64, 128 positions 4.1 / 4.1, 256 5.1 / 4.5; 16 heads of
     // 192 / 128, 8 rows at 30 5.4 / 6.1, 2 rows at 100 7.6 / 6.2).
