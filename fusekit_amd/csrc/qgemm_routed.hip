@@ -42,6 +42,7 @@ struct QgemmRoutedArgs {
     uint32_t N, K, gshift;        // gshift: 64-code groups per scale: 0 (group 64), 1 (group 128)
     uint32_t n_routes, n_experts, n_x_rows;
     uint32_t tiles;               // pieces of one expert
+    uint32_t cus;
 };
 
 // The sorted list: row << 16 | route by expert; routes of an expert (then their first place); the pieces' experts, first
@@ -308,10 +309,10 @@ __global__ __launch_bounds__(kRtThreads, 2) void qgemm_routed_kernel(const Qgemm
     fetch_x(now, 0u, x0);
     fetch_x(now, 1u, x1);
     fetch_w(now, 1u, w1);
-    // The waves of a CU's three workgroups go first in turn, a piece each: left to their age the third one's first piece was done 5 us
-    // after the first one's and its last so much later, the others' memory idle meanwhile (8 rows x 6 routes, below: 31.6 / 31.4 us; 96 rows
-    // 60.9 / 60.0).
-    uint32_t turn = blockIdx.x >> 8;
+    // The waves of a CU's three workgroups (the grid deals one to each CU before the next) go first in turn, a piece each: left to their age
+    // the third one's first piece was done 5 us after the first one's and its last so much later, the others' memory idle meanwhile (64
+    // experts, pair of 1408 x 2048 int4, runs differ by 0.1: 48 routes 30.1 / 29.9 us, 96 40.0 / 39.6, 192 48.4 / 47.8, 576 58.1 / 57.3).
+    uint32_t turn = blockIdx.x < a.cus ? 0u : (blockIdx.x < 2u * a.cus ? 1u : 2u);
     while (true) {
         switch (turn++ % 3u) {   // uniform
             case 0: __builtin_amdgcn_s_setprio(0); break;
@@ -450,6 +451,7 @@ fk_status plan_qgemm_routed(const uint16_t* x, uint32_t n_x_rows, const fk_weigh
     a.n_experts = n_experts;
     a.n_x_rows = n_x_rows;
     a.tiles = rt_pieces_of_an_expert(a.N, pair);
+    a.cus = (uint32_t)dev->cus;
     const uint64_t most = (uint64_t)(n_routes < n_experts ? n_routes : n_experts + n_routes / kRtRows) * a.tiles;
     const uint32_t resident = 3u * (uint32_t)dev->cus;   // by LDS four; two were 1 %, four 0 .. 1 % slower
     out->func = Wa->bits == 4 ? routed_func<W_Q4>(pair) : routed_func<W_Q8>(pair);
