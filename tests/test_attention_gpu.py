@@ -321,7 +321,7 @@ def test_rope_store_sdpa_rejects_bad_arguments(fk):
     (8, 8, 64, 64, 1, 193), (6, 2, 64, 64, 1, 256), (10, 2, 64, 64, 1, 257), (24, 2, 64, 64, 1, 769),       # groups of 1, 3, 5 and 12; round edges
     (32, 8, 128, 128, 1, 255), (3, 1, 128, 128, 1, 512), (7, 1, 128, 128, 1, 513), (16, 1, 128, 128, 1, 4097),
     (32, 8, 128, 128, 1, 705), (3, 1, 128, 128, 1, 1025), (7, 1, 128, 128, 1, 1793), (56, 8, 128, 128, 1, 1089),   # one past the vector form's lines
-    (2, 1, 64, 64, 1, 9000), (5, 1, 128, 128, 1, 33000),                                                      # merges of up to 64 partials
+    (2, 1, 64, 64, 1, 9000), (5, 1, 128, 128, 1, 33000),                                                      # merges of 18 and 43 partials
     (14, 2, 64, 64, 3, 200), (32, 8, 128, 128, 2, 223), (64, 2, 64, 64, 13, 500), (128, 8, 128, 128, 17, 300),  # tiles of 8 and of 16, last ones not full
     (16, 16, 192, 128, 2, 30), (16, 16, 192, 128, 8, 225), (4, 2, 192, 128, 9, 700), (64, 64, 192, 128, 33, 128),
 ])
@@ -427,7 +427,7 @@ class _At:
         return self.ptr
 
 
-@pytest.mark.parametrize("norm,table,offset", [(False, True, 0), (True, True, 0), (True, False, 2), (True, True, 4), (False, True, 8)])
+@pytest.mark.parametrize("norm,table,offset", [(False, True, 0), (True, True, 0), (True, False, 0), (True, False, 2), (True, True, 4), (False, True, 8)])
 @pytest.mark.parametrize("n_heads,n_kv,dim,rope_dims,cap,kv_len", [
     (14, 2, 64, 62, 1024, 300), (8, 8, 64, 64, 512, 512), (32, 2, 64, 32, 1024, 700),         # groups of 7, 1 and 16: tiles of 8 and 4, two tiles
     (32, 8, 128, 126, 1024, 1000), (56, 8, 128, 64, 2048, 2048), (7, 1, 128, 128, 2304, 1), (16, 1, 128, 66, 4096, 3000),
@@ -446,6 +446,7 @@ def test_rope_store_sdpa_takes_the_form_of_the_pair(fk, norm, table, offset, n_h
     fk.qkv_rope_store_decode(dq, dev(k), dev(v), dev(qw) if norm else None, dev(kw) if norm else None, n_heads, n_kv, dim, rope_dims, theta,
                              eps, _u32(fk, pos), 0, cap, ck1, cv1)
     fk.sdpa_decode(dq, ck1, cv1, out1, _u32(fk, kv_len), 0, cap, n_heads, n_kv, dim, dim, cap, scale, part, cnt)
+    assert _matrix_core_grid(fk, n_heads, n_kv, dim, dim, 1, cap)
     at = lambda a: _At(fk, a, offset)
     tab = None
     if table:
@@ -463,3 +464,29 @@ def test_rope_store_sdpa_takes_the_form_of_the_pair(fk, norm, table, offset, n_h
                              dim, dim, kv_len, cap, scale)
     assert rel_l2(out2.to_numpy(np.uint16), oracle.bf16_to_f32(ref)) <= REL_L2_BAR
     assert not cnt.to_numpy(np.uint32).any()
+
+
+def _matrix_core_grid(fk, n_heads, n_kv, qk, vd, rows, max_len):
+    """The grid of the attention launch planned for max_len positions where it is the form on the matrix cores, which stages keys and
+    values in 64 KB of LDS and more (the form on vector instructions holds scores and sums, 20 KB at most over a bf16 cache); else None."""
+    from fusekit_amd.runtime import Dispatch, Dispatcher
+    pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, qk, vd, max_len)
+    sizes = [rows * n_heads * qk * 2, n_kv * max_len * qk * 2, n_kv * max_len * vd * 2, 4, rows * n_heads * vd * 2, pb * rows, cb * rows]
+    d = Dispatch("fusekit_sdpa_decode_f0", [((i + 1) << 40, n) for i, n in enumerate(sizes)],   # (planned, not run: any aligned addresses)
+                 {"n_heads": n_heads, "n_kv": n_kv, "qk_dim": qk, "v_dim": vd, "capacity": max_len, "rows": rows})
+    g = Dispatcher().plan_geometry(d)
+    return tuple(g.grid[0]) if g.lds_bytes[0] > 60000 else None
+
+
+@pytest.mark.parametrize("n_heads,n_kv,qk,vd,rows,kv_len,splits", [
+    (3, 1, 128, 128, 1, 1024, 0), (3, 1, 128, 128, 1, 1025, 9), (2, 2, 128, 128, 1, 1280, 0), (2, 2, 128, 128, 1, 1281, 11), (7, 1, 128, 128, 1, 1792, 0), (7, 1, 128, 128, 1, 1793, 8),   # at and past the lines
+    (7, 1, 128, 128, 1, 2048, 8), (7, 1, 128, 128, 1, 2049, 9), (3, 1, 128, 128, 1, 3072, 12), (3, 1, 128, 128, 1, 3073, 13),  # round edges
+    (16, 16, 192, 128, 2, 63, 0), (16, 16, 192, 128, 2, 64, 1),
+    (5, 1, 128, 128, 1, 4096, 16), (3, 1, 128, 128, 1, 8193, 17), (5, 1, 128, 128, 1, 16384, 32), (5, 1, 128, 128, 1, 16385, 33),
+    (5, 1, 128, 128, 1, 32768, 64), (2, 1, 64, 64, 1, 4096, 16), (2, 1, 64, 64, 1, 8193, 17), (2, 1, 64, 64, 1, 32768, 64),    # edges of the merge
+])
+def test_sdpa_form_and_number_of_ranges(fk, n_heads, n_kv, qk, vd, rows, kv_len, splits):
+    """Lengths at which the form or the merge changes; splits 0: the form on vector instructions."""
+    grid = _matrix_core_grid(fk, n_heads, n_kv, qk, vd, rows, kv_len + rows - 1)
+    assert (grid is not None) == (splits > 0) and (grid is None or grid[0] == splits), grid
+    test_sdpa_on_the_matrix_cores_at_the_edges_of_its_tiles(fk, n_heads, n_kv, qk, vd, rows, kv_len)
