@@ -94,10 +94,25 @@ def _close_rows(got, ref_bits, x64, W, frac=0.02):
                          [(b, h, i, v) for b in (4, 8, 16) for h, i, v in ((512, 1024, 0), (2560, 9728, 1), (1024, 3072, 2))] +
                          [(4, 4096, 14336, 1)])
 def test_xcd_mlp_block(fk, bits, hidden, inter, variant):
-    """(4096 x 14336 is the 8B class: in 4 bits its tiles hold up to 1792 quantisation groups and take the flavour with
-    the pass loop; in 8 bits and bf16 two workgroups do not fit a CU and the shape is refused.)"""
+    """(4096 x 14336 is the 8B class: in 4 bits its tiles hold up to 1792 quantisation groups and 14 requests a thread, one
+    pass; in 8 bits and bf16 two workgroups do not fit a CU and the shape is refused.)"""
     assert fk.xcd_layer_supported(hidden, inter, 32, 8, 128, 256, bits, 64), fk.lib.fk_last_error().decode()
     _run_mlp_block(fk, bits, hidden, inter, variant)
+
+
+@pytest.mark.parametrize("bits,hidden,inter,requests", [
+    (4, 4096, 12288, 12), (8, 4096, 7168, 14),                          # one pass of 12 and of 14, with 2048 groups a tile
+    (4, 4096, 15360, 15), (8, 4096, 7680, 15), (16, 1024, 10240, 10),   # passes of 5
+    (4, 4096, 16384, 16), (16, 1024, 6144, 6),                          # passes of 6, the last not full; one full pass of 6
+])
+def test_xcd_mlp_block_of_every_depth(fk, bits, hidden, inter, requests):
+    """Launches compiled for the requests a thread that a tile of either projection has: those that no other test's shape takes."""
+    values = 128 // bits   # of a 16-byte request
+    gate = -(-(-(-inter // 512) * hidden // values) // 256)
+    down = -(-(hidden // 64) * (inter // 8 // values) // 256)
+    assert gate == down == requests
+    assert fk.xcd_layer_supported(hidden, inter, 32, 8, 128, 256, bits, 64), fk.lib.fk_last_error().decode()
+    _run_mlp_block(fk, bits, hidden, inter, 1)
 
 
 @pytest.mark.parametrize("gain,lo,hi", [(3.0e3, 2.0 ** 20, 2.0 ** 27), (1.5e-6, 0.0, 2.0 ** -26)])
@@ -183,7 +198,7 @@ def test_xcd_attn_block(fk, bits, n_heads, head_dim, qk_norm, hidden):
     attention over the growing context, o_proj partial rows; against the oracle's composition of the same
     dispatches.  Context crosses several key ranges (capacity 256 -> ranges of 64 or 128 positions)."""
     from fusekit_amd.runtime import Dispatch, Dispatcher, arg
-    n_kv, inter, capacity, theta = 8, 1024, 256, 1e6   # (hidden 4096: the 8B class, q / k / v tiles of 13 rows x 64 groups)
+    n_kv, inter, capacity, theta = 8, 1024, 256, 1e6   # (hidden 4096: the 8B class, q / k / v tiles of 12 rows x 64 groups)
     if not fk.xcd_layer_supported(hidden, inter, n_heads, n_kv, head_dim, capacity, bits, 64):
         pytest.skip("shape not supported: " + fk.lib.fk_last_error().decode())
     d = Dispatcher()
@@ -265,6 +280,16 @@ def test_xcd_attn_block(fk, bits, n_heads, head_dim, qk_norm, hidden):
         worst = max(worst, rel)
         assert rel <= 1e-2, (pos, rel)
     print("worst rel-L2 of the o_proj sums over the sampled positions: %.3e" % worst)
+
+
+@pytest.mark.parametrize("bits,n_heads,head_dim,hidden", [
+    (8, 32, 128, 1024),    # tiles of 12 rows: one of q and k, one of k and v
+    (8, 16, 64, 1024), (8, 8, 128, 512),
+    (16, 8, 128, 4096),    # o_proj in a pass of 5
+])
+def test_xcd_attn_block_of_other_tiles(fk, bits, n_heads, head_dim, hidden):
+    assert fk.xcd_layer_supported(hidden, 1024, n_heads, 8, head_dim, 256, bits, 64), fk.lib.fk_last_error().decode()
+    test_xcd_attn_block(fk, bits, n_heads, head_dim, True, hidden)
 
 
 @pytest.mark.parametrize("kv_len", [512, 4096, 32768])
