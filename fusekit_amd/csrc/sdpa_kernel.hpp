@@ -92,7 +92,7 @@ __device__ __forceinline__ void each_index(F&& f) {
         each_index<N, F, I + 1>(static_cast<F&&>(f));
     }
 }
-// Lane J of the caller's 16-lane row (row_newbcast); a value moved as a DPP control says.
+// Lane J of the caller's 16-lane row (row_newbcast).
 template <int J>
 __device__ __forceinline__ uint32_t row_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + J, 0xF, 0xF, false); }
 // Lane J of the caller's half of a 16-lane row.
@@ -100,15 +100,6 @@ template <int J>
 __device__ __forceinline__ uint32_t half_row_lane(uint32_t v) {
     const int low = __builtin_amdgcn_update_dpp(0, (int)v, 0x150 + J, 0xF, 0x3, false);
     return (uint32_t)__builtin_amdgcn_update_dpp(low, (int)v, 0x158 + J, 0xF, 0xC, false);
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false)); }
-// The maximum over the wave's four 16-lane rows, lane by lane.
-__device__ __forceinline__ float rows_max(float v) {
-    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
 // One (range, kv head, head tile) work item.  Uniform per block; `kv_len` already read.

@@ -82,20 +82,12 @@ constexpr uint32_t mma_lds_bytes(uint32_t qk, uint32_t vd, uint32_t qt, uint32_t
     return mma_input_bytes(qk, qt, fused) + (stages > meet ? stages : meet);
 }
 
-__device__ __forceinline__ float mma_rows_max(float v) {   // over the wave's four 16-lane rows, lane by lane
-    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float mma_rows_sum(float v) {
+__device__ __forceinline__ float mma_rows_sum(float v) {   // over the wave's four 16-lane rows, lane by lane
     const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
     const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
-template <int CTRL>
-__device__ __forceinline__ float mma_dpp(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true)); }
 // what another block of this launch wrote, or is to read, moves past every cache that the two do not share (sc1)
 constexpr int kShared = 16;
 
@@ -363,7 +355,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const std::conditi
 #pragma unroll
         for (int i = 1; i < 8; ++i) mx = fmaxf(mx, x[i]);
         if (__builtin_amdgcn_ballot_w64(mx > m_run + kLagLog2) != 0) {   // rare after the first steps
-            mx = mma_rows_max(mx);
+            mx = rows_max(mx);
             const bool grow = mx > m_run + kLagLog2;
             const float alpha = grow ? __builtin_amdgcn_exp2f(m_run - mx) : 1.0f;
             m_run = grow ? mx : m_run;
@@ -501,8 +493,8 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const std::conditi
         for (int r = 0; r < 4; ++r) {
             const float hi = acc[0][i][r];
             float rest;
-            if constexpr (QT == 4) rest = mma_dpp<0x104>(hi) + mma_dpp<0x108>(hi);            // the columns 4 and 8 on
-            else if constexpr (QT == 8) rest = mma_dpp<0x108>(hi) + acc[1][i][r];
+            if constexpr (QT == 4) rest = dpp_move<0x104>(hi) + dpp_move<0x108>(hi);            // the columns 4 and 8 on
+            else if constexpr (QT == 8) rest = dpp_move<0x108>(hi) + acc[1][i][r];
             else rest = acc[1][i][r] + acc[2][i][r];
             o[r] = __builtin_fabsf(hi) < INFINITY ? hi + rest : hi;   // (an infinite value: its products with zero parts are no numbers)
         }
