@@ -58,7 +58,8 @@ fk_status sdpa_workspace_bytes(uint32_t n_heads, uint32_t n_kv, uint32_t qk_dim,
 namespace {
 
 // The kernels by tile, cache and row form.  A bf16 cache has tiles of 1 and 2 heads (rows of up to 512 dims fit a wave, so that keys and
-// values always share their lanes); those of 4 and 8 belong to quantised caches.
+// values always share their lanes); those of 4 and 8 belong to quantised caches.  Two heads come over a bf16 cache beyond 4096 positions:
+// of 64 and 128 dims those are rows that are not 16-byte aligned and calls without a workspace.
 template <int GT, int Q>
 const void* decode_func(int row) {
     if (row == 16) return reinterpret_cast<const void*>(&sdpa_decode_kernel<GT, Q, 16>);
@@ -144,6 +145,9 @@ fk_status plan_sdpa_decode(const uint16_t* q, const uint16_t* k, const uint16_t*
     const uint32_t lpk0 = pow2_ceil(qk_dim / 8), lpv0 = pow2_ceil(v_dim / 8), lp_wide = lpk0 > lpv0 ? lpk0 : lpv0;
     const bool same_lanes = lpk0 == lpv0 || (!kvq && lp_wide <= (uint32_t)kWave);
     int gt = !same_lanes ? 8 : (G >= 8 ? 8 : (G >= 4 ? (G == 4 ? 4 : 8) : (G >= 2 ? (G == 2 ? 2 : 4) : 1)));
+    // What of a bf16 cache comes here: 64 and 128 dims up to the matrix-core form's lines (192 positions; one row of 128 dims 704 .. 1792), unaligned
+    // or without a workspace beyond them; other widths and one row of 192 / 128 at any length.  Figures of 64 and 128 dims beyond those lines
+    // are what the lines of this form were drawn from, for the widths that keep it.
     // Groups of 2 .. 4 query heads per KV head: smaller tiles mean more blocks with fewer registers each, and the
     // repeated K / V reads of a KV head's tiles hit the L2.  Measured (32 q / 8 kv heads x 128, cold caches), tiles
     // of 1 / 2 / 4 heads: 512 positions 7.2 / 7.9 / 8.3 us, 4096 12.6 / 13.5 / 14.2, 8192 17.3 / 18.4 / 17.5, 32768 47.8 / 37.8 / 37.6.
