@@ -88,6 +88,8 @@ __device__ __forceinline__ float mma_rows_sum(float v) {   // over the wave's fo
     const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
+template <int CTRL>   // (lanes without a source get zero, and no register to clear first as dpp_move has: 0.1 us of a block of 128 dims)
+__device__ __forceinline__ float mma_dpp(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true)); }
 // what another block of this launch wrote, or is to read, moves past every cache that the two do not share (sc1)
 constexpr int kShared = 16;
 
@@ -493,8 +495,8 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const std::conditi
         for (int r = 0; r < 4; ++r) {
             const float hi = acc[0][i][r];
             float rest;
-            if constexpr (QT == 4) rest = dpp_move<0x104>(hi) + dpp_move<0x108>(hi);            // the columns 4 and 8 on
-            else if constexpr (QT == 8) rest = dpp_move<0x108>(hi) + acc[1][i][r];
+            if constexpr (QT == 4) rest = mma_dpp<0x104>(hi) + mma_dpp<0x108>(hi);            // the columns 4 and 8 on
+            else if constexpr (QT == 8) rest = mma_dpp<0x108>(hi) + acc[1][i][r];
             else rest = acc[1][i][r] + acc[2][i][r];
             o[r] = __builtin_fabsf(hi) < INFINITY ? hi + rest : hi;   // (an infinite value: its products with zero parts are no numbers)
         }
