@@ -2079,6 +2079,51 @@ fk_status build_token_kernel(std::vector<Node>& nodes, uint32_t spin_limit, Grap
     return FK_OK;
 }
 
+// The executable graph of g's nodes as they are planned: one kernel node per launch, one per fused run.
+fk_status instantiate(Graph* g) {
+    const size_t n = g->nodes.size();
+    FK_HIP(hipGraphCreate(&g->graph, 0));
+    for (size_t i = 0; i < n; ++i) {
+        Node& nd = g->nodes[i];
+        const int fr = g->fused_of[i];
+        if (fr >= 0) {
+            Graph::FusedRun& run = g->fused[fr];
+            if (i != run.first) {
+                nd.node = run.node;  // later dispatches that depend on any member wait for the run's launch
+                continue;
+            }
+            std::vector<hipGraphNode_t> deps;
+            for (size_t m = run.first; m < run.first + run.count; ++m)
+                for (uint32_t j : g->nodes[m].deps)
+                    if (j < run.first) {
+                        hipGraphNode_t dn = g->nodes[j].last();
+                        if (std::find(deps.begin(), deps.end(), dn) == deps.end()) deps.push_back(dn);
+                    }
+            void* slot[kMaxKernelParams];
+            hipKernelNodeParams p = launch_params(run.launch, slot);
+            FK_HIP(hipGraphAddKernelNode(&run.node, g->graph, deps.data(), deps.size(), &p));
+            nd.node = run.node;
+            continue;
+        }
+        std::vector<hipGraphNode_t> deps;
+        for (uint32_t j : nd.deps) {
+            hipGraphNode_t dn = g->nodes[j].last();
+            if (std::find(deps.begin(), deps.end(), dn) == deps.end()) deps.push_back(dn);
+        }
+        void* slot[kMaxKernelParams];
+        hipKernelNodeParams p = node_params(nd, slot);
+        FK_HIP(hipGraphAddKernelNode(&nd.node, g->graph, deps.data(), deps.size(), &p));
+        nd.tail.resize(nd.launch.then.size());
+        for (size_t f = 0; f < nd.launch.then.size(); ++f) {
+            hipGraphNode_t prev = f ? nd.tail[f - 1] : nd.node;
+            hipKernelNodeParams fp = launch_params(nd.launch.then[f], slot);
+            FK_HIP(hipGraphAddKernelNode(&nd.tail[f], g->graph, &prev, 1, &fp));
+        }
+    }
+    FK_HIP(hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0));
+    return FK_OK;
+}
+
 // Called with the stream idle.  A failed XCD-resident launch leaves partial sums behind: the control block is reset
 // by the check, the graph's sum rows are zeroed here (every token starts from zero rows), and the error text tells the
 // caller to decode the token again, which rewrites the cache rows of its position.
@@ -2338,45 +2383,7 @@ fk_status fk_build_graph(fk_handle h, const fk_dispatch* list, size_t n, const u
         }
     }
     FK_TRY(find_fused_runs(g.get()));
-    FK_HIP(hipGraphCreate(&g->graph, 0));
-    for (size_t i = 0; i < n; ++i) {
-        Node& nd = g->nodes[i];
-        const int fr = g->fused_of[i];
-        if (fr >= 0) {
-            Graph::FusedRun& run = g->fused[fr];
-            if (i != run.first) {
-                nd.node = run.node;  // later dispatches that depend on any member wait for the run's launch
-                continue;
-            }
-            std::vector<hipGraphNode_t> deps;
-            for (size_t m = run.first; m < run.first + run.count; ++m)
-                for (uint32_t j : g->nodes[m].deps)
-                    if (j < run.first) {
-                        hipGraphNode_t dn = g->nodes[j].last();
-                        if (std::find(deps.begin(), deps.end(), dn) == deps.end()) deps.push_back(dn);
-                    }
-            void* slot[kMaxKernelParams];
-            hipKernelNodeParams p = launch_params(run.launch, slot);
-            FK_HIP(hipGraphAddKernelNode(&run.node, g->graph, deps.data(), deps.size(), &p));
-            nd.node = run.node;
-            continue;
-        }
-        std::vector<hipGraphNode_t> deps;
-        for (uint32_t j : nd.deps) {
-            hipGraphNode_t dn = g->nodes[j].last();
-            if (std::find(deps.begin(), deps.end(), dn) == deps.end()) deps.push_back(dn);
-        }
-        void* slot[kMaxKernelParams];
-        hipKernelNodeParams p = node_params(nd, slot);
-        FK_HIP(hipGraphAddKernelNode(&nd.node, g->graph, deps.data(), deps.size(), &p));
-        nd.tail.resize(nd.launch.then.size());
-        for (size_t f = 0; f < nd.launch.then.size(); ++f) {
-            hipGraphNode_t prev = f ? nd.tail[f - 1] : nd.node;
-            hipKernelNodeParams fp = launch_params(nd.launch.then[f], slot);
-            FK_HIP(hipGraphAddKernelNode(&nd.tail[f], g->graph, &prev, 1, &fp));
-        }
-    }
-    FK_HIP(hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0));
+    FK_TRY(instantiate(g.get()));
     ds->graphs.push_back(std::move(g));
     *graph_id = (uint32_t)ds->graphs.size() - 1;
     return FK_OK;
@@ -2544,6 +2551,15 @@ fk_status fk_update_graph_bindings(fk_handle h, uint32_t graph_id, const fk_bind
     }
     // all checks passed: apply.  A HIP failure below can still leave the executable graph partly updated;
     // the error is reported and the caller must rebuild.
+    // Another kernel for a task (a rule that looks at alignment): the runtime holds the new launch against the bounds of the one that the node
+    // has and refuses a larger workgroup, so the executable graph is made anew.
+    bool other_kernel = false;
+    for (size_t k = 0; k < touched.size(); ++k) {
+        if (!g->fused_of.empty() && g->fused_of[touched[k]] >= 0) continue;
+        const Launch& was = g->nodes[touched[k]].launch;
+        other_kernel |= was.func != launches[k].func;
+        for (size_t f = 0; f < was.then.size(); ++f) other_kernel |= was.then[f].func != launches[k].then[f].func;
+    }
     std::vector<int> replan;
     for (size_t k = 0; k < touched.size(); ++k) {
         Node& nd = g->nodes[touched[k]];
@@ -2565,6 +2581,7 @@ fk_status fk_update_graph_bindings(fk_handle h, uint32_t graph_id, const fk_bind
             FK_HIP(hipMemcpy(dst, lt.args, lt.args_size, hipMemcpyHostToDevice));
             continue;
         }
+        if (other_kernel) continue;
         void* slot[kMaxKernelParams];
         hipKernelNodeParams p = node_params(nd, slot);
         FK_HIP(hipGraphExecKernelNodeSetParams(g->exec, nd.node, &p));
@@ -2578,9 +2595,19 @@ fk_status fk_update_graph_bindings(fk_handle h, uint32_t graph_id, const fk_bind
     for (int fr : replan) {
         Graph::FusedRun& run = g->fused[fr];
         FK_TRY(plan_xcd_layer(g->nodes[run.first].launch, g->nodes[run.first + 1].launch, &run.launch));
+        if (other_kernel) continue;
         void* slot[kMaxKernelParams];
         hipKernelNodeParams p = launch_params(run.launch, slot);
         FK_HIP(hipGraphExecKernelNodeSetParams(g->exec, run.node, &p));
+    }
+    if (other_kernel) {
+        FK_HIP(hipStreamSynchronize(ds->stream));   // nothing of the old one may be under way
+        const hipGraph_t graph = g->graph;
+        const hipGraphExec_t exec = g->exec;
+        const fk_status made = instantiate(g);
+        if (g->graph != graph) (void)hipGraphDestroy(graph);
+        if (g->exec != exec) (void)hipGraphExecDestroy(exec);
+        FK_TRY(made);
     }
     return FK_OK;
 }

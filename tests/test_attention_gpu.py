@@ -490,3 +490,31 @@ def test_sdpa_form_and_number_of_ranges(fk, n_heads, n_kv, qk, vd, rows, kv_len,
     grid = _matrix_core_grid(fk, n_heads, n_kv, qk, vd, rows, kv_len + rows - 1)
     assert (grid is not None) == (splits > 0) and (grid is None or grid[0] == splits), grid
     test_sdpa_on_the_matrix_cores_at_the_edges_of_its_tiles(fk, n_heads, n_kv, qk, vd, rows, kv_len)
+
+
+def test_graph_binding_moves_a_launch_to_the_other_form_and_back(fk):
+    """A query row bound two bytes off its alignment takes the form on vector instructions, an aligned one the matrix cores: the graph
+    replays what the binding plans, eager work between the replays."""
+    from fusekit_amd.runtime import Dispatch, Dispatcher, arg
+    n_heads, n_kv, dim, cap = 14, 2, 64, 700
+    q, ck, cv = normal_bf16(51, n_heads * dim), normal_bf16(52, n_kv * cap * dim), normal_bf16(53, n_kv * cap * dim)
+    pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, dim, dim, cap)
+    aligned, odd = _At(fk, q, 0), _At(fk, q, 2)
+    bufs = [fk.DeviceBuffer.from_numpy(a) for a in (ck, cv, np.array([cap], np.uint32))]
+    out, part, cnt = fk.DeviceBuffer(q.nbytes), fk.DeviceBuffer(pb), fk.zeros(cb)
+    d = Dispatcher()
+    task = lambda at: Dispatch("fusekit_sdpa_decode_f0", [(at.ptr, q.nbytes)] + [arg(b) for b in bufs + [out, part, cnt]],
+                               {"n_heads": n_heads, "n_kv": n_kv, "head_dim": dim, "capacity": cap})
+    want = []
+    for at in (aligned, odd):
+        d.dispatch_kernel(task(at))
+        want.append(out.to_numpy(np.uint16))
+    assert d.plan_geometry(task(aligned)).lds_bytes[0] > 60000 > d.plan_geometry(task(odd)).lds_bytes[0]
+    g = d.build_graph([task(aligned)])
+    for at, ref in ((aligned, want[0]), (odd, want[1]), (aligned, want[0])):
+        d.update_graph_bindings(g, [(0, 0, at.ptr, q.nbytes)])
+        for _ in range(2):
+            out.upload(np.zeros_like(q))
+            d.execute_graph(g)
+            assert np.array_equal(out.to_numpy(np.uint16), ref)
+    assert rel_l2(want[0], oracle.bf16_to_f32(oracle.sdpa_decode(q, ck, cv, n_heads, n_kv, dim, dim, cap, cap, dim ** -0.5))) <= 3e-3
