@@ -488,9 +488,12 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const std::conditi
         wm[wave * QT + n] = m_run;
         wl[wave * QT + n] = l_all;
     }
+    // An infinite value's products with zero parts are no numbers: where a sum of the first parts is infinite it stands alone.  Looked for once, over
+    // the tile, and the sums formed by all lanes ahead of one test of the column; value by value / this, us: 32 / 8 heads x 128, 1024 positions
+    // 8.07 / 7.93, 50 of 1024 5.51 / 5.29, 256 6.01 / 5.97; 14 / 2 x 64, 544 5.11 / 5.02, 12000 8.04 / 7.94.
+    float o[DT][4], far = 0.f;
 #pragma unroll
-    for (int i = 0; i < DT; ++i) {
-        float o[4];
+    for (int i = 0; i < DT; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const float hi = acc[0][i][r];
@@ -498,9 +501,19 @@ __global__ __launch_bounds__(NW * 64, 1) void sdpa_mma_kernel(const std::conditi
             if constexpr (QT == 4) rest = mma_dpp<0x104>(hi) + mma_dpp<0x108>(hi);            // the columns 4 and 8 on
             else if constexpr (QT == 8) rest = mma_dpp<0x108>(hi) + acc[1][i][r];
             else rest = acc[1][i][r] + acc[2][i][r];
-            o[r] = __builtin_fabsf(hi) < INFINITY ? hi + rest : hi;   // (an infinite value: its products with zero parts are no numbers)
+            o[i][r] = hi + rest;
+            far = fmaxf(far, __builtin_fabsf(hi));
         }
-        if (n < (uint32_t)QT) *reinterpret_cast<float4*>(red + (wave * QT + n) * OS + (uint32_t)i * 16u + 4u * g) = make_float4(o[0], o[1], o[2], o[3]);
+    if (__builtin_amdgcn_ballot_w64(far == INFINITY) != 0) {
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[i][r] = __builtin_fabsf(acc[0][i][r]) < INFINITY ? o[i][r] : acc[0][i][r];
+    }
+    if (n < (uint32_t)QT) {
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+            *reinterpret_cast<float4*>(red + (wave * QT + n) * OS + (uint32_t)i * 16u + 4u * g) = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
     }
     __syncthreads();
     const bool direct = n_active == 1u;
