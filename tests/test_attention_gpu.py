@@ -481,7 +481,7 @@ def _matrix_core_grid(fk, n_heads, n_kv, qk, vd, rows, max_len):
 @pytest.mark.parametrize("n_heads,n_kv,qk,vd,rows,kv_len,splits", [
     (3, 1, 128, 128, 1, 1024, 0), (3, 1, 128, 128, 1, 1025, 9), (2, 2, 128, 128, 1, 1280, 0), (2, 2, 128, 128, 1, 1281, 11), (7, 1, 128, 128, 1, 1792, 0), (7, 1, 128, 128, 1, 1793, 8),   # at and past the lines
     (7, 1, 128, 128, 1, 2048, 8), (7, 1, 128, 128, 1, 2049, 9), (3, 1, 128, 128, 1, 3072, 12), (3, 1, 128, 128, 1, 3073, 13),  # round edges
-    (16, 16, 192, 128, 2, 63, 0), (16, 16, 192, 128, 2, 64, 1),
+    (16, 16, 192, 128, 2, 63, 0), (16, 16, 192, 128, 2, 64, 1), (64, 8, 64, 64, 41, 300, 1), (64, 8, 64, 64, 33, 1100, 1),     # (tiles of 16 of 64 dims)
     (5, 1, 128, 128, 1, 4096, 16), (3, 1, 128, 128, 1, 8193, 17), (5, 1, 128, 128, 1, 16384, 32), (5, 1, 128, 128, 1, 16385, 33),
     (5, 1, 128, 128, 1, 32768, 64), (2, 1, 64, 64, 1, 4096, 16), (2, 1, 64, 64, 1, 8193, 17), (2, 1, 64, 64, 1, 32768, 64),    # edges of the merge
 ])
