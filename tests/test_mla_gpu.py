@@ -143,6 +143,26 @@ def test_split_store_and_attention_in_one_launch_of_square_heads(fk, n_heads, k0
     test_split_store_and_attention_in_one_launch(fk, n_heads, k0d, k1d, vd, rope, kv_len, cap, traditional, table)
 
 
+@pytest.mark.parametrize("n_heads,n_kv,k0d,k1d,cap,kv_len", [(14, 2, 48, 16, 600, 421), (32, 8, 64, 64, 1024, 1024), (9, 1, 40, 24, 700, 700)])
+def test_split_store_in_one_launch_of_grouped_heads(fk, n_heads, n_kv, k0d, k1d, cap, kv_len):
+    """Groups of heads, a second key part of each key head's own, value rows apart from the keys'."""
+    qk, vd, theta, pos, rope = k0d + k1d, k0d + k1d, 1e4, kv_len - 1, k1d
+    q, ck, cv = normal_bf16(60, (n_heads, qk)), normal_bf16(61, n_kv * cap * qk), normal_bf16(62, n_kv * cap * vd)
+    k0, k1, v = normal_bf16(63, (n_kv, k0d)), normal_bf16(64, (n_kv, k1d)), normal_bf16(65, (n_kv, vd + 8))
+    pb, cb = fk.sdpa_workspace_bytes(n_heads, n_kv, qk, vd, cap)
+    part, cnt = fk.DeviceBuffer(pb), fk.zeros(cb)
+    d_q, d_ck, d_cv, d_k0, d_k1, d_v = (_dev(fk, a) for a in (q, ck, cv, k0, k1, v))
+    fk.kv_cache_store_split_decode(d_q, n_heads, k0d, k1d, d_k0, k0d, d_k1, n_kv, d_v, vd + 8, n_kv, k0d, k1d, vd, rope, False, theta, None, pos,
+                                   None, pos, cap, d_ck, d_cv)
+    ref, out = fk.DeviceBuffer(2 * n_heads * vd), fk.DeviceBuffer(2 * n_heads * vd)
+    fk.sdpa_decode(d_q, d_ck, d_cv, ref, None, kv_len, cap, n_heads, n_kv, qk, vd, cap, qk ** -0.5, part, cnt)
+    f_q, f_ck, f_cv = (_dev(fk, a) for a in (q, ck, cv))
+    fk.split_store_sdpa_decode(f_q, n_heads, k0d, k1d, d_k0, k0d, d_k1, n_kv, d_v, vd + 8, n_kv, vd, rope, False, theta, None, f_ck, f_cv, out,
+                               None, kv_len, cap, cap, qk ** -0.5, part, cnt)
+    for got, want in ((out, ref), (f_ck, d_ck), (f_cv, d_cv)):
+        assert np.array_equal(got.to_numpy(np.uint16), want.to_numpy(np.uint16))
+
+
 @pytest.mark.parametrize("rows,row_n,top_k,per_route", [(1, 64, 6, False), (8, 64, 6, True), (3, 256, 32, False),
                                                         (5, 2, 1, False), (2, 128, 8, True)])
 def test_softmax_topk_route(fk, rows, row_n, top_k, per_route):
